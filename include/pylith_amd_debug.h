@@ -25,6 +25,11 @@ extern "C" {
 int plx_debug_plan_info(plx_dm dm, int label_value, int part, int *num_tiles, int64_t *halo_slots,
                         int *reordered);
 
+/* Z = M R: one multigrid V-cycle on k columns (k in {1, 8, 16, 32, 64}) of a Green's-function handle
+ * with the multigrid preconditioner; R, Z: DEVICE [dof][k] in DM order.  R must be complete when the
+ * call is made (the handle's own stream reads it); synchronises. */
+int plx_debug_gf_precondition(plx_gf g, int k, const float *R, float *Z);
+
 int plx_debug_emulate_apply(int cell_type, int num_cells, int num_vertices, int num_nodes,
                             const int32_t *closure, const int32_t *cone, const double *coords,
                             const int32_t *labels, int label_value, const double *lam_mu,

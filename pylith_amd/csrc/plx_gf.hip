@@ -22,6 +22,7 @@
 #include <thread>
 #include <vector>
 
+#include "../../include/pylith_amd_debug.h"
 #include "plx_amg.hpp"
 #include "plx_element.hpp"
 #include "plx_internal.hpp"
@@ -556,6 +557,88 @@ __global__ void __launch_bounds__(256) amg_bsr1(int nrows, const int32_t *__rest
     }
 }
 
+// The block-row products of amg_bsr where there are too few rows to fill the chip with a wave
+// each (coarse levels, restrictions onto them, small meshes) or rows are long (a restriction row
+// gathers an aggregate's whole neighbourhood): one workgroup per block row, its NT threads as NT / K
+// entry slots x K columns, each slot every (NT / K)-th entry, the slots' partial rows summed in LDS
+// in slot order.  Latency-bound: a row's entries form NT / K short chains in place of one long one.
+// Measured at 16 columns on a 16^3 mesh: restriction to the first coarse level 68 -> 6.8 us, its
+// operator products 14.7 -> 3.7 us, the fine level's 9.8 -> 7.7 us; at 64 columns on 44^3 (125 rows
+// at the second coarse level): transfers to and from it 88 -> 13 us on average.
+template <int BR, int BC, int K, int MODE, int NT>
+__global__ void __launch_bounds__(NT) amg_bsr_split(int nrows, const int32_t *__restrict__ ptr,
+                                                     const int32_t *__restrict__ col, const float *__restrict__ val,
+                                                     const float *__restrict__ X, const float *__restrict__ Bv,
+                                                     const float *__restrict__ Dinv, float *Y, float s,
+                                                     int accumulate) {
+    constexpr int S = NT / K;
+    constexpr int U = 3;  // entries whose operands are loaded together
+    __shared__ float sy[S][BR][K];
+    __shared__ float sr[BR][K];
+    const int row = blockIdx.x;
+    if (row >= nrows) return;
+    const int c = (int)(threadIdx.x % K);
+    int slot = (int)(threadIdx.x / K);
+    if (K == 64) slot = __builtin_amdgcn_readfirstlane(slot);
+    const int e1 = ptr[row + 1];
+    float y[BR];
+#pragma unroll
+    for (int a = 0; a < BR; ++a) y[a] = 0.f;
+    int e = ptr[row] + slot;
+    for (; e + (U - 1) * S < e1; e += U * S) {
+        float x[U][BC];
+#pragma unroll
+        for (int m = 0; m < U; ++m) {
+            const size_t j = (size_t)col[e + m * S];
+#pragma unroll
+            for (int q = 0; q < BC; ++q) x[m][q] = X[(BC * j + q) * K + c];
+        }
+#pragma unroll
+        for (int m = 0; m < U; ++m) {
+            const float *A = val + (size_t)BR * BC * (e + m * S);
+#pragma unroll
+            for (int a = 0; a < BR; ++a)
+#pragma unroll
+                for (int q = 0; q < BC; ++q) y[a] += A[a * BC + q] * x[m][q];
+        }
+    }
+    for (; e < e1; e += S) {
+        const size_t j = (size_t)col[e];
+        const float *A = val + (size_t)BR * BC * e;
+        float x[BC];
+#pragma unroll
+        for (int q = 0; q < BC; ++q) x[q] = X[(BC * j + q) * K + c];
+#pragma unroll
+        for (int a = 0; a < BR; ++a)
+#pragma unroll
+            for (int q = 0; q < BC; ++q) y[a] += A[a * BC + q] * x[q];
+    }
+#pragma unroll
+    for (int a = 0; a < BR; ++a) sy[threadIdx.x / K][a][c] = y[a];
+    __syncthreads();
+    const size_t o = (size_t)BR * row * K;
+    for (int t = threadIdx.x; t < BR * K; t += NT) {
+        const int a = t / K, r = t % K;
+        float v = 0.f;
+#pragma unroll
+        for (int q = 0; q < S; ++q) v += sy[q][a][r];
+        if (MODE == kBsrPlain) Y[o + t] = accumulate ? Y[o + t] + v : v;
+        else if (MODE == kBsrResid) Y[o + t] = Bv[o + t] - v;
+        else sr[a][r] = Bv[o + t] - v;
+    }
+    if (MODE == kBsrPost) {
+        __syncthreads();
+        const float *Di = Dinv + (size_t)BR * BR * row;
+        for (int t = threadIdx.x; t < BR * K; t += NT) {
+            const int a = t / K, r = t % K;
+            float z = 0.f;
+#pragma unroll
+            for (int q = 0; q < BR; ++q) z += Di[a * BR + q] * sr[q][r];
+            Y[o + t] = X[o + t] + s * z;
+        }
+    }
+}
+
 // r = b - t (the fine residual over a matrix-free product t = A x)
 __global__ void __launch_bounds__(256) amg_sub(int64_t n, const float *__restrict__ b, const float *__restrict__ t,
                                                float *r) {
@@ -578,11 +661,11 @@ __global__ void __launch_bounds__(256) amg_post0(int n, const float *__restrict_
 }
 
 // coarsest level, one column: a wave per row of the dense inverse
-__global__ void __launch_bounds__(256) amg_dense1(int m, const float *__restrict__ Ainv, const float *__restrict__ Bv,
-                                                  float *X) {
+__global__ void __launch_bounds__(256) amg_dense1(int m, int ld, const float *__restrict__ Ainv,
+                                                  const float *__restrict__ Bv, float *X) {
     const int lane = threadIdx.x & 63;
     for (int i = blockIdx.x * 4 + (int)(threadIdx.x >> 6); i < m; i += gridDim.x * 4) {
-        const float *a = Ainv + (size_t)m * i;
+        const float *a = Ainv + (size_t)ld * i;
         float acc = 0.f;
         for (int jj = lane; jj < m; jj += 64) acc += a[jj] * Bv[jj];
 #pragma unroll
@@ -613,18 +696,54 @@ __global__ void __launch_bounds__(256) amg_jacobi0(int n, const float *__restric
     }
 }
 
-// coarsest level: x = Ainv b (dense, m x m)
+// coarsest level, K columns: X = Ainv B on the matrix cores, FP32 products and sums.  Ainv is
+// [ld][ld], ld a multiple of 16, zero beyond the operator's m rows and columns (the rows of B read
+// for the padding are clamped to its last).  One workgroup per 16 rows, its 8 waves taking every 8th chunk of 16 of
+// the inner dimension, summed in LDS in wave order.  The product is a contraction of ~750 x 750 by
+// K: a thread per output read B through L2 once per row and was bound by that (177 us at 64
+// columns, m = 752, 10 us here).
+// v_mfma_f32_16x16x4: lane l holds A[l % 16][l / 16] and B[l / 16][l % 16]; the order of the inner
+// index is free, so lane group g = l / 16 takes the four consecutive inner indices 4 g .. 4 g + 3 of
+// a chunk (one 16-byte load of A), and tile n of the columns is every (K / 16)-th column from n
+// (one wide load of B).
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 template <int K>
-__global__ void __launch_bounds__(256) amg_dense(int m, const float *__restrict__ Ainv, const float *__restrict__ Bv,
-                                                 float *X) {
-    const int64_t nt = (int64_t)m * K;
-    const int r = (int)(threadIdx.x % K);
-    for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < nt; t += (int64_t)gridDim.x * 256) {
-        const int64_t i = t / K;
-        const float *a = Ainv + (size_t)m * i;
-        float acc = 0.f;
-        for (int j = 0; j < m; ++j) acc += a[j] * Bv[(size_t)j * K + r];
-        X[i * K + r] = acc;
+__global__ void __launch_bounds__(512) amg_dense(int m, int ld, const float *__restrict__ Ainv,
+                                                 const float *__restrict__ Bv, float *X) {
+    constexpr int NT = K >= 16 ? K / 16 : 1;
+    __shared__ float red[8][16][16 * NT];
+    const int lane = threadIdx.x & 63, w = (int)(threadIdx.x >> 6);
+    const int c = lane & 15, g = lane >> 4;
+    const int row0 = blockIdx.x * 16;
+    f32x4 acc[NT];
+#pragma unroll
+    for (int n = 0; n < NT; ++n) acc[n] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const float *arow = Ainv + (size_t)(row0 + c) * ld + 4 * g;
+    for (int k0 = 16 * w; k0 < ld; k0 += 128) {
+        const f32x4 a = *reinterpret_cast<const f32x4 *>(arow + k0);
+        float b[4][NT];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float *brow = Bv + (size_t)min(k0 + 4 * g + i, m - 1) * K;
+#pragma unroll
+            for (int n = 0; n < NT; ++n) b[i][n] = K >= 16 ? brow[NT * c + n] : (c < K ? brow[c] : 0.f);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int n = 0; n < NT; ++n) acc[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[i][n], acc[n], 0, 0, 0);
+    }
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) red[w][4 * g + r][NT * c + n] = acc[n][r];
+    __syncthreads();
+    for (int t = threadIdx.x; t < 16 * K; t += 512) {
+        const int r = t / K, q = t % K;
+        float v = 0.f;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v += red[j][r][q];
+        if (row0 + r < m) X[(size_t)(row0 + r) * K + q] = v;
     }
 }
 
@@ -807,7 +926,7 @@ struct plx_gf_s {
         float *r = nullptr, *d = nullptr, *bv = nullptr, *xv = nullptr;  // workspace, 64 columns
     };
     std::vector<Level> lv;
-    int coarse_m = 0;
+    int coarse_m = 0, coarse_ld = 0;  // unknowns of the coarsest level; its rows padded to a multiple of 16
     float *coarse_inv = nullptr, *cb = nullptr, *cx = nullptr;
     float *vr1 = nullptr, *vz1 = nullptr;  // single-column V-cycle operands in row order
     // the finest level's transfer operators and inverse diagonal blocks with DM-ordered fine
@@ -949,6 +1068,13 @@ static dim3 amg_grid(int nrows, int rows_per_wave) {
     return dim3((unsigned)blocks);
 }
 
+// Block products with fewer waves of rows than kSplitWaves (four per SIMD of the chip) take a
+// workgroup per row (amg_bsr_split): fewer waves do not hide a row's chain of gathers.  At 3375 rows x 64
+// columns the 6 x 6 products took 26.7 / 19.3 us a wave per row and 22.2 / 17.9 us split; at 91,000 rows
+// a wave per row already fills the chip.  Up to kSplitRows rows (two per CU) the workgroup has 16 waves.
+constexpr int64_t kSplitWaves = 16384;
+constexpr int kSplitRows = 512;
+
 // G: lanes per block row of the single-column kernel (operator rows ~25-50 blocks, restriction
 // rows up to a few hundred, prolongation rows ~4-8)
 template <int BR, int BC, int K, int MODE, int G = 16>
@@ -957,7 +1083,14 @@ static void amg_bsr_launch(plx_gf g, int nrows, const int32_t *ptr, const int32_
     if (K == 1)
         hipLaunchKernelGGL((amg_bsr1<BR, BC, G, MODE>), amg_grid(nrows, 64 / G), dim3(256), 0, g->stream, nrows, ptr,
                            col, val, X, Bv, Dinv, Y, s, accumulate);
-    else
+    else if ((int64_t)nrows * K < 64 * kSplitWaves) {
+        if (nrows <= kSplitRows)
+            hipLaunchKernelGGL((amg_bsr_split<BR, BC, K == 1 ? 64 : K, MODE, 1024>), dim3(nrows), dim3(1024), 0,
+                               g->stream, nrows, ptr, col, val, X, Bv, Dinv, Y, s, accumulate);
+        else
+            hipLaunchKernelGGL((amg_bsr_split<BR, BC, K == 1 ? 64 : K, MODE, 256>), dim3(nrows), dim3(256), 0,
+                               g->stream, nrows, ptr, col, val, X, Bv, Dinv, Y, s, accumulate);
+    } else
         hipLaunchKernelGGL((amg_bsr<BR, BC, K, MODE>), amg_grid(nrows, 64 / K), dim3(256), 0, g->stream, nrows, ptr,
                            col, val, X, Bv, Dinv, Y, s, accumulate);
 }
@@ -970,10 +1103,10 @@ static void amg_vcycle(plx_gf g, int l, const float *bv, float *xv) {
     if (l == (int)g->lv.size()) {
         if (K == 1)
             hipLaunchKernelGGL(amg_dense1, dim3((g->coarse_m + 3) / 4), dim3(256), 0, g->stream, g->coarse_m,
-                               g->coarse_inv, bv, xv);
+                               g->coarse_ld, g->coarse_inv, bv, xv);
         else
-            hipLaunchKernelGGL(amg_dense<K>, dim3(std::max(1, std::min(kGfRed, (g->coarse_m * K + 255) / 256))),
-                               dim3(256), 0, g->stream, g->coarse_m, g->coarse_inv, bv, xv);
+            hipLaunchKernelGGL(amg_dense<K>, dim3(g->coarse_ld / 16), dim3(512), 0, g->stream, g->coarse_m,
+                               g->coarse_ld, g->coarse_inv, bv, xv);
         return;
     }
     if (g->lv[l].b == 3) amg_level<3, K>(g, l, bv, xv);
@@ -1139,7 +1272,7 @@ static void gf_amg_free(plx_gf g) {
         if (p) (void)hipFree(p);
     g->coarse_inv = g->cb = g->cx = g->vr1 = g->vz1 = g->Pval_dm = g->Dinv_dm = nullptr;
     g->Rcol_dm = g->Pptr_dm = g->Pcol_dm = nullptr;
-    g->coarse_m = 0;
+    g->coarse_m = g->coarse_ld = 0;
 }
 
 // Build the multigrid hierarchy of the merged FP64 operator on the host and upload it in FP32
@@ -1276,8 +1409,12 @@ static int gf_amg_setup(plx_gf g) {
         if (l > 0 && ((err = ws(&L.bv, nd)) || (err = ws(&L.xv, nd)))) return err;
     }
     g->coarse_m = h.coarse_n;
-    if ((err = upf(&g->coarse_inv, h.coarse_inv)) || (err = ws(&g->cb, h.coarse_n)) || (err = ws(&g->cx, h.coarse_n)))
-        return err;
+    g->coarse_ld = (h.coarse_n + 15) / 16 * 16;
+    const size_t cm = (size_t)g->coarse_m, ld = (size_t)g->coarse_ld;
+    std::vector<float> inv(ld * ld, 0.f);
+    for (size_t i = 0; i < cm; ++i)
+        for (size_t j = 0; j < cm; ++j) inv[ld * i + j] = (float)h.coarse_inv[cm * i + j];
+    if ((err = upf(&g->coarse_inv, inv)) || (err = ws(&g->cb, cm)) || (err = ws(&g->cx, cm))) return err;
     PLX_HIP(dm, hipMalloc((void **)&g->vr1, (size_t)g->ndof * sizeof(float)));
     PLX_HIP(dm, hipMalloc((void **)&g->vz1, (size_t)g->ndof * sizeof(float)));
     {  // the finest level in DM order: Dinv and P rows moved to their nodes, R columns renamed
@@ -1858,6 +1995,36 @@ int plx_gf_apply(plx_gf g, int k, int scalar_type, const void *X, void *Y) {
     const hipError_t e1 = hipGetLastError(), e2 = hipStreamSynchronize(g->stream);
     (void)hipFree(Xr);
     (void)hipFree(Yr);
+    PLX_HIP(dm, e1);
+    PLX_HIP(dm, e2);
+    return 0;
+}
+
+int plx_debug_gf_precondition(plx_gf g, int k, const float *R, float *Z) {
+    if (!g || !R || !Z) return 1;
+    plx_dm dm = g->dm;
+    if (k != 1 && k != 8 && k != 16 && k != 32 && k != 64) return set_error(dm, 1, "k must be 1, 8, 16, 32 or 64");
+    if (g->lv.empty()) return set_error(dm, 1, "multigrid hierarchy not built");
+    float *Rr = nullptr, *Zr = nullptr;
+    PLX_HIP(dm, hipMalloc(&Rr, (size_t)g->ndof * k * sizeof(float)));
+    if (hipMalloc(&Zr, (size_t)g->ndof * k * sizeof(float)) != hipSuccess) {
+        (void)hipFree(Rr);
+        return set_error(dm, 1, "out of device memory");
+    }
+    hipLaunchKernelGGL(gf_permute_block<float>, gf_grid(g->ndof * k), dim3(256), 0, g->stream, g->ndof, k, g->d_perm,
+                       true, R, Rr);
+    switch (k) {
+    case 1: amg_vcycle<1>(g, 0, Rr, Zr); break;
+    case 8: amg_vcycle<8>(g, 0, Rr, Zr); break;
+    case 16: amg_vcycle<16>(g, 0, Rr, Zr); break;
+    case 32: amg_vcycle<32>(g, 0, Rr, Zr); break;
+    default: amg_vcycle<64>(g, 0, Rr, Zr); break;
+    }
+    hipLaunchKernelGGL(gf_permute_block<float>, gf_grid(g->ndof * k), dim3(256), 0, g->stream, g->ndof, k, g->d_perm,
+                       false, (const float *)Zr, Z);
+    const hipError_t e1 = hipGetLastError(), e2 = hipStreamSynchronize(g->stream);
+    (void)hipFree(Rr);
+    (void)hipFree(Zr);
     PLX_HIP(dm, e1);
     PLX_HIP(dm, e2);
     return 0;

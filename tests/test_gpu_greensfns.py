@@ -163,6 +163,36 @@ def test_multigrid_preconditioner_matches_jacobi(block):
         gf.set_preconditioner(7)
 
 
+# few rows (a workgroup per row), rows past the line where a wave takes a row; coarsest levels of one
+# and of several 16-row tiles with a remainder
+@pytest.mark.parametrize("n", [(4, 4, 4), (12, 9, 7), (30, 25, 22)])
+def test_vcycle_is_the_same_operator_at_every_block_width(n):
+    """The block V-cycle's kernels against the single-column ones, column by column.  All are FP32 sums
+    of at most some hundred products a row, in different orders: 1e-4 of the largest entry."""
+    import ctypes
+    from pylith_amd.greensfns import GreensFunctions
+    m, f, dm, dofs = faulted_problem(n)
+    gf = GreensFunctions(dm)
+    gf.set_preconditioner("amg")
+    nd = 3 * m.num_nodes
+    mu = 2500.0 * 3000.0 ** 2 * 1000.0  # stiffness scale: solutions of order one
+    R = mu * torch.randn(nd, 64, generator=torch.Generator().manual_seed(3)).cuda()
+
+    def cycle(k, cols):
+        r = R[:, cols].contiguous()
+        z = torch.empty_like(r)
+        torch.cuda.synchronize()
+        assert gf.lib.plx_debug_gf_precondition(gf.h, k, ctypes.c_void_p(r.data_ptr()), ctypes.c_void_p(z.data_ptr())) == 0
+        return z.double()
+
+    ref = torch.cat([cycle(1, [c]) for c in range(64)], 1)
+    for k in (8, 16, 32, 64):
+        got = torch.cat([cycle(k, list(range(c, c + k))) for c in range(0, 64, k)], 1)
+        err = ((got - ref).abs().amax(0) / ref.abs().amax(0)).max().item()
+        print(f"[gf-vcycle] n={n} k={k} err={err:.2e}", flush=True)
+        assert err <= 1e-4, (k, err)
+
+
 def test_autotune_picks_a_candidate():
     from pylith_amd.greensfns import GreensFunctions
     m, f, dm, dofs = faulted_problem((6, 4, 4))
