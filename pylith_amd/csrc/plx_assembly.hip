@@ -127,18 +127,13 @@ struct Shape<PLX_HEX_Q1, Real> {
     // RECW: uint4 words per cell record (8 x uint16 closure)
     static constexpr int NT = 256, CPT = 2, NB = 8, NV = 8, PFN = 3, PFV = 0, RECW = 1;
 };
-// P2 FP64: 4-wave workgroups over the 384-cell tile (cells 0-255 on the first pass, 256-383 on
-// the second), two workgroups per CU at the kernel's register count (2 waves per SIMD: every
-// wave slot of the CU busy; measured 6 % faster than 3-wave workgroups with two full passes).
-// FP32 takes the same shape (three workgroups per CU at its 142 VGPRs): two cells a thread give
-// the two-phase fetch its split point (3 % faster than 6-wave workgroups of one cell a thread).
+// P2: 4-wave workgroups over the 384-cell tile (cells 0-255 on the first pass, 256-383 on the
+// second), two workgroups per CU at the FP64 kernel's register count (2 waves per SIMD).  One cell
+// per thread in 6-wave workgroups measured slower (63 x 66 x 61 x 6 cells, FP64: 92 us, 96 us with
+// the registers cut to three waves per SIMD, against 80 us).
 // record: 10 x uint16 closure, 4 x uint16 cone, 2 padding = 2 uint4 words
-template <>
-struct Shape<PLX_TET_P2, double> {
-    static constexpr int NT = 256, CPT = 2, NB = 10, NV = 4, PFN = 3, PFV = 1, RECW = 2;
-};
-template <>
-struct Shape<PLX_TET_P2, float> {
+template <typename Real>
+struct Shape<PLX_TET_P2, Real> {
     static constexpr int NT = 256, CPT = 2, NB = 10, NV = 4, PFN = 3, PFV = 1, RECW = 2;
 };
 
@@ -243,7 +238,8 @@ __device__ __forceinline__ void fetch_values(Stage<Real, CT> &T, const ApplyArgs
     }
 }
 
-// One phase (the first tile of every kernel; the kernels that keep one phase throughout).
+// One phase (the first tile; the Q1 quadrature-point kernels throughout).  Kept apart from the two
+// phases: with those for the first tile too, the P2 kernels take 30 registers more.
 template <typename Real, int CT, int ACC>
 __device__ __forceinline__ void fetch(Stage<Real, CT> &T, const ApplyArgs &A, int tile, int tid) {
     using S = Shape<CT, Real>;
@@ -260,16 +256,15 @@ __device__ __forceinline__ void fetch(Stage<Real, CT> &T, const ApplyArgs &A, in
     T.hoff = P.tile_halo_off[tile];
     if constexpr (CT == PLX_HEX_Q1) {
         // every node id first, then the values: one wait between the two, not one per slot
-        int gn[S::PFN];
 #pragma unroll
         for (int j = 0; j < S::PFN; ++j) {
             const int k = tid + j * S::NT;
-            gn[j] = k < T.nn ? P.tile_nodes[T.n0 + k] : -1;
+            T.gn[j] = k < T.nn ? P.tile_nodes[T.n0 + k] : -1;
         }
 #pragma unroll
         for (int j = 0; j < S::PFN; ++j) {
-            if (gn[j] >= 0) {
-                const size_t g = (size_t)gn[j];
+            if (T.gn[j] >= 0) {
+                const size_t g = (size_t)T.gn[j];
 #pragma unroll
                 for (int c = 0; c < 3; ++c) T.pu[j][c] = u[3 * g + c];
 #pragma unroll
@@ -277,12 +272,13 @@ __device__ __forceinline__ void fetch(Stage<Real, CT> &T, const ApplyArgs &A, in
             }
         }
     } else {
-        // P2: id and values slot by slot (measured faster here than all ids first)
+        // P2: id and values slot by slot
 #pragma unroll
         for (int j = 0; j < S::PFN; ++j) {
             const int k = tid + j * S::NT;
             if (k < T.nn) {
-                const size_t g = (size_t)P.tile_nodes[T.n0 + k];
+                T.gn[j] = P.tile_nodes[T.n0 + k];
+                const size_t g = (size_t)T.gn[j];
 #pragma unroll
                 for (int c = 0; c < 3; ++c) T.pu[j][c] = u[3 * g + c];
             }
@@ -384,26 +380,11 @@ __global__ void __launch_bounds__((Shape<CT, Real>::NT), MINW) apply_tiles(Apply
         }
         __syncthreads();
 
-        // The next tile's loads go out in two phases (see Stage) in the factored Q1 kernels and
-        // the P2 kernels (measured -3 % each for the factored kernels with LDS atomics or colour
-        // phases, FP64 and FP32, -1.7 % for the P2 quadrature-point kernel); the Q1
-        // quadrature-point kernels overflow their registers with it and keep one phase.  The P2 kernel makes room by
-        // loading its write-out ids after the cells (below) instead of early.
-        constexpr bool P2SPLIT = CT != PLX_HEX_Q1 && (PATH == kPathFactored || PATH == kPathQpAffine);
-        constexpr bool SPLIT = (CT == PLX_HEX_Q1 && PATH == kPathFactored && S::CPT > 1) || P2SPLIT;
-        // node ids of this tile's owned write-out, loaded before the next tile's gathers so that
-        // waiting for them does not wait for those (not for the FP64 Q1 kernel: its registers
-        // are full, and the extra ids spill; not for the two-phase P2 kernel)
-        constexpr bool EARLY = (CT != PLX_HEX_Q1 || sizeof(Real) == 4) && !P2SPLIT;
-        constexpr int NW = EARLY ? S::PFN : 1;
-        int wn[NW];
-        if constexpr (EARLY) {
-#pragma unroll
-            for (int j = 0; j < NW; ++j) {
-                const int k = tid + j * NT;
-                wn[j] = k < cur.nown ? A.p.tile_nodes[cur.n0 + k] : 0;
-            }
-        }
+        // The next tile's loads go out in two phases (see Stage): its ids here, the values at them after
+        // the first of the thread's two cells; the Q1 quadrature-point kernels issue both here (their
+        // registers overflow otherwise)
+        constexpr bool SPLIT = CT != PLX_HEX_Q1 || PATH == kPathFactored;
+        constexpr bool DIRECT = CT != PLX_HEX_Q1 && PATH == kPathFactored && ACC == kAccAtomic;
         const int next_slot = slot + G;
         const bool has_next = next_slot < A.num_list;
         Stage<Real, CT> nxt;
@@ -416,6 +397,13 @@ __global__ void __launch_bounds__((Shape<CT, Real>::NT), MINW) apply_tiles(Apply
             else fetch<Real, CT, ACC>(nxt, A, tile_of(next_slot), tid);
         }
         __builtin_amdgcn_s_setprio(0);
+        const auto next_values = [&] {
+            if (has_next) {
+                __builtin_amdgcn_s_setprio(2);
+                fetch_values<Real, CT>(nxt, A);
+                __builtin_amdgcn_s_setprio(0);
+            }
+        };
 
 #pragma unroll
         for (int i = 0; i < S::CPT; ++i) {
@@ -453,8 +441,12 @@ __global__ void __launch_bounds__((Shape<CT, Real>::NT), MINW) apply_tiles(Apply
                         for (int d = 0; d < 3; ++d) X[v][d] = sX[3 * lv + d];
                     }
                     if constexpr (PATH == kPathFactored) {
-                        LdsAcc<Real, 10> acc{sU, {lc[0], lc[1], lc[2], lc[3], lc[4], lc[5], lc[6], lc[7], lc[8], lc[9]}};
-                        p2_element_linear<Real>(X, acc, lam, mu, c_p2.wdiag, c_p2.woff, re);
+                        const LdsAcc<Real, 10> acc{sU, {lc[0], lc[1], lc[2], lc[3], lc[4], lc[5], lc[6], lc[7], lc[8], lc[9]}};
+                        // LDS atomics take an entry as soon as it is formed
+                        p2_element_linear<Real>(X, acc, lam, mu, [&](int c, int b, Real v) {
+                            if constexpr (DIRECT) atomicAdd(&sR[3 * lc[b] + c], (Acc)v);
+                            else re[c][b] = v;
+                        });
                     } else {
                         Real U[3][10];
 #pragma unroll
@@ -467,7 +459,7 @@ __global__ void __launch_bounds__((Shape<CT, Real>::NT), MINW) apply_tiles(Apply
             }
             if constexpr (ACC == kAccAtomic) {
                 // LDS atomics: no colour phases; the order of the additions into a node varies
-                if (active) {
+                if (!DIRECT && active) {
 #pragma unroll
                     for (int b = 0; b < NB; ++b)
 #pragma unroll
@@ -487,50 +479,24 @@ __global__ void __launch_bounds__((Shape<CT, Real>::NT), MINW) apply_tiles(Apply
                     }
                 }
             }
-            if constexpr (SPLIT) {
-                if (i == 0 && has_next) {
-                    __builtin_amdgcn_s_setprio(2);
-                    fetch_values<Real, CT>(nxt, A);
-                    __builtin_amdgcn_s_setprio(0);
-                }
-            }
+            if constexpr (SPLIT)
+                if (i == 0) next_values();
         }
         __syncthreads();
         __builtin_amdgcn_s_setprio(1);
 
-        if constexpr (EARLY) {
+        // owned nodes: the ids are those this thread gathered by; the quadrature-point kernels, whose
+        // registers are full, read them again (all slots at once, clamped positions, no branch)
+        constexpr bool KEEP = PATH == kPathFactored;
+        int wl[S::PFN];
 #pragma unroll
-            for (int j = 0; j < NW; ++j) {
-                const int k = tid + j * NT;
-                if (k < cur.nown) {
-                    const size_t g = (size_t)wn[j];
+        for (int j = 0; j < S::PFN; ++j)
+            wl[j] = KEEP ? cur.gn[j] : A.p.tile_nodes[cur.n0 + min(tid + j * NT, max(cur.nown - 1, 0))];
 #pragma unroll
-                    for (int c = 0; c < 3; ++c) {
-                        const Real v = (Real)sR[3 * k + c];
-                        r[3 * g + c] = insert ? v : r[3 * g + c] + v;
-                    }
-                }
-            }
-        } else if constexpr (P2SPLIT) {
-            // the write-out ids, all slots at once (clamped positions, no branch)
-            int wl[S::PFN];
-#pragma unroll
-            for (int j = 0; j < S::PFN; ++j) wl[j] = A.p.tile_nodes[cur.n0 + min(tid + j * NT, max(cur.nown - 1, 0))];
-#pragma unroll
-            for (int j = 0; j < S::PFN; ++j) {
-                const int k = tid + j * NT;
-                if (k < cur.nown) {
-                    const size_t g = (size_t)wl[j];
-#pragma unroll
-                    for (int c = 0; c < 3; ++c) {
-                        const Real v = (Real)sR[3 * k + c];
-                        r[3 * g + c] = insert ? v : r[3 * g + c] + v;
-                    }
-                }
-            }
-        } else {
-            for (int k = tid; k < cur.nown; k += NT) {
-                const size_t g = (size_t)A.p.tile_nodes[cur.n0 + k];
+        for (int j = 0; j < S::PFN; ++j) {
+            const int k = tid + j * NT;
+            if (k < cur.nown) {
+                const size_t g = (size_t)wl[j];
 #pragma unroll
                 for (int c = 0; c < 3; ++c) {
                     const Real v = (Real)sR[3 * k + c];

@@ -12,7 +12,6 @@ struct P2Tables {
     double w[kP2Quad];
     double dphi[kP2Quad][10][3];
     double lam[kP2Quad][4];  // barycentric coordinates of the points
-    double wdiag, woff;      // P1 moments of the rule: sum_q w_q l_c l_d = wdiag (c == d), woff (c != d)
 };
 
 // Reference tables of the P2 tetrahedron at the 14-point degree-5 rule (two S31 orbits and
@@ -37,12 +36,8 @@ inline void p2_fill_tables(P2Tables *t) {
         t->w[q] = W3;
     }
     const double dl[4][3] = {{-1, -1, -1}, {1, 0, 0}, {0, 1, 0}, {0, 0, 1}};
-    t->wdiag = t->woff = 0.0;
-    for (q = 0; q < kP2Quad; ++q) {
+    for (q = 0; q < kP2Quad; ++q)
         for (int v = 0; v < 4; ++v) t->lam[q][v] = lam[q][v];
-        t->wdiag += t->w[q] * lam[q][0] * lam[q][0];
-        t->woff += t->w[q] * lam[q][0] * lam[q][1];
-    }
     for (q = 0; q < kP2Quad; ++q) {
         for (int v = 0; v < 4; ++v)
             for (int d = 0; d < 3; ++d) t->dphi[q][v][d] = (4.0 * lam[q][v] - 1.0) * dl[v][d];
@@ -633,46 +628,167 @@ __host__ __device__ inline void q1_element_qp(const XAcc &X, const UAcc &U, Real
     for (int c = 0; c < 3; ++c) iwht8<Real>(R[c], re[c]);
 }
 
-// P2 affine element, factorized through the P1 structure of the gradient: G(q) = sum_c l_c(q) G_c
-// with G_c the reference gradient at vertex c, so P(q) = sum_c l_c(q) P_c and
-//   r_i = sum_d M_d : dphi_i(vertex d),  M_d = sum_c W_dc P_c,  W_dc = sum_q w_q l_d(q) l_c(q)
-// (W from the 14-point rule: wdiag on the diagonal, woff off it).
-template <typename Real, typename UAcc>
-__host__ __device__ inline void p2_element_linear(const double X[4][3], const UAcc &U, Real lam,
-                                                  Real mu, double wdiag, double woff, Real re[3][10]) {
-    double J[9], Jid[9];
+// --------------------------------------------------------------------------------------------
+// P2 tetrahedron (affine), factorized.  Between the solution side and the test side it holds only one symmetric 3 x 3 per vertex (24 values): strains built component by component of u, turned into
+// stresses, and contracted component by component, each entry of the element vector handed to
+// emit(c, b, value) when it is formed.  That is 48 registers where the vertex fluxes (36 values) and
+// the whole element vector (30) took 132.
+// Jinv is only used as the adjugate A = det Jinv; the powers of det go into the stress scale.
+// e_0 = (-1, -1, -1), e_k = unit k: the reference gradients of the barycentric coordinates.
+// --------------------------------------------------------------------------------------------
+
+// pin(x) forms x here: without it the compiler reads every component's operands up front (in pairs) and
+// sinks the arithmetic to its last use, and the registers that the parts are cut to save go to operands.
+// schedule_barrier() keeps the instruction scheduler from mixing the parts again.
+template <typename Real>
+__host__ __device__ inline void pin(Real &x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" : "+v"(x));
+#endif
+}
+__host__ __device__ inline void schedule_barrier() {
+#if defined(__HIP_DEVICE_COMPILE__)
+    __builtin_amdgcn_sched_barrier(0);
+#endif
+}
+
+// Position of entry (c, d) of a symmetric 3 x 3 stored xx, yy, zz, xy, yz, xz.
+__host__ __device__ constexpr int sym6(int c, int d) { return c == d ? c : (c + d == 1 ? 3 : c + d == 3 ? 4 : 5); }
+
+__host__ __device__ inline double p2_adjugate(const double X[4][3], double A[9]) {
+    double J[9];
 #pragma unroll
     for (int d = 0; d < 3; ++d)
 #pragma unroll
         for (int k = 0; k < 3; ++k) J[3 * d + k] = X[k + 1][d] - X[0][d];
-    const double det = inv3(J, Jid);
-    Real Ji[9];
-#pragma unroll
-    for (int i = 0; i < 9; ++i) Ji[i] = (Real)Jid[i];
-    Real P[4][9];
-    p2_vertex_grads<Real>(U, P);
-    // vertex fluxes, in place
+    A[0] = J[4] * J[8] - J[5] * J[7];
+    A[1] = J[2] * J[7] - J[1] * J[8];
+    A[2] = J[1] * J[5] - J[2] * J[4];
+    A[3] = J[5] * J[6] - J[3] * J[8];
+    A[4] = J[0] * J[8] - J[2] * J[6];
+    A[5] = J[2] * J[3] - J[0] * J[5];
+    A[6] = J[3] * J[7] - J[4] * J[6];
+    A[7] = J[1] * J[6] - J[0] * J[7];
+    A[8] = J[0] * J[4] - J[1] * J[3];
+    return J[0] * A[0] + J[1] * A[3] + J[2] * A[6];
+}
+
+// Strains at the four vertices times det (xx, yy, zz and twice xy, yz, xz), the part of solution
+// component c (0, 1, 2 in turn; u: its ten nodal values).  With S the vertex differences u_k - u_0,
+// the reference gradient at vertex v is 4 d_v - S, d_0 = (u01 - u0, u02 - u0, u03 - u0),
+// d_1 = (u1 - u01, u12 - u01, u13 - u01), d_2 = (u12 - u02, u2 - u02, u23 - u02),
+// d_3 = (u13 - u03, u23 - u03, u3 - u03).
+template <int C, bool PIN, typename Real>
+__host__ __device__ inline void p2_strain_component(const Real u[10], const Real A[9], Real S[4][6]) {
+    const Real s0 = u[1] - u[0], s1 = u[2] - u[0], s2 = u[3] - u[0];
+    const Real far[4][3] = {{u[4], u[5], u[6]}, {u[1], u[7], u[8]}, {u[7], u[2], u[9]}, {u[8], u[9], u[3]}};
+    const Real near[4] = {u[0], u[4], u[5], u[6]};
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
-        Real G[9];
+        const Real g0 = Real(4) * (far[v][0] - near[v]) - s0, g1 = Real(4) * (far[v][1] - near[v]) - s1,
+                   g2 = Real(4) * (far[v][2] - near[v]) - s2;
 #pragma unroll
-        for (int i = 0; i < 9; ++i) G[i] = P[v][i];
-        iso_flux<Real>(G, Ji, lam, mu, (Real)det, P[v]);
+        for (int d = 0; d < 3; ++d) {
+            const Real g = g0 * A[d] + g1 * A[3 + d] + g2 * A[6 + d];
+            // the first component to reach an entry assigns it
+            if (C <= d) S[v][sym6(C, d)] = g;
+            else S[v][sym6(C, d)] += g;
+            if (PIN) pin(S[v][sym6(C, d)]);
+        }
     }
-    // M_d = wdiag' P_d + woff SP with wdiag' = wdiag - woff; sum_d M_d = (wdiag' + 4 woff) SP
-    Real SP[9];
+}
+
+template <bool PIN, typename Real, typename UAcc>
+__host__ __device__ inline void p2_vertex_strains(const UAcc &U, const Real A[9], Real S[4][6]) {
+    Real u[10];
 #pragma unroll
-    for (int i = 0; i < 9; ++i) SP[i] = P[0][i] + P[1][i] + P[2][i] + P[3][i];
-    const Real a = (Real)(wdiag - woff), b = (Real)woff;
+    for (int b = 0; b < 10; ++b) u[b] = U(0, b);
+    p2_strain_component<0, PIN, Real>(u, A, S);
+    if (PIN) schedule_barrier();
 #pragma unroll
-    for (int v = 0; v < 4; ++v)
+    for (int b = 0; b < 10; ++b) u[b] = U(1, b);
+    p2_strain_component<1, PIN, Real>(u, A, S);
+    if (PIN) schedule_barrier();
 #pragma unroll
-        for (int i = 0; i < 9; ++i) P[v][i] = a * P[v][i] + b * SP[i];
-    const Real sa = a + Real(4) * b;
-    Real SM[9];
+    for (int b = 0; b < 10; ++b) u[b] = U(2, b);
+    p2_strain_component<2, PIN, Real>(u, A, S);
+    if (PIN) schedule_barrier();
+}
+
+// Stresses of the linear kernels in place of the strains of p2_vertex_strains (isotropic, scaled by q).
+template <typename Real>
+__host__ __device__ inline void p2_vertex_stresses(Real q, Real lam, Real mu, Real S[4][6]) {
+    const Real ql = q * lam, qm = q * mu, qm2 = Real(2) * qm;
 #pragma unroll
-    for (int i = 0; i < 9; ++i) SM[i] = sa * SP[i];
-    p2_vertex_contract<Real>(P, SM, re);
+    for (int v = 0; v < 4; ++v) {
+        const Real ls = ql * (S[v][0] + S[v][1] + S[v][2]);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) S[v][i] = ls + qm2 * S[v][i];
+#pragma unroll
+        for (int i = 3; i < 6; ++i) S[v][i] *= qm;
+    }
+}
+
+// Test side, component c: with P_v = S_v A^T = -(stress at vertex v) Jinv^T det / 30 and h = sum_v P_v,
+//     vertex a:    P_a e_a - h e_a / 4
+//     edge (a, b): P_a e_b + P_b e_a + h (e_a + e_b).
+// This is r_i = sum_v M_v : dphi_i(vertex v) (vertex gradients (4 delta - 1) e_a, edge gradients 4 e_b
+// at a and 4 e_a at b) with the vertex moments of any rule exact to degree 2, M_v = sum_w W_vw (30 P_w),
+// W_vw = sum_q w_q l_v l_w = (1 + delta_vw) / 120: 4 M_a = P_a + h, sum_v M_v = 5 h / 4.
+template <typename Real>
+__host__ __device__ inline void p2_contract_component(int c, const Real S[4][6], const Real A[9], Real re[10]) {
+    Real P[4][3], t[4];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+            P[v][k] = S[v][sym6(c, 0)] * A[3 * k] + S[v][sym6(c, 1)] * A[3 * k + 1] + S[v][sym6(c, 2)] * A[3 * k + 2];
+        t[v] = P[v][0] + P[v][1] + P[v][2];  // -P_v e_0
+    }
+    const Real h0 = P[0][0] + P[1][0] + P[2][0] + P[3][0], h1 = P[0][1] + P[1][1] + P[2][1] + P[3][1],
+               h2 = P[0][2] + P[1][2] + P[2][2] + P[3][2];
+    const Real q = Real(0.25);
+    re[0] = q * (h0 + h1 + h2) - t[0];
+    re[1] = P[1][0] - q * h0;
+    re[2] = P[2][1] - q * h1;
+    re[3] = P[3][2] - q * h2;
+    const Real h01 = h0 + h1, h02 = h0 + h2, h12 = h1 + h2;
+    re[4] = P[0][0] - t[1] - h12;
+    re[5] = P[0][1] - t[2] - h02;
+    re[6] = P[0][2] - t[3] - h01;
+    re[7] = P[1][1] + P[2][0] + h01;
+    re[8] = P[1][2] + P[3][0] + h02;
+    re[9] = P[2][2] + P[3][1] + h12;
+}
+
+template <bool PIN, typename Real, typename Emit>
+__host__ __device__ inline void p2_sym_contract(const Real S[4][6], const Real A[9], const Emit &emit) {
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        Real re[10];
+        p2_contract_component<Real>(c, S, A, re);
+#pragma unroll
+        for (int b = 0; b < 10; ++b) emit(c, b, re[b]);
+        if (PIN) schedule_barrier();
+    }
+}
+
+// Factorized through the P1 structure of the gradient: stresses at the four vertices and the exact
+// moments of the barycentric coordinates in place of the points.
+template <typename Real, typename UAcc, typename Emit>
+__host__ __device__ inline void p2_element_linear(const double X[4][3], const UAcc &U, Real lam, Real mu,
+                                                  const Emit &emit) {
+    Real A[9], S[4][6];
+    Real scale;
+    {
+        double Ad[9];
+        scale = (Real)(-1.0 / (30.0 * p2_adjugate(X, Ad)));
+#pragma unroll
+        for (int i = 0; i < 9; ++i) A[i] = (Real)Ad[i];
+    }
+    p2_vertex_strains<sizeof(Real) == 8, Real>(U, A, S);
+    p2_vertex_stresses<Real>(scale, lam, mu, S);
+    p2_sym_contract<sizeof(Real) == 8, Real>(S, A, emit);
 }
 
 }  // namespace plx

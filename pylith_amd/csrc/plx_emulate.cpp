@@ -118,8 +118,9 @@ int emulate(const plx::MeshView &mv, const double *coords, const plx::HostPlan &
                 }
                 for (int b = 0; b < nb; ++b)
                     for (int c = 0; c < 3; ++c) U[c][b] = sU[3 * lc[b] + c];
+                const auto emit = [&](int c, int b, Real v) { rl[c][b] = v; };
                 if (linear)
-                    plx::p2_element_linear<Real>(X, plx::ArrayAcc3<Real>{U}, lam, mu, HostTab::t().wdiag, HostTab::t().woff, rl);
+                    plx::p2_element_linear<Real>(X, plx::ArrayAcc3<Real>{U}, lam, mu, emit);
                 else
                     plx::p2_element<Real, HostTab>(X, U, lam, mu, rl);
                 for (int b = 0; b < nb; ++b)
