@@ -81,14 +81,13 @@ int device_setup(plx_dm dm) {
 struct ApplyArgs {
     TilePlanDev p;
     const uint8_t *color;   // [stride] colour of each key cell (tile-local greedy colouring)
-    const int32_t *tile_ncolor;
     const void *mat;        // [2][stride] lambda, mu
     const void *u;
     void *r;
     void *halo;
     int mode;
     double scale;           // multiplies the element vectors (e.g. -1 for the SPD operator -J)
-    const int32_t *tile_list;  // tiles this launch covers (nullptr: all, in order)
+    const int32_t *heads;      // TileHead of the tiles this launch covers, in order
     int num_list;
     const void *records;       // packed 16-bit local closure (+ cone) per key cell
     const double *prestress;   // Q1: per-point stress added to sigma, [6][8][stride] (nullptr: none)
@@ -109,6 +108,51 @@ struct LdsAccQ1 {
 };
 
 constexpr int kAccColored = 0, kAccAtomic = 1;
+
+// Tile extents (TileHead), loaded one word per lane two tiles ahead and read from the lanes when the
+// tile's ids go out.  Read in place, each tile began with a wait for its extents that also waited for
+// the previous tile's stores (loads and stores complete in order): 137 -> 128 us on 153 x 149 x 157
+// hexes.
+__device__ __forceinline__ int head_word(const int32_t *heads, int tile) { return heads[8 * (size_t)tile + (threadIdx.x & 7)]; }
+__device__ __forceinline__ TileHead head_of(int word) {
+    TileHead h;
+    h.c0 = __builtin_amdgcn_readlane(word, 0);
+    h.nc = __builtin_amdgcn_readlane(word, 1);
+    h.n0 = __builtin_amdgcn_readlane(word, 2);
+    h.nn = __builtin_amdgcn_readlane(word, 3);
+    h.v0 = __builtin_amdgcn_readlane(word, 4);
+    h.nvt = __builtin_amdgcn_readlane(word, 5);
+    h.nown = __builtin_amdgcn_readlane(word, 6);
+    h.hoff = __builtin_amdgcn_readlane(word, 7);
+    return h;
+}
+
+// A tile's node sums to the output: owned nodes to their rows (the ids in gn), shared ones to the
+// halo slots.  All of a thread's sums are read before the first is stored.
+template <typename Real, typename Acc, int SLOTS, int NT>
+__device__ __forceinline__ void write_out(const Acc *sR, const int (&gn)[SLOTS], int nn, int nown, int hoff, int tid,
+                                          Real *r, Real *halo, bool insert) {
+    Real w[SLOTS][3];
+#pragma unroll
+    for (int j = 0; j < SLOTS; ++j) {
+        const int k = min(tid + j * NT, nn - 1);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) w[j][c] = (Real)sR[3 * k + c];
+    }
+#pragma unroll
+    for (int j = 0; j < SLOTS; ++j) {
+        const int k = tid + j * NT;
+        if (k < nn) {
+            Real *dst = k < nown ? r + 3 * (size_t)gn[j] : halo + 3 * ((size_t)hoff + (size_t)(k - nown));
+            if (!insert && k < nown) {
+#pragma unroll
+                for (int c = 0; c < 3; ++c) w[j][c] += dst[c];
+            }
+#pragma unroll
+            for (int c = 0; c < 3; ++c) dst[c] = w[j][c];
+        }
+    }
+}
 
 // Map slot i to a tile so that each of the 8 XCDs (round-robin workgroup dispatch) walks a
 // contiguous range of tiles: neighbouring tiles then share that XCD's L2.
@@ -146,168 +190,90 @@ __device__ __forceinline__ int rec_get(const uint4 (&r)[W], int k) {
     return (k & 1) ? (int)(v >> 16) : (int)(v & 0xffffu);
 }
 
-// One tile's data on its way from HBM: gathered node values and coordinates, the cells'
-// local closures, moduli and colours (registers; the next tile's loads overlap the current
-// tile's arithmetic).  The gathers go out in two phases: the node / vertex ids (with the cells'
-// records and moduli) before the current tile's first cell, the values at those ids after it,
-// so the ids' latency hides behind that cell's arithmetic.
+// One tile's data on its way from HBM: gathered node values and coordinates, the cells' local
+// closures, moduli and colours (registers).  The gathers go out in two phases: the node / vertex ids
+// before the previous tile's cells, whose arithmetic hides their latency, and the values at them later.
+// Every load is unconditional, at positions clamped into the tile: slots past its end repeat its last
+// entry.  (A branch around each load keeps its destination registers alive around the loop: 30 to 60
+// registers, and with them the spills of the Q1 quadrature-point kernels.)
 template <typename Real, int CT>
 struct Stage {
     using S = Shape<CT, Real>;
-    int tile, c0, nc, n0, nn, v0, nvt, nown, hoff;
-    int gn[S::PFN];                          // node ids between the two phases (-1: past the tile)
+    int c0, nc, ncolor, n0, nn, v0, nvt, nown, hoff;
+    int gn[S::PFN];                          // node ids (the write-out uses them again)
     int gv[CT == PLX_HEX_Q1 ? 1 : S::PFV];   // P2 vertex ids
     Real pu[S::PFN][3];
     double px[CT == PLX_HEX_Q1 ? S::PFN : S::PFV][3];
     uint4 rec[S::CPT][S::RECW];  // packed 16-bit local closure (and cone) of each cell
     Real lam[S::CPT], mu[S::CPT];
     int color[S::CPT];
+    __device__ __forceinline__ void extents(const TileHead &h) {
+        c0 = h.c0;
+        nc = h.nc & 0xffff;
+        ncolor = h.nc >> 16;
+        n0 = h.n0;
+        nn = h.nn;
+        v0 = h.v0;
+        nvt = h.nvt;
+        nown = h.nown;
+        hoff = h.hoff;
+    }
 };
 
-// First phase of the two-phase fetch: extents, node (and P2 vertex) ids, the cells' records and
-// moduli.
-template <typename Real, int CT, int ACC>
-__device__ __forceinline__ void fetch_ids(Stage<Real, CT> &T, const ApplyArgs &A, int tile, int tid) {
+template <typename Real, int CT>
+__device__ __forceinline__ void fetch_ids(Stage<Real, CT> &T, const ApplyArgs &A, const TileHead &h, int tid) {
     using S = Shape<CT, Real>;
-    const TilePlanDev &P = A.p;
-    T.tile = tile;
-    T.c0 = P.tile_cell_ptr[tile];
-    T.nc = P.tile_cell_ptr[tile + 1] - T.c0;
-    T.n0 = P.tile_node_ptr[tile];
-    T.nn = P.tile_node_ptr[tile + 1] - T.n0;
-    T.v0 = P.tile_vert_ptr[tile];
-    T.nvt = P.tile_vert_ptr[tile + 1] - T.v0;
-    T.nown = P.tile_nown[tile];
-    T.hoff = P.tile_halo_off[tile];
+    T.extents(h);
 #pragma unroll
-    for (int j = 0; j < S::PFN; ++j) {
-        const int k = tid + j * S::NT;
-        T.gn[j] = k < T.nn ? P.tile_nodes[T.n0 + k] : -1;
-    }
-    if constexpr (CT != PLX_HEX_Q1) {
-#pragma unroll
-        for (int j = 0; j < S::PFV; ++j) {
-            const int k = tid + j * S::NT;
-            T.gv[j] = k < T.nvt ? P.tile_verts[T.v0 + k] : -1;
-        }
-    }
+    for (int j = 0; j < S::PFN; ++j) T.gn[j] = A.p.tile_nodes[h.n0 + min(tid + j * S::NT, h.nn - 1)];
+    if constexpr (CT != PLX_HEX_Q1) T.gv[0] = A.p.tile_verts[h.v0 + min(tid, h.nvt - 1)];
+}
+
+template <typename Real, int CT, int ACC>
+__device__ __forceinline__ void fetch_cells(Stage<Real, CT> &T, const ApplyArgs &A, int tid) {
+    using S = Shape<CT, Real>;
     const Real *mat = static_cast<const Real *>(A.mat);
+    const uint4 *recs = reinterpret_cast<const uint4 *>(A.records);
 #pragma unroll
     for (int i = 0; i < S::CPT; ++i) {
-        const int cell = tid + i * S::NT;
-        if (cell < T.nc) {
-            const int pos = T.c0 + cell;
-            const uint4 *recs = reinterpret_cast<const uint4 *>(A.records);
+        const int pos = T.c0 + min(tid + i * S::NT, T.nc - 1);
 #pragma unroll
-            for (int w = 0; w < S::RECW; ++w) T.rec[i][w] = recs[(size_t)pos * S::RECW + w];
-            // unscaled here (scaled where used): the fetch then has no use of these loads to wait for
-            T.lam[i] = mat[pos];
-            T.mu[i] = mat[P.stride + pos];
-            if (ACC == kAccColored) T.color[i] = A.color[pos];
-        }
+        for (int w = 0; w < S::RECW; ++w) T.rec[i][w] = recs[(size_t)pos * S::RECW + w];
+        // unscaled here (scaled where used): the fetch then has no use of these loads to wait for
+        T.lam[i] = mat[pos];
+        T.mu[i] = mat[A.p.stride + pos];
+        if (ACC == kAccColored) T.color[i] = A.color[pos];
     }
 }
 
-// Second phase: the values and coordinates at the ids of fetch_ids.
 template <typename Real, int CT>
 __device__ __forceinline__ void fetch_values(Stage<Real, CT> &T, const ApplyArgs &A) {
     using S = Shape<CT, Real>;
-    const TilePlanDev &P = A.p;
     const Real *u = static_cast<const Real *>(A.u);
+    const double *coords = A.p.coords;
 #pragma unroll
     for (int j = 0; j < S::PFN; ++j) {
-        if (T.gn[j] >= 0) {
-            const size_t g = (size_t)T.gn[j];
+        const size_t g = (size_t)T.gn[j];
 #pragma unroll
-            for (int c = 0; c < 3; ++c) T.pu[j][c] = u[3 * g + c];
-            if constexpr (CT == PLX_HEX_Q1) {
+        for (int c = 0; c < 3; ++c) T.pu[j][c] = u[3 * g + c];
+        if constexpr (CT == PLX_HEX_Q1) {
 #pragma unroll
-                for (int d = 0; d < 3; ++d) T.px[j][d] = P.coords[3 * g + d];
-            }
+            for (int d = 0; d < 3; ++d) T.px[j][d] = coords[3 * g + d];
         }
     }
     if constexpr (CT != PLX_HEX_Q1) {
 #pragma unroll
-        for (int j = 0; j < S::PFV; ++j) {
-            if (T.gv[j] >= 0) {
-                const size_t g = (size_t)T.gv[j];
-#pragma unroll
-                for (int d = 0; d < 3; ++d) T.px[j][d] = P.coords[3 * g + d];
-            }
-        }
+        for (int d = 0; d < 3; ++d) T.px[0][d] = coords[3 * (size_t)T.gv[0] + d];
     }
 }
 
-// One phase (the first tile; the Q1 quadrature-point kernels throughout).  Kept apart from the two
-// phases: with those for the first tile too, the P2 kernels take 30 registers more.
-template <typename Real, int CT, int ACC>
-__device__ __forceinline__ void fetch(Stage<Real, CT> &T, const ApplyArgs &A, int tile, int tid) {
+// LDS of a tile kernel: nodal values, the accumulator and coordinates at fixed places (the addresses
+// then differ by constants), sized for every thread's slots.
+template <typename Real, int CT, typename Acc>
+constexpr size_t tile_lds_bytes() {
     using S = Shape<CT, Real>;
-    const TilePlanDev &P = A.p;
-    const Real *u = static_cast<const Real *>(A.u);
-    T.tile = tile;
-    T.c0 = P.tile_cell_ptr[tile];
-    T.nc = P.tile_cell_ptr[tile + 1] - T.c0;
-    T.n0 = P.tile_node_ptr[tile];
-    T.nn = P.tile_node_ptr[tile + 1] - T.n0;
-    T.v0 = P.tile_vert_ptr[tile];
-    T.nvt = P.tile_vert_ptr[tile + 1] - T.v0;
-    T.nown = P.tile_nown[tile];
-    T.hoff = P.tile_halo_off[tile];
-    if constexpr (CT == PLX_HEX_Q1) {
-        // every node id first, then the values: one wait between the two, not one per slot
-#pragma unroll
-        for (int j = 0; j < S::PFN; ++j) {
-            const int k = tid + j * S::NT;
-            T.gn[j] = k < T.nn ? P.tile_nodes[T.n0 + k] : -1;
-        }
-#pragma unroll
-        for (int j = 0; j < S::PFN; ++j) {
-            if (T.gn[j] >= 0) {
-                const size_t g = (size_t)T.gn[j];
-#pragma unroll
-                for (int c = 0; c < 3; ++c) T.pu[j][c] = u[3 * g + c];
-#pragma unroll
-                for (int d = 0; d < 3; ++d) T.px[j][d] = P.coords[3 * g + d];
-            }
-        }
-    } else {
-        // P2: id and values slot by slot
-#pragma unroll
-        for (int j = 0; j < S::PFN; ++j) {
-            const int k = tid + j * S::NT;
-            if (k < T.nn) {
-                T.gn[j] = P.tile_nodes[T.n0 + k];
-                const size_t g = (size_t)T.gn[j];
-#pragma unroll
-                for (int c = 0; c < 3; ++c) T.pu[j][c] = u[3 * g + c];
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < S::PFV; ++j) {
-            const int k = tid + j * S::NT;
-            if (k < T.nvt) {
-                const size_t g = (size_t)P.tile_verts[T.v0 + k];
-#pragma unroll
-                for (int d = 0; d < 3; ++d) T.px[j][d] = P.coords[3 * g + d];
-            }
-        }
-    }
-    const Real *mat = static_cast<const Real *>(A.mat);
-#pragma unroll
-    for (int i = 0; i < S::CPT; ++i) {
-        const int cell = tid + i * S::NT;
-        if (cell < T.nc) {
-            const int pos = T.c0 + cell;
-            const uint4 *recs = reinterpret_cast<const uint4 *>(A.records);
-#pragma unroll
-            for (int w = 0; w < S::RECW; ++w) T.rec[i][w] = recs[(size_t)pos * S::RECW + w];
-            // unscaled here (scaled where used): the fetch then has no use of these loads to wait for
-            T.lam[i] = mat[pos];
-            T.mu[i] = mat[P.stride + pos];
-            if (ACC == kAccColored) T.color[i] = A.color[pos];
-        }
-    }
+    return (size_t)S::PFN * S::NT * 3 * (sizeof(Real) + sizeof(Acc)) +
+           (size_t)(CT == PLX_HEX_Q1 ? S::PFN * S::NT : S::PFV * S::NT) * 3 * sizeof(double);
 }
 
 // Element paths of the tile kernel: the factorized form (kernels linear in the gradient with
@@ -323,68 +289,53 @@ __global__ void __launch_bounds__((Shape<CT, Real>::NT), MINW) apply_tiles(Apply
     using S = Shape<CT, Real>;
     constexpr int NT = S::NT, NB = S::NB, NV = S::NV;
     static_assert(S::PFN * NT >= 768 && S::CPT * NT >= (CT == PLX_HEX_Q1 ? 512 : 384), "tile limits");
-    static_assert(CT == PLX_HEX_Q1 || S::PFV * NT >= 192, "vertex limit");
+    static_assert(CT == PLX_HEX_Q1 || (S::PFV == 1 && NT >= 192), "vertex limit");
     extern __shared__ __align__(16) unsigned char smem[];
     const int tid = threadIdx.x;
     const int G = gridDim.x;
     int slot = blockIdx.x;
     if (slot >= A.num_list) return;
-    auto tile_of = [&](int s) {
-        const int t = xcd_tile(s, A.num_list);
-        return A.tile_list ? A.tile_list[t] : t;
-    };
+    auto word_of = [&](int s) { return head_word(A.heads, xcd_tile(s, A.num_list)); };
     Stage<Real, CT> cur;
-    fetch<Real, CT, ACC>(cur, A, tile_of(slot), tid);
-    // Q1: the first tile's loads complete here, as every later tile's complete before the
-    // loop's back edge, so the loop is entered with nothing in flight.  Otherwise the wait
-    // analysis, merging this path into the loop, puts a wait for them inside the cell
-    // arithmetic, where in every later tile it also waits for the next tile's gathers
-    // (Q1 192^3 FP64: 0.300 -> 0.275 ms; the P2 kernels measured no gain)
-    if constexpr (CT == PLX_HEX_Q1) __builtin_amdgcn_s_waitcnt(0);
+    int next_word = slot + G < A.num_list ? word_of(slot + G) : 0;
+    fetch_ids<Real, CT>(cur, A, head_of(word_of(slot)), tid);
+    fetch_cells<Real, CT, ACC>(cur, A, tid);
+    fetch_values<Real, CT>(cur, A);
     Real *r = static_cast<Real *>(A.r);
     Real *halo = static_cast<Real *>(A.halo);
     const bool insert = A.mode == PLX_INSERT_VALUES;
     // LDS atomics accumulate in FP64 whatever the vector type (native ds_add_f64; FP32 calls
     // round once at the write-out)
     using Acc = typename std::conditional<ACC == kAccAtomic, double, Real>::type;
+    Acc *sR = reinterpret_cast<Acc *>(smem);
+    Real *sU = reinterpret_cast<Real *>(sR + 3 * S::PFN * NT);
+    double *sX = reinterpret_cast<double *>(sU + 3 * S::PFN * NT);
+    constexpr bool DIRECT = CT != PLX_HEX_Q1 && PATH == kPathFactored && ACC == kAccAtomic;
+    // The next tile's node values go out between the thread's two cells and arrive during the second
+    // (153 x 149 x 157 hexes, factored: 128 us; after both cells 146 us).  The Q1 quadrature-point
+    // kernels, whose elements fill the registers, load them and the cells' data after both (80 x 71 x 66
+    // non-affine hexes: 44.5 us, 45.6 us between the cells).
+    constexpr bool LATE = CT == PLX_HEX_Q1 && PATH != kPathFactored;
     while (true) {
-        // LDS layout of this tile: coordinates, the accumulator, then nodal values
-        const int nxv = CT == PLX_HEX_Q1 ? cur.nn : cur.nvt;
-        double *sX = reinterpret_cast<double *>(smem);
-        Acc *sR = reinterpret_cast<Acc *>(sX + 3 * nxv);
-        Real *sU = reinterpret_cast<Real *>(sR + 3 * cur.nn);
 #pragma unroll
         for (int j = 0; j < S::PFN; ++j) {
             const int k = tid + j * NT;
-            if (k < cur.nn) {
 #pragma unroll
-                for (int c = 0; c < 3; ++c) {
-                    sU[3 * k + c] = cur.pu[j][c];
-                    sR[3 * k + c] = Acc(0);
-                }
-                if constexpr (CT == PLX_HEX_Q1) {
+            for (int c = 0; c < 3; ++c) {
+                sU[3 * k + c] = cur.pu[j][c];
+                sR[3 * k + c] = Acc(0);
+            }
+            if constexpr (CT == PLX_HEX_Q1) {
 #pragma unroll
-                    for (int d = 0; d < 3; ++d) sX[3 * k + d] = cur.px[j][d];
-                }
+                for (int d = 0; d < 3; ++d) sX[3 * k + d] = cur.px[j][d];
             }
         }
         if constexpr (CT != PLX_HEX_Q1) {
 #pragma unroll
-            for (int j = 0; j < S::PFV; ++j) {
-                const int k = tid + j * NT;
-                if (k < cur.nvt) {
-#pragma unroll
-                    for (int d = 0; d < 3; ++d) sX[3 * k + d] = cur.px[j][d];
-                }
-            }
+            for (int d = 0; d < 3; ++d) sX[3 * tid + d] = cur.px[0][d];
         }
         __syncthreads();
 
-        // The next tile's loads go out in two phases (see Stage): its ids here, the values at them after
-        // the first of the thread's two cells; the Q1 quadrature-point kernels issue both here (their
-        // registers overflow otherwise)
-        constexpr bool SPLIT = CT != PLX_HEX_Q1 || PATH == kPathFactored;
-        constexpr bool DIRECT = CT != PLX_HEX_Q1 && PATH == kPathFactored && ACC == kAccAtomic;
         const int next_slot = slot + G;
         const bool has_next = next_slot < A.num_list;
         Stage<Real, CT> nxt;
@@ -393,17 +344,12 @@ __global__ void __launch_bounds__((Shape<CT, Real>::NT), MINW) apply_tiles(Apply
         // at priority 1: Q1 -1.4 %)
         __builtin_amdgcn_s_setprio(2);
         if (has_next) {
-            if constexpr (SPLIT) fetch_ids<Real, CT, ACC>(nxt, A, tile_of(next_slot), tid);
-            else fetch<Real, CT, ACC>(nxt, A, tile_of(next_slot), tid);
+            const TileHead h = head_of(next_word);
+            if (next_slot + G < A.num_list) next_word = word_of(next_slot + G);
+            fetch_ids<Real, CT>(nxt, A, h, tid);
+            if constexpr (!LATE) fetch_cells<Real, CT, ACC>(nxt, A, tid);
         }
         __builtin_amdgcn_s_setprio(0);
-        const auto next_values = [&] {
-            if (has_next) {
-                __builtin_amdgcn_s_setprio(2);
-                fetch_values<Real, CT>(nxt, A);
-                __builtin_amdgcn_s_setprio(0);
-            }
-        };
 
 #pragma unroll
         for (int i = 0; i < S::CPT; ++i) {
@@ -468,8 +414,7 @@ __global__ void __launch_bounds__((Shape<CT, Real>::NT), MINW) apply_tiles(Apply
             } else {
                 // cells of one colour share no node: fixed summation order (cells i = 0 of the
                 // workgroup colour by colour, then cells i = 1), reproducible bits
-                const int ncolor = A.tile_ncolor[cur.tile];
-                for (int col = 0; col < ncolor; ++col) {
+                for (int col = 0; col < cur.ncolor; ++col) {
                     __syncthreads();
                     if (active && cur.color[i] == col) {
 #pragma unroll
@@ -479,37 +424,177 @@ __global__ void __launch_bounds__((Shape<CT, Real>::NT), MINW) apply_tiles(Apply
                     }
                 }
             }
-            if constexpr (SPLIT)
-                if (i == 0) next_values();
+            if (!LATE && i == 0 && has_next) {
+                __builtin_amdgcn_s_setprio(2);
+                fetch_values<Real, CT>(nxt, A);
+                __builtin_amdgcn_s_setprio(0);
+            }
         }
         __syncthreads();
         __builtin_amdgcn_s_setprio(1);
+        if (LATE && has_next) {
+            fetch_cells<Real, CT, ACC>(nxt, A, tid);
+            fetch_values<Real, CT>(nxt, A);
+        }
+        write_out<Real, Acc, S::PFN, NT>(sR, cur.gn, cur.nn, cur.nown, cur.hoff, tid, r, halo, insert);
+        __builtin_amdgcn_s_setprio(0);
+        if (!has_next) break;
+        __syncthreads();  // every read of this tile's LDS precedes the next tile's staging
+        cur = nxt;
+        slot = next_slot;
+    }
+}
 
-        // owned nodes: the ids are those this thread gathered by; the quadrature-point kernels, whose
-        // registers are full, read them again (all slots at once, clamped positions, no branch)
-        constexpr bool KEEP = PATH == kPathFactored;
-        int wl[S::PFN];
+// --------------------------------------------------------------------------------------------
+// P2 pair kernel: the factored residual / action with LDS atomics, one pair of face-sharing cells per
+// thread (PairPlan).  A pair reads 14 nodes and 5 vertices from LDS and adds to 14 nodes where two
+// cells take 20, 8 and 20, its record is 24 bytes where theirs are 64, and 512-cell tiles leave fewer
+// shared nodes.  63 x 66 x 61 x 6 cells: 74 us against 84 us for the tile kernel (FP32, 40 x 44 x 37 x 6:
+// 17 us against 19 us).
+// The tile kernel above was bound on chip (63 x 66 x 61 x 6 cells: 80 us, 68 us with every gather
+// served from L2, 57 us without its atomics, 42 us without the element): LDS accesses are what
+// pairing cuts.  Same pipeline, with everything but the next tile's ids after the cells: two cells at
+// once leave no registers for it (between the two halves of the element: 79 us against 74).
+// --------------------------------------------------------------------------------------------
+struct PairArgs {
+    int num_tiles;
+    const int32_t *heads, *nodes, *verts;
+    const uint2 *rec;   // [pairs][3]
+    const void *mat;    // [pairs][4] lambda, mu of the two cells
+    const double *coords;
+    const void *u;
+    void *r, *halo;
+    int mode;
+    double scale;
+};
+
+constexpr int kPairThreads = 256, kPairSlots = kPairTileNodes / kPairThreads;
+static_assert(kPairThreads == kPairTilePairs && kPairThreads >= kPairTileVerts, "one pair and one vertex per thread");
+
+template <typename Real>
+constexpr size_t pair_lds_bytes() {
+    return (size_t)kPairTileNodes * 3 * (sizeof(double) + sizeof(Real)) + (size_t)kPairTileVerts * 3 * sizeof(double);
+}
+
+template <typename Real>
+struct PairStage {
+    int p0, np, nn, nown, hoff;
+    int gn[kPairSlots], gv;
+    Real pu[kPairSlots][3];
+    double px[3];
+    uint2 rec[3];
+    Real mat[4];
+};
+
+// Every load is unconditional, at positions clamped into the tile: slots past its end repeat its last
+// entry (a branch around each load keeps its destination registers alive around the loop).
+template <typename Real>
+__device__ __forceinline__ void pair_fetch_ids(PairStage<Real> &T, const PairArgs &A, const TileHead &h, int tid) {
+    T.p0 = h.c0;
+    T.np = h.nc;
+    T.nn = h.nn;
+    T.nown = h.nown;
+    T.hoff = h.hoff;
 #pragma unroll
-        for (int j = 0; j < S::PFN; ++j)
-            wl[j] = KEEP ? cur.gn[j] : A.p.tile_nodes[cur.n0 + min(tid + j * NT, max(cur.nown - 1, 0))];
+    for (int j = 0; j < kPairSlots; ++j) T.gn[j] = A.nodes[h.n0 + min(tid + j * kPairThreads, h.nn - 1)];
+    T.gv = A.verts[h.v0 + min(tid, h.nvt - 1)];
+}
+
+template <typename Real>
+__device__ __forceinline__ void pair_fetch_values(PairStage<Real> &T, const PairArgs &A, int tid) {
+    const Real *u = static_cast<const Real *>(A.u);
+    const size_t p = (size_t)T.p0 + (size_t)min(tid, T.np - 1);
 #pragma unroll
-        for (int j = 0; j < S::PFN; ++j) {
-            const int k = tid + j * NT;
-            if (k < cur.nown) {
-                const size_t g = (size_t)wl[j];
+    for (int w = 0; w < 3; ++w) T.rec[w] = A.rec[3 * p + w];
+    const Real *m = static_cast<const Real *>(A.mat) + 4 * p;
 #pragma unroll
-                for (int c = 0; c < 3; ++c) {
-                    const Real v = (Real)sR[3 * k + c];
-                    r[3 * g + c] = insert ? v : r[3 * g + c] + v;
-                }
+    for (int i = 0; i < 4; ++i) T.mat[i] = m[i];
+#pragma unroll
+    for (int j = 0; j < kPairSlots; ++j)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) T.pu[j][c] = u[3 * (size_t)T.gn[j] + c];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) T.px[d] = A.coords[3 * (size_t)T.gv + d];
+}
+
+template <typename Real>
+__global__ void __launch_bounds__(kPairThreads, 2) apply_pairs(PairArgs A) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    double *sR = reinterpret_cast<double *>(smem);
+    double *sX = sR + 3 * kPairTileNodes;
+    Real *sU = reinterpret_cast<Real *>(sX + 3 * kPairTileVerts);
+    const int tid = threadIdx.x;
+    const int G = gridDim.x;
+    int slot = blockIdx.x;
+    if (slot >= A.num_tiles) return;
+    PairStage<Real> cur;
+    auto word_of = [&](int s) { return head_word(A.heads, xcd_tile(s, A.num_tiles)); };
+    int next_word = slot + G < A.num_tiles ? word_of(slot + G) : 0;
+    pair_fetch_ids<Real>(cur, A, head_of(word_of(slot)), tid);
+    pair_fetch_values<Real>(cur, A, tid);
+    Real *r = static_cast<Real *>(A.r);
+    Real *halo = static_cast<Real *>(A.halo);
+    const bool insert = A.mode == PLX_INSERT_VALUES;
+    while (true) {
+#pragma unroll
+        for (int j = 0; j < kPairSlots; ++j) {
+            const int k = tid + j * kPairThreads;
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                sU[3 * k + c] = cur.pu[j][c];
+                sR[3 * k + c] = 0.0;
             }
         }
-        const size_t hoff = (size_t)cur.hoff;
-        for (int k = cur.nown + tid; k < cur.nn; k += NT) {
-            const size_t s = hoff + (size_t)(k - cur.nown);
 #pragma unroll
-            for (int c = 0; c < 3; ++c) halo[3 * s + c] = (Real)sR[3 * k + c];
+        for (int d = 0; d < 3; ++d) sX[3 * tid + d] = cur.px[d];
+        __syncthreads();
+        const int next_slot = slot + G;
+        const bool has_next = next_slot < A.num_tiles;
+        PairStage<Real> nxt;
+        // the next tile's loads at a raised wave priority, ahead of the other waves' arithmetic
+        __builtin_amdgcn_s_setprio(2);
+        if (has_next) {
+            const TileHead h = head_of(next_word);
+            if (next_slot + G < A.num_tiles) next_word = word_of(next_slot + G);
+            pair_fetch_ids<Real>(nxt, A, h, tid);
         }
+        __builtin_amdgcn_s_setprio(0);
+        if (tid < cur.np) {
+            int n[14];
+            Real AA[9], AB[9], SA[4][6], SB[4][6], qa, qb;
+            {
+                const unsigned w[6] = {cur.rec[0].x, cur.rec[0].y, cur.rec[1].x, cur.rec[1].y, cur.rec[2].x, cur.rec[2].y};
+#pragma unroll
+                for (int j = 0; j < 12; ++j) n[j] = (int)((w[j / 3] >> (10 * (j % 3))) & 1023u);
+                n[12] = (int)(w[4] & 1023u);
+                n[13] = (int)((w[4] >> 10) & 1023u);
+                double X[5][3];
+#pragma unroll
+                for (int v = 0; v < 5; ++v) {
+                    const int lv = v < 4 ? (int)((w[5] >> (8 * v)) & 255u) : (int)((w[4] >> 20) & 255u);
+#pragma unroll
+                    for (int d = 0; d < 3; ++d) X[v][d] = sX[3 * lv + d];
+                }
+                double Ad[9];
+                qa = (Real)(-A.scale / (30.0 * p2_adjugate(X, Ad)));
+#pragma unroll
+                for (int i = 0; i < 9; ++i) AA[i] = (Real)Ad[i];
+                const double XB[4][3] = {{X[4][0], X[4][1], X[4][2]}, {X[1][0], X[1][1], X[1][2]},
+                                         {X[3][0], X[3][1], X[3][2]}, {X[2][0], X[2][1], X[2][2]}};
+                qb = (Real)(-A.scale / (30.0 * p2_adjugate(XB, Ad)));
+#pragma unroll
+                for (int i = 0; i < 9; ++i) AB[i] = (Real)Ad[i];
+            }
+            p2_pair_strains<sizeof(Real) == 8, Real>([&](int c, int j) { return sU[3 * n[j] + c]; }, AA, AB, SA, SB);
+            p2_vertex_stresses<Real>(qa, cur.mat[0], cur.mat[1], SA);
+            p2_vertex_stresses<Real>(qb, cur.mat[2], cur.mat[3], SB);
+            p2_pair_contract<sizeof(Real) == 8, Real>(
+                SA, SB, AA, AB, [&](int c, int j, Real v) { atomicAdd(&sR[3 * n[j] + c], (double)v); });
+        }
+        __syncthreads();
+        __builtin_amdgcn_s_setprio(1);
+        if (has_next) pair_fetch_values<Real>(nxt, A, tid);
+        write_out<Real, double, kPairSlots, kPairThreads>(sR, cur.gn, cur.nn, cur.nown, cur.hoff, tid, r, halo, insert);
         __builtin_amdgcn_s_setprio(0);
         if (!has_next) break;
         __syncthreads();  // every read of this tile's LDS precedes the next tile's staging
@@ -593,14 +678,59 @@ static int resident_per_cu(const void *kernel, int nt, size_t lds, int fallback)
 }
 
 template <typename Real>
+static int reduce_shared(plx_dm dm, int n, const int32_t *node, const int32_t *ptr, const int32_t *slot,
+                         const void *halo, void *r, int mode, bool log) {
+    if (n == 0) return 0;
+    ScopedEvent ev(dm, log ? "plx:reduce_halo" : nullptr);
+    hipLaunchKernelGGL(reduce_halo<Real>, dim3((n + 255) / 256), dim3(256), 0, dm->stream, n, node, ptr, slot,
+                       static_cast<const Real *>(halo), static_cast<Real *>(r), mode);
+    PLX_HIP(dm, hipGetLastError());
+    return 0;
+}
+
+bool takes_pairs(plx_dm dm, const KeyPlan *kp) {
+    return kp->pairs.num_tiles > 0 && kp->pairs.d_mat64 && dm->algorithm != PLX_ALGO_QUADRATURE_POINTS &&
+           dm->accumulate != PLX_ACCUMULATE_COLORED && dm->min_waves <= 2;
+}
+
+template <typename Real>
+static int apply_pairs_typed(plx_dm dm, KeyPlan *kp, const void *u, void *r, int mode, double scale, void *halo,
+                             bool log) {
+    const PairDev &P = kp->pairs;
+    PairArgs A;
+    A.num_tiles = P.num_tiles;
+    A.heads = P.d_heads;
+    A.nodes = P.d_nodes;
+    A.verts = P.d_verts;
+    A.rec = reinterpret_cast<const uint2 *>(P.d_records);
+    A.mat = std::is_same<Real, double>::value ? (const void *)P.d_mat64 : (const void *)P.d_mat32;
+    A.coords = dm->d_coords;
+    A.u = u;
+    A.r = r;
+    A.halo = halo ? halo : kp->d_halo;
+    A.mode = mode;
+    A.scale = scale;
+    if (dm->num_cu <= 0) PLX_HIP(dm, hipDeviceGetAttribute(&dm->num_cu, hipDeviceAttributeMultiprocessorCount, 0));
+    const size_t lds = pair_lds_bytes<Real>();
+    const int per_cu = resident_per_cu(reinterpret_cast<const void *>(&apply_pairs<Real>), kPairThreads, lds, 2);
+    const int resident = ((std::max(dm->num_cu, 8) * per_cu + 7) / 8) * 8;
+    {
+        ScopedEvent ev(dm, log ? "plx:apply_tiles" : nullptr);
+        hipLaunchKernelGGL(apply_pairs<Real>, dim3(std::min(P.num_tiles, resident)), dim3(kPairThreads), lds, dm->stream, A);
+    }
+    PLX_HIP(dm, hipGetLastError());
+    return reduce_shared<Real>(dm, P.num_shared, P.d_shared_node, P.d_shared_ptr, P.d_shared_slot, A.halo, r, mode, log);
+}
+
+template <typename Real>
 static int apply_typed(plx_dm dm, KeyPlan *kp, const void *u, void *r, int mode, double scale,
                        const double *prestress, void *halo, bool log) {
+    if (!prestress && takes_pairs(dm, kp)) return apply_pairs_typed<Real>(dm, kp, u, r, mode, scale, halo, log);
     ApplyArgs A;
     A.scale = scale;
     A.prestress = prestress;
     A.p = plan_dev(dm, kp);
     A.color = kp->d_color;
-    A.tile_ncolor = kp->d_tile_ncolor;
     A.mat = std::is_same<Real, double>::value ? (const void *)kp->d_mat64 : (const void *)kp->d_mat32;
     A.u = u;
     A.r = r;
@@ -611,8 +741,6 @@ static int apply_typed(plx_dm dm, KeyPlan *kp, const void *u, void *r, int mode,
     const bool linear = dm->algorithm != PLX_ALGO_QUADRATURE_POINTS && !prestress;
     // AUTO: LDS atomics (FP64 accumulator, native ds_add_f64) for both vector types
     const bool atomic = dm->accumulate != PLX_ACCUMULATE_COLORED;
-    const size_t lds = (size_t)kp->max_verts * 3 * sizeof(double) +
-                       (size_t)kp->max_nodes * 3 * (sizeof(Real) + (atomic ? sizeof(double) : sizeof(Real)));
     // persistent grid: as many workgroups per CU as the kernel's registers and LDS let reside
     // (a multiple of 8 in all keeps each workgroup on the XCD whose tile range it walks), never
     // more than there are tiles
@@ -623,6 +751,8 @@ static int apply_typed(plx_dm dm, KeyPlan *kp, const void *u, void *r, int mode,
 #define PLX_LAUNCH_W(CT, PATH, ACC, W, N)                                                             \
     do {                                                                                             \
         const void *kfn = reinterpret_cast<const void *>(&apply_tiles<Real, CT, PATH, ACC, W>);       \
+        constexpr size_t lds =                                                                       \
+            tile_lds_bytes<Real, CT, typename std::conditional<ACC == kAccAtomic, double, Real>::type>(); \
         const int per_cu = resident_per_cu(kfn, Shape<CT, Real>::NT, lds, dm->wg_per_cu);            \
         const int resident = ((ncu * per_cu + 7) / 8) * 8;                                           \
         hipLaunchKernelGGL((apply_tiles<Real, CT, PATH, ACC, W>), dim3(std::min(N, resident)),         \
@@ -630,7 +760,7 @@ static int apply_typed(plx_dm dm, KeyPlan *kp, const void *u, void *r, int mode,
     } while (0)
 #define PLX_LAUNCH(CT, PATH, ACC, LIST, N)                                                           \
     do {                                                                                             \
-        A.tile_list = LIST;                                                                          \
+        A.heads = LIST;                                                                              \
         A.num_list = N;                                                                              \
         if (N > 0) {                                                                                 \
             if (minw <= 2) PLX_LAUNCH_W(CT, PATH, ACC, 2, N);                                          \
@@ -644,43 +774,36 @@ static int apply_typed(plx_dm dm, KeyPlan *kp, const void *u, void *r, int mode,
         // rest: the quadrature-point kernel with the Jacobian at each point
         if (linear) {
             if (atomic) {
-                PLX_LAUNCH(PLX_HEX_Q1, kPathFactored, kAccAtomic, kp->d_tiles_affine, kp->num_tiles_affine);
-                PLX_LAUNCH(PLX_HEX_Q1, kPathQpGeneral, kAccAtomic, kp->d_tiles_general, kp->num_tiles_general);
+                PLX_LAUNCH(PLX_HEX_Q1, kPathFactored, kAccAtomic, kp->d_heads_affine, kp->num_tiles_affine);
+                PLX_LAUNCH(PLX_HEX_Q1, kPathQpGeneral, kAccAtomic, kp->d_heads_general, kp->num_tiles_general);
             } else {
-                PLX_LAUNCH(PLX_HEX_Q1, kPathFactored, kAccColored, kp->d_tiles_affine, kp->num_tiles_affine);
-                PLX_LAUNCH(PLX_HEX_Q1, kPathQpGeneral, kAccColored, kp->d_tiles_general, kp->num_tiles_general);
+                PLX_LAUNCH(PLX_HEX_Q1, kPathFactored, kAccColored, kp->d_heads_affine, kp->num_tiles_affine);
+                PLX_LAUNCH(PLX_HEX_Q1, kPathQpGeneral, kAccColored, kp->d_heads_general, kp->num_tiles_general);
             }
         } else {
             if (atomic) {
-                PLX_LAUNCH(PLX_HEX_Q1, kPathQpAffine, kAccAtomic, kp->d_tiles_affine, kp->num_tiles_affine);
-                PLX_LAUNCH(PLX_HEX_Q1, kPathQpGeneral, kAccAtomic, kp->d_tiles_general, kp->num_tiles_general);
+                PLX_LAUNCH(PLX_HEX_Q1, kPathQpAffine, kAccAtomic, kp->d_heads_affine, kp->num_tiles_affine);
+                PLX_LAUNCH(PLX_HEX_Q1, kPathQpGeneral, kAccAtomic, kp->d_heads_general, kp->num_tiles_general);
             } else {
-                PLX_LAUNCH(PLX_HEX_Q1, kPathQpAffine, kAccColored, kp->d_tiles_affine, kp->num_tiles_affine);
-                PLX_LAUNCH(PLX_HEX_Q1, kPathQpGeneral, kAccColored, kp->d_tiles_general, kp->num_tiles_general);
+                PLX_LAUNCH(PLX_HEX_Q1, kPathQpAffine, kAccColored, kp->d_heads_affine, kp->num_tiles_affine);
+                PLX_LAUNCH(PLX_HEX_Q1, kPathQpGeneral, kAccColored, kp->d_heads_general, kp->num_tiles_general);
             }
         }
     } else {
         if (linear) {
-            if (atomic) PLX_LAUNCH(PLX_TET_P2, kPathFactored, kAccAtomic, nullptr, kp->num_tiles);
-            else PLX_LAUNCH(PLX_TET_P2, kPathFactored, kAccColored, nullptr, kp->num_tiles);
+            if (atomic) PLX_LAUNCH(PLX_TET_P2, kPathFactored, kAccAtomic, kp->d_heads, kp->num_tiles);
+            else PLX_LAUNCH(PLX_TET_P2, kPathFactored, kAccColored, kp->d_heads, kp->num_tiles);
         } else {
-            if (atomic) PLX_LAUNCH(PLX_TET_P2, kPathQpAffine, kAccAtomic, nullptr, kp->num_tiles);
-            else PLX_LAUNCH(PLX_TET_P2, kPathQpAffine, kAccColored, nullptr, kp->num_tiles);
+            if (atomic) PLX_LAUNCH(PLX_TET_P2, kPathQpAffine, kAccAtomic, kp->d_heads, kp->num_tiles);
+            else PLX_LAUNCH(PLX_TET_P2, kPathQpAffine, kAccColored, kp->d_heads, kp->num_tiles);
         }
     }
 #undef PLX_LAUNCH_W
 #undef PLX_LAUNCH
     }
     PLX_HIP(dm, hipGetLastError());
-    if (kp->num_shared > 0) {
-        ScopedEvent ev(dm, log ? "plx:reduce_halo" : nullptr);
-        hipLaunchKernelGGL(reduce_halo<Real>, dim3((kp->num_shared + 255) / 256), dim3(256), 0,
-                           dm->stream, kp->num_shared, kp->d_shared_node, kp->d_shared_ptr,
-                           kp->d_shared_slot, static_cast<const Real *>(A.halo),
-                           static_cast<Real *>(r), mode);
-        PLX_HIP(dm, hipGetLastError());
-    }
-    return 0;
+    return reduce_shared<Real>(dm, kp->num_shared, kp->d_shared_node, kp->d_shared_ptr, kp->d_shared_slot, A.halo, r, mode,
+                               log);
 }
 
 // Residual and Jacobian action share the element operator: for isotropic linear elasticity
@@ -899,7 +1022,7 @@ int plx_compute_residual_noalloc(plx_dm dm, int label_value, int part, int scala
     if (kp->pf_residual || !kp->f1)
         return set_error(dm, 1, "PetscPointFn-form keys are not served allocation-free: use plx_compute_residual");
     if (scalar_type != PLX_FP64 && scalar_type != PLX_FP32) return set_error(dm, 1, "bad scalar type");
-    const size_t need = (size_t)kp->halo_slots * 3 * (scalar_type == PLX_FP64 ? sizeof(double) : sizeof(float));
+    const size_t need = (size_t)(takes_pairs(dm, kp) ? kp->pairs.halo_slots : kp->halo_slots) * 3 * (scalar_type == PLX_FP64 ? sizeof(double) : sizeof(float));
     if (need > kScratchBytes)
         return set_error(dm, 1, "the key's shared-node partial sums (" + std::to_string(need) +
                                     " bytes) exceed the allocation-free scratch (" +

@@ -773,6 +773,52 @@ __host__ __device__ inline void p2_sym_contract(const Real S[4][6], const Real A
     }
 }
 
+// The two cells of a pair (PairPlan's 14 slots: U(c, j), emit(c, j, value)); the second cell's local
+// basis is slots 10, 1, 3, 2, 11, 13, 12, 8, 7, 9.
+template <bool PIN, typename Real, typename UAcc>
+__host__ __device__ inline void p2_pair_strains(const UAcc &U, const Real AA[9], const Real AB[9], Real SA[4][6],
+                                                Real SB[4][6]) {
+    Real u[14];
+#define PLX_PAIR_COMPONENT(C)                                                                               \
+    {                                                                                                       \
+        for (int j = 0; j < 14; ++j) u[j] = U(C, j);                                                        \
+        const Real ub[10] = {u[10], u[1], u[3], u[2], u[11], u[13], u[12], u[8], u[7], u[9]};               \
+        p2_strain_component<C, PIN, Real>(u, AA, SA);                                                       \
+        p2_strain_component<C, PIN, Real>(ub, AB, SB);                                                      \
+        if (PIN) schedule_barrier();                                                                        \
+    }
+    PLX_PAIR_COMPONENT(0)
+    PLX_PAIR_COMPONENT(1)
+    PLX_PAIR_COMPONENT(2)
+#undef PLX_PAIR_COMPONENT
+}
+
+template <bool PIN, typename Real, typename Emit>
+__host__ __device__ inline void p2_pair_contract(const Real SA[4][6], const Real SB[4][6], const Real AA[9],
+                                                 const Real AB[9], const Emit &emit) {
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        Real a[10], b[10];
+        p2_contract_component<Real>(c, SA, AA, a);
+        emit(c, 0, a[0]);
+        emit(c, 4, a[4]);
+        emit(c, 5, a[5]);
+        emit(c, 6, a[6]);
+        p2_contract_component<Real>(c, SB, AB, b);
+        emit(c, 1, a[1] + b[1]);
+        emit(c, 2, a[2] + b[3]);
+        emit(c, 3, a[3] + b[2]);
+        emit(c, 7, a[7] + b[8]);
+        emit(c, 8, a[8] + b[7]);
+        emit(c, 9, a[9] + b[9]);
+        emit(c, 10, b[0]);
+        emit(c, 11, b[4]);
+        emit(c, 12, b[6]);
+        emit(c, 13, b[5]);
+        if (PIN) schedule_barrier();
+    }
+}
+
 // Factorized through the P1 structure of the gradient: stresses at the four vertices and the exact
 // moments of the barycentric coordinates in place of the points.
 template <typename Real, typename UAcc, typename Emit>

@@ -165,6 +165,94 @@ int emulate(const plx::MeshView &mv, const double *coords, const plx::HostPlan &
     return 0;
 }
 
+// The pair kernel (apply_pairs + reduce_halo) over the pair plan; also checks that every cell of
+// the key is in exactly one pair.
+template <typename Real>
+int emulate_pairs(const plx::MeshView &mv, const double *coords, const plx::HostPlan &hp, const plx::PairPlan &pp,
+                  const double *lam_mu, const Real *u, Real *r, int mode) {
+    std::vector<double> halo(3 * (size_t)pp.halo_slots);
+    std::vector<int> seen(mv.num_cells, 0);
+    CHECK(pp.halo_slots <= hp.halo_slots);
+    CHECK((int)pp.tile_pair_ptr.size() == pp.num_tiles + 1 && pp.tile_pair_ptr.back() == pp.num_pairs);
+    for (int slot = 0; slot < pp.num_tiles; ++slot) {
+        const int tile = xcd_tile(slot, pp.num_tiles);
+        const int p0 = pp.tile_pair_ptr[tile], np = pp.tile_pair_ptr[tile + 1] - p0;
+        const int n0 = pp.tile_node_ptr[tile], nn = pp.tile_node_ptr[tile + 1] - n0;
+        const int v0 = pp.tile_vert_ptr[tile], nvt = pp.tile_vert_ptr[tile + 1] - v0;
+        CHECK(np >= 1 && np <= plx::kPairTilePairs && nn >= 1 && nn <= plx::kPairTileNodes);
+        CHECK(nvt >= 1 && nvt <= plx::kPairTileVerts && pp.tile_nown[tile] <= nn);
+        std::vector<Real> sU(3 * (size_t)nn);
+        std::vector<double> sX(3 * (size_t)nvt), sR(3 * (size_t)nn, 0.0);
+        for (int k = 0; k < nn; ++k) {
+            const int g = pp.tile_nodes[n0 + k];
+            CHECK(g >= 0 && g < mv.num_nodes);
+            for (int c = 0; c < 3; ++c) sU[3 * k + c] = u[3 * (size_t)g + c];
+        }
+        for (int k = 0; k < nvt; ++k) {
+            const int g = pp.tile_verts[v0 + k];
+            CHECK(g >= 0 && g < mv.num_vertices);
+            for (int d = 0; d < 3; ++d) sX[3 * k + d] = coords[3 * (size_t)g + d];
+        }
+        for (int i = 0; i < np; ++i) {
+            const uint32_t *w = &pp.records[6 * (size_t)(p0 + i)];
+            int n[14];
+            double X[5][3];
+            for (int j = 0; j < 14; ++j) CHECK((n[j] = plx::pair_node(w, j)) < nn);
+            for (int j = 0; j < 5; ++j) {
+                const int v = plx::pair_vert(w, j);
+                CHECK(v < nvt);
+                for (int d = 0; d < 3; ++d) X[j][d] = sX[3 * v + d];
+            }
+            double m[4] = {0.0, 0.0, 0.0, 0.0};
+            for (int k = 0; k < 2; ++k) {
+                const int32_t cell = pp.cells[2 * (size_t)(p0 + i) + k];
+                CHECK(k == 1 || cell >= 0);
+                if (cell < 0) continue;
+                CHECK(cell < mv.num_cells);
+                ++seen[cell];
+                m[2 * k] = lam_mu[2 * (size_t)cell];
+                m[2 * k + 1] = lam_mu[2 * (size_t)cell + 1];
+            }
+            double Ad[9];
+            Real AA[9], AB[9], SA[4][6], SB[4][6];
+            const double da = plx::p2_adjugate(X, Ad);
+            for (int k = 0; k < 9; ++k) AA[k] = (Real)Ad[k];
+            const double XB[4][3] = {{X[4][0], X[4][1], X[4][2]}, {X[1][0], X[1][1], X[1][2]},
+                                     {X[3][0], X[3][1], X[3][2]}, {X[2][0], X[2][1], X[2][2]}};
+            const double db = plx::p2_adjugate(XB, Ad);
+            for (int k = 0; k < 9; ++k) AB[k] = (Real)Ad[k];
+            plx::p2_pair_strains<false, Real>([&](int c, int j) { return sU[3 * n[j] + c]; }, AA, AB, SA, SB);
+            plx::p2_vertex_stresses<Real>((Real)(-1.0 / (30.0 * da)), (Real)m[0], (Real)m[1], SA);
+            plx::p2_vertex_stresses<Real>((Real)(-1.0 / (30.0 * db)), (Real)m[2], (Real)m[3], SB);
+            plx::p2_pair_contract<false, Real>(SA, SB, AA, AB,
+                                               [&](int c, int j, Real v) { sR[3 * n[j] + c] += (double)v; });
+        }
+        for (int k = 0; k < nn; ++k) {
+            const size_t g = (size_t)pp.tile_nodes[n0 + k], h = (size_t)pp.tile_halo_off[tile] + (size_t)(k - pp.tile_nown[tile]);
+            for (int c = 0; c < 3; ++c) {
+                if (k < pp.tile_nown[tile])
+                    r[3 * g + c] = (Real)sR[3 * k + c] + (mode == PLX_INSERT_VALUES ? Real(0) : r[3 * g + c]);
+                else {
+                    CHECK((int64_t)h < pp.halo_slots);
+                    halo[3 * h + c] = (Real)sR[3 * k + c];
+                }
+            }
+        }
+    }
+    for (size_t s = 0; s < pp.shared_node.size(); ++s)
+        for (int c = 0; c < 3; ++c) {
+            Real a = 0;
+            for (int j = pp.shared_ptr[s]; j < pp.shared_ptr[s + 1]; ++j) {
+                CHECK(pp.shared_slot[j] >= 0 && pp.shared_slot[j] < pp.halo_slots);
+                a += (Real)halo[3 * (size_t)pp.shared_slot[j] + c];
+            }
+            const size_t g = 3 * (size_t)pp.shared_node[s] + c;
+            r[g] = a + (mode == PLX_INSERT_VALUES ? Real(0) : r[g]);
+        }
+    for (int32_t c : hp.cells) CHECK(seen[c] == 1);
+    return 0;
+}
+
 }  // namespace
 
 extern "C" int plx_debug_emulate_apply(int cell_type, int num_cells, int num_vertices,
@@ -184,6 +272,13 @@ extern "C" int plx_debug_emulate_apply(int cell_type, int num_cells, int num_ver
     plx::HostPlan hp;
     std::string msg;
     if (plx::build_host_plan(mv, label_value, plx::tile_limits(cell_type), &hp, &msg)) return 1;
+    if (algorithm == PLX_EMULATE_PAIRS) {
+        plx::PairPlan pp;
+        if (cell_type != PLX_TET_P2 || plx::build_pair_plan(mv, hp, &pp, &msg)) return 1;
+        if (scalar_type == PLX_FP64)
+            return emulate_pairs<double>(mv, coords, hp, pp, lam_mu, (const double *)u, (double *)r, mode);
+        return emulate_pairs<float>(mv, coords, hp, pp, lam_mu, (const float *)u, (float *)r, mode);
+    }
     if (scalar_type == PLX_FP64)
         return emulate<double>(mv, coords, hp, lam_mu, (const double *)u, (double *)r, mode, cell_type,
                                algorithm != PLX_ALGO_QUADRATURE_POINTS);

@@ -26,6 +26,13 @@ namespace plx {
 constexpr int kMaxQuad = 14;
 
 // Device-side arrays of one key's tile plan (passed by value to kernels).
+// Extents of one tile for the tile kernels: cells (or pairs) c0 .. c0 + nc (the colour count in nc's
+// upper half), its nn nodes from n0 (nown owned ones first) and nvt vertices from v0 in the tile
+// lists, first halo slot hoff.
+struct TileHead {
+    int32_t c0, nc, n0, nn, v0, nvt, nown, hoff;
+};
+
 struct TilePlanDev {
     int num_tiles;
     int stride;                      // SoA stride of per-cell arrays (= number of key cells)
@@ -39,6 +46,20 @@ struct TilePlanDev {
     const uint16_t *lclosure;        // [nb][stride] tile-local node index
     const uint16_t *lcone;           // [nv][stride] tile-local vertex index
     const double *coords;            // [num_vertices][3]
+};
+
+// Device arrays of a key's pair plan (PairPlan; num_tiles = 0: none).  Its halo partials share the
+// key's halo buffer (the pair plan has no more halo slots than the tile plan).
+struct PairDev {
+    int num_tiles = 0, num_pairs = 0, num_shared = 0;
+    int64_t halo_slots = 0;
+    std::vector<int32_t> cells;      // [num_pairs][2] mesh cells (-1: none)
+    int32_t *d_heads = nullptr;      // TileHead of each tile (pairs in place of cells)
+    int32_t *d_nodes = nullptr, *d_verts = nullptr;
+    int32_t *d_shared_node = nullptr, *d_shared_ptr = nullptr, *d_shared_slot = nullptr;
+    uint32_t *d_records = nullptr;   // [num_pairs][6]
+    double *d_mat64 = nullptr;       // [num_pairs][4] lambda, mu of the two cells
+    float *d_mat32 = nullptr;
 };
 
 struct KeyPlan {
@@ -60,11 +81,12 @@ struct KeyPlan {
     uint16_t *d_lclosure = nullptr, *d_lcone = nullptr;
     uint16_t *d_records = nullptr;   // [ncells][8 or 16] packed local closure (+ cone) per cell
     uint8_t *d_color = nullptr;      // [ncells] colour within the tile (cells sorted by colour)
-    int32_t *d_tile_ncolor = nullptr;
+    int32_t *d_heads = nullptr;      // TileHead of each tile
     int max_colors = 0;
     bool sorted_by_color = true;
-    int32_t *d_tiles_affine = nullptr, *d_tiles_general = nullptr;  // Q1: tiles of affine cells / others
+    int32_t *d_heads_affine = nullptr, *d_heads_general = nullptr;  // Q1: those of affine cells / the others
     int num_tiles_affine = 0, num_tiles_general = 0;
+    PairDev pairs;                   // P2: the factored path with LDS atomics
     int32_t *d_shared_node = nullptr, *d_shared_ptr = nullptr, *d_shared_slot = nullptr;
     void *d_halo = nullptr;          // halo partial sums, sized for FP64
     // auxiliary field, repacked per key cell (SoA, tile order)
@@ -222,6 +244,7 @@ void pointfn_release(plx_dm dm, KeyPlan *kp);
 // kernels' event timers when the handle's logging is on
 int launch_apply(plx_dm dm, KeyPlan *kp, int scalar_type, bool jacobian, const void *u,
                  void *r, int mode, double scale = 1.0, void *halo = nullptr, bool log = true);
+bool takes_pairs(plx_dm dm, const KeyPlan *kp);  // whether the factored apply runs over the pair plan
 // Per-device set-up at plx_dm_create with the DM's device current: the element tables in
 // constant memory and the device address of the allocation-free entry point's scratch array.
 int device_setup(plx_dm dm);

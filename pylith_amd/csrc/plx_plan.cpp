@@ -8,6 +8,7 @@
 #include <algorithm>
 #include <array>
 #include <cmath>
+#include <thread>
 
 #include "plx_plan.hpp"
 
@@ -48,6 +49,40 @@ std::vector<int32_t> morton_permutation(const double *xyz, size_t n) {
     std::vector<int32_t> out(n);
     for (size_t i = 0; i < n; ++i) out[i] = key[i].second;
     return out;
+}
+
+// body(i) for i in [0, n) on host threads, in contiguous ranges.
+template <typename F>
+static void parallel_for(int n, const F &body) {
+    const int nt = std::max(1, std::min({(int)std::thread::hardware_concurrency(), 16, n / 64 + 1}));
+    if (nt == 1) {
+        for (int i = 0; i < n; ++i) body(i);
+        return;
+    }
+    std::vector<std::thread> th;
+    for (int t = 0; t < nt; ++t)
+        th.emplace_back([&, t] {
+            for (int i = (int)((int64_t)n * t / nt); i < (int)((int64_t)n * (t + 1) / nt); ++i) body(i);
+        });
+    for (auto &x : th) x.join();
+}
+
+static int distinct(std::vector<int32_t> &v) {
+    std::sort(v.begin(), v.end());
+    v.erase(std::unique(v.begin(), v.end()), v.end());
+    return (int)v.size();
+}
+
+// Nodes that several tiles touch, ascending, and the ranges of their halo slots (empty: none).
+static void shared_map(int num_nodes, const std::vector<int32_t> &tile_count, std::vector<int32_t> &node,
+                       std::vector<int32_t> &ptr) {
+    node.clear();
+    ptr.assign(1, 0);
+    for (int i = 0; i < num_nodes; ++i)
+        if (tile_count[i] > 1) {
+            node.push_back(i);
+            ptr.push_back(ptr.back() + tile_count[i]);
+        }
 }
 
 // The cells in Morton order of their centroids.
@@ -227,149 +262,133 @@ static int plan_cells(const MeshView &m, const TileLimits &lim, HostPlan *hp, st
     const int ntiles = (int)tile_cell_ptr.size() - 1;
     hp->num_tiles = ntiles;
 
-    // How many tiles touch each node.
-    std::vector<int32_t> tile_count(m.num_nodes, 0);
-    std::fill(node_mark.begin(), node_mark.end(), -1);
-    for (int t = 0; t < ntiles; ++t)
-        for (int i = tile_cell_ptr[t]; i < tile_cell_ptr[t + 1]; ++i) {
-            const int32_t *cl = m.closure + (size_t)cells[i] * nb;
-            for (int b = 0; b < nb; ++b)
-                if (node_mark[cl[b]] != t) {
-                    node_mark[cl[b]] = t;
-                    ++tile_count[cl[b]];
-                }
-        }
-
-    // Greedy colouring inside each tile, then cells sorted by colour.
+    // Each tile by itself, on host threads: its sorted nodes, colouring, node and vertex lists, local
+    // closures; then the tiles one after another.
+    struct Tile {
+        std::vector<int32_t> nodes, own, ids, verts;  // sorted nodes; owned ones; local order (owned, shared); vertices
+        int ncolor = 0;
+    };
+    std::vector<Tile> tiles(ntiles);
+    parallel_for(ntiles, [&](int t) {
+        std::vector<int32_t> &v = tiles[t].nodes;
+        for (int i = tile_cell_ptr[t]; i < tile_cell_ptr[t + 1]; ++i)
+            v.insert(v.end(), m.closure + (size_t)cells[i] * nb, m.closure + (size_t)(cells[i] + 1) * nb);
+        distinct(v);
+    });
+    std::vector<int32_t> tile_count(m.num_nodes, 0);  // how many tiles touch each node
+    for (const Tile &T : tiles)
+        for (int32_t x : T.nodes) ++tile_count[x];
     hp->color.assign(ncells, 0);
-    hp->tile_ncolor.assign(ntiles, 0);
-    hp->max_colors = 0;
-    {
-        std::vector<uint64_t> used(2 * (size_t)m.num_nodes, 0);
-        std::vector<std::pair<int, int32_t>> order;
-        for (int t = 0; t < ntiles; ++t) {
-            const int b0 = tile_cell_ptr[t], b1 = tile_cell_ptr[t + 1];
-            order.clear();
-            int nc = 0;
-            for (int i = b0; i < b1; ++i) {
-                const int32_t *cl = m.closure + (size_t)cells[i] * nb;
-                uint64_t m0 = 0, m1 = 0;
-                for (int b = 0; b < nb; ++b) {
-                    m0 |= used[2 * (size_t)cl[b]];
-                    m1 |= used[2 * (size_t)cl[b] + 1];
-                }
-                int c = 0;
-                while (c < 128 && ((c < 64 ? (m0 >> c) : (m1 >> (c - 64))) & 1)) ++c;
-                if (c >= 128) {
-                    *err = "tile colouring needs more than 128 colours";
-                    return 1;
-                }
-                for (int b = 0; b < nb; ++b)
-                    used[2 * (size_t)cl[b] + (c >> 6)] |= (uint64_t)1 << (c & 63);
-                order.emplace_back(c, cells[i]);
-                nc = std::max(nc, c + 1);
+    hp->lclosure.assign((size_t)nb * ncells, 0);
+    hp->lcone.assign((size_t)nv * ncells, 0);
+    std::vector<char> too_many(ntiles, 0);
+    parallel_for(ntiles, [&](int t) {
+        Tile &T = tiles[t];
+        const int c0 = tile_cell_ptr[t], tc = tile_cell_ptr[t + 1] - c0;
+        auto local = [](const std::vector<int32_t> &v, int32_t x) {
+            return (int32_t)(std::lower_bound(v.begin(), v.end(), x) - v.begin());
+        };
+        // greedy colouring, then cells sorted by colour
+        std::vector<int32_t> lc((size_t)tc * nb);  // sorted position of each closure node
+        for (int i = 0; i < tc; ++i)
+            for (int b = 0; b < nb; ++b) lc[(size_t)i * nb + b] = local(T.nodes, m.closure[(size_t)cells[c0 + i] * nb + b]);
+        std::vector<std::array<uint64_t, 2>> used(T.nodes.size(), {0, 0});
+        std::vector<std::pair<int, int32_t>> order;  // colour, cell of the tile
+        for (int i = 0; i < tc; ++i) {
+            uint64_t m0 = 0, m1 = 0;
+            for (int b = 0; b < nb; ++b) {
+                m0 |= used[lc[(size_t)i * nb + b]][0];
+                m1 |= used[lc[(size_t)i * nb + b]][1];
             }
-            for (int i = b0; i < b1; ++i) {
-                const int32_t *cl = m.closure + (size_t)cells[i] * nb;
-                for (int b = 0; b < nb; ++b) used[2 * (size_t)cl[b]] = used[2 * (size_t)cl[b] + 1] = 0;
+            int c = 0;
+            while (c < 128 && ((c < 64 ? (m0 >> c) : (m1 >> (c - 64))) & 1)) ++c;
+            if (c >= 128) {
+                too_many[t] = 1;
+                return;
             }
-            if (sort_by_color)
-                std::stable_sort(order.begin(), order.end(),
-                                 [](const std::pair<int, int32_t> &a, const std::pair<int, int32_t> &b) {
-                                     return a.first < b.first;
-                                 });
-            for (int i = b0; i < b1; ++i) {
-                hp->color[i] = (uint8_t)order[i - b0].first;
-                cells[i] = order[i - b0].second;
-            }
-            hp->tile_ncolor[t] = nc;
-            hp->max_colors = std::max(hp->max_colors, nc);
+            for (int b = 0; b < nb; ++b) used[lc[(size_t)i * nb + b]][c >> 6] |= (uint64_t)1 << (c & 63);
+            order.emplace_back(c, i);
+            T.ncolor = std::max(T.ncolor, c + 1);
         }
-    }
-
-    // Per-tile node / vertex lists and local closures.
+        if (sort_by_color)
+            std::stable_sort(order.begin(), order.end(),
+                             [](const std::pair<int, int32_t> &a, const std::pair<int, int32_t> &b) {
+                                 return a.first < b.first;
+                             });
+        {
+            std::vector<int32_t> sorted(tc), lsorted(lc.size());
+            for (int i = 0; i < tc; ++i) {
+                hp->color[c0 + i] = (uint8_t)order[i].first;
+                sorted[i] = cells[c0 + order[i].second];
+                std::copy_n(&lc[(size_t)order[i].second * nb], nb, &lsorted[(size_t)i * nb]);
+            }
+            std::copy(sorted.begin(), sorted.end(), cells.begin() + c0);
+            lc.swap(lsorted);
+        }
+        // local numbering: owned nodes, then shared ones.  Colour-sorted tiles put scattered cells in
+        // each half-wave: their owned nodes are numbered for LDS bank balance around the shared
+        // ones, which keep node order (the halo reduction reads their partials in node order).
+        // Tiles in mesh order keep node order: neighbouring lanes already touch spread-out banks.
+        std::vector<int32_t> sh;
+        for (int32_t x : T.nodes) (tile_count[x] == 1 ? T.own : sh).push_back(x);
+        T.ids = T.own;
+        T.ids.insert(T.ids.end(), sh.begin(), sh.end());
+        std::vector<int32_t> rank(T.ids.size());  // sorted position -> local index
+        auto ranks = [&] {
+            for (size_t k = 0; k < T.ids.size(); ++k) rank[local(T.nodes, T.ids[k])] = (int32_t)k;
+        };
+        ranks();
+        if (sort_by_color) {
+            std::vector<std::vector<int32_t>> slot(nb, std::vector<int32_t>(tc));
+            for (int i = 0; i < tc; ++i)
+                for (int b = 0; b < nb; ++b) slot[b][i] = rank[lc[(size_t)i * nb + b]];
+            balance_banks(T.ids, {0, (int)T.own.size(), (int)T.ids.size()}, slot, tc, kFixShared);
+            ranks();
+        }
+        for (int i = 0; i < tc; ++i)
+            for (int b = 0; b < nb; ++b) hp->lclosure[(size_t)b * ncells + c0 + i] = (uint16_t)rank[lc[(size_t)i * nb + b]];
+        if (m.cone_is_closure) return;
+        std::vector<int32_t> vs;
+        for (int i = 0; i < tc; ++i)
+            vs.insert(vs.end(), m.cone + (size_t)cells[c0 + i] * nv, m.cone + (size_t)(cells[c0 + i] + 1) * nv);
+        distinct(vs);
+        T.verts = vs;
+        std::vector<std::vector<int32_t>> slot(nv, std::vector<int32_t>(tc));
+        for (int i = 0; i < tc; ++i)
+            for (int b = 0; b < nv; ++b) slot[b][i] = local(vs, m.cone[(size_t)cells[c0 + i] * nv + b]);
+        if (sort_by_color && vs.size() > 16) balance_banks(T.verts, {0, (int)vs.size()}, slot, tc);
+        std::vector<int32_t> vrank(vs.size());
+        for (size_t k = 0; k < vs.size(); ++k) vrank[local(vs, T.verts[k])] = (int32_t)k;
+        for (int i = 0; i < tc; ++i)
+            for (int b = 0; b < nv; ++b) hp->lcone[(size_t)b * ncells + c0 + i] = (uint16_t)vrank[slot[b][i]];
+    });
+    hp->tile_ncolor.clear();
+    hp->max_colors = 0;
     hp->tile_node_ptr.assign(1, 0);
     hp->tile_vert_ptr.assign(1, 0);
     hp->tile_nown.clear();
     hp->tile_nodes.clear();
     hp->tile_verts.clear();
     hp->tile_halo_off.clear();
-    hp->lclosure.assign((size_t)nb * ncells, 0);
-    hp->lcone.assign((size_t)nv * ncells, 0);
-    std::vector<int32_t> local_of(m.num_nodes, -1), vlocal_of(m.num_vertices, -1);
-    std::vector<std::pair<int32_t, int32_t>> shared_pairs;  // (node, halo slot)
     int64_t halo = 0;
     int max_nodes = 0, max_verts = 0;
-    std::vector<int32_t> own, sh, vl;
     for (int t = 0; t < ntiles; ++t) {
-        own.clear();
-        sh.clear();
-        vl.clear();
-        for (int i = tile_cell_ptr[t]; i < tile_cell_ptr[t + 1]; ++i) {
-            const int32_t *cl = m.closure + (size_t)cells[i] * nb;
-            const int32_t *cn = m.cone + (size_t)cells[i] * nv;
-            for (int b = 0; b < nb; ++b)
-                if (local_of[cl[b]] == -1) {
-                    local_of[cl[b]] = 0;
-                    (tile_count[cl[b]] == 1 ? own : sh).push_back(cl[b]);
-                }
-            for (int b = 0; b < nv; ++b)
-                if (vlocal_of[cn[b]] == -1) {
-                    vlocal_of[cn[b]] = 0;
-                    vl.push_back(cn[b]);
-                }
+        if (too_many[t]) {
+            *err = "tile colouring needs more than 128 colours";
+            return 1;
         }
-        std::sort(own.begin(), own.end());
-        std::sort(sh.begin(), sh.end());
-        std::sort(vl.begin(), vl.end());
-        const int c0 = tile_cell_ptr[t], tc = tile_cell_ptr[t + 1] - c0;
-        // local numbering: owned nodes, then shared ones.  Colour-sorted tiles put scattered cells in
-        // each half-wave: their owned nodes are numbered for LDS bank balance around the shared
-        // ones, which keep node order (the halo reduction reads their partials in node order).
-        // Tiles in mesh order keep node order: neighbouring lanes already touch spread-out banks.
-        std::vector<int32_t> ids(own);
-        ids.insert(ids.end(), sh.begin(), sh.end());
-        if (sort_by_color) {
-            for (size_t q = 0; q < ids.size(); ++q) local_of[ids[q]] = (int32_t)q;
-            std::vector<std::vector<int32_t>> slot(nb, std::vector<int32_t>(tc));
-            for (int i = 0; i < tc; ++i)
-                for (int b = 0; b < nb; ++b) slot[b][i] = local_of[m.closure[(size_t)cells[c0 + i] * nb + b]];
-            balance_banks(ids, {0, (int)own.size(), (int)ids.size()}, slot, tc, kFixShared);
-        }
-        if (sort_by_color && !m.cone_is_closure && vl.size() > 16) {
-            for (size_t q = 0; q < vl.size(); ++q) vlocal_of[vl[q]] = (int32_t)q;
-            std::vector<std::vector<int32_t>> slot(nv, std::vector<int32_t>(tc));
-            for (int i = 0; i < tc; ++i)
-                for (int b = 0; b < nv; ++b) slot[b][i] = vlocal_of[m.cone[(size_t)cells[c0 + i] * nv + b]];
-            balance_banks(vl, {0, (int)vl.size()}, slot, tc);
-        }
-        int k = 0;
-        for (int32_t n : ids) {
-            if (k >= (int)own.size()) shared_pairs.emplace_back(n, (int32_t)(halo + (k - (int)own.size())));
-            local_of[n] = k++;
-            hp->tile_nodes.push_back(n);
-        }
-        hp->tile_nown.push_back((int32_t)own.size());
+        const Tile &T = tiles[t];
+        hp->tile_ncolor.push_back(T.ncolor);
+        hp->max_colors = std::max(hp->max_colors, T.ncolor);
+        hp->tile_nown.push_back((int32_t)T.own.size());
         hp->tile_halo_off.push_back((int32_t)halo);
-        halo += (int64_t)sh.size();
+        halo += (int64_t)(T.ids.size() - T.own.size());
+        hp->tile_nodes.insert(hp->tile_nodes.end(), T.ids.begin(), T.ids.end());
+        hp->tile_verts.insert(hp->tile_verts.end(), T.verts.begin(), T.verts.end());
         hp->tile_node_ptr.push_back((int32_t)hp->tile_nodes.size());
-        int kv = 0;
-        for (int32_t v : vl) {
-            vlocal_of[v] = kv++;
-            hp->tile_verts.push_back(v);
-        }
         hp->tile_vert_ptr.push_back((int32_t)hp->tile_verts.size());
-        max_nodes = std::max(max_nodes, k);
-        max_verts = std::max(max_verts, kv);
-        for (int i = tile_cell_ptr[t]; i < tile_cell_ptr[t + 1]; ++i) {
-            const int32_t *cl = m.closure + (size_t)cells[i] * nb;
-            const int32_t *cn = m.cone + (size_t)cells[i] * nv;
-            for (int b = 0; b < nb; ++b) hp->lclosure[(size_t)b * ncells + i] = (uint16_t)local_of[cl[b]];
-            for (int b = 0; b < nv; ++b) hp->lcone[(size_t)b * ncells + i] = (uint16_t)vlocal_of[cn[b]];
-        }
-        for (int32_t n : own) local_of[n] = -1;
-        for (int32_t n : sh) local_of[n] = -1;
-        for (int32_t v : vl) vlocal_of[v] = -1;
+        max_nodes = std::max(max_nodes, (int)T.ids.size());
+        max_verts = std::max(max_verts, (int)T.verts.size());
     }
     if (m.cone_is_closure) {
         hp->tile_verts = hp->tile_nodes;
@@ -385,22 +404,343 @@ static int plan_cells(const MeshView &m, const TileLimits &lim, HostPlan *hp, st
     hp->max_nodes = max_nodes;
     hp->max_verts = max_verts;
 
-    // Shared-node reduction map: nodes ascending, slots in tile order (stable sort).
-    std::stable_sort(shared_pairs.begin(), shared_pairs.end(),
-                     [](const std::pair<int32_t, int32_t> &a, const std::pair<int32_t, int32_t> &b) {
-                         return a.first < b.first;
-                     });
-    hp->shared_node.clear();
-    hp->shared_slot.clear();
-    hp->shared_ptr.assign(1, 0);
-    for (size_t i = 0; i < shared_pairs.size(); ++i) {
-        if (i > 0 && shared_pairs[i].first != shared_pairs[i - 1].first)
-            hp->shared_ptr.push_back((int32_t)i);
-        if (i == 0 || shared_pairs[i].first != shared_pairs[i - 1].first)
-            hp->shared_node.push_back(shared_pairs[i].first);
-        hp->shared_slot.push_back(shared_pairs[i].second);
+    // Shared-node reduction map: nodes ascending, slots in tile order.
+    shared_map(m.num_nodes, tile_count, hp->shared_node, hp->shared_ptr);
+    std::vector<int32_t> place(m.num_nodes, -1);
+    for (size_t i = 0; i < hp->shared_node.size(); ++i) place[hp->shared_node[i]] = hp->shared_ptr[i];
+    hp->shared_slot.resize((size_t)halo);
+    int32_t slot = 0;
+    for (const Tile &T : tiles)
+        for (size_t k = T.own.size(); k < T.ids.size(); ++k) hp->shared_slot[place[T.ids[k]]++] = slot++;
+    return 0;
+}
+
+// --------------------------------------------------------------------------------------------
+// Pair plan.
+// --------------------------------------------------------------------------------------------
+
+// Cells order[0 .. n) cut into tiles by recursive bisection of their centroids along the longest
+// axis; tile sizes are appended to `sizes` in order.  A cut may move by a sixteenth of its range
+// to the widest gap between centroids there: between layers of cells where the mesh has them.
+static void bisect(const MeshView &m, const std::vector<double> &cen, int32_t *order, int n, std::vector<int32_t> &sizes,
+                   int depth) {
+    const int most = 2 * kPairTilePairs;
+    if (n <= most) {
+        std::vector<int32_t> nodes, verts;
+        nodes.reserve((size_t)n * m.nb);
+        verts.reserve((size_t)n * m.nv);
+        for (int i = 0; i < n; ++i) {
+            const int32_t c = order[i];
+            nodes.insert(nodes.end(), m.closure + (size_t)c * m.nb, m.closure + (size_t)(c + 1) * m.nb);
+            verts.insert(verts.end(), m.cone + (size_t)c * m.nv, m.cone + (size_t)(c + 1) * m.nv);
+        }
+        if (n == 1 || (distinct(nodes) <= kPairTileNodes && distinct(verts) <= kPairTileVerts)) {
+            sizes.push_back(n);
+            return;
+        }
     }
-    if (!shared_pairs.empty()) hp->shared_ptr.push_back((int32_t)shared_pairs.size());
+    double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
+    for (int i = 0; i < n; ++i)
+        for (int d = 0; d < 3; ++d) {
+            lo[d] = std::min(lo[d], cen[3 * (size_t)order[i] + d]);
+            hi[d] = std::max(hi[d], cen[3 * (size_t)order[i] + d]);
+        }
+    int ax = 0;
+    for (int d = 1; d < 3; ++d)
+        if (hi[d] - lo[d] > hi[ax] - lo[ax]) ax = d;
+    auto less = [&](int32_t a, int32_t b) {
+        const double x = cen[3 * (size_t)a + ax], y = cen[3 * (size_t)b + ax];
+        return x < y || (x == y && a < b);
+    };
+    // two parts holding whole numbers of nearly full tiles (15 / 16 of the bound)
+    const int tiles = std::max(2, (n + most * 15 / 16 - 1) / (most * 15 / 16));
+    const int ideal = std::min(n - 1, std::max(1, (int)((int64_t)n * (tiles / 2) / tiles)));
+    const int w = n / 16;
+    const int a = std::max(1, ideal - w), b = std::min(n - 1, ideal + w);
+    std::nth_element(order, order + a, order + n, less);
+    if (b > a) std::nth_element(order + a, order + b, order + n, less);
+    std::sort(order + a, order + b, less);
+    int cut = ideal;
+    double widest = 0.0;
+    for (int i = a; i <= b; ++i) {
+        if (i > a && i >= b && b == a) break;
+        const double below = i == a ? -1e300 : cen[3 * (size_t)order[i - 1] + ax];
+        const double gap = i == a ? 0.0 : cen[3 * (size_t)order[i] + ax] - below;
+        if (gap > 1.001 * widest || (gap > 0.999 * widest && std::abs(i - ideal) < std::abs(cut - ideal) && gap > 0.0)) {
+            widest = std::max(widest, gap);
+            cut = i;
+        }
+    }
+    if (depth < 3) {
+        std::vector<int32_t> right;
+        std::thread t([&] { bisect(m, cen, order + cut, n - cut, right, depth + 1); });
+        bisect(m, cen, order, cut, sizes, depth + 1);
+        t.join();
+        sizes.insert(sizes.end(), right.begin(), right.end());
+    } else {
+        bisect(m, cen, order, cut, sizes, depth + 1);
+        bisect(m, cen, order + cut, n - cut, sizes, depth + 1);
+    }
+}
+
+namespace {
+struct PairTile {
+    std::vector<int32_t> nodes;  // sorted distinct, then in local order (owned, shared)
+    std::vector<int32_t> verts;
+    int nown = 0;
+    std::vector<int32_t> cells;  // [pairs][2]
+    std::vector<uint32_t> rec;
+};
+}  // namespace
+
+// Pairs, numbering and records of one tile (cells ids[0 .. n); T.nodes its sorted nodes).
+static void build_pair_tile(const MeshView &m, const int32_t *ids, int n, const std::vector<int32_t> &tile_count,
+                            PairTile &T) {
+    auto local = [](const std::vector<int32_t> &v, int32_t x) {
+        return (int)(std::lower_bound(v.begin(), v.end(), x) - v.begin());
+    };
+    std::vector<int32_t> verts;
+    for (int i = 0; i < n; ++i) verts.insert(verts.end(), m.cone + 4 * (size_t)ids[i], m.cone + 4 * (size_t)(ids[i] + 1));
+    distinct(verts);
+    std::vector<std::array<int, 4>> cv(n);  // tile vertices of each cell
+    for (int i = 0; i < n; ++i)
+        for (int k = 0; k < 4; ++k) cv[i][k] = local(verts, m.cone[4 * (size_t)ids[i] + k]);
+    // faces of the tile: (vertices sorted) -> cell and the vertex opposite
+    std::vector<std::pair<uint64_t, int32_t>> faces;
+    for (int i = 0; i < n; ++i)
+        for (int k = 0; k < 4; ++k) {
+            std::array<int, 3> f{cv[i][(k + 1) & 3], cv[i][(k + 2) & 3], cv[i][(k + 3) & 3]};
+            std::sort(f.begin(), f.end());
+            faces.push_back({((uint64_t)f[0] << 40) | ((uint64_t)f[1] << 20) | (uint64_t)f[2], 4 * i + k});
+        }
+    std::sort(faces.begin(), faces.end());
+    std::vector<std::array<std::array<int, 3>, 4>> nbr(n);  // (neighbour, my opposite vertex, its)
+    std::vector<int> deg(n, 0);
+    for (size_t f = 0; f + 1 < faces.size(); ++f)
+        if (faces[f].first == faces[f + 1].first) {
+            const int a = faces[f].second >> 2, b = faces[f + 1].second >> 2;
+            if (a != b && deg[a] < 4 && deg[b] < 4) {
+                nbr[a][deg[a]++] = {b, faces[f].second & 3, faces[f + 1].second & 3};
+                nbr[b][deg[b]++] = {a, faces[f + 1].second & 3, faces[f].second & 3};
+            }
+            ++f;
+        }
+    // the second cell's face turned so that its first vertex is the first cell's; the other two then
+    // run the opposite way round in a consistently oriented mesh (else the cells are not paired)
+    static const int kApex[4][4] = {{0, 1, 2, 3}, {1, 0, 3, 2}, {2, 0, 1, 3}, {3, 0, 2, 1}};  // even permutations
+    auto orient = [&](int a, int oa, int b, int ob, int pa[4], int pb[4]) {
+        for (int k = 0; k < 4; ++k) pa[k] = kApex[oa][k];
+        for (int r = 0; r < 3; ++r) {
+            pb[0] = kApex[ob][0];
+            for (int k = 0; k < 3; ++k) pb[1 + k] = kApex[ob][1 + (k + r) % 3];
+            if (cv[b][pb[1]] == cv[a][pa[1]]) break;
+        }
+        return cv[b][pb[1]] == cv[a][pa[1]] && cv[b][pb[2]] == cv[a][pa[3]] && cv[b][pb[3]] == cv[a][pa[2]];
+    };
+    // matching: cells with the fewest free neighbours first, each to its neighbour with the fewest
+    std::vector<int> mate(n, -1), free_deg(deg);
+    std::vector<std::array<int, 2>> opp(n);
+    std::array<std::vector<int>, 5> bucket;
+    for (int i = n - 1; i >= 0; --i) bucket[free_deg[i]].push_back(i);
+    std::vector<std::array<int, 2>> pairs;  // (first, second)
+    for (int d = 1; d <= 4;) {
+        if (bucket[d].empty()) {
+            ++d;
+            continue;
+        }
+        const int a = bucket[d].back();
+        bucket[d].pop_back();
+        if (mate[a] >= 0 || free_deg[a] != d) continue;
+        int best = -1;
+        for (int k = 0; k < deg[a]; ++k) {
+            const int b = nbr[a][k][0];
+            if (mate[b] >= 0) continue;
+            int pa[4], pb[4];
+            if (!orient(a, nbr[a][k][1], b, nbr[a][k][2], pa, pb)) continue;
+            if (best < 0 || free_deg[b] < free_deg[nbr[a][best][0]]) best = k;
+        }
+        if (best < 0) continue;  // no neighbour it can be turned to: stays single
+        const int b = nbr[a][best][0];
+        mate[a] = b;
+        mate[b] = a;
+        opp[a] = {nbr[a][best][1], nbr[a][best][2]};
+        pairs.push_back({a, b});
+        for (int c : {a, b})
+            for (int k = 0; k < deg[c]; ++k) {
+                const int e = nbr[c][k][0];
+                if (mate[e] >= 0) continue;
+                if (--free_deg[e] > 0) bucket[free_deg[e]].push_back(e);
+                if (free_deg[e] > 0 && free_deg[e] < d) d = free_deg[e];
+            }
+    }
+    const int npaired = (int)pairs.size();
+    for (int i = 0; i < n; ++i)
+        if (mate[i] < 0) pairs.push_back({i, -1});
+    const int np = (int)pairs.size();
+    // slots: mesh nodes [14] and tile vertices [5] of each pair
+    static const int kEdge[4][4] = {{-1, 4, 5, 6}, {4, -1, 7, 8}, {5, 7, -1, 9}, {6, 8, 9, -1}};
+    std::vector<std::array<int32_t, 14>> pn(np);
+    std::vector<std::array<int, 5>> pv(np);
+    for (int p = 0; p < np; ++p) {
+        const int a = pairs[p][0], b = pairs[p][1];
+        int pa[4] = {0, 1, 2, 3}, pb[4] = {0, 1, 3, 2};
+        if (b >= 0) (void)orient(a, opp[a][0], b, opp[a][1], pa, pb);
+        const int q = b >= 0 ? b : a;  // alone: the second cell is the mirror image of the first
+        const int32_t *ca = m.closure + 10 * (size_t)ids[a], *cb = m.closure + 10 * (size_t)ids[q];
+        for (int k = 0; k < 4; ++k) {
+            pn[p][k] = ca[pa[k]];
+            pv[p][k] = cv[a][pa[k]];
+        }
+        for (int k = 0; k < 3; ++k) pn[p][4 + k] = ca[kEdge[pa[0]][pa[1 + k]]];
+        pn[p][7] = ca[kEdge[pa[1]][pa[2]]];
+        pn[p][8] = ca[kEdge[pa[1]][pa[3]]];
+        pn[p][9] = ca[kEdge[pa[2]][pa[3]]];
+        pn[p][10] = cb[pb[0]];
+        pv[p][4] = cv[q][pb[0]];
+        pn[p][11] = cb[kEdge[pb[0]][pb[1]]];  // to x
+        pn[p][12] = cb[kEdge[pb[0]][pb[3]]];  // to y
+        pn[p][13] = cb[kEdge[pb[0]][pb[2]]];  // to z
+    }
+    // pairs of one colour share no node; sorted by colour (paired ones first) a wave's atomic
+    // targets are distinct
+    std::vector<std::array<int32_t, 14>> pl(np);
+    for (int p = 0; p < np; ++p)
+        for (int j = 0; j < 14; ++j) pl[p][j] = local(T.nodes, pn[p][j]);
+    std::vector<int> color(np), order(np);
+    {
+        std::vector<std::array<uint64_t, 2>> used(T.nodes.size(), {0, 0});
+        for (int p = 0; p < np; ++p) {
+            uint64_t m0 = 0, m1 = 0;
+            for (int32_t k : pl[p]) {
+                m0 |= used[k][0];
+                m1 |= used[k][1];
+            }
+            int c = 0;
+            while (c < 127 && ((c < 64 ? (m0 >> c) : (m1 >> (c - 64))) & 1)) ++c;
+            for (int32_t k : pl[p]) used[k][c >> 6] |= (uint64_t)1 << (c & 63);
+            color[p] = c + (p < npaired ? 0 : 128);
+            order[p] = p;
+        }
+        std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return color[a] < color[b]; });
+    }
+    // local numbering: owned nodes balanced over the LDS banks around the shared ones, which keep node
+    // order (the halo reduction reads their partials in that order); vertices balanced
+    std::vector<int32_t> own, sh, ord;
+    for (int32_t x : T.nodes) (tile_count[x] == 1 ? own : sh).push_back(x);
+    T.nown = (int)own.size();
+    ord = own;
+    ord.insert(ord.end(), sh.begin(), sh.end());
+    std::vector<int32_t> rank(T.nodes.size());  // sorted position -> local index
+    auto ranks = [&](const std::vector<int32_t> &v) {
+        for (size_t k = 0; k < v.size(); ++k) rank[local(T.nodes, v[k])] = (int32_t)k;
+    };
+    ranks(ord);
+    std::vector<std::vector<int32_t>> slot(14, std::vector<int32_t>(np));
+    for (int i = 0; i < np; ++i)
+        for (int j = 0; j < 14; ++j) slot[j][i] = rank[pl[order[i]][j]];
+    balance_banks(ord, {0, T.nown, (int)ord.size()}, slot, np, kFixShared);
+    ranks(ord);
+    std::vector<int32_t> vo(verts.size()), vslot_id(verts.size());
+    for (size_t k = 0; k < verts.size(); ++k) vo[k] = (int32_t)k;
+    std::vector<std::vector<int32_t>> vslot(5, std::vector<int32_t>(np));
+    for (int i = 0; i < np; ++i)
+        for (int j = 0; j < 5; ++j) vslot[j][i] = pv[order[i]][j];
+    balance_banks(vo, {0, (int)vo.size()}, vslot, np);
+    for (size_t k = 0; k < vo.size(); ++k) vslot_id[vo[k]] = (int32_t)k;
+    T.verts.resize(verts.size());
+    for (size_t k = 0; k < vo.size(); ++k) T.verts[k] = verts[vo[k]];
+    T.rec.assign(6 * (size_t)np, 0);
+    T.cells.resize(2 * (size_t)np);
+    for (int i = 0; i < np; ++i) {
+        const int p = order[i];
+        uint32_t *w = &T.rec[6 * (size_t)i];
+        for (int j = 0; j < 12; ++j) w[j / 3] |= (uint32_t)rank[pl[p][j]] << (10 * (j % 3));
+        w[4] = (uint32_t)rank[pl[p][12]] | (uint32_t)rank[pl[p][13]] << 10 | (uint32_t)vslot_id[pv[p][4]] << 20;
+        for (int j = 0; j < 4; ++j) w[5] |= (uint32_t)vslot_id[pv[p][j]] << (8 * j);
+        T.cells[2 * (size_t)i] = ids[pairs[p][0]];
+        T.cells[2 * (size_t)i + 1] = pairs[p][1] >= 0 ? ids[pairs[p][1]] : -1;
+    }
+    T.nodes = std::move(ord);
+}
+
+// Halo slots of cells cut into the given tiles; per tile its sorted nodes, per node its tiles.
+static int64_t tile_nodes_of(const MeshView &m, const std::vector<int32_t> &cells, const std::vector<int32_t> &ptr,
+                             std::vector<PairTile> &tiles, std::vector<int32_t> &tile_count) {
+    const int nt = (int)ptr.size() - 1;
+    tiles.assign(nt, PairTile());
+    parallel_for(nt, [&](int t) {
+        std::vector<int32_t> &v = tiles[t].nodes;
+        for (int i = ptr[t]; i < ptr[t + 1]; ++i)
+            v.insert(v.end(), m.closure + (size_t)cells[i] * m.nb, m.closure + (size_t)(cells[i] + 1) * m.nb);
+        distinct(v);
+    });
+    tile_count.assign(m.num_nodes, 0);
+    for (const PairTile &T : tiles)
+        for (int32_t x : T.nodes) ++tile_count[x];
+    int64_t halo = 0;
+    for (int32_t c : tile_count) halo += c > 1 ? c : 0;
+    return halo;
+}
+
+int build_pair_plan(const MeshView &m, const HostPlan &base, PairPlan *pp, std::string *err) {
+    if (m.nb != 10 || m.nv != 4 || !m.coords) {
+        *err = "pair plans are for P2 tetrahedra";
+        return 1;
+    }
+    const int n = (int)base.cells.size();
+    std::vector<int32_t> cells(base.cells), ptr(1, 0);
+    std::vector<PairTile> tiles;
+    std::vector<int32_t> tile_count;
+    {
+        std::vector<double> cen(3 * (size_t)m.num_cells);
+        for (int32_t c : cells)
+            for (int d = 0; d < 3; ++d) {
+                double acc = 0.0;
+                for (int v = 0; v < 4; ++v) acc += m.coords[3 * (size_t)m.cone[4 * (size_t)c + v] + d];
+                cen[3 * (size_t)c + d] = 0.25 * acc;
+            }
+        std::vector<int32_t> sizes;
+        bisect(m, cen, cells.data(), n, sizes, 0);
+        for (int32_t s : sizes) ptr.push_back(ptr.back() + s);
+    }
+    int64_t halo = tile_nodes_of(m, cells, ptr, tiles, tile_count);
+    if (halo > base.halo_slots) {
+        cells = base.cells;
+        ptr = base.tile_cell_ptr;
+        halo = tile_nodes_of(m, cells, ptr, tiles, tile_count);
+    }
+    const int nt = (int)ptr.size() - 1;
+    parallel_for(nt, [&](int t) { build_pair_tile(m, &cells[ptr[t]], ptr[t + 1] - ptr[t], tile_count, tiles[t]); });
+    *pp = PairPlan();
+    pp->num_tiles = nt;
+    pp->halo_slots = halo;
+    pp->tile_pair_ptr.assign(1, 0);
+    pp->tile_node_ptr.assign(1, 0);
+    pp->tile_vert_ptr.assign(1, 0);
+    // shared nodes ascending, their slots in tile order
+    shared_map(m.num_nodes, tile_count, pp->shared_node, pp->shared_ptr);
+    std::vector<int32_t> place(m.num_nodes, -1);
+    for (size_t i = 0; i < pp->shared_node.size(); ++i) place[pp->shared_node[i]] = pp->shared_ptr[i];
+    pp->shared_slot.resize((size_t)halo);
+    int64_t off = 0;
+    for (PairTile &T : tiles) {
+        if ((int)T.nodes.size() > kPairTileNodes || (int)T.verts.size() > kPairTileVerts ||
+            (int)T.cells.size() > 2 * kPairTilePairs || off > INT32_MAX) {
+            *err = "pair tile over its bounds";
+            return 1;
+        }
+        pp->tile_nown.push_back(T.nown);
+        pp->tile_halo_off.push_back((int32_t)off);
+        for (size_t k = (size_t)T.nown; k < T.nodes.size(); ++k) pp->shared_slot[place[T.nodes[k]]++] = (int32_t)off++;
+        pp->tile_nodes.insert(pp->tile_nodes.end(), T.nodes.begin(), T.nodes.end());
+        pp->tile_verts.insert(pp->tile_verts.end(), T.verts.begin(), T.verts.end());
+        pp->cells.insert(pp->cells.end(), T.cells.begin(), T.cells.end());
+        pp->records.insert(pp->records.end(), T.rec.begin(), T.rec.end());
+        pp->tile_pair_ptr.push_back((int32_t)(pp->cells.size() / 2));
+        pp->tile_node_ptr.push_back((int32_t)pp->tile_nodes.size());
+        pp->tile_vert_ptr.push_back((int32_t)pp->tile_verts.size());
+    }
+    pp->num_pairs = (int)(pp->cells.size() / 2);
     return 0;
 }
 

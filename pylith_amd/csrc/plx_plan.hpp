@@ -45,6 +45,36 @@ struct HostPlan {
     bool reordered = false;  // cells taken in Morton order of their centroids instead of input order
 };
 
+// Tile plan of the P2 pair kernel: the key's cells in tiles of up to kPairTilePairs pairs of cells
+// that share a face (a pair has 14 distinct nodes and 5 vertices where two cells have 20 and 8), one
+// pair per thread.  A cell left without a partner is paired with its own mirror image, whose
+// moduli the kernel reads as zero.
+constexpr int kPairTilePairs = 256, kPairTileNodes = 1024, kPairTileVerts = 256;
+struct PairPlan {
+    int num_tiles = 0, num_pairs = 0;
+    int64_t halo_slots = 0;
+    std::vector<int32_t> tile_pair_ptr, tile_node_ptr, tile_nown, tile_nodes, tile_vert_ptr, tile_verts, tile_halo_off;
+    // six words per pair: 14 node indices of 10 bits (three a word, the last two with the fifth
+    // vertex index above them), four vertex indices of 8 bits.  Nodes: first cell's apex, the
+    // face's vertices x, y, z, the apex's edges to them, edges xy, xz, yz, then the second cell's
+    // apex and its edges to x, y, z; vertices: first apex, x, y, z, second apex.
+    std::vector<uint32_t> records;
+    std::vector<int32_t> cells;  // [num_pairs][2] mesh cells, -1: no second cell
+    std::vector<int32_t> shared_node, shared_ptr, shared_slot;
+};
+// First cell's local basis -> pair slot is the identity; the second's (apex, x, z, y in its own
+// orientation; edges (0,1), (0,2), (0,3), (1,2), (1,3), (2,3)):
+constexpr int kPairSecond[10] = {10, 1, 3, 2, 11, 13, 12, 8, 7, 9};
+// The slot indices of a record.
+inline int pair_node(const uint32_t *w, int j) {
+    return j < 12 ? (int)((w[j / 3] >> (10 * (j % 3))) & 1023u) : (int)((w[4] >> (10 * (j - 12))) & 1023u);
+}
+inline int pair_vert(const uint32_t *w, int j) { return j < 4 ? (int)((w[5] >> (8 * j)) & 255u) : (int)((w[4] >> 20) & 255u); }
+
+// Pair plan of the base plan's cells (P2).  The cells are cut by recursive coordinate bisection of their
+// centroids; where that gives no fewer halo slots than the base plan's tiles, those are kept.
+int build_pair_plan(const MeshView &m, const HostPlan &base, PairPlan *pp, std::string *err);
+
 // sort_by_color: order each tile's cells by colour (colour-phase accumulation activates
 // contiguous threads); otherwise cells keep their mesh order inside the tile (neighbouring
 // threads then touch neighbouring nodes: structured LDS access for atomic accumulation).

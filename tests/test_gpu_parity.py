@@ -164,6 +164,30 @@ def test_p2_tets_config2_64cube(oracle):
     check_residual(oracle, m, u, aux=(aux, sizes))
 
 
+# meshes over the line where P2 keys take the pair kernel (65,536 cells): bricks with a remainder, no
+# locality in the numbering, and a key of scattered cells with a second key beside it
+@pytest.mark.parametrize("kind", ["bricks", "random", "scattered_key"])
+def test_p2_pair_kernel(oracle, kind):
+    m = mg.tet_p2_box((27, 23, 21), (0, 0, 0), (2700.0, 2300.0, 2100.0))
+    if kind == "random":
+        m = mg.renumbered(m, 5)
+    label = 0
+    if kind == "scattered_key":
+        m.labels = (np.random.default_rng(2).random(m.num_cells) < 0.9).astype(np.int32)
+        label = 1
+    assert int((m.labels == label).sum()) >= 65536
+    aux, sizes = mg.elastic_aux(m.num_cells, seed=6, vs_sigma=0.2, vp_vs=1.8)
+    u = mg.random_field(m.num_nodes, 9)
+    dm, ref = check_residual(oracle, m, u, label=label, aux=(aux, sizes))
+    dm.set_kernel_options()
+    for dt, tol in ((torch.float64, TOL64), (torch.float32, TOL32)):
+        x = dev(u, dt)
+        r = torch.zeros_like(x)
+        dm.compute_residual_noalloc(label, 0, x, r, mode=1)
+        torch.cuda.synchronize()
+        assert relerr(r.double().cpu().numpy(), ref) <= tol
+
+
 def test_deterministic_bitwise(oracle):
     m = mg.tet_p2_box(8, (0, 0, 0), (1.0, 1.0, 1.0))
     aux, sizes = mg.elastic_aux(m.num_cells)
