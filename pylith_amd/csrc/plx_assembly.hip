@@ -695,7 +695,7 @@ bool takes_pairs(plx_dm dm, const KeyPlan *kp) {
 
 template <typename Real>
 static int apply_pairs_typed(plx_dm dm, KeyPlan *kp, const void *u, void *r, int mode, double scale, void *halo,
-                             bool log) {
+                             bool log, bool reduce) {
     const PairDev &P = kp->pairs;
     PairArgs A;
     A.num_tiles = P.num_tiles;
@@ -719,13 +719,14 @@ static int apply_pairs_typed(plx_dm dm, KeyPlan *kp, const void *u, void *r, int
         hipLaunchKernelGGL(apply_pairs<Real>, dim3(std::min(P.num_tiles, resident)), dim3(kPairThreads), lds, dm->stream, A);
     }
     PLX_HIP(dm, hipGetLastError());
+    if (!reduce) return 0;
     return reduce_shared<Real>(dm, P.num_shared, P.d_shared_node, P.d_shared_ptr, P.d_shared_slot, A.halo, r, mode, log);
 }
 
 template <typename Real>
 static int apply_typed(plx_dm dm, KeyPlan *kp, const void *u, void *r, int mode, double scale,
-                       const double *prestress, void *halo, bool log) {
-    if (!prestress && takes_pairs(dm, kp)) return apply_pairs_typed<Real>(dm, kp, u, r, mode, scale, halo, log);
+                       const double *prestress, void *halo, bool log, bool reduce) {
+    if (!prestress && takes_pairs(dm, kp)) return apply_pairs_typed<Real>(dm, kp, u, r, mode, scale, halo, log, reduce);
     ApplyArgs A;
     A.scale = scale;
     A.prestress = prestress;
@@ -802,6 +803,7 @@ static int apply_typed(plx_dm dm, KeyPlan *kp, const void *u, void *r, int mode,
 #undef PLX_LAUNCH
     }
     PLX_HIP(dm, hipGetLastError());
+    if (!reduce) return 0;
     return reduce_shared<Real>(dm, kp->num_shared, kp->d_shared_node, kp->d_shared_ptr, kp->d_shared_slot, A.halo, r, mode,
                                log);
 }
@@ -810,13 +812,23 @@ static int apply_typed(plx_dm dm, KeyPlan *kp, const void *u, void *r, int mode,
 // J v = F(v); for generalized Maxwell F(u) = J u + (the state term), with J the elastic operator
 // at the effective shear modulus (the residual adds the per-point state stress).
 int launch_apply(plx_dm dm, KeyPlan *kp, int scalar_type, bool jacobian, const void *u, void *r,
-                 int mode, double scale, void *halo, bool log) {
+                 int mode, double scale, void *halo, bool log, bool reduce) {
     if (mode != PLX_ADD_VALUES && mode != PLX_INSERT_VALUES) return set_error(dm, 1, "bad insert mode");
     const double *pre = (!jacobian && kp->genmax) ? kp->d_prestress : nullptr;
     if (pre && scalar_type != PLX_FP64) return set_error(dm, 1, "the viscoelastic residual is FP64");
-    if (scalar_type == PLX_FP64) return apply_typed<double>(dm, kp, u, r, mode, scale, pre, halo, log);
-    if (scalar_type == PLX_FP32) return apply_typed<float>(dm, kp, u, r, mode, scale, pre, halo, log);
+    if (scalar_type == PLX_FP64) return apply_typed<double>(dm, kp, u, r, mode, scale, pre, halo, log, reduce);
+    if (scalar_type == PLX_FP32) return apply_typed<float>(dm, kp, u, r, mode, scale, pre, halo, log, reduce);
     return set_error(dm, 1, "bad scalar type");
+}
+
+SharedSums shared_sums(plx_dm dm, KeyPlan *kp, bool jacobian) {
+    SharedSums S;
+    const bool pre = !jacobian && kp->genmax && kp->d_prestress;
+    if (!pre && takes_pairs(dm, kp))
+        S = {kp->pairs.num_shared, kp->pairs.d_shared_node, kp->pairs.d_shared_ptr, kp->pairs.d_shared_slot, kp->d_halo};
+    else
+        S = {kp->num_shared, kp->d_shared_node, kp->d_shared_ptr, kp->d_shared_slot, kp->d_halo};
+    return S;
 }
 
 // Body force / gravity load (fixed per node): r[node] += load.

@@ -639,27 +639,6 @@ __global__ void __launch_bounds__(NT) amg_bsr_split(int nrows, const int32_t *__
     }
 }
 
-// r = b - t (the fine residual over a matrix-free product t = A x)
-__global__ void __launch_bounds__(256) amg_sub(int64_t n, const float *__restrict__ b, const float *__restrict__ t,
-                                               float *r) {
-    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) r[i] = b[i] - t[i];
-}
-
-// z = x + s Dinv (b - t), 3 x 3 blocks (the fine post-smoothing over a matrix-free t = A x)
-__global__ void __launch_bounds__(256) amg_post0(int n, const float *__restrict__ Dinv, const float *__restrict__ b,
-                                                 const float *__restrict__ t, const float *__restrict__ x, float *z,
-                                                 float s) {
-    for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
-        const float *Di = Dinv + 9 * (size_t)i;
-        float rv[3];
-#pragma unroll
-        for (int q = 0; q < 3; ++q) rv[q] = b[3 * (size_t)i + q] - t[3 * (size_t)i + q];
-#pragma unroll
-        for (int a = 0; a < 3; ++a)
-            z[3 * (size_t)i + a] = x[3 * (size_t)i + a] + s * (Di[3 * a] * rv[0] + Di[3 * a + 1] * rv[1] + Di[3 * a + 2] * rv[2]);
-    }
-}
-
 // coarsest level, one column: a wave per row of the dense inverse
 __global__ void __launch_bounds__(256) amg_dense1(int m, int ld, const float *__restrict__ Ainv,
                                                   const float *__restrict__ Bv, float *X) {
@@ -1695,9 +1674,8 @@ static int gf_vcycle1_matfree(plx_gf g, const float *r, float *z) {
     float *nb = nl > 1 ? g->lv[1].bv : g->cb;
     float *nx = nl > 1 ? g->lv[1].xv : g->cx;
     hipLaunchKernelGGL((amg_jacobi0<3, 1>), gf_grid((int64_t)L.n), dim3(256), 0, g->stream, L.n, g->Dinv_dm, r, x, s);
-    int err = g->fine_op(g->fine_ctx, x, t);
+    int err = g->fine_op(g->fine_ctx, x, r, nullptr, 0.f, t, r1);
     if (err) return err;
-    hipLaunchKernelGGL(amg_sub, gf_grid(g->ndof), dim3(256), 0, g->stream, g->ndof, r, (const float *)t, r1);
     if (L.bc == 3) {  // P2 -> P1 transfer
         amg_bsr_launch<3, 3, 1, kBsrPlain, 16>(g, L.nc, L.Rptr, g->Rcol_dm, L.Rval, r1, nullptr, nullptr, nb, 0.f, 0);
         amg_vcycle<1>(g, 1, nb, nx);
@@ -1709,9 +1687,7 @@ static int gf_vcycle1_matfree(plx_gf g, const float *r, float *z) {
         amg_bsr_launch<3, 6, 1, kBsrPlain, 8>(g, L.n, g->Pptr_dm, g->Pcol_dm, g->Pval_dm, nx, nullptr, nullptr, x, 0.f,
                                               1);
     }
-    if ((err = g->fine_op(g->fine_ctx, x, t))) return err;
-    hipLaunchKernelGGL(amg_post0, gf_grid(L.n), dim3(256), 0, g->stream, L.n, (const float *)g->Dinv_dm, r,
-                       (const float *)t, (const float *)x, z, s);
+    if ((err = g->fine_op(g->fine_ctx, x, r, g->Dinv_dm, s, t, z))) return err;
     PLX_HIP(g->dm, hipGetLastError());
     return 0;
 }

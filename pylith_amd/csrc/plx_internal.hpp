@@ -242,8 +242,16 @@ void pointfn_release(plx_dm dm, KeyPlan *kp);
 // Kernel launchers (plx_assembly.hip).
 // halo: the shared-node partial-sum buffer (nullptr: the key's own d_halo); log: record the
 // kernels' event timers when the handle's logging is on
+// reduce: sum the shared nodes' partials into r (false: the caller does, from shared_sums)
 int launch_apply(plx_dm dm, KeyPlan *kp, int scalar_type, bool jacobian, const void *u,
-                 void *r, int mode, double scale = 1.0, void *halo = nullptr, bool log = true);
+                 void *r, int mode, double scale = 1.0, void *halo = nullptr, bool log = true, bool reduce = true);
+// Where an apply leaves the shared nodes' partial sums, under the DM's present options.
+struct SharedSums {
+    int num_shared = 0;
+    const int32_t *node = nullptr, *ptr = nullptr, *slot = nullptr;
+    const void *halo = nullptr;
+};
+SharedSums shared_sums(plx_dm dm, KeyPlan *kp, bool jacobian);
 bool takes_pairs(plx_dm dm, const KeyPlan *kp);  // whether the factored apply runs over the pair plan
 // Per-device set-up at plx_dm_create with the DM's device current: the element tables in
 // constant memory and the device address of the allocation-free entry point's scratch array.
@@ -271,11 +279,12 @@ int launch_fault_slip_rhs(plx_dm dm, double *lag_out);
 void free_fault(FaultData *f);
 
 // Multigrid V-cycle of a Green's-function handle on one column (plx_gf.hip), r and z in DM
-// node order.  gf_set_fine_operator gives it a matrix-free fine-level operator y = A x (FP32,
-// DM order, queued on the V-cycle's stream, constrained rows zero): the fine level then smooths
-// with it instead of the assembled operator (null: back to the assembled one).
+// node order.  gf_set_fine_operator gives it a matrix-free fine-level operator A (FP32, DM order,
+// queued on the V-cycle's stream, constrained rows zero): the fine level then smooths with it
+// instead of the assembled operator (null: back to the assembled one).  The operator writes
+// out = b - A x, or out = x + s Dinv (b - A x) when Dinv ([node][9]) is given; t is scratch.
 int gf_vcycle1(plx_gf g, hipStream_t stream, const float *r, float *z);
-using GfFineOp = int (*)(void *ctx, const float *x, float *y);
+using GfFineOp = int (*)(void *ctx, const float *x, const float *b, const float *Dinv, float s, float *t, float *out);
 int gf_set_fine_operator(plx_gf g, GfFineOp op, void *ctx);
 
 // Vector kernels (plx_vector.hip).

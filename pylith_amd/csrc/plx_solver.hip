@@ -29,7 +29,7 @@
 namespace plx {
 
 constexpr int kRedBlocks = 512;
-enum { S_RZ = 0, S_PQ, S_ALPHA, S_BETA, S_RR, S_RZNEW, S_COUNT };
+enum { S_RZ = 0, S_PQ, S_ALPHA, S_BETA, S_RR, S_RZOLD, S_COUNT };
 
 template <typename Real>
 __global__ void __launch_bounds__(256) mask_kernel(int n, const int32_t *__restrict__ dofs, Real *v) {
@@ -37,21 +37,21 @@ __global__ void __launch_bounds__(256) mask_kernel(int n, const int32_t *__restr
     if (i < n) v[dofs[i]] = Real(0);
 }
 
-// Block-reduce helper (256 threads): returns the block sum in thread 0.
+// Block sum of 256 threads (every thread gets it; fixed order): shuffles inside the waves, then the four
+// wave sums.
 __device__ __forceinline__ double block_sum(double v, double *s) {
-    s[threadIdx.x] = v;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
     __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) s[threadIdx.x] += s[threadIdx.x + w];
-        __syncthreads();
-    }
-    return s[0];
+    if ((threadIdx.x & 63) == 0) s[threadIdx.x >> 6] = v;
+    __syncthreads();
+    return (s[0] + s[1]) + (s[2] + s[3]);
 }
 
 template <typename Real>
 __global__ void __launch_bounds__(256) dot_partials(int64_t n, const Real *__restrict__ a,
                                                     const Real *__restrict__ b, double *partials) {
-    __shared__ double s[256];
+    __shared__ double s[4];
     double acc = 0.0;
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256)
         acc += (double)a[i] * (double)b[i];
@@ -61,7 +61,7 @@ __global__ void __launch_bounds__(256) dot_partials(int64_t n, const Real *__res
 
 // scal[S_PQ] = sum(partials); scal[S_ALPHA] = scal[S_RZ] / scal[S_PQ]
 __global__ void __launch_bounds__(256) finish_alpha(const double *__restrict__ partials, double *scal) {
-    __shared__ double s[256];
+    __shared__ double s[4];
     double acc = 0.0;
     for (int i = threadIdx.x; i < kRedBlocks; i += 256) acc += partials[i];
     const double t = block_sum(acc, s);
@@ -78,7 +78,7 @@ __global__ void __launch_bounds__(256) cg_update(int nnodes, const Real *__restr
                                                  const Real *__restrict__ q, Real *z,
                                                  const double *__restrict__ scal, double *part_rz,
                                                  double *part_rr) {
-    __shared__ double s[256];
+    __shared__ double s[4];
     const Real alpha = (Real)scal[S_ALPHA];
     double rz = 0.0, rr = 0.0;
     for (int node = blockIdx.x * 256 + threadIdx.x; node < nnodes; node += gridDim.x * 256) {
@@ -111,7 +111,7 @@ __global__ void __launch_bounds__(256) cg_update(int nnodes, const Real *__restr
 // beta = rz_new / rz; rz = rz_new; rr
 __global__ void __launch_bounds__(256) finish_beta(const double *__restrict__ part_rz,
                                                    const double *__restrict__ part_rr, double *scal) {
-    __shared__ double s[256];
+    __shared__ double s[4];
     double a = 0.0, b = 0.0;
     for (int i = threadIdx.x; i < kRedBlocks; i += 256) {
         a += part_rz[i];
@@ -142,7 +142,7 @@ template <typename Real>
 __global__ void __launch_bounds__(256) cg_update_xr(int64_t n, Real *x, Real *r, const Real *__restrict__ p,
                                                     const Real *__restrict__ q, const double *__restrict__ scal,
                                                     double *part_rr) {
-    __shared__ double s[256];
+    __shared__ double s[4];
     const Real alpha = (Real)scal[S_ALPHA];
     double rr = 0.0;
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
@@ -159,7 +159,7 @@ __global__ void __launch_bounds__(256) cg_update_xr(int64_t n, Real *x, Real *r,
 template <typename Real>
 __global__ void __launch_bounds__(256) rz_partials(int64_t n, const Real *__restrict__ r, const Real *__restrict__ z,
                                                    Real *p, double *part_rz, double *part_rr) {
-    __shared__ double s[256];
+    __shared__ double s[4];
     double rz = 0.0, rr = 0.0;
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
         const double rv = (double)r[i], zv = (double)z[i];
@@ -181,7 +181,7 @@ template <typename Real>
 __global__ void __launch_bounds__(256) pc_start(int nnodes, const Real *__restrict__ Binv,
                                                 const Real *__restrict__ r, Real *z, Real *p,
                                                 double *part_rz, double *part_rr) {
-    __shared__ double s[256];
+    __shared__ double s[4];
     double rz = 0.0, rr = 0.0;
     for (int node = blockIdx.x * 256 + threadIdx.x; node < nnodes; node += gridDim.x * 256) {
         const size_t o = 3 * (size_t)node;
@@ -208,7 +208,7 @@ __global__ void __launch_bounds__(256) pc_start(int nnodes, const Real *__restri
 
 __global__ void __launch_bounds__(256) finish_start(const double *__restrict__ part_rz,
                                                     const double *__restrict__ part_rr, double *scal) {
-    __shared__ double s[256];
+    __shared__ double s[4];
     double a = 0.0, b = 0.0;
     for (int i = threadIdx.x; i < kRedBlocks; i += 256) {
         a += part_rz[i];
@@ -222,6 +222,182 @@ __global__ void __launch_bounds__(256) finish_start(const double *__restrict__ p
         scal[S_RR] = rr;
         scal[S_BETA] = 0.0;
     }
+}
+
+// --------------------------------------------------------------------------------------------
+// The PCG iteration of one key without a fault in four kernels (multigrid: four around the V-cycle)
+// where it took eight (eleven): at a few 10,000 dofs each kernel is launch and latency, about 3 us
+// whatever it does.  The apply leaves the shared nodes' partial sums; node_finish adds them, masks and
+// takes the dot product in one pass over the nodes; the reductions' last step, a sum of at most
+// kRedBlocks partials, is done by every block of the kernel that needs it instead of by a kernel of
+// its own.  24 x 22 x 25 hexes, FP32 point-block Jacobi: 26 -> 21 us an iteration; multigrid CG on
+// 22 x 24 x 21 x 6 tets: 5.8 -> 5.0 ms a solve.
+// --------------------------------------------------------------------------------------------
+
+// Sum of n partials by the whole block.
+__device__ __forceinline__ double total(const double *__restrict__ part, int n, double *s) {
+    double acc = 0.0;
+    for (int i = threadIdx.x; i < n; i += 256) acc += part[i];
+    return block_sum(acc, s);
+}
+
+enum { kFinishDot = 0, kFinishResid, kFinishPost };
+// One thread per node: q = A x there (its row of y, or the sum of its halo slots range[node] when
+// tiles share it), zero at constrained dofs.  Dot: y = q, partials of x.q; Resid: out = b - q;
+// Post: out = x + s Dinv (b - q).
+template <typename Real, int MODE>
+__global__ void __launch_bounds__(256) node_finish(int nnodes, const int2 *__restrict__ range,
+                                                   const int32_t *__restrict__ slot, const Real *__restrict__ halo,
+                                                   const uint8_t *__restrict__ fixed, Real *y,
+                                                   const Real *__restrict__ x, const Real *__restrict__ b,
+                                                   const Real *__restrict__ Dinv, Real sc, Real *out, double *part) {
+    __shared__ double s[4];
+    double acc = 0.0;
+    for (int node = blockIdx.x * 256 + threadIdx.x; node < nnodes; node += gridDim.x * 256) {
+        const size_t o = 3 * (size_t)node;
+        const int2 r = range[node];
+        Real q[3];
+        if (r.x < r.y) {
+            q[0] = q[1] = q[2] = Real(0);
+            for (int j = r.x; j < r.y; ++j) {
+                const size_t h = 3 * (size_t)slot[j];
+#pragma unroll
+                for (int c = 0; c < 3; ++c) q[c] += halo[h + c];
+            }
+        } else {
+#pragma unroll
+            for (int c = 0; c < 3; ++c) q[c] = y[o + c];
+        }
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+            if (fixed[o + c]) q[c] = Real(0);
+        if (MODE == kFinishDot) {
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                y[o + c] = q[c];
+                acc += (double)x[o + c] * (double)q[c];
+            }
+        } else {
+            Real rv[3];
+#pragma unroll
+            for (int c = 0; c < 3; ++c) rv[c] = b[o + c] - q[c];
+            if (MODE == kFinishPost) {
+                const Real *D = Dinv + 9 * (size_t)node;
+#pragma unroll
+                for (int c = 0; c < 3; ++c)
+                    out[o + c] = x[o + c] + sc * (D[3 * c] * rv[0] + D[3 * c + 1] * rv[1] + D[3 * c + 2] * rv[2]);
+            } else {
+#pragma unroll
+                for (int c = 0; c < 3; ++c) out[o + c] = rv[c];
+            }
+        }
+    }
+    if (MODE == kFinishDot) {
+        const double t = block_sum(acc, s);
+        if (threadIdx.x == 0) part[blockIdx.x] = t;
+    }
+}
+
+__global__ void __launch_bounds__(256) fill_ranges(int n, const int32_t *__restrict__ node,
+                                                   const int32_t *__restrict__ ptr, int2 *range) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n) range[node[i]] = make_int2(ptr[i], ptr[i + 1]);
+}
+
+// alpha = rz / p.q (partials part_pq), kept in scal by the first block with the rz it used
+__device__ __forceinline__ double alpha_of(const double *part_pq, int nblk, double *scal, double *s) {
+    const double pq = total(part_pq, nblk, s), rz = scal[S_RZ];
+    if (blockIdx.x == 0 && threadIdx.x == 0) scal[S_RZOLD] = rz;
+    return pq != 0.0 ? rz / pq : 0.0;
+}
+
+// x += alpha p; r -= alpha q; z = Binv r (per node); partials of r.z and r.r
+template <typename Real>
+__global__ void __launch_bounds__(256) cg_step(int nnodes, const Real *__restrict__ Binv, Real *x, Real *r,
+                                               const Real *__restrict__ p, const Real *__restrict__ q, Real *z,
+                                               const double *__restrict__ part_pq, int nblk, double *scal,
+                                               double *part_rz, double *part_rr) {
+    __shared__ double s[4];
+    const Real alpha = (Real)alpha_of(part_pq, nblk, scal, s);
+    double rz = 0.0, rr = 0.0;
+    for (int node = blockIdx.x * 256 + threadIdx.x; node < nnodes; node += gridDim.x * 256) {
+        const size_t o = 3 * (size_t)node;
+        Real rv[3];
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            x[o + c] += alpha * p[o + c];
+            rv[c] = r[o + c] - alpha * q[o + c];
+            r[o + c] = rv[c];
+        }
+        const Real *B = Binv + 9 * (size_t)node;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            const Real zc = B[3 * c] * rv[0] + B[3 * c + 1] * rv[1] + B[3 * c + 2] * rv[2];
+            z[o + c] = zc;
+            rz += (double)rv[c] * (double)zc;
+            rr += (double)rv[c] * (double)rv[c];
+        }
+    }
+    __syncthreads();
+    const double a = block_sum(rz, s);
+    __syncthreads();
+    const double b = block_sum(rr, s);
+    if (threadIdx.x == 0) {
+        part_rz[blockIdx.x] = a;
+        part_rr[blockIdx.x] = b;
+    }
+}
+
+// x += alpha p; r -= alpha q, and r in FP32 for the V-cycle (r32, unless r is that vector); partials of r.r
+template <typename Real>
+__global__ void __launch_bounds__(256) cg_step_xr(int64_t n, Real *x, Real *r, const Real *__restrict__ p,
+                                                  const Real *__restrict__ q, float *r32,
+                                                  const double *__restrict__ part_pq, int nblk, double *scal,
+                                                  double *part_rr) {
+    __shared__ double s[4];
+    const Real alpha = (Real)alpha_of(part_pq, nblk, scal, s);
+    double rr = 0.0;
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
+        x[i] += alpha * p[i];
+        const Real rv = r[i] - alpha * q[i];
+        r[i] = rv;
+        if (sizeof(Real) == 8) r32[i] = (float)rv;
+        rr += (double)rv * (double)rv;
+    }
+    __syncthreads();
+    const double b = block_sum(rr, s);
+    if (threadIdx.x == 0) part_rr[blockIdx.x] = b;
+}
+
+// partials of r.z over an FP32 z
+template <typename Real>
+__global__ void __launch_bounds__(256) rz_partials32(int64_t n, const Real *__restrict__ r, const float *__restrict__ z,
+                                                     double *part_rz) {
+    __shared__ double s[4];
+    double rz = 0.0;
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256)
+        rz += (double)r[i] * (double)z[i];
+    const double a = block_sum(rz, s);
+    if (threadIdx.x == 0) part_rz[blockIdx.x] = a;
+}
+
+// beta = rz_new / rz_old; p = z + beta p; the first block keeps rz and rr
+template <typename Real, typename ZReal>
+__global__ void __launch_bounds__(256) p_step(int64_t n, const ZReal *__restrict__ z, Real *p,
+                                              const double *__restrict__ part_rz, const double *__restrict__ part_rr,
+                                              int nblk, double *scal) {
+    __shared__ double s[4];
+    const double rz = total(part_rz, nblk, s), old = scal[S_RZOLD];
+    const Real beta = (Real)(old != 0.0 ? rz / old : 0.0);
+    if (blockIdx.x == 0) {
+        const double rr = total(part_rr, nblk, s);
+        if (threadIdx.x == 0) {
+            scal[S_RZ] = rz;
+            scal[S_RR] = rr;
+        }
+    }
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256)
+        p[i] = (Real)z[i] + beta * p[i];
 }
 
 template <typename Src, typename Dst>
@@ -296,7 +472,13 @@ struct plx_solver_s {
     // FGMRES bases
     int restart = 30;
     std::vector<double *> V, Z;
-    double *scal = nullptr, *part_a = nullptr, *part_b = nullptr;
+    double *scal = nullptr, *part_a = nullptr, *part_b = nullptr, *part_c = nullptr;
+    // one key without a fault: where its apply leaves each node's sum (range: halo slots, empty for nodes
+    // of one tile) and the constrained dofs, made at the DM's epoch
+    int2 *range = nullptr;
+    uint8_t *fixed = nullptr;
+    uint64_t finish_epoch = ~0ull;
+    SharedSums sums;
     double inner_rtol = 1e-4;
     int inner_maxit = 2000;
     plx_solve_stats last{};
@@ -330,6 +512,50 @@ static int apply_keys(plx_solver s, int st, const void *x, void *y, double scale
     PLX_HIP(dm, hipGetLastError());
     for (KeyPlan *kp : s->keys)
         if (int err = launch_apply(dm, kp, st, true, x, y, PLX_ADD_VALUES, scale)) return err;
+    return 0;
+}
+
+// Whether iterations take the fused kernels (one key, no fault).
+static bool fused(const plx_solver_s *s) { return s->keys.size() == 1 && !s->fault; }
+
+// The node map and mask of the fused kernels, for the DM's present options and constraints (before a
+// solve, outside any capture).
+static int ensure_finish(plx_solver s) {
+    plx_dm dm = s->dm;
+    if (!fused(s) || s->finish_epoch == dm->epoch) return 0;
+    if (!s->range) PLX_HIP(dm, hipMalloc(&s->range, (size_t)s->nnodes * sizeof(int2)));
+    if (!s->fixed) PLX_HIP(dm, hipMalloc(&s->fixed, (size_t)s->n));
+    std::vector<uint8_t> mask(s->n, 0);
+    for (int32_t d : dm->con.dofs)
+        if (d < s->n) mask[d] = 1;
+    PLX_HIP(dm, hipMemcpyAsync(s->fixed, mask.data(), mask.size(), hipMemcpyHostToDevice, dm->stream));
+    PLX_HIP(dm, hipMemsetAsync(s->range, 0, (size_t)s->nnodes * sizeof(int2), dm->stream));
+    s->sums = shared_sums(dm, s->keys[0], true);
+    if (s->sums.num_shared > 0)
+        hipLaunchKernelGGL(fill_ranges, dim3((s->sums.num_shared + 255) / 256), dim3(256), 0, dm->stream,
+                           s->sums.num_shared, s->sums.node, s->sums.ptr, s->range);
+    PLX_HIP(dm, hipGetLastError());
+    PLX_HIP(dm, hipStreamSynchronize(dm->stream));  // the host mask outlives its copy
+    s->finish_epoch = dm->epoch;
+    return 0;
+}
+
+// Blocks of the fused kernels: one node per thread up to kRedBlocks blocks (so that a reduction's last
+// step, repeated by every block, stays short on small meshes).
+static int node_blocks(const plx_solver_s *s) { return std::max(1, std::min(kRedBlocks, (s->nnodes + 255) / 256)); }
+
+// t = A x (tile kernel), then node_finish over it.
+template <typename Real, int MODE>
+static int apply_finish(plx_solver s, const Real *x, Real *t, const Real *b, const Real *Dinv, Real sc, Real *out,
+                        double *part) {
+    plx_dm dm = s->dm;
+    const int st = std::is_same<Real, double>::value ? PLX_FP64 : PLX_FP32;
+    if (int err = launch_apply(dm, s->keys[0], st, true, x, t, PLX_INSERT_VALUES, -1.0, nullptr, true, false)) return err;
+    // a sum over the whole mesh needs its partials bounded; the others take a thread per node
+    const int blocks = MODE == kFinishDot ? node_blocks(s) : std::max(1, (s->nnodes + 255) / 256);
+    hipLaunchKernelGGL((node_finish<Real, MODE>), dim3(blocks), dim3(256), 0, dm->stream, s->nnodes, s->range,
+                       s->sums.slot, static_cast<const Real *>(s->sums.halo), s->fixed, t, x, b, Dinv, sc, out, part);
+    PLX_HIP(dm, hipGetLastError());
     return 0;
 }
 
@@ -411,10 +637,41 @@ static int dot64(plx_solver s, const double *a, const double *b, double *out) {
     return read_scalar(s, S_RZ, out);
 }
 
-// The V-cycle's fine-level operator: the masked matrix-free FP32 apply (no fault: x is not
-// touched; with a fault the V-cycle keeps the assembled merged operator).
-static int amg_fine_apply(void *ctx, const float *x, float *y) {
-    return masked_apply<float>((plx_solver)ctx, const_cast<float *>(x), y);
+// out = b - t (the V-cycle's fine residual where the fused kernels do not apply)
+__global__ void __launch_bounds__(256) fine_resid(int64_t n, const float *__restrict__ b, const float *__restrict__ t,
+                                                  float *out) {
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) out[i] = b[i] - t[i];
+}
+
+// out = x + s Dinv (b - t), 3 x 3 blocks
+__global__ void __launch_bounds__(256) fine_post(int n, const float *__restrict__ Dinv, const float *__restrict__ b,
+                                                 const float *__restrict__ t, const float *__restrict__ x, float *out,
+                                                 float s) {
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
+        const float *D = Dinv + 9 * (size_t)i;
+        float rv[3];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) rv[q] = b[3 * (size_t)i + q] - t[3 * (size_t)i + q];
+#pragma unroll
+        for (int a = 0; a < 3; ++a)
+            out[3 * (size_t)i + a] = x[3 * (size_t)i + a] + s * (D[3 * a] * rv[0] + D[3 * a + 1] * rv[1] + D[3 * a + 2] * rv[2]);
+    }
+}
+
+// The V-cycle's fine-level operator (GfFineOp) over the masked matrix-free FP32 apply (no fault: x is
+// not touched; with a fault the V-cycle keeps the assembled merged operator).
+static int amg_fine_apply(void *ctx, const float *x, const float *b, const float *Dinv, float sc, float *t, float *out) {
+    plx_solver s = (plx_solver)ctx;
+    if (fused(s))
+        return Dinv ? apply_finish<float, kFinishPost>(s, x, t, b, Dinv, sc, out, nullptr)
+                    : apply_finish<float, kFinishResid>(s, x, t, b, nullptr, 0.f, out, nullptr);
+    if (int err = masked_apply<float>(s, const_cast<float *>(x), t)) return err;
+    if (Dinv)
+        hipLaunchKernelGGL(fine_post, red_grid(), dim3(256), 0, s->dm->stream, s->nnodes, Dinv, b, t, x, out, sc);
+    else
+        hipLaunchKernelGGL(fine_resid, red_grid(), dim3(256), 0, s->dm->stream, s->n, b, t, out);
+    PLX_HIP(s->dm, hipGetLastError());
+    return 0;
 }
 
 // z = M r with the multigrid V-cycle (FP32; an FP64 pair goes through the FP32 work vectors,
@@ -450,6 +707,21 @@ static int pcg_amg(plx_solver s, Real *x, Real *r, Real *p, Real *q, Real *z, do
     double rr = rr0;
     const int check = 2;  // a V-cycle iteration is expensive next to a convergence check
     auto iteration = [&]() -> int {
+        if (fused(s)) {
+            const int nblk = node_blocks(s);
+            int e = apply_finish<Real, kFinishDot>(s, p, q, nullptr, nullptr, Real(0), nullptr, s->part_c);
+            if (e) return e;
+            float *r32 = std::is_same<Real, float>::value ? (float *)r : s->r32;
+            float *z32 = std::is_same<Real, float>::value ? (float *)z : s->z32;
+            hipLaunchKernelGGL(cg_step_xr<Real>, dim3(nblk), dim3(256), 0, dm->stream, s->n, x, r, p, q, r32, s->part_c,
+                               nblk, s->scal, s->part_b);
+            if ((e = gf_vcycle1(s->amg, dm->stream, r32, z32))) return e;
+            hipLaunchKernelGGL(rz_partials32<Real>, dim3(nblk), dim3(256), 0, dm->stream, s->n, r, z32, s->part_a);
+            hipLaunchKernelGGL((p_step<Real, float>), dim3(nblk), dim3(256), 0, dm->stream, s->n, z32, p, s->part_a,
+                               s->part_b, nblk, s->scal);
+            PLX_HIP(dm, hipGetLastError());
+            return 0;
+        }
         int e = masked_apply<Real>(s, p, q);
         if (e) return e;
         hipLaunchKernelGGL(dot_partials<Real>, red_grid(), dim3(256), 0, dm->stream, s->n, p, q, s->part_a);
@@ -504,6 +776,17 @@ static int pcg(plx_solver s, Real *x, Real *r, Real *p, Real *q, Real *z, const 
     double rr = rr0;
     const int check = 10;
     auto iteration = [&]() -> int {
+        if (fused(s)) {
+            const int nblk = node_blocks(s);
+            const int e = apply_finish<Real, kFinishDot>(s, p, q, nullptr, nullptr, Real(0), nullptr, s->part_c);
+            if (e) return e;
+            hipLaunchKernelGGL(cg_step<Real>, dim3(nblk), dim3(256), 0, dm->stream, s->nnodes, Binv, x, r, p, q, z,
+                               s->part_c, nblk, s->scal, s->part_a, s->part_b);
+            hipLaunchKernelGGL((p_step<Real, Real>), dim3(nblk), dim3(256), 0, dm->stream, s->n, z, p, s->part_a,
+                               s->part_b, nblk, s->scal);
+            PLX_HIP(dm, hipGetLastError());
+            return 0;
+        }
         int e = masked_apply<Real>(s, p, q);
         if (e) return e;
         hipLaunchKernelGGL(dot_partials<Real>, red_grid(), dim3(256), 0, dm->stream, s->n, p, q, s->part_a);
@@ -711,7 +994,8 @@ int plx_solver_create(plx_solver *out, plx_dm dm, int label_value, int part) {
               hipMalloc(&s->Binv32, 9 * (size_t)s->nnodes * sizeof(float)) == hipSuccess &&
               hipMalloc(&s->scal, 16 * sizeof(double)) == hipSuccess &&
               hipMalloc(&s->part_a, kRedBlocks * sizeof(double)) == hipSuccess &&
-              hipMalloc(&s->part_b, kRedBlocks * sizeof(double)) == hipSuccess;
+              hipMalloc(&s->part_b, kRedBlocks * sizeof(double)) == hipSuccess &&
+              hipMalloc(&s->part_c, kRedBlocks * sizeof(double)) == hipSuccess;
     for (float **v : {&s->x32, &s->r32, &s->p32, &s->q32, &s->z32})
         ok = ok && hipMalloc(v, n * sizeof(float)) == hipSuccess;
     for (double **v : {&s->r64, &s->p64, &s->q64, &s->z64, &s->t64})
@@ -732,7 +1016,8 @@ int plx_solver_create(plx_solver *out, plx_dm dm, int label_value, int part) {
 
 int plx_solver_destroy(plx_solver s) {
     if (!s) return 0;
-    void *ptrs[] = {s->Binv64, s->Binv32, s->scal, s->part_a, s->part_b, s->x32, s->r32, s->p32,
+    void *ptrs[] = {s->range,  s->fixed,  s->part_c,
+                    s->Binv64, s->Binv32, s->scal, s->part_a, s->part_b, s->x32, s->r32, s->p32,
                     s->q32,    s->z32,    s->r64,  s->p64,    s->q64,    s->z64, s->t64};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
@@ -990,7 +1275,8 @@ int plx_solver_solve(plx_solver s, int method, const double *b, double *x, doubl
         return set_error(dm, 76, "solver stream ordering failed");
     }
     dm->stream = s->stream;
-    const int err = solve_impl(s, method, b, x, rtol, maxit, stats);
+    int err = ensure_finish(s);
+    if (!err) err = solve_impl(s, method, b, x, rtol, maxit, stats);
     dm->stream = caller;
     const bool ordered = hipEventRecord(ev, s->stream) == hipSuccess && hipStreamWaitEvent(caller, ev, 0) == hipSuccess;
     (void)hipEventDestroy(ev);
