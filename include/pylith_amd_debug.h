@@ -30,8 +30,9 @@ int plx_debug_plan_info(plx_dm dm, int label_value, int part, int *num_tiles, in
  * call is made (the handle's own stream reads it); synchronises. */
 int plx_debug_gf_precondition(plx_gf g, int k, const float *R, float *Z);
 
-/* algorithm: a plx_algorithm, or PLX_EMULATE_PAIRS for the P2 pair kernel over its pair plan. */
-enum { PLX_EMULATE_PAIRS = 100 };
+/* algorithm: a plx_algorithm, PLX_EMULATE_PAIRS for the P2 pair kernel over its pair plan, or
+ * PLX_EMULATE_GATHER for the tile kernel over the gather plan (an error where there is none). */
+enum { PLX_EMULATE_PAIRS = 100, PLX_EMULATE_GATHER = 101 };
 int plx_debug_emulate_apply(int cell_type, int num_cells, int num_vertices, int num_nodes,
                             const int32_t *closure, const int32_t *cone, const double *coords,
                             const int32_t *labels, int label_value, const double *lam_mu,

@@ -1,6 +1,6 @@
 // plx_assembly.hip -- gfx950 kernels of the residual / Jacobian-action apply.
 //
-// One persistent workgroup walks a sequence of tiles of cells (one or two cells per thread):
+// One persistent workgroup walks a sequence of tiles of cells (one or two cells, or a pair, per thread):
 //   1. the tile's nodal field and vertex coordinates are staged in LDS through the tile's
 //      node / vertex lists (coalesced where node numbers run contiguously); the next tile's
 //      gathers are issued into registers before the current tile's arithmetic;
@@ -12,6 +12,7 @@
 //      (the default; the order of the additions into one node, and so the last bits, may vary);
 //   4. nodes owned by the tile are written straight to the output vector; shared nodes leave
 //      as partial sums in the halo buffer, reduced in slot order by a node-ordered second kernel.
+//      Small meshes take a gather plan instead: overlapping tiles that own nodes, and no halo.
 // No global atomics are used.
 #include <algorithm>
 #include <map>
@@ -436,7 +437,8 @@ __global__ void __launch_bounds__((Shape<CT, Real>::NT), MINW) apply_tiles(Apply
             fetch_cells<Real, CT, ACC>(nxt, A, tid);
             fetch_values<Real, CT>(nxt, A);
         }
-        write_out<Real, Acc, S::PFN, NT>(sR, cur.gn, cur.nn, cur.nown, cur.hoff, tid, r, halo, insert);
+        // a gather plan (no halo) has nothing to store for the nodes that other tiles own
+        write_out<Real, Acc, S::PFN, NT>(sR, cur.gn, halo ? cur.nn : cur.nown, cur.nown, cur.hoff, tid, r, halo, insert);
         __builtin_amdgcn_s_setprio(0);
         if (!has_next) break;
         __syncthreads();  // every read of this tile's LDS precedes the next tile's staging
@@ -693,6 +695,12 @@ bool takes_pairs(plx_dm dm, const KeyPlan *kp) {
            dm->accumulate != PLX_ACCUMULATE_COLORED && dm->min_waves <= 2;
 }
 
+// (build_plan makes a gather plan only where it is the faster one)
+bool takes_gather(plx_dm dm, const KeyPlan *kp) {
+    return kp->gather.num_tiles > 0 && kp->gather.d_mat64 && dm->algorithm != PLX_ALGO_QUADRATURE_POINTS &&
+           dm->accumulate != PLX_ACCUMULATE_COLORED;
+}
+
 template <typename Real>
 static int apply_pairs_typed(plx_dm dm, KeyPlan *kp, const void *u, void *r, int mode, double scale, void *halo,
                              bool log, bool reduce) {
@@ -738,6 +746,20 @@ static int apply_typed(plx_dm dm, KeyPlan *kp, const void *u, void *r, int mode,
     A.halo = halo ? halo : kp->d_halo;
     A.mode = mode;
     A.records = kp->d_records;
+    int n_affine = kp->num_tiles_affine, n_tiles = kp->num_tiles;
+    const int32_t *affine = kp->d_heads_affine, *tiles = kp->d_heads;
+    const bool gather = !prestress && takes_gather(dm, kp);
+    if (gather) {
+        const GatherDev &G = kp->gather;
+        n_affine = n_tiles = G.num_tiles;  // a Q1 key with a gather plan has affine tiles only
+        affine = tiles = G.d_heads;
+        A.p.tile_nodes = G.d_nodes;
+        A.p.tile_verts = G.d_verts;
+        A.p.stride = (int)G.cells.size();
+        A.mat = std::is_same<Real, double>::value ? (const void *)G.d_mat64 : (const void *)G.d_mat32;
+        A.records = G.d_records;
+        A.halo = nullptr;
+    }
     // a per-point prestress needs the quadrature-point path
     const bool linear = dm->algorithm != PLX_ALGO_QUADRATURE_POINTS && !prestress;
     // AUTO: LDS atomics (FP64 accumulator, native ds_add_f64) for both vector types
@@ -775,35 +797,35 @@ static int apply_typed(plx_dm dm, KeyPlan *kp, const void *u, void *r, int mode,
         // rest: the quadrature-point kernel with the Jacobian at each point
         if (linear) {
             if (atomic) {
-                PLX_LAUNCH(PLX_HEX_Q1, kPathFactored, kAccAtomic, kp->d_heads_affine, kp->num_tiles_affine);
+                PLX_LAUNCH(PLX_HEX_Q1, kPathFactored, kAccAtomic, affine, n_affine);
                 PLX_LAUNCH(PLX_HEX_Q1, kPathQpGeneral, kAccAtomic, kp->d_heads_general, kp->num_tiles_general);
             } else {
-                PLX_LAUNCH(PLX_HEX_Q1, kPathFactored, kAccColored, kp->d_heads_affine, kp->num_tiles_affine);
+                PLX_LAUNCH(PLX_HEX_Q1, kPathFactored, kAccColored, affine, n_affine);
                 PLX_LAUNCH(PLX_HEX_Q1, kPathQpGeneral, kAccColored, kp->d_heads_general, kp->num_tiles_general);
             }
         } else {
             if (atomic) {
-                PLX_LAUNCH(PLX_HEX_Q1, kPathQpAffine, kAccAtomic, kp->d_heads_affine, kp->num_tiles_affine);
+                PLX_LAUNCH(PLX_HEX_Q1, kPathQpAffine, kAccAtomic, affine, n_affine);
                 PLX_LAUNCH(PLX_HEX_Q1, kPathQpGeneral, kAccAtomic, kp->d_heads_general, kp->num_tiles_general);
             } else {
-                PLX_LAUNCH(PLX_HEX_Q1, kPathQpAffine, kAccColored, kp->d_heads_affine, kp->num_tiles_affine);
+                PLX_LAUNCH(PLX_HEX_Q1, kPathQpAffine, kAccColored, affine, n_affine);
                 PLX_LAUNCH(PLX_HEX_Q1, kPathQpGeneral, kAccColored, kp->d_heads_general, kp->num_tiles_general);
             }
         }
     } else {
         if (linear) {
-            if (atomic) PLX_LAUNCH(PLX_TET_P2, kPathFactored, kAccAtomic, kp->d_heads, kp->num_tiles);
-            else PLX_LAUNCH(PLX_TET_P2, kPathFactored, kAccColored, kp->d_heads, kp->num_tiles);
+            if (atomic) PLX_LAUNCH(PLX_TET_P2, kPathFactored, kAccAtomic, tiles, n_tiles);
+            else PLX_LAUNCH(PLX_TET_P2, kPathFactored, kAccColored, tiles, n_tiles);
         } else {
-            if (atomic) PLX_LAUNCH(PLX_TET_P2, kPathQpAffine, kAccAtomic, kp->d_heads, kp->num_tiles);
-            else PLX_LAUNCH(PLX_TET_P2, kPathQpAffine, kAccColored, kp->d_heads, kp->num_tiles);
+            if (atomic) PLX_LAUNCH(PLX_TET_P2, kPathQpAffine, kAccAtomic, tiles, n_tiles);
+            else PLX_LAUNCH(PLX_TET_P2, kPathQpAffine, kAccColored, tiles, n_tiles);
         }
     }
 #undef PLX_LAUNCH_W
 #undef PLX_LAUNCH
     }
     PLX_HIP(dm, hipGetLastError());
-    if (!reduce) return 0;
+    if (!reduce || gather) return 0;
     return reduce_shared<Real>(dm, kp->num_shared, kp->d_shared_node, kp->d_shared_ptr, kp->d_shared_slot, A.halo, r, mode,
                                log);
 }
@@ -826,7 +848,7 @@ SharedSums shared_sums(plx_dm dm, KeyPlan *kp, bool jacobian) {
     const bool pre = !jacobian && kp->genmax && kp->d_prestress;
     if (!pre && takes_pairs(dm, kp))
         S = {kp->pairs.num_shared, kp->pairs.d_shared_node, kp->pairs.d_shared_ptr, kp->pairs.d_shared_slot, kp->d_halo};
-    else
+    else if (pre || !takes_gather(dm, kp))
         S = {kp->num_shared, kp->d_shared_node, kp->d_shared_ptr, kp->d_shared_slot, kp->d_halo};
     return S;
 }
@@ -1034,7 +1056,11 @@ int plx_compute_residual_noalloc(plx_dm dm, int label_value, int part, int scala
     if (kp->pf_residual || !kp->f1)
         return set_error(dm, 1, "PetscPointFn-form keys are not served allocation-free: use plx_compute_residual");
     if (scalar_type != PLX_FP64 && scalar_type != PLX_FP32) return set_error(dm, 1, "bad scalar type");
-    const size_t need = (size_t)(takes_pairs(dm, kp) ? kp->pairs.halo_slots : kp->halo_slots) * 3 * (scalar_type == PLX_FP64 ? sizeof(double) : sizeof(float));
+    // (a viscoelastic residual takes the tile plan)
+    const int64_t slots = kp->genmax ? kp->halo_slots
+                          : takes_pairs(dm, kp) ? kp->pairs.halo_slots
+                          : takes_gather(dm, kp) ? 0 : kp->halo_slots;
+    const size_t need = (size_t)slots * 3 * (scalar_type == PLX_FP64 ? sizeof(double) : sizeof(float));
     if (need > kScratchBytes)
         return set_error(dm, 1, "the key's shared-node partial sums (" + std::to_string(need) +
                                     " bytes) exceed the allocation-free scratch (" +

@@ -43,7 +43,9 @@ static void free_plan_arrays(KeyPlan *k) {
                     k->d_state,       k->d_gm_mat,        k->d_prestress,     k->d_load_node,
                     k->d_load64,      k->d_load32,        k->pairs.d_heads,
                     k->pairs.d_nodes, k->pairs.d_verts,   k->pairs.d_shared_node, k->pairs.d_shared_ptr,
-                    k->pairs.d_shared_slot, k->pairs.d_records, k->pairs.d_mat64, k->pairs.d_mat32};
+                    k->pairs.d_shared_slot, k->pairs.d_records, k->pairs.d_mat64, k->pairs.d_mat32,
+                    k->gather.d_heads, k->gather.d_nodes, k->gather.d_verts,  k->gather.d_records,
+                    k->gather.d_mat64, k->gather.d_mat32};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     KeyPlan fresh;
@@ -71,6 +73,28 @@ static void free_key(KeyPlan *k) {
     delete k;
 }
 
+// Packed per-cell records in tile order: Q1 8 x uint16 closure; P2 10 closure + 4 cone + 2 pad.
+static std::vector<uint16_t> cell_records(plx_dm dm, const HostPlan &hp) {
+    const int recw = dm->cell_type == PLX_HEX_Q1 ? 8 : 16;
+    const size_t n = hp.cells.size();
+    std::vector<uint16_t> rec(n * recw, 0);
+    for (size_t i = 0; i < n; ++i) {
+        for (int b = 0; b < dm->nb; ++b) rec[i * recw + b] = hp.lclosure[(size_t)b * n + i];
+        if (dm->cell_type != PLX_HEX_Q1)
+            for (int v = 0; v < dm->nv; ++v) rec[i * recw + dm->nb + v] = hp.lcone[(size_t)v * n + i];
+    }
+    return rec;
+}
+
+static std::vector<TileHead> tile_heads(const HostPlan &hp) {
+    std::vector<TileHead> heads(hp.num_tiles);
+    for (int t = 0; t < hp.num_tiles; ++t)
+        heads[t] = {hp.tile_cell_ptr[t], (hp.tile_cell_ptr[t + 1] - hp.tile_cell_ptr[t]) | hp.tile_ncolor[t] << 16,
+                    hp.tile_node_ptr[t], hp.tile_node_ptr[t + 1] - hp.tile_node_ptr[t], hp.tile_vert_ptr[t],
+                    hp.tile_vert_ptr[t + 1] - hp.tile_vert_ptr[t], hp.tile_nown[t], hp.tile_halo_off[t]};
+    return heads;
+}
+
 // Keys with fewer cells keep the tile kernel alone: two cells one after another per thread leave too few
 // waves there.  FP64 / FP32 apply, pairs against tiles: 48,000 cells 10.2 / 9.4 against 9.5 / 9.0 us, 83,000
 // 11.6 / 9.9 against 12.1 / 10.7 us, 196,000 17.2 / 14.5 against 20.9 / 17.5 us.
@@ -91,11 +115,11 @@ static int build_plan(plx_dm dm, KeyPlan *kp) {
     // tile (fewer halo nodes).  Measured on Q1 32^3: 10.5 us per apply at 256-cell tiles against
     // 13.1 us at 512; at 48^3 smaller tiles no longer pay.
     TileLimits lim = tile_limits(dm->cell_type);
+    int ncu = 0;
     {
         int64_t nkey = 0;
         for (int c = 0; c < dm->num_cells; ++c)
             if ((dm->labels.empty() ? 0 : dm->labels[c]) == kp->label_value) ++nkey;
-        int ncu = 0;
         if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, 0) != hipSuccess || ncu <= 0) ncu = 256;
         int cells = lim.cells;
         while (cells > 64 && nkey < (int64_t)cells * (ncu / 2)) cells >>= 1;
@@ -124,22 +148,10 @@ static int build_plan(plx_dm dm, KeyPlan *kp) {
     if ((err = upload(dm, &kp->d_lcone, hp.lcone.data(), hp.lcone.size()))) return err;
     if ((err = upload(dm, &kp->d_color, hp.color.data(), hp.color.size()))) return err;
     {
-        // packed per-cell records: Q1 8 x uint16 closure; P2 10 closure + 4 cone + 2 pad
-        const int recw = dm->cell_type == PLX_HEX_Q1 ? 8 : 16;
-        const size_t n = hp.cells.size();
-        std::vector<uint16_t> rec(n * recw, 0);
-        for (size_t i = 0; i < n; ++i) {
-            for (int b = 0; b < dm->nb; ++b) rec[i * recw + b] = hp.lclosure[(size_t)b * n + i];
-            if (dm->cell_type != PLX_HEX_Q1)
-                for (int v = 0; v < dm->nv; ++v) rec[i * recw + dm->nb + v] = hp.lcone[(size_t)v * n + i];
-        }
+        const std::vector<uint16_t> rec = cell_records(dm, hp);
         if ((err = upload(dm, &kp->d_records, rec.data(), rec.size()))) return err;
     }
-    std::vector<TileHead> heads(hp.num_tiles);
-    for (int t = 0; t < hp.num_tiles; ++t)
-        heads[t] = {hp.tile_cell_ptr[t], (hp.tile_cell_ptr[t + 1] - hp.tile_cell_ptr[t]) | hp.tile_ncolor[t] << 16,
-                    hp.tile_node_ptr[t], hp.tile_node_ptr[t + 1] - hp.tile_node_ptr[t], hp.tile_vert_ptr[t],
-                    hp.tile_vert_ptr[t + 1] - hp.tile_vert_ptr[t], hp.tile_nown[t], hp.tile_halo_off[t]};
+    const std::vector<TileHead> heads = tile_heads(hp);
     auto upload_heads = [&](int32_t **d, const std::vector<TileHead> &h) {
         return upload(dm, reinterpret_cast<TileHead **>(d), h.data(), h.size());
     };
@@ -191,6 +203,71 @@ static int build_plan(plx_dm dm, KeyPlan *kp) {
         kp->num_tiles_general = (int)gen.size();
         if ((err = upload_heads(&kp->d_heads_affine, aff))) return err;
         if ((err = upload_heads(&kp->d_heads_general, gen))) return err;
+    }
+    // Small keys whose elements are cheap (P2, affine hexes): a gather plan of two tiles per CU, all resident at
+    // once.  It evaluates the cells on tile boundaries several times but saves the second launch and the
+    // halo's way through memory.  FP64 / FP32 apply, gather against tiles + reduce_halo: 12^3 hexes 4.5 / 4.8
+    // against 8.0 / 8.3 us, 28^3 5.9 / 5.7 against 8.3 / 8.5, 38^3 (about the largest that fits) 7.3 / 6.6
+    // against 9.1 / 8.1; 6 x 8^3 tets 4.7 / 4.7 against 7.4 / 7.2, 6 x 16^3 7.0 / 7.0 against 8.3 / 7.8.  Not for
+    // the quadrature-point element of other hexes: 28^3 16.9 against 14.1 us.
+    if (dm->cell_type != PLX_HEX_Q1 || kp->num_tiles_general == 0) {
+        HostPlan gp;
+        bool fits = false;
+        if (build_gather_plan(mv, hp, 2 * ncu, &gp, &fits)) return set_error(dm, 1, "gather plan");
+        if (fits) {
+            GatherDev &G = kp->gather;
+            G.num_tiles = gp.num_tiles;
+            const std::vector<uint16_t> rec = cell_records(dm, gp);
+            if ((err = upload_heads(&G.d_heads, tile_heads(gp))) ||
+                (err = upload(dm, &G.d_nodes, gp.tile_nodes.data(), gp.tile_nodes.size())) ||
+                (err = upload(dm, &G.d_verts, gp.tile_verts.data(), gp.tile_verts.size())) ||
+                (err = upload(dm, &G.d_records, rec.data(), rec.size())))
+                return err;
+            G.cells = std::move(gp.cells);
+        }
+    }
+    return 0;
+}
+
+int repack_plans(plx_dm dm, KeyPlan *kp, const std::vector<double> &m64, const std::vector<float> &m32) {
+    const int n = (int)kp->cells.size();
+    int err = 0;
+    if (kp->pairs.num_tiles == 0 && kp->gather.num_tiles == 0) return 0;
+    std::vector<int32_t> at(dm->num_cells, -1);  // mesh cell -> key cell
+    for (int i = 0; i < n; ++i) at[kp->cells[i]] = i;
+    if (kp->gather.num_tiles > 0) {
+        GatherDev &G = kp->gather;
+        const size_t ng = G.cells.size();
+        std::vector<double> g64(2 * ng);
+        std::vector<float> g32(2 * ng);
+        for (size_t i = 0; i < ng; ++i)
+            for (size_t k = 0; k < 2; ++k) {
+                g64[k * ng + i] = m64[k * n + at[G.cells[i]]];
+                g32[k * ng + i] = m32[k * n + at[G.cells[i]]];
+            }
+        if (G.d_mat64) (void)hipFree(G.d_mat64);
+        if (G.d_mat32) (void)hipFree(G.d_mat32);
+        G.d_mat64 = nullptr;
+        G.d_mat32 = nullptr;
+        if ((err = upload(dm, &G.d_mat64, g64.data(), g64.size()))) return err;
+        if ((err = upload(dm, &G.d_mat32, g32.data(), g32.size()))) return err;
+    }
+    if (kp->pairs.num_tiles > 0) {
+        PairDev &P = kp->pairs;
+        std::vector<double> p64(4 * (size_t)P.num_pairs, 0.0);
+        std::vector<float> p32(4 * (size_t)P.num_pairs, 0.0f);
+        for (size_t i = 0; i < P.cells.size(); ++i)
+            if (P.cells[i] >= 0)
+                for (int k = 0; k < 2; ++k) {
+                    p64[2 * i + k] = m64[(size_t)k * n + at[P.cells[i]]];
+                    p32[2 * i + k] = m32[(size_t)k * n + at[P.cells[i]]];
+                }
+        if (P.d_mat64) (void)hipFree(P.d_mat64);
+        if (P.d_mat32) (void)hipFree(P.d_mat32);
+        P.d_mat64 = nullptr;
+        P.d_mat32 = nullptr;
+        if ((err = upload(dm, &P.d_mat64, p64.data(), p64.size()))) return err;
+        if ((err = upload(dm, &P.d_mat32, p32.data(), p32.size()))) return err;
     }
     return 0;
 }
@@ -386,25 +463,7 @@ static int repack_aux(plx_dm dm, KeyPlan *kp) {
     int err = 0;
     if ((err = upload(dm, &kp->d_mat64, m64.data(), m64.size()))) return err;
     if ((err = upload(dm, &kp->d_mat32, m32.data(), m32.size()))) return err;
-    if (kp->pairs.num_tiles > 0) {
-        PairDev &P = kp->pairs;
-        std::vector<int32_t> at(dm->num_cells, -1);  // mesh cell -> key cell
-        for (int i = 0; i < n; ++i) at[kp->cells[i]] = i;
-        std::vector<double> p64(4 * (size_t)P.num_pairs, 0.0);
-        std::vector<float> p32(4 * (size_t)P.num_pairs, 0.0f);
-        for (size_t i = 0; i < P.cells.size(); ++i)
-            if (P.cells[i] >= 0)
-                for (int k = 0; k < 2; ++k) {
-                    p64[2 * i + k] = m64[(size_t)k * n + at[P.cells[i]]];
-                    p32[2 * i + k] = m32[(size_t)k * n + at[P.cells[i]]];
-                }
-        if (P.d_mat64) (void)hipFree(P.d_mat64);
-        if (P.d_mat32) (void)hipFree(P.d_mat32);
-        P.d_mat64 = nullptr;
-        P.d_mat32 = nullptr;
-        if ((err = upload(dm, &P.d_mat64, p64.data(), p64.size()))) return err;
-        if ((err = upload(dm, &P.d_mat32, p32.data(), p32.size()))) return err;
-    }
+    if ((err = repack_plans(dm, kp, m64, m32))) return err;
     kp->has_aux = true;
     return build_load(dm, kp);
 }

@@ -62,6 +62,16 @@ struct PairDev {
     float *d_mat32 = nullptr;
 };
 
+// Device arrays of a small key's gather plan (build_gather_plan; num_tiles = 0: none).
+struct GatherDev {
+    int num_tiles = 0;
+    std::vector<int32_t> cells;      // tile order, cells on tile boundaries repeated
+    int32_t *d_heads = nullptr, *d_nodes = nullptr, *d_verts = nullptr;
+    uint16_t *d_records = nullptr;
+    double *d_mat64 = nullptr;       // [2][cells]
+    float *d_mat32 = nullptr;
+};
+
 struct KeyPlan {
     int label_value = 0;
     int part = 0;
@@ -87,6 +97,7 @@ struct KeyPlan {
     int32_t *d_heads_affine = nullptr, *d_heads_general = nullptr;  // Q1: those of affine cells / the others
     int num_tiles_affine = 0, num_tiles_general = 0;
     PairDev pairs;                   // P2: the factored path with LDS atomics
+    GatherDev gather;                // small keys: the default algorithm with LDS atomics
     int32_t *d_shared_node = nullptr, *d_shared_ptr = nullptr, *d_shared_slot = nullptr;
     void *d_halo = nullptr;          // halo partial sums, sized for FP64
     // auxiliary field, repacked per key cell (SoA, tile order)
@@ -252,7 +263,9 @@ struct SharedSums {
     const void *halo = nullptr;
 };
 SharedSums shared_sums(plx_dm dm, KeyPlan *kp, bool jacobian);
-bool takes_pairs(plx_dm dm, const KeyPlan *kp);  // whether the factored apply runs over the pair plan
+// Whether the apply without a state stress runs over the key's pair plan / gather plan.
+bool takes_pairs(plx_dm dm, const KeyPlan *kp);
+bool takes_gather(plx_dm dm, const KeyPlan *kp);
 // Per-device set-up at plx_dm_create with the DM's device current: the element tables in
 // constant memory and the device address of the allocation-free entry point's scratch array.
 int device_setup(plx_dm dm);
@@ -264,6 +277,8 @@ int launch_genmax_prestress(plx_dm dm, KeyPlan *kp);
 int launch_genmax_update(plx_dm dm, KeyPlan *kp, const double *u);
 int genmax_capture(plx_dm dm, KeyPlan *kp);
 int genmax_refresh(plx_dm dm, KeyPlan *kp);
+// The moduli (lambda, mu: [2][key cells], tile order) in the order of the key's pair and gather plans.
+int repack_plans(plx_dm dm, KeyPlan *kp, const std::vector<double> &m64, const std::vector<float> &m32);
 int validate_geometry(plx_dm dm, int *num_bad);
 
 // Cohesive cells and split-node maps (plx_fault.hip).

@@ -8,6 +8,7 @@
 #include <algorithm>
 #include <array>
 #include <cmath>
+#include <system_error>
 #include <thread>
 
 #include "plx_plan.hpp"
@@ -60,10 +61,17 @@ static void parallel_for(int n, const F &body) {
         return;
     }
     std::vector<std::thread> th;
-    for (int t = 0; t < nt; ++t)
-        th.emplace_back([&, t] {
+    th.reserve(nt);
+    for (int t = 0; t < nt; ++t) {
+        auto range = [&, t] {
             for (int i = (int)((int64_t)n * t / nt); i < (int)((int64_t)n * (t + 1) / nt); ++i) body(i);
-        });
+        };
+        try {
+            th.emplace_back(range);
+        } catch (const std::system_error &) {  // no thread to be had: this range runs here
+            range();
+        }
+    }
     for (auto &x : th) x.join();
 }
 
@@ -473,9 +481,15 @@ static void bisect(const MeshView &m, const std::vector<double> &cen, int32_t *o
     }
     if (depth < 3) {
         std::vector<int32_t> right;
-        std::thread t([&] { bisect(m, cen, order + cut, n - cut, right, depth + 1); });
+        auto upper = [&] { bisect(m, cen, order + cut, n - cut, right, depth + 1); };
+        std::thread t;
+        try {
+            t = std::thread(upper);
+        } catch (const std::system_error &) {
+            upper();
+        }
         bisect(m, cen, order, cut, sizes, depth + 1);
-        t.join();
+        if (t.joinable()) t.join();
         sizes.insert(sizes.end(), right.begin(), right.end());
     } else {
         bisect(m, cen, order, cut, sizes, depth + 1);
@@ -741,6 +755,181 @@ int build_pair_plan(const MeshView &m, const HostPlan &base, PairPlan *pp, std::
         pp->tile_vert_ptr.push_back((int32_t)pp->tile_verts.size());
     }
     pp->num_pairs = (int)(pp->cells.size() / 2);
+    return 0;
+}
+
+// --------------------------------------------------------------------------------------------
+// Gather plan.
+// --------------------------------------------------------------------------------------------
+
+// order[0 .. n) cut into `parts` equal parts by bisection along the longest axis; sizes appended in order.
+static void bisect_equal(const std::vector<double> &x, int32_t *order, int n, int parts, std::vector<int32_t> &sizes,
+                         int depth = 0) {
+    if (parts <= 1 || n <= 1) {
+        sizes.push_back(n);
+        return;
+    }
+    double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
+    for (int i = 0; i < n; ++i)
+        for (int d = 0; d < 3; ++d) {
+            lo[d] = std::min(lo[d], x[3 * (size_t)order[i] + d]);
+            hi[d] = std::max(hi[d], x[3 * (size_t)order[i] + d]);
+        }
+    int ax = 0;
+    for (int d = 1; d < 3; ++d)
+        if (hi[d] - lo[d] > hi[ax] - lo[ax]) ax = d;
+    const int left = parts / 2;
+    const int cut = std::max(1, (int)((int64_t)n * left / parts));
+    std::nth_element(order, order + cut, order + n, [&](int32_t a, int32_t b) {
+        const double u = x[3 * (size_t)a + ax], v = x[3 * (size_t)b + ax];
+        return u < v || (u == v && a < b);
+    });
+    std::vector<int32_t> right;
+    auto upper = [&] { bisect_equal(x, order + cut, n - cut, parts - left, right, depth + 1); };
+    std::thread t;
+    if (depth < 3 && n > 2000) try {
+            t = std::thread(upper);
+        } catch (const std::system_error &) {
+        }
+    bisect_equal(x, order, cut, left, sizes, depth + 1);
+    if (t.joinable()) t.join();
+    else upper();
+    sizes.insert(sizes.end(), right.begin(), right.end());
+}
+
+int build_gather_plan(const MeshView &m, const HostPlan &base, int max_tiles, HostPlan *gp, bool *fits) {
+    *fits = false;
+    *gp = HostPlan();
+    const int nb = m.nb, nv = m.nv;
+    // (an early way out: boxes of up to 38^3 hexes or 6 x 16^3 tets fit 512 tiles)
+    if (!m.coords || (int64_t)base.cells.size() > (int64_t)max_tiles * (nb == 8 ? 128 : 64)) return 0;
+    // the key's nodes, their positions (mean of the incident cells' centroids) and incident cells
+    std::vector<int32_t> cells(base.cells), nodes;
+    std::sort(cells.begin(), cells.end());
+    std::vector<double> x(3 * (size_t)m.num_nodes, 0.0);
+    std::vector<int32_t> ptr(m.num_nodes + 1, 0), inc;
+    for (int32_t c : cells) {
+        const int32_t *cl = m.closure + (size_t)c * nb, *cn = m.cone + (size_t)c * nv;
+        double mid[3] = {0.0, 0.0, 0.0};
+        for (int v = 0; v < nv; ++v)
+            for (int d = 0; d < 3; ++d) mid[d] += m.coords[3 * (size_t)cn[v] + d] / nv;
+        for (int b = 0; b < nb; ++b) {
+            for (int d = 0; d < 3; ++d) x[3 * (size_t)cl[b] + d] += mid[d];
+            ++ptr[cl[b] + 1];
+        }
+    }
+    for (int i = 0; i < m.num_nodes; ++i)
+        for (int d = 0; d < 3; ++d)
+            if (ptr[i + 1] > 0) x[3 * (size_t)i + d] /= ptr[i + 1];
+    for (int i = 0; i < m.num_nodes; ++i) {
+        if (ptr[i + 1] > 0) nodes.push_back(i);
+        ptr[i + 1] += ptr[i];
+    }
+    inc.resize(ptr[m.num_nodes]);
+    {
+        std::vector<int32_t> fill(ptr.begin(), ptr.end() - 1);
+        for (int32_t c : cells)
+            for (int b = 0; b < nb; ++b) inc[fill[m.closure[(size_t)c * nb + b]]++] = c;
+    }
+    // as many tiles as allowed (the work of a tile is what a call waits for), not below 32 nodes each
+    const int parts = std::max(1, std::min(max_tiles, (int)nodes.size() / 32));
+    std::vector<int32_t> order(nodes), sizes;
+    bisect_equal(x, order.data(), (int)order.size(), parts, sizes);
+    const TileLimits lim = tile_limits(nb == 8 ? 1 : 2);
+    gp->tile_cell_ptr.assign(1, 0);
+    gp->tile_node_ptr.assign(1, 0);
+    gp->tile_vert_ptr.assign(1, 0);
+    sizes.erase(std::remove(sizes.begin(), sizes.end(), 0), sizes.end());
+    std::vector<int32_t> first(1, 0);
+    for (int32_t sz : sizes) first.push_back(first.back() + sz);
+    struct Tile {
+        std::vector<int32_t> cells, nodes, verts;
+        std::vector<uint16_t> lcl, lcn;  // [cells][nb], [cells][nv]
+    };
+    std::vector<Tile> tiles(sizes.size());
+    parallel_for((int)tiles.size(), [&](int t) {
+        Tile &T = tiles[t];
+        std::vector<int32_t> tc, &tn = T.nodes, &tv = T.verts;
+        tn.assign(order.begin() + first[t], order.begin() + first[t + 1]);
+        std::sort(tn.begin(), tn.end());
+        for (int32_t i : tn) tc.insert(tc.end(), inc.begin() + ptr[i], inc.begin() + ptr[i + 1]);
+        distinct(tc);
+        // the other nodes and the vertices of the tile's cells, and every entry's place in the lists
+        std::vector<int32_t> other, own(tn);
+        for (int32_t c : tc) other.insert(other.end(), m.closure + (size_t)c * nb, m.closure + (size_t)(c + 1) * nb);
+        distinct(other);
+        for (int32_t g : other)
+            if (!std::binary_search(own.begin(), own.end(), g)) tn.push_back(g);
+        const auto node_at = [&](int32_t g) {
+            const auto i = std::lower_bound(own.begin(), own.end(), g);
+            if (i != own.end() && *i == g) return (size_t)(i - own.begin());
+            return (size_t)(std::lower_bound(tn.begin() + own.size(), tn.end(), g) - tn.begin());
+        };
+        if (!m.cone_is_closure) {
+            for (int32_t c : tc) tv.insert(tv.end(), m.cone + (size_t)c * nv, m.cone + (size_t)(c + 1) * nv);
+            distinct(tv);
+        }
+        std::vector<uint16_t> at;
+        for (int32_t c : tc)
+            for (int b = 0; b < nb; ++b) at.push_back((uint16_t)node_at(m.closure[(size_t)c * nb + b]));
+        // tets sorted by colour, so that a wave's atomic targets are mostly distinct (hexes keep mesh order:
+        // neighbouring lanes, spread banks)
+        std::vector<std::pair<int, int>> by;
+        std::vector<uint64_t> used(tn.size(), 0);
+        for (size_t i = 0; i < tc.size(); ++i) {
+            uint64_t mask = 0;
+            for (int b = 0; b < nb; ++b) mask |= used[at[i * nb + b]];
+            int k = 0;
+            while (k < 63 && ((mask >> k) & 1)) ++k;
+            for (int b = 0; b < nb; ++b) used[at[i * nb + b]] |= (uint64_t)1 << k;
+            by.emplace_back(nb == 8 ? 0 : k, (int)i);
+        }
+        std::sort(by.begin(), by.end());
+        for (const auto &e : by) {
+            const int32_t c = tc[e.second];
+            T.cells.push_back(c);
+            for (int b = 0; b < nb; ++b) T.lcl.push_back(at[(size_t)e.second * nb + b]);
+            for (int b = 0; b < nv && !m.cone_is_closure; ++b)
+                T.lcn.push_back((uint16_t)(std::lower_bound(tv.begin(), tv.end(), m.cone[(size_t)c * nv + b]) - tv.begin()));
+        }
+    });
+    for (size_t t = 0; t < tiles.size(); ++t) {
+        const Tile &T = tiles[t];
+        if ((int)T.cells.size() > kGatherCells || (int)T.nodes.size() > lim.nodes || (int)T.verts.size() > lim.verts) {
+            *gp = HostPlan();
+            return 0;
+        }
+        gp->cells.insert(gp->cells.end(), T.cells.begin(), T.cells.end());
+        gp->tile_nodes.insert(gp->tile_nodes.end(), T.nodes.begin(), T.nodes.end());
+        gp->tile_verts.insert(gp->tile_verts.end(), T.verts.begin(), T.verts.end());
+        gp->tile_cell_ptr.push_back((int32_t)gp->cells.size());
+        gp->tile_node_ptr.push_back((int32_t)gp->tile_nodes.size());
+        gp->tile_vert_ptr.push_back((int32_t)gp->tile_verts.size());
+        gp->tile_nown.push_back(sizes[t]);
+        gp->tile_halo_off.push_back(0);
+        gp->tile_ncolor.push_back(1);
+        gp->max_nodes = std::max(gp->max_nodes, (int)T.nodes.size());
+        gp->max_verts = std::max(gp->max_verts, (int)T.verts.size());
+    }
+    gp->num_tiles = (int)gp->tile_nown.size();
+    const size_t n = gp->cells.size();
+    gp->color.assign(n, 0);
+    gp->lclosure.resize(nb * n);
+    gp->lcone.resize(nv * n);
+    for (int t = 0; t < gp->num_tiles; ++t)
+        for (int i = gp->tile_cell_ptr[t]; i < gp->tile_cell_ptr[t + 1]; ++i) {
+            const size_t k = (size_t)(i - gp->tile_cell_ptr[t]);
+            for (int b = 0; b < nb; ++b) gp->lclosure[(size_t)b * n + i] = tiles[t].lcl[k * nb + b];
+            if (!m.cone_is_closure)
+                for (int b = 0; b < nv; ++b) gp->lcone[(size_t)b * n + i] = tiles[t].lcn[k * nv + b];
+        }
+    if (m.cone_is_closure) {
+        gp->tile_verts = gp->tile_nodes;
+        gp->tile_vert_ptr = gp->tile_node_ptr;
+        gp->lcone = gp->lclosure;
+        gp->max_verts = gp->max_nodes;
+    }
+    *fits = true;
     return 0;
 }
 

@@ -75,6 +75,15 @@ inline int pair_vert(const uint32_t *w, int j) { return j < 4 ? (int)((w[5] >> (
 // centroids; where that gives no fewer halo slots than the base plan's tiles, those are kept.
 int build_pair_plan(const MeshView &m, const HostPlan &base, PairPlan *pp, std::string *err);
 
+// Gather plan of a small key: tiles own nodes instead of cells.  Each tile holds every cell that touches
+// one of its nodes (cells on tile boundaries appear in several tiles and are evaluated in each), so
+// its sums are complete and nothing is left for a second pass: halo_slots = 0, and only the first
+// tile_nown nodes of a tile's list are written.  `cells` repeats the duplicated cells.  At most
+// max_tiles tiles of at most kGatherCells cells (one per thread); *fits is false, and the plan empty, when the key is too
+// large for that.
+constexpr int kGatherCells = 256;
+int build_gather_plan(const MeshView &m, const HostPlan &base, int max_tiles, HostPlan *gp, bool *fits);
+
 // sort_by_color: order each tile's cells by colour (colour-phase accumulation activates
 // contiguous threads); otherwise cells keep their mesh order inside the tile (neighbouring
 // threads then touch neighbouring nodes: structured LDS access for atomic accumulation).

@@ -106,3 +106,34 @@ def test_emulated_pair_kernel_matches_tile_kernel(name):
     assert relerr(r32.astype(np.float64), ref) <= 2e-5
     radd = emulate(m, aux, u, label, mode=L.ADD_VALUES, r0=np.ones_like(u), algo=EMULATE_PAIRS)
     assert relerr(radd - 1.0, ref) <= 1e-11
+
+
+EMULATE_GATHER = 101  # PLX_EMULATE_GATHER
+
+
+def gather_cases():
+    big = mg.tet_p2_box(6, (0, 0, 0), (1.0, 1.0, 1.0))
+    big.labels = (np.arange(big.num_cells) % 3 == 0).astype(np.int32)
+    return {
+        "one_hex": (mg.hex_box(1, (0, 0, 0), (1.0, 1.0, 1.0)), 0),
+        "one_cube": (mg.tet_p2_box(1, (0, 0, 0), (1.0, 1.0, 1.0)), 0),
+        "tet_label": (big, 1),  # nodes of the mesh outside the key
+        "hex_max": (mg.hex_box(38, (0, 0, 0), (1.0, 1.0, 1.0)), 0),  # about the largest that fits 512 tiles
+        "tet_large": (mg.tet_p2_box(16, (0, 0, 0), (1.0, 1.0, 1.0)), 0),
+        **cases(),
+    }
+
+
+@pytest.mark.parametrize("name", list(gather_cases()))
+def test_emulated_gather_plan_matches_tile_plan(name):
+    """The tile kernel over the gather plan against the tile plan's emulation: the same sums in another
+    order (rounding of at most some 24 additions per node in FP64, of the element products in FP32)."""
+    m, label = gather_cases()[name]
+    aux, _ = mg.elastic_aux(m.num_cells, seed=5, vs_sigma=0.2, vp_vs=1.8)
+    u = mg.random_field(m.num_nodes, 3)
+    ref = emulate(m, aux, u, label)
+    assert relerr(emulate(m, aux, u, label, algo=EMULATE_GATHER), ref) <= 1e-13
+    r32 = emulate(m, aux, u, label, scalar=L.FP32, algo=EMULATE_GATHER)
+    assert relerr(r32.astype(np.float64), ref) <= 2e-5
+    radd = emulate(m, aux, u, label, mode=L.ADD_VALUES, r0=np.ones_like(u), algo=EMULATE_GATHER)
+    assert relerr(radd - 1.0, ref) <= 1e-11

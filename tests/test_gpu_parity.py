@@ -188,6 +188,32 @@ def test_p2_pair_kernel(oracle, kind):
         assert relerr(r.double().cpu().numpy(), ref) <= tol
 
 
+# either side of the line where a key takes the gather plan (38^3 hexes and 6 x 16^3 tets are about the
+# largest), non-affine hexes, and a mesh of affine and other hex tiles
+@pytest.mark.parametrize("kind", ["hex38", "hex41", "hex_warped", "hex_mixed", "tet16", "tet18"])
+def test_gather_plan(oracle, kind):
+    n = int(kind[3:]) if kind[3:].isdigit() else 14
+    if kind.startswith("tet"):
+        m = mg.tet_p2_box(n, (0, 0, 0), (100.0 * n,) * 3)
+    else:
+        m = mg.hex_box(n, (0, 0, 0), (100.0 * n,) * 3)
+    if n == 14:
+        x = m.coords.copy()
+        move = x[:, 0] > (0.0 if kind == "hex_warped" else 700.0)
+        x[move] += np.random.default_rng(4).uniform(-15, 15, (int(move.sum()), 3))
+        m.coords = m.node_coords = x
+    aux, sizes = mg.elastic_aux(m.num_cells, seed=6, vs_sigma=0.2, vp_vs=1.8)
+    u = mg.random_field(m.num_nodes, 9)
+    dm, ref = check_residual(oracle, m, u, aux=(aux, sizes))
+    dm.set_kernel_options()
+    for dt, tol in ((torch.float64, TOL64), (torch.float32, TOL32)):
+        x = dev(u, dt)
+        r = torch.zeros_like(x)
+        dm.compute_residual_noalloc(0, 0, x, r, mode=1)
+        torch.cuda.synchronize()
+        assert relerr(r.double().cpu().numpy(), ref) <= tol
+
+
 def test_deterministic_bitwise(oracle):
     m = mg.tet_p2_box(8, (0, 0, 0), (1.0, 1.0, 1.0))
     aux, sizes = mg.elastic_aux(m.num_cells)
