@@ -217,6 +217,7 @@ static int build_plan(plx_dm dm, KeyPlan *kp) {
         if (fits) {
             GatherDev &G = kp->gather;
             G.num_tiles = gp.num_tiles;
+            for (int32_t k : gp.tile_nown) G.num_owned += k;
             const std::vector<uint16_t> rec = cell_records(dm, gp);
             if ((err = upload_heads(&G.d_heads, tile_heads(gp))) ||
                 (err = upload(dm, &G.d_nodes, gp.tile_nodes.data(), gp.tile_nodes.size())) ||

@@ -64,7 +64,7 @@ struct PairDev {
 
 // Device arrays of a small key's gather plan (build_gather_plan; num_tiles = 0: none).
 struct GatherDev {
-    int num_tiles = 0;
+    int num_tiles = 0, num_owned = 0;  // num_owned: the key's nodes
     std::vector<int32_t> cells;      // tile order, cells on tile boundaries repeated
     int32_t *d_heads = nullptr, *d_nodes = nullptr, *d_verts = nullptr;
     uint16_t *d_records = nullptr;
@@ -266,6 +266,21 @@ SharedSums shared_sums(plx_dm dm, KeyPlan *kp, bool jacobian);
 // Whether the apply without a state stress runs over the key's pair plan / gather plan.
 bool takes_pairs(plx_dm dm, const KeyPlan *kp);
 bool takes_gather(plx_dm dm, const KeyPlan *kp);
+
+// The vector work that rides on a gather-plan apply in a CG iteration: beta = rz / *rz_old with rz the sum
+// of nblk partials (kept in *rz), p_out = z + beta u, r = scale A p_out with zeros at fixed dofs, and
+// the partials of p_out.r, one per tile.
+struct CgArgs {
+    const void *z;
+    void *p_out;
+    const uint8_t *fixed;  // per node, bit c: component c
+    const double *part_rz;
+    int nblk;
+    double *rz;
+    const double *rz_old;
+    double *part_pq;  // [gather.num_tiles]
+};
+int launch_cg_apply(plx_dm dm, KeyPlan *kp, int scalar_type, const void *u, void *r, double scale, const CgArgs &C);
 // Per-device set-up at plx_dm_create with the DM's device current: the element tables in
 // constant memory and the device address of the allocation-free entry point's scratch array.
 int device_setup(plx_dm dm);

@@ -25,6 +25,7 @@
 
 #include "plx_element.hpp"
 #include "plx_internal.hpp"
+#include "plx_reduce.hpp"
 
 namespace plx {
 
@@ -35,17 +36,6 @@ template <typename Real>
 __global__ void __launch_bounds__(256) mask_kernel(int n, const int32_t *__restrict__ dofs, Real *v) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) v[dofs[i]] = Real(0);
-}
-
-// Block sum of 256 threads (every thread gets it; fixed order): shuffles inside the waves, then the four
-// wave sums.
-__device__ __forceinline__ double block_sum(double v, double *s) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0) s[threadIdx.x >> 6] = v;
-    __syncthreads();
-    return (s[0] + s[1]) + (s[2] + s[3]);
 }
 
 template <typename Real>
@@ -234,13 +224,6 @@ __global__ void __launch_bounds__(256) finish_start(const double *__restrict__ p
 // 22 x 24 x 21 x 6 tets: 5.8 -> 5.0 ms a solve.
 // --------------------------------------------------------------------------------------------
 
-// Sum of n partials by the whole block.
-__device__ __forceinline__ double total(const double *__restrict__ part, int n, double *s) {
-    double acc = 0.0;
-    for (int i = threadIdx.x; i < n; i += 256) acc += part[i];
-    return block_sum(acc, s);
-}
-
 enum { kFinishDot = 0, kFinishResid, kFinishPost };
 // One thread per node: q = A x there (its row of y, or the sum of its halo slots range[node] when
 // tiles share it), zero at constrained dofs.  Dot: y = q, partials of x.q; Resid: out = b - q;
@@ -268,9 +251,10 @@ __global__ void __launch_bounds__(256) node_finish(int nnodes, const int2 *__res
 #pragma unroll
             for (int c = 0; c < 3; ++c) q[c] = y[o + c];
         }
+        const int fx = fixed[node];
 #pragma unroll
         for (int c = 0; c < 3; ++c)
-            if (fixed[o + c]) q[c] = Real(0);
+            if ((fx >> c) & 1) q[c] = Real(0);
         if (MODE == kFinishDot) {
 #pragma unroll
             for (int c = 0; c < 3; ++c) {
@@ -318,21 +302,35 @@ __global__ void __launch_bounds__(256) cg_step(int nnodes, const Real *__restric
                                                const double *__restrict__ part_pq, int nblk, double *scal,
                                                double *part_rz, double *part_rr) {
     __shared__ double s[4];
+    // the first node's loads go out before the sum is waited for
+    int node = blockIdx.x * 256 + threadIdx.x;
+    Real xv[3], rv[3], pv[3], qv[3], Bv[9];
+    auto load = [&]() {
+        const size_t o = 3 * (size_t)min(node, nnodes - 1);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            xv[c] = x[o + c];
+            rv[c] = r[o + c];
+            pv[c] = p[o + c];
+            qv[c] = q[o + c];
+        }
+#pragma unroll
+        for (int c = 0; c < 9; ++c) Bv[c] = Binv[3 * o + c];
+    };
+    load();
     const Real alpha = (Real)alpha_of(part_pq, nblk, scal, s);
     double rz = 0.0, rr = 0.0;
-    for (int node = blockIdx.x * 256 + threadIdx.x; node < nnodes; node += gridDim.x * 256) {
+    for (; node < nnodes; node += gridDim.x * 256, load()) {
         const size_t o = 3 * (size_t)node;
-        Real rv[3];
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
-            x[o + c] += alpha * p[o + c];
-            rv[c] = r[o + c] - alpha * q[o + c];
+            x[o + c] = xv[c] + alpha * pv[c];
+            rv[c] -= alpha * qv[c];
             r[o + c] = rv[c];
         }
-        const Real *B = Binv + 9 * (size_t)node;
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
-            const Real zc = B[3 * c] * rv[0] + B[3 * c + 1] * rv[1] + B[3 * c + 2] * rv[2];
+            const Real zc = Bv[3 * c] * rv[0] + Bv[3 * c + 1] * rv[1] + Bv[3 * c + 2] * rv[2];
             z[o + c] = zc;
             rz += (double)rv[c] * (double)zc;
             rr += (double)rv[c] * (double)rv[c];
@@ -398,6 +396,19 @@ __global__ void __launch_bounds__(256) p_step(int64_t n, const ZReal *__restrict
     }
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256)
         p[i] = (Real)z[i] + beta * p[i];
+}
+
+// rz and rr from their partials; at the start of a solve also rz_old = inf, so that the first
+// direction is p = z + 0 p.
+__global__ void __launch_bounds__(256) cg_totals(const double *__restrict__ part_rz, const double *__restrict__ part_rr,
+                                                 int nblk, double *scal, bool start) {
+    __shared__ double s[4];
+    const double rz = total(part_rz, nblk, s), rr = total(part_rr, nblk, s);
+    if (threadIdx.x == 0) {
+        scal[S_RZ] = rz;
+        scal[S_RR] = rr;
+        if (start) scal[S_RZOLD] = __builtin_inf();
+    }
 }
 
 template <typename Src, typename Dst>
@@ -472,6 +483,7 @@ struct plx_solver_s {
     // FGMRES bases
     int restart = 30;
     std::vector<double *> V, Z;
+    double *p2 = nullptr;            // the other direction buffer of the two-kernel iteration (either type)
     double *scal = nullptr, *part_a = nullptr, *part_b = nullptr, *part_c = nullptr;
     // one key without a fault: where its apply leaves each node's sum (range: halo slots, empty for nodes
     // of one tile) and the constrained dofs, made at the DM's epoch
@@ -518,16 +530,25 @@ static int apply_keys(plx_solver s, int st, const void *x, void *y, double scale
 // Whether iterations take the fused kernels (one key, no fault).
 static bool fused(const plx_solver_s *s) { return s->keys.size() == 1 && !s->fault; }
 
+// Whether point-block Jacobi iterations take the two-kernel form: the direction update and the dot product
+// ride on the gather plan's apply.
+static bool gathered(const plx_solver_s *s) {
+    const KeyPlan *kp = s->keys[0];
+    return fused(s) && !s->amg && takes_gather(s->dm, kp) && kp->gather.num_owned == s->nnodes &&
+           kp->gather.num_tiles <= kRedBlocks;
+}
+
 // The node map and mask of the fused kernels, for the DM's present options and constraints (before a
 // solve, outside any capture).
 static int ensure_finish(plx_solver s) {
     plx_dm dm = s->dm;
     if (!fused(s) || s->finish_epoch == dm->epoch) return 0;
     if (!s->range) PLX_HIP(dm, hipMalloc(&s->range, (size_t)s->nnodes * sizeof(int2)));
-    if (!s->fixed) PLX_HIP(dm, hipMalloc(&s->fixed, (size_t)s->n));
-    std::vector<uint8_t> mask(s->n, 0);
+    if (!s->fixed) PLX_HIP(dm, hipMalloc(&s->fixed, (size_t)s->nnodes));
+    if (gathered(s) && !s->p2) PLX_HIP(dm, hipMalloc(&s->p2, (size_t)s->n * sizeof(double)));
+    std::vector<uint8_t> mask(s->nnodes, 0);
     for (int32_t d : dm->con.dofs)
-        if (d < s->n) mask[d] = 1;
+        if (d < 3 * s->nnodes) mask[d / 3] |= (uint8_t)(1 << d % 3);
     PLX_HIP(dm, hipMemcpyAsync(s->fixed, mask.data(), mask.size(), hipMemcpyHostToDevice, dm->stream));
     PLX_HIP(dm, hipMemsetAsync(s->range, 0, (size_t)s->nnodes * sizeof(int2), dm->stream));
     s->sums = shared_sums(dm, s->keys[0], true);
@@ -764,9 +785,14 @@ static int pcg(plx_solver s, Real *x, Real *r, Real *p, Real *q, Real *z, const 
     if (s->amg) return pcg_amg<Real>(s, x, r, p, q, z, rtol, maxit, its, rnorm_out);
     plx_dm dm = s->dm;
     // r = b - A x  (caller stored b in r; x == 0 guess skips the apply)
-    hipLaunchKernelGGL(pc_start<Real>, red_grid(), dim3(256), 0, dm->stream, s->nnodes, Binv, r, z, p,
+    const bool two = gathered(s);
+    const int nblk = node_blocks(s);
+    hipLaunchKernelGGL(pc_start<Real>, two ? dim3(nblk) : red_grid(), dim3(256), 0, dm->stream, s->nnodes, Binv, r, z, p,
                        s->part_a, s->part_b);
-    hipLaunchKernelGGL(finish_start, dim3(1), dim3(256), 0, dm->stream, s->part_a, s->part_b, s->scal);
+    if (two)
+        hipLaunchKernelGGL(cg_totals, dim3(1), dim3(256), 0, dm->stream, s->part_a, s->part_b, nblk, s->scal, true);
+    else
+        hipLaunchKernelGGL(finish_start, dim3(1), dim3(256), 0, dm->stream, s->part_a, s->part_b, s->scal);
     PLX_HIP(dm, hipGetLastError());
     double rr0 = 0.0;
     int err = read_scalar(s, S_RR, &rr0);
@@ -774,10 +800,21 @@ static int pcg(plx_solver s, Real *x, Real *r, Real *p, Real *q, Real *z, const 
     const double target = rtol * rtol * rr0;
     int it = 0;
     double rr = rr0;
-    const int check = 10;
-    auto iteration = [&]() -> int {
+    constexpr int check = 10;
+    // k: parity of the iteration in its chunk (the two-kernel form alternates between two direction buffers)
+    static_assert(check % 2 == 0, "a chunk ends on the buffer it began with");
+    auto iteration = [&](int k) -> int {
+        if (two) {
+            Real *pa = (k & 1) ? reinterpret_cast<Real *>(s->p2) : p, *pb = (k & 1) ? p : reinterpret_cast<Real *>(s->p2);
+            const CgArgs C{z, pb, s->fixed, s->part_a, nblk, s->scal + S_RZ, s->scal + S_RZOLD, s->part_c};
+            const int st = std::is_same<Real, double>::value ? PLX_FP64 : PLX_FP32;
+            if (const int e = launch_cg_apply(dm, s->keys[0], st, pa, q, -1.0, C)) return e;
+            hipLaunchKernelGGL(cg_step<Real>, dim3(nblk), dim3(256), 0, dm->stream, s->nnodes, Binv, x, r, pb, q, z,
+                               s->part_c, s->keys[0]->gather.num_tiles, s->scal, s->part_a, s->part_b);
+            PLX_HIP(dm, hipGetLastError());
+            return 0;
+        }
         if (fused(s)) {
-            const int nblk = node_blocks(s);
             const int e = apply_finish<Real, kFinishDot>(s, p, q, nullptr, nullptr, Real(0), nullptr, s->part_c);
             if (e) return e;
             hipLaunchKernelGGL(cg_step<Real>, dim3(nblk), dim3(256), 0, dm->stream, s->nnodes, Binv, x, r, p, q, z,
@@ -798,18 +835,25 @@ static int pcg(plx_solver s, Real *x, Real *r, Real *p, Real *q, Real *z, const 
         PLX_HIP(dm, hipGetLastError());
         return 0;
     };
+    auto totals = [&]() -> int {  // the residual norm after the last iteration, for the host
+        if (!two) return 0;
+        hipLaunchKernelGGL(cg_totals, dim3(1), dim3(256), 0, dm->stream, s->part_a, s->part_b, nblk, s->scal, false);
+        PLX_HIP(dm, hipGetLastError());
+        return 0;
+    };
     while (it < maxit && rr > target && rr0 > 0.0) {
         if (it + check <= maxit) {
             err = run_chunk(s, 10 * sizeof(Real) + 1, x, r, [&]() -> int {
                 for (int k = 0; k < check; ++k)
-                    if (int e = iteration()) return e;
-                return 0;
+                    if (int e = iteration(k)) return e;
+                return totals();
             });
             if (err) return err;
             it += check;
         } else {
             for (; it < maxit; ++it)
-                if ((err = iteration())) return err;
+                if ((err = iteration(it))) return err;
+            if ((err = totals())) return err;
         }
         if ((err = read_scalar(s, S_RR, &rr))) return err;
     }
@@ -1016,7 +1060,7 @@ int plx_solver_create(plx_solver *out, plx_dm dm, int label_value, int part) {
 
 int plx_solver_destroy(plx_solver s) {
     if (!s) return 0;
-    void *ptrs[] = {s->range,  s->fixed,  s->part_c,
+    void *ptrs[] = {s->range,  s->fixed,  s->part_c, s->p2,
                     s->Binv64, s->Binv32, s->scal, s->part_a, s->part_b, s->x32, s->r32, s->p32,
                     s->q32,    s->z32,    s->r64,  s->p64,    s->q64,    s->z64, s->t64};
     for (void *p : ptrs)

@@ -231,3 +231,30 @@ def test_two_materials_solve_matches_dense_direct(oracle, method, pc, kind):
     assert st["converged"], st
     err = np.abs(x.cpu().numpy() - ref).max() / np.abs(ref).max()
     assert err <= 1e-9, err
+
+
+@pytest.mark.parametrize("kind", ["hex", "hex44", "tet", "tet_pairs"])
+@pytest.mark.parametrize("maxit", [1, 13, 20])
+def test_iterates_agree_over_plans(kind, maxit):
+    """The same number of CG iterations over the default plan (gather: two kernels an iteration, or tiles,
+    or pairs: four), over the coloured tiles after a change of options on the same solver, and back.
+    Rounding differs by some 1e-16 per operation, which 20 iterations amplify little: 1e-10."""
+    if kind.startswith("hex"):
+        m = mg.hex_box((44, 41, 42) if kind == "hex44" else (9, 14, 11), (0, 0, 0), (6000.0, 6000.0, 6000.0))
+    else:
+        m = mg.tet_p2_box((27, 21, 22) if kind == "tet_pairs" else (5, 8, 6), (0, 0, 0), (6000.0, 6000.0, 6000.0))
+    aux, sizes = mg.elastic_aux(m.num_cells, seed=4, vs_sigma=0.2, vp_vs=1.732)
+    dofs, vals = mg.shear_bcs(m.node_coords, 0.0, 6000.0)
+    dm, solver = build(m, aux, sizes, dofs)
+    out = []
+    for acc in (L.ACCUMULATE_AUTO, L.ACCUMULATE_COLORED, L.ACCUMULATE_AUTO):
+        dm.set_kernel_options(L.ALGO_AUTO, acc)
+        x = torch.zeros(3 * m.num_nodes, dtype=torch.float64, device="cuda")
+        dm.insert_boundary_values(torch.from_numpy(vals).cuda(), x)
+        st = solver.solve(x, method=L.KSP_CG, rtol=1e-30, maxit=maxit)
+        torch.cuda.synchronize()
+        out.append((x.cpu().numpy(), (st["outer_iterations"], st["inner_iterations"])))
+    scale = np.abs(out[0][0]).max()
+    for x, its in out[1:]:
+        assert np.abs(x - out[0][0]).max() / scale <= 1e-10
+        assert its == out[0][1]
