@@ -20,6 +20,7 @@
 #include <chrono>
 #include <cmath>
 #include <thread>
+#include <utility>
 #include <vector>
 
 #include "../../include/pylith_amd_debug.h"
@@ -307,9 +308,52 @@ __global__ void __launch_bounds__(256) gfk_spmm_dot(int nrows, const int32_t *__
     if ((int)threadIdx.x < K) ppq[(size_t)blockIdx.x * K + threadIdx.x] = s[threadIdx.x];
 }
 
-// K = 64: one wavefront per block row, lane = column.  The row index is wave-uniform, so the
-// row's column indices and 3x3 blocks come through scalar loads and each neighbour's three
-// values are one coalesced 256-byte vector load per component.
+// Block row times a 64-column block on the matrix cores: y (rows 0 .. 2 in the vector's entries, lane =
+// column) += sum over the row's blocks e of val[e] X[col[e]].  v_mfma_f32_4x4x1 multiplies sixteen 4 x 1 by
+// 1 x 4 pairs; with the first operand broadcast (CBSZ = 4, ABID = k: lanes 4k .. 4k + 3 to all sixteen) it adds one
+// column of a 3 x 3 block times one component of the neighbour's 64 values as they lie in memory.  One vector
+// load brings U blocks (lane 4 (BC m + q) + i: entry (i, q) of block m; the fourth row is not used).
+// The products were bound by the blocks' scalar loads, 9 words a block through the scalar caches: 91,000 rows of
+// 27 blocks 195 us (residual) and 180 us (with the dot product), here 158 and 146 us, which the neighbours' vectors
+// (1.9 GB, from L2 for the most part) bound; 3 x 6 prolongation 86 us, here 70.  Sharing the vectors between
+// four rows of a wave did not help: 160 us with zero blocks where a row lacks a column, 315 us with scalar
+// blocks and a branch.
+typedef float gf_f4 __attribute__((ext_vector_type(4)));
+
+template <int... T>
+__device__ __forceinline__ void gf_mfma_columns(std::integer_sequence<int, T...>, float a, const float *x, gf_f4 &y) {
+    ((y = __builtin_amdgcn_mfma_f32_4x4x1f32(a, x[T], y, 4, T, 0)), ...);
+}
+
+template <int BC>
+__device__ __forceinline__ gf_f4 gf_row64(int e0, int e1, const int32_t *__restrict__ col, const float *__restrict__ val,
+                                          const float *__restrict__ X, int lane) {
+    constexpr int U = 16 / BC;                 // blocks per vector load
+    constexpr int C = 2;                       // loads, and their columns, in flight
+    const int m = (lane >> 2) / BC, q = (lane >> 2) % BC, i = min(lane & 3, 2);
+    gf_f4 y = {0.f, 0.f, 0.f, 0.f};
+    for (int e = e0; e < e1; e += C * U) {
+        float a[C], x[C][U * BC];
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+            const int em = e + c * U + m;
+            a[c] = val[3 * BC * (size_t)min(em, e1 - 1) + BC * i + q];
+            if (m >= U || em >= e1) a[c] = 0.f;  // no block there (its column repeats the row's last)
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const size_t j = (size_t)col[min(e + c * U + u, e1 - 1)];
+#pragma unroll
+                for (int p = 0; p < BC; ++p) x[c][u * BC + p] = X[(BC * j + p) * 64 + lane];
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < C; ++c) gf_mfma_columns(std::make_integer_sequence<int, U * BC>(), a[c], x[c], y);
+    }
+    return y;
+}
+
+// K = 64: one wavefront per block row, lane = column: the row's column indices come through scalar
+// loads and each neighbour's three values are one coalesced 256-byte vector load per component.
 __global__ void __launch_bounds__(256) gfk_spmm_dot64(int nrows, const int32_t *__restrict__ row_ptr,
                                                       const int32_t *__restrict__ col,
                                                       const float *__restrict__ val, const float *__restrict__ P,
@@ -321,39 +365,12 @@ __global__ void __launch_bounds__(256) gfk_spmm_dot64(int nrows, const int32_t *
     gf_xcd_slab(nrows, lo, hi, jb, nbx);
     for (int row0 = lo + jb * 4 + (int)(threadIdx.x >> 6); row0 < hi; row0 += nbx * 4) {
         const int row = __builtin_amdgcn_readfirstlane(row0);
-        const int e0 = row_ptr[row], e1 = row_ptr[row + 1];
-        float y0 = 0.f, y1 = 0.f, y2 = 0.f;
-        int e = e0;
-        // groups of 9 neighbours: all 27 loads of a group are issued before the arithmetic
-        for (; e + 9 <= e1; e += 9) {
-            float x[9][3];
-#pragma unroll
-            for (int m = 0; m < 9; ++m) {
-                const size_t j = (size_t)col[e + m];
-#pragma unroll
-                for (int c = 0; c < 3; ++c) x[m][c] = P[(3 * j + c) * 64 + lane];
-            }
-#pragma unroll
-            for (int m = 0; m < 9; ++m) {
-                const float *A = val + 9 * (size_t)(e + m);
-                y0 += A[0] * x[m][0] + A[1] * x[m][1] + A[2] * x[m][2];
-                y1 += A[3] * x[m][0] + A[4] * x[m][1] + A[5] * x[m][2];
-                y2 += A[6] * x[m][0] + A[7] * x[m][1] + A[8] * x[m][2];
-            }
-        }
-        for (; e < e1; ++e) {
-            const size_t j = (size_t)col[e];
-            const float *A = val + 9 * (size_t)e;
-            const float x0 = P[(3 * j) * 64 + lane], x1 = P[(3 * j + 1) * 64 + lane], x2 = P[(3 * j + 2) * 64 + lane];
-            y0 += A[0] * x0 + A[1] * x1 + A[2] * x2;
-            y1 += A[3] * x0 + A[4] * x1 + A[5] * x2;
-            y2 += A[6] * x0 + A[7] * x1 + A[8] * x2;
-        }
+        const gf_f4 y = gf_row64<3>(row_ptr[row], row_ptr[row + 1], col, val, P, lane);
         const size_t o = (3 * (size_t)row) * 64 + lane;
-        Q[o] = y0;
-        Q[o + 64] = y1;
-        Q[o + 128] = y2;
-        acc += (double)P[o] * y0 + (double)P[o + 64] * y1 + (double)P[o + 128] * y2;
+        Q[o] = y[0];
+        Q[o + 64] = y[1];
+        Q[o + 128] = y[2];
+        acc += (double)P[o] * y[0] + (double)P[o + 64] * y[1] + (double)P[o + 128] * y[2];
     }
     s[threadIdx.x] = acc;
     __syncthreads();
@@ -446,6 +463,12 @@ __global__ void __launch_bounds__(256) amg_bsr(int nrows, const int32_t *__restr
 #pragma unroll
         for (int a = 0; a < BR; ++a) y[a] = 0.f;
         int e = e0;
+        if constexpr (K == 64 && BR == 3) {
+            const gf_f4 v = gf_row64<BC>(e0, e1, col, val, X, lane);
+#pragma unroll
+            for (int a = 0; a < 3; ++a) y[a] = v[a];
+            e = e1;
+        }
         for (; e + U <= e1; e += U) {
             float x[U][BC];
 #pragma unroll
