@@ -30,7 +30,9 @@
 
 namespace plx {
 
-constexpr int kGfRed = 2048;  // blocks of the grid-stride block kernels (= per-column partials)
+// Blocks of the grid-stride block kernels, and of one column's partials ([column][kGfRed]): a thread per
+// (node, column), at most kGfRed blocks.
+constexpr int kGfRed = 2048;
 enum { G_RZ = 0, G_PQ, G_ALPHA, G_BETA, G_RR, G_COUNT };
 
 // ---------------------------------------------------------------------------------------------
@@ -212,14 +214,14 @@ __global__ void __launch_bounds__(256) gf_dot(int64_t ndof, int k, const Real *_
         acc += (double)a[t] * (double)b[t];
     s[threadIdx.x] = acc;
     col_reduce(s, k);
-    if ((int)threadIdx.x < k) partials[(size_t)blockIdx.x * k + threadIdx.x] = s[threadIdx.x];
+    if ((int)threadIdx.x < k) partials[(size_t)threadIdx.x * kGfRed + blockIdx.x] = s[threadIdx.x];
 }
 
 // Column r of the per-block partials summed by block r (256 threads, fixed-order tree).
-__device__ __forceinline__ double col_sum(const double *partials, int k, int r) {
+__device__ __forceinline__ double col_sum(const double *partials, int nblk, int r) {
     __shared__ double s[256];
     double acc = 0.0;
-    for (int b = threadIdx.x; b < kGfRed; b += 256) acc += partials[(size_t)b * k + r];
+    for (int b = threadIdx.x; b < nblk; b += 256) acc += partials[(size_t)r * kGfRed + b];
     s[threadIdx.x] = acc;
     __syncthreads();
     for (int w = 128; w > 0; w >>= 1) {
@@ -230,27 +232,27 @@ __device__ __forceinline__ double col_sum(const double *partials, int k, int r) 
 }
 
 // grid = k blocks of 256 threads: block r finishes column r
-__global__ void __launch_bounds__(256) gf_finish_norm(int k, const double *__restrict__ partials, double *out) {
+__global__ void __launch_bounds__(256) gf_finish_norm(int nblk, const double *__restrict__ partials, double *out) {
     const int r = blockIdx.x;
-    const double v = col_sum(partials, k, r);
+    const double v = col_sum(partials, nblk, r);
     if (threadIdx.x == 0) out[r] = sqrt(v);
 }
 
-__global__ void __launch_bounds__(256) gf_finish_alpha(int k, const double *__restrict__ partials, double *scal) {
+__global__ void __launch_bounds__(256) gf_finish_alpha(int nblk, const double *__restrict__ partials, double *scal) {
     const int r = blockIdx.x;
-    const double pq = col_sum(partials, k, r);
+    const double pq = col_sum(partials, nblk, r);
     if (threadIdx.x == 0) {
         scal[G_PQ * 64 + r] = pq;
         scal[G_ALPHA * 64 + r] = pq != 0.0 ? scal[G_RZ * 64 + r] / pq : 0.0;
     }
 }
 
-__global__ void __launch_bounds__(256) gf_finish_beta(int k, const double *__restrict__ prz,
+__global__ void __launch_bounds__(256) gf_finish_beta(int nblk, const double *__restrict__ prz,
                                                       const double *__restrict__ prr, double *scal, int start) {
     const int r = blockIdx.x;
-    const double rz = col_sum(prz, k, r);
+    const double rz = col_sum(prz, nblk, r);
     __syncthreads();
-    const double rr = col_sum(prr, k, r);
+    const double rr = col_sum(prr, nblk, r);
     if (threadIdx.x == 0) {
         const double old = scal[G_RZ * 64 + r];
         scal[G_BETA * 64 + r] = (!start && old != 0.0) ? rz / old : 0.0;
@@ -274,7 +276,7 @@ __device__ __forceinline__ void gf_xcd_slab(int n, int &lo, int &hi, int &j, int
 
 // ---- FP32 block PCG kernels with a compile-time block width K (thread = (node, column)) ----
 // q = A p and the per-column partial sums of p.q
-template <int K>
+template <int K, int U>
 __global__ void __launch_bounds__(256) gfk_spmm_dot(int nrows, const int32_t *__restrict__ row_ptr,
                                                     const int32_t *__restrict__ col, const float *__restrict__ val,
                                                     const float *__restrict__ P, float *Q, double *ppq) {
@@ -289,13 +291,28 @@ __global__ void __launch_bounds__(256) gfk_spmm_dot(int nrows, const int32_t *__
         if (i >= hi) continue;
         float y0 = 0.f, y1 = 0.f, y2 = 0.f;
         const int e1 = row_ptr[i + 1];
-        for (int e = row_ptr[i]; e < e1; ++e) {
-            const int64_t j = col[e];
-            const float *A = val + 9 * (size_t)e;
-            const float x0 = P[(3 * j) * K + r], x1 = P[(3 * j + 1) * K + r], x2 = P[(3 * j + 2) * K + r];
-            y0 += A[0] * x0 + A[1] * x1 + A[2] * x2;
-            y1 += A[3] * x0 + A[4] * x1 + A[5] * x2;
-            y2 += A[6] * x0 + A[7] * x1 + A[8] * x2;
+        // U neighbours at a time, their loads before the arithmetic (past the row's end the last block
+        // again, times zero)
+        for (int e = row_ptr[i]; e < e1; e += U) {
+            float a[U][9], x[U][3];
+#pragma unroll
+            for (int m = 0; m < U; ++m) {
+                const int em = min(e + m, e1 - 1);
+                const int64_t j = col[em];
+#pragma unroll
+                for (int q = 0; q < 9; ++q) a[m][q] = val[9 * (size_t)em + q];
+#pragma unroll
+                for (int c = 0; c < 3; ++c) {
+                    x[m][c] = P[(3 * j + c) * K + r];
+                    if (e + m >= e1) x[m][c] = 0.f;
+                }
+            }
+#pragma unroll
+            for (int m = 0; m < U; ++m) {
+                y0 += a[m][0] * x[m][0] + a[m][1] * x[m][1] + a[m][2] * x[m][2];
+                y1 += a[m][3] * x[m][0] + a[m][4] * x[m][1] + a[m][5] * x[m][2];
+                y2 += a[m][6] * x[m][0] + a[m][7] * x[m][1] + a[m][8] * x[m][2];
+            }
         }
         const size_t o = (3 * (size_t)i) * K + r;
         Q[o] = y0;
@@ -305,7 +322,7 @@ __global__ void __launch_bounds__(256) gfk_spmm_dot(int nrows, const int32_t *__
     }
     s[threadIdx.x] = acc;
     col_reduce(s, K);
-    if ((int)threadIdx.x < K) ppq[(size_t)blockIdx.x * K + threadIdx.x] = s[threadIdx.x];
+    if ((int)threadIdx.x < K) ppq[(size_t)threadIdx.x * kGfRed + blockIdx.x] = s[threadIdx.x];
 }
 
 // Block row times a 64-column block on the matrix cores: y (rows 0 .. 2 in the vector's entries, lane =
@@ -375,7 +392,7 @@ __global__ void __launch_bounds__(256) gfk_spmm_dot64(int nrows, const int32_t *
     s[threadIdx.x] = acc;
     __syncthreads();
     if (threadIdx.x < 64)
-        ppq[(size_t)blockIdx.x * 64 + threadIdx.x] = (s[threadIdx.x] + s[threadIdx.x + 64]) +
+        ppq[(size_t)threadIdx.x * kGfRed + blockIdx.x] = (s[threadIdx.x] + s[threadIdx.x + 64]) +
                                                      (s[threadIdx.x + 128] + s[threadIdx.x + 192]);
 }
 
@@ -420,8 +437,8 @@ __global__ void __launch_bounds__(256) gfk_update(int nrows, const float *__rest
     s2[threadIdx.x] = rr;
     col_reduce(s2, K);
     if ((int)threadIdx.x < K) {
-        prz[(size_t)blockIdx.x * K + threadIdx.x] = s1[threadIdx.x];
-        prr[(size_t)blockIdx.x * K + threadIdx.x] = s2[threadIdx.x];
+        prz[(size_t)threadIdx.x * kGfRed + blockIdx.x] = s1[threadIdx.x];
+        prr[(size_t)threadIdx.x * kGfRed + blockIdx.x] = s2[threadIdx.x];
     }
 }
 
@@ -767,7 +784,7 @@ __global__ void __launch_bounds__(256) gfk_update_xr(int64_t ndof, const double 
     }
     s[threadIdx.x] = rr;
     col_reduce(s, K);
-    if ((int)threadIdx.x < K) prr[(size_t)blockIdx.x * K + threadIdx.x] = s[threadIdx.x];
+    if ((int)threadIdx.x < K) prr[(size_t)threadIdx.x * kGfRed + blockIdx.x] = s[threadIdx.x];
 }
 
 // per-column partials of a.b (and, when bb is set, of b.b) -- fixed column per thread
@@ -786,8 +803,8 @@ __global__ void __launch_bounds__(256) gfk_dot2(int64_t ndof, const float *__res
     s2[threadIdx.x] = bb;
     col_reduce(s2, K);
     if ((int)threadIdx.x < K) {
-        pab[(size_t)blockIdx.x * K + threadIdx.x] = s1[threadIdx.x];
-        if (pbb) pbb[(size_t)blockIdx.x * K + threadIdx.x] = s2[threadIdx.x];
+        pab[(size_t)threadIdx.x * kGfRed + blockIdx.x] = s1[threadIdx.x];
+        if (pbb) pbb[(size_t)threadIdx.x * kGfRed + blockIdx.x] = s2[threadIdx.x];
     }
 }
 
@@ -976,6 +993,12 @@ static int gf_alloc(plx_gf g, int k) {
     return 0;
 }
 
+// Blocks of a k-column kernel with a thread per (node, column); a multiple of the 8 XCDs.  2048 whatever the size left
+// the column sums (a block per column) 2048 partials of mostly idle blocks to add: 16^3 hexes x 16 columns 9.2 -> 4.2 us.
+static int red_blocks(plx_gf g, int k) {
+    return (int)std::min<int64_t>(kGfRed, (((int64_t)g->nrows * k + 255) / 256 + 7) / 8 * 8);
+}
+
 template <typename Real>
 static void gf_spmm_launch(plx_gf g, int k, const Real *val, const Real *X, Real *Y) {
     const int64_t n = (int64_t)g->nrows * k;
@@ -983,15 +1006,22 @@ static void gf_spmm_launch(plx_gf g, int k, const Real *val, const Real *X, Real
                        g->d_row_ptr, g->d_col, val, X, Y);
 }
 
-// q = A p and the per-column partials of p.q for the k-column block
+// q = A p and the per-column partials of p.q for the k-column block.  With fewer than kBatchWaves waves of
+// rows (eight per SIMD) the neighbours' loads go out in batches: 16^3 hexes x 16 columns 15.6 -> 11.3 us; a solve with
+// point-block Jacobi on 16^3 x 32 9.0 -> 7.0 ms, 26^3 x 8 12.6 -> 9.8 ms.  More waves hide the loads by
+// themselves: 30^3 x 16 29.2 ms either way, 36^3 x 32 79.5 ms in batches, 75.5 ms without.
+constexpr int64_t kBatchWaves = 8192;
 template <int K>
 static void gf_spmm_dot_launch(plx_gf g) {
     if (K == 64)
-        hipLaunchKernelGGL(gfk_spmm_dot64, dim3(kGfRed), dim3(256), 0, g->stream, g->nrows, g->d_row_ptr, g->d_col,
+        hipLaunchKernelGGL(gfk_spmm_dot64, dim3(red_blocks(g, K)), dim3(256), 0, g->stream, g->nrows, g->d_row_ptr, g->d_col,
                            g->d_val32, g->P32, g->Q32, g->prz);
+    else if ((int64_t)g->nrows * K < 64 * kBatchWaves)
+        hipLaunchKernelGGL((gfk_spmm_dot<K, 5>), dim3(red_blocks(g, K)), dim3(256), 0, g->stream, g->nrows, g->d_row_ptr,
+                           g->d_col, g->d_val32, g->P32, g->Q32, g->prz);
     else
-        hipLaunchKernelGGL(gfk_spmm_dot<K>, dim3(kGfRed), dim3(256), 0, g->stream, g->nrows, g->d_row_ptr, g->d_col,
-                           g->d_val32, g->P32, g->Q32, g->prz);
+        hipLaunchKernelGGL((gfk_spmm_dot<K, 1>), dim3(red_blocks(g, K)), dim3(256), 0, g->stream, g->nrows, g->d_row_ptr,
+                           g->d_col, g->d_val32, g->P32, g->Q32, g->prz);
 }
 
 // Ten iterations of the FP32 block PCG (p, z, scalars carried on the device): per iteration
@@ -1000,11 +1030,11 @@ template <int K>
 static void gf_pcg_chunk_k(plx_gf g) {
     for (int it = 0; it < 10; ++it) {
         gf_spmm_dot_launch<K>(g);
-        hipLaunchKernelGGL(gf_finish_alpha, dim3(K), dim3(256), 0, g->stream, K, g->prz, g->scal);
-        hipLaunchKernelGGL((gfk_update<K, false>), dim3(kGfRed), dim3(256), 0, g->stream, g->nrows, g->d_Binv32,
+        hipLaunchKernelGGL(gf_finish_alpha, dim3(K), dim3(256), 0, g->stream, red_blocks(g, K), g->prz, g->scal);
+        hipLaunchKernelGGL((gfk_update<K, false>), dim3(red_blocks(g, K)), dim3(256), 0, g->stream, g->nrows, g->d_Binv32,
                            g->scal, g->X32, g->R32, g->P32, g->Q32, g->Z32, g->prz, g->prr);
-        hipLaunchKernelGGL(gf_finish_beta, dim3(K), dim3(256), 0, g->stream, K, g->prz, g->prr, g->scal, 0);
-        hipLaunchKernelGGL(gfk_pupdate<K>, dim3(kGfRed), dim3(256), 0, g->stream, g->ndof * K, g->scal, g->Z32,
+        hipLaunchKernelGGL(gf_finish_beta, dim3(K), dim3(256), 0, g->stream, red_blocks(g, K), g->prz, g->prr, g->scal, 0);
+        hipLaunchKernelGGL(gfk_pupdate<K>, dim3(red_blocks(g, K)), dim3(256), 0, g->stream, g->ndof * K, g->scal, g->Z32,
                            g->P32);
     }
 }
@@ -1044,7 +1074,7 @@ static void gf_pcg_start(plx_gf g, int k) {
         return;
     }
 #define PLX_GF_START(K)                                                                                      \
-    hipLaunchKernelGGL((gfk_update<K, true>), dim3(kGfRed), dim3(256), 0, g->stream, g->nrows, g->d_Binv32, \
+    hipLaunchKernelGGL((gfk_update<K, true>), dim3(red_blocks(g, K)), dim3(256), 0, g->stream, g->nrows, g->d_Binv32, \
                        g->scal, g->X32, g->R32, g->P32, g->Q32, g->Z32, g->prz, g->prr)
     switch (k) {
     case 8: PLX_GF_START(8); break;
@@ -1053,7 +1083,7 @@ static void gf_pcg_start(plx_gf g, int k) {
     default: PLX_GF_START(64); break;
     }
 #undef PLX_GF_START
-    hipLaunchKernelGGL(gf_finish_beta, dim3(k), dim3(256), 0, g->stream, k, g->prz, g->prr, g->scal, 1);
+    hipLaunchKernelGGL(gf_finish_beta, dim3(k), dim3(256), 0, g->stream, red_blocks(g, k), g->prz, g->prr, g->scal, 1);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1147,14 +1177,14 @@ template <int K>
 static void gf_pcg_chunk_amg(plx_gf g) {
     for (int it = 0; it < kAmgChunk; ++it) {
         gf_spmm_dot_launch<K>(g);
-        hipLaunchKernelGGL(gf_finish_alpha, dim3(K), dim3(256), 0, g->stream, K, g->prz, g->scal);
-        hipLaunchKernelGGL(gfk_update_xr<K>, dim3(kGfRed), dim3(256), 0, g->stream, g->ndof, g->scal, g->X32, g->R32,
+        hipLaunchKernelGGL(gf_finish_alpha, dim3(K), dim3(256), 0, g->stream, red_blocks(g, K), g->prz, g->scal);
+        hipLaunchKernelGGL(gfk_update_xr<K>, dim3(red_blocks(g, K)), dim3(256), 0, g->stream, g->ndof, g->scal, g->X32, g->R32,
                            g->P32, g->Q32, g->prr);
         amg_vcycle<K>(g, 0, g->R32, g->Z32);
-        hipLaunchKernelGGL(gfk_dot2<K>, dim3(kGfRed), dim3(256), 0, g->stream, g->ndof, g->Z32, g->R32, g->prz,
+        hipLaunchKernelGGL(gfk_dot2<K>, dim3(red_blocks(g, K)), dim3(256), 0, g->stream, g->ndof, g->Z32, g->R32, g->prz,
                            (double *)nullptr);
-        hipLaunchKernelGGL(gf_finish_beta, dim3(K), dim3(256), 0, g->stream, K, g->prz, g->prr, g->scal, 0);
-        hipLaunchKernelGGL(gfk_pupdate<K>, dim3(kGfRed), dim3(256), 0, g->stream, g->ndof * K, g->scal, g->Z32,
+        hipLaunchKernelGGL(gf_finish_beta, dim3(K), dim3(256), 0, g->stream, red_blocks(g, K), g->prz, g->prr, g->scal, 0);
+        hipLaunchKernelGGL(gfk_pupdate<K>, dim3(red_blocks(g, K)), dim3(256), 0, g->stream, g->ndof * K, g->scal, g->Z32,
                            g->P32);
     }
 }
@@ -1164,8 +1194,8 @@ template <int K>
 static void gf_pcg_start_amg(plx_gf g) {
     amg_vcycle<K>(g, 0, g->R32, g->Z32);
     hipLaunchKernelGGL(gf_copyf, gf_grid(g->ndof * K), dim3(256), 0, g->stream, g->ndof * K, g->Z32, g->P32);
-    hipLaunchKernelGGL(gfk_dot2<K>, dim3(kGfRed), dim3(256), 0, g->stream, g->ndof, g->Z32, g->R32, g->prz, g->prr);
-    hipLaunchKernelGGL(gf_finish_beta, dim3(K), dim3(256), 0, g->stream, K, g->prz, g->prr, g->scal, 1);
+    hipLaunchKernelGGL(gfk_dot2<K>, dim3(red_blocks(g, K)), dim3(256), 0, g->stream, g->ndof, g->Z32, g->R32, g->prz, g->prr);
+    hipLaunchKernelGGL(gf_finish_beta, dim3(K), dim3(256), 0, g->stream, red_blocks(g, K), g->prz, g->prr, g->scal, 1);
 }
 
 static int gf_run_chunk(plx_gf g, int k) {
@@ -1215,8 +1245,8 @@ static int gf_inner(plx_gf g, int k, int *its) {
 // Column norms of an FP64 block -> g->nrm (device) and host copy.
 static int gf_norms(plx_gf g, int k, const double *V, std::vector<double> &out) {
     plx_dm dm = g->dm;
-    hipLaunchKernelGGL(gf_dot<double>, dim3(kGfRed), dim3(256), 0, g->stream, g->ndof, k, V, V, g->prz);
-    hipLaunchKernelGGL(gf_finish_norm, dim3(k), dim3(256), 0, g->stream, k, g->prz, g->nrm);
+    hipLaunchKernelGGL(gf_dot<double>, dim3(red_blocks(g, k)), dim3(256), 0, g->stream, g->ndof, k, V, V, g->prz);
+    hipLaunchKernelGGL(gf_finish_norm, dim3(k), dim3(256), 0, g->stream, red_blocks(g, k), g->prz, g->nrm);
     PLX_HIP(dm, hipGetLastError());
     out.resize(k);
     PLX_HIP(dm, hipMemcpyAsync(out.data(), g->nrm, k * sizeof(double), hipMemcpyDeviceToHost, g->stream));
@@ -2228,13 +2258,13 @@ __global__ void __launch_bounds__(256) gfk_zjacobi(int nrows, const float *__res
 
 // PCG start of the selected columns: beta = 0, r.z and r.r from the partials; r.r also kept as the
 // column's starting residual (rr0) for its convergence test
-__global__ void __launch_bounds__(256) gf_finish_start_mask(int k, const double *__restrict__ prz,
+__global__ void __launch_bounds__(256) gf_finish_start_mask(int nblk, const double *__restrict__ prz,
                                                             const double *__restrict__ prr, double *scal,
                                                             uint64_t mask, double *rr0) {
     const int r = blockIdx.x;
-    const double rz = col_sum(prz, k, r);
+    const double rz = col_sum(prz, nblk, r);
     __syncthreads();
-    const double rr = col_sum(prr, k, r);
+    const double rr = col_sum(prr, nblk, r);
     if (threadIdx.x == 0 && col_on(mask, r)) {
         scal[G_BETA * 64 + r] = 0.0;
         scal[G_RZ * 64 + r] = rz;
@@ -2310,11 +2340,11 @@ static void gf_start_mask_k(plx_gf g, uint64_t mask) {
     if (g->pc == PLX_GF_PC_AMG)
         amg_vcycle<K>(g, 0, g->R32, g->Z32);
     else
-        hipLaunchKernelGGL(gfk_zjacobi<K>, dim3(kGfRed), dim3(256), 0, g->stream, g->nrows, g->d_Binv32, g->R32, g->Z32);
+        hipLaunchKernelGGL(gfk_zjacobi<K>, dim3(red_blocks(g, K)), dim3(256), 0, g->stream, g->nrows, g->d_Binv32, g->R32, g->Z32);
     hipLaunchKernelGGL(gf_copy_cols<float>, gf_grid(g->ndof * K), dim3(256), 0, g->stream, g->ndof, K, mask,
                        g->Z32, g->P32);
-    hipLaunchKernelGGL(gfk_dot2<K>, dim3(kGfRed), dim3(256), 0, g->stream, g->ndof, g->Z32, g->R32, g->prz, g->prr);
-    hipLaunchKernelGGL(gf_finish_start_mask, dim3(K), dim3(256), 0, g->stream, K, g->prz, g->prr, g->scal, mask,
+    hipLaunchKernelGGL(gfk_dot2<K>, dim3(red_blocks(g, K)), dim3(256), 0, g->stream, g->ndof, g->Z32, g->R32, g->prz, g->prr);
+    hipLaunchKernelGGL(gf_finish_start_mask, dim3(K), dim3(256), 0, g->stream, red_blocks(g, K), g->prz, g->prr, g->scal, mask,
                        g->d_rr0);
 }
 
