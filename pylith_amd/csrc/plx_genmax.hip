@@ -115,14 +115,27 @@ __global__ void __launch_bounds__(256) genmax_prestress_kernel(GmArgs A) {
     for (int k = 0; k < 6; ++k) A.pre[(size_t)(8 * k + q) * n + pos] = s[k];
 }
 
-// State update at the new displacement u, fused with the next step's state stress.
-__global__ void __launch_bounds__(256) genmax_update_kernel(GmArgs A, const double *__restrict__ u) {
-    const int pos = blockIdx.x * blockDim.x + threadIdx.x;
-    const int q = blockIdx.y;
+// State update at the new displacement u, fused with the next step's state stress.  One thread per cell and
+// point; bound by the state's way through HBM.  The eight blocks of a chunk of cells (one per point) follow one
+// another on one XCD, so that the cells' indices, moduli and nodes come from its L2 for seven of them, and the
+// state is read before the first store.  STREAM: the state passes by the caches; for keys whose state and
+// state stress exceed half of the 256 MB Infinity Cache, which the solve between two updates fills with its
+// own.  Update and residual, out of the cache, 48 x 45 x 43 cells (178 MB): 118 -> 108 us, streamed 104; 60^3:
+// 236, streamed 228 (191 at once again, 233 not streamed); 32^3 (63 MB): 38, streamed 42.
+template <bool STREAM>
+__global__ void __launch_bounds__(256, STREAM ? 4 : 3) genmax_update_kernel(GmArgs A, const double *__restrict__ u) {
+    const int j = blockIdx.x >> 3, q = j & 7;
+    const int pos = ((j >> 3) * 8 + (blockIdx.x & 7)) * 256 + threadIdx.x;
     if (pos >= A.n) return;
     const size_t n = (size_t)A.n;
     auto at = [&](int k) { return (size_t)(8 * k + q) * n + pos; };
-    double e[6], de[6], et[6], det[6];
+    auto put = [&](int k, double v) {
+        if (STREAM) __builtin_nontemporal_store(v, &A.state[at(k)]);
+        else A.state[at(k)] = v;
+    };
+    double ov[18], e[6], de[6], et[6], det[6];
+#pragma unroll
+    for (int k = 0; k < 18; ++k) ov[k] = STREAM ? __builtin_nontemporal_load(&A.state[at(k)]) : A.state[at(k)];
     q1_point_strain(A.closure + 8 * (size_t)A.cells[pos], A.coords, u, q, e);
     dev6(e, de);
 #pragma unroll
@@ -137,14 +150,14 @@ __global__ void __launch_bounds__(256) genmax_update_kernel(GmArgs A, const doub
         const double w = 2.0 * mu * ri;
 #pragma unroll
         for (int k = 0; k < 6; ++k) {
-            const double ev = x * A.state[at(6 * i + k)] + dq * (de[k] - det[k]);
-            A.state[at(6 * i + k)] = ev;
+            const double ev = x * ov[6 * i + k] + dq * (de[k] - det[k]);
+            put(6 * i + k, ev);
             s[k] += w * (x * ev - dq * de[k]);
         }
     }
 #pragma unroll
     for (int k = 0; k < 6; ++k) {
-        A.state[at(18 + k)] = e[k];
+        put(18 + k, e[k]);
         A.pre[(size_t)(8 * k + q) * n + pos] = s[k];
     }
 }
@@ -177,7 +190,10 @@ int launch_genmax_update(plx_dm dm, KeyPlan *kp, const double *u) {
     const GmArgs A = gm_args(dm, kp);
     if (A.n == 0) return 0;
     ScopedEvent ev(dm, "plx:genmax_update");
-    hipLaunchKernelGGL(genmax_update_kernel, dim3((A.n + 255) / 256, 8), dim3(256), 0, dm->stream, A, u);
+    const dim3 grid(64 * ((A.n + 2047) / 2048));
+    const bool stream = (int64_t)A.n * (24 + 6) * 8 * sizeof(double) > (int64_t)128 << 20;
+    if (stream) hipLaunchKernelGGL(genmax_update_kernel<true>, grid, dim3(256), 0, dm->stream, A, u);
+    else hipLaunchKernelGGL(genmax_update_kernel<false>, grid, dim3(256), 0, dm->stream, A, u);
     PLX_HIP(dm, hipGetLastError());
     return 0;
 }

@@ -199,3 +199,20 @@ def test_axial_strain_rate_solve(oracle):
     assert worst["u"] <= 1e-11, worst
     assert worst["szz"] <= 1e-11, worst
     assert worst["visc"] <= 1e-11, worst
+
+
+def test_state_update_of_a_key_larger_than_the_caches(oracle):
+    """Over 128 MB of state the update streams it; the last chunk of cells is ragged."""
+    m = mg.hex_box((43, 42, 41), (0, 0, 0), (4300.0, 4200.0, 4100.0))
+    assert m.num_cells * 30 * 8 * 8 > 128 << 20
+    aux, sizes = mg.genmax_aux(m.num_cells, 8, seed=5, log_eta_range=(1e17, 1e19), ratios=(0.3, 0.3, 0.3))
+    aux[:, 9:33] = np.random.default_rng(7).standard_normal((aux.shape[0], 24)) * 1e-4
+    dt = 0.1 * mg.YEAR
+    dm = gm_dm(m, aux, sizes, dt)
+    u = mg.random_field(m.num_nodes, 100)
+    P = oracle.Problem(m, aux, sizes, per_qp=True, constants=[dt])
+    dm.update_state_vars(0, 0, dev(u))
+    got = dm.get_auxiliary(0, 0, aux)
+    aux = gm_update(P, u)
+    assert relerr(got[:, 9:27], aux[:, 9:27]) <= TOL64
+    assert relerr(got[:, 27:33], aux[:, 27:33]) <= TOL64
