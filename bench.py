@@ -700,12 +700,12 @@ def main():
         },
         "roofline": {
             "bound": "hbm",
-            "kernel": "apply_tiles<double, TET_P2, factored, lds-atomic>",
+            "kernel": "apply_pairs<double> (P2 factored, LDS atomics)",
             "achieved": achieved,
             "peak": HBM_PEAK_GBS,
             "unit": "GB/s",
             "frac": achieved / HBM_PEAK_GBS,
-            "frac_basis": "the apply_tiles kernel alone (HIP events on its stream)",
+            "frac_basis": "the tile kernel alone (HIP events on its stream)",
             "frac_apply_kernels": B / ((kms + hms) * 1e-3) / 1e9 / HBM_PEAK_GBS,
             "frac_apply_wall": B / sec / 1e9 / HBM_PEAK_GBS,
             "traffic": traffic,

@@ -454,7 +454,7 @@ __global__ void __launch_bounds__(256) gfk_pupdate(int64_t n, const double *__re
 
 // ---- multigrid preconditioner kernels ([dof][K] layout) ----
 // Block-sparse products of the V-cycle, one wave per (64 / K) block rows, lane = (row, column);
-// with K = 64 the row is wave-uniform and the matrix words are scalar loads.  Rows follow the
+// with K = 64 the row is wave-uniform and the matrix words are scalar loads (BR = 3: on the matrix cores, gf_row64).  Rows follow the
 // per-XCD slab schedule of the fine-level product.
 //   kBsrPlain: Y = T X (or Y += T X with accumulate)          transfers (P, R = P^T)
 //   kBsrResid: Y = B - A X                                    pre-smoother residual
