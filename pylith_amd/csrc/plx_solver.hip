@@ -542,10 +542,11 @@ static bool gathered(const plx_solver_s *s) {
 // solve, outside any capture).
 static int ensure_finish(plx_solver s) {
     plx_dm dm = s->dm;
+    // (by the preconditioner as well, which changes without the DM's epoch)
+    if (gathered(s) && !s->p2) PLX_HIP(dm, hipMalloc(&s->p2, (size_t)s->n * sizeof(double)));
     if (!fused(s) || s->finish_epoch == dm->epoch) return 0;
     if (!s->range) PLX_HIP(dm, hipMalloc(&s->range, (size_t)s->nnodes * sizeof(int2)));
     if (!s->fixed) PLX_HIP(dm, hipMalloc(&s->fixed, (size_t)s->nnodes));
-    if (gathered(s) && !s->p2) PLX_HIP(dm, hipMalloc(&s->p2, (size_t)s->n * sizeof(double)));
     std::vector<uint8_t> mask(s->nnodes, 0);
     for (int32_t d : dm->con.dofs)
         if (d < 3 * s->nnodes) mask[d / 3] |= (uint8_t)(1 << d % 3);
@@ -571,6 +572,7 @@ static int apply_finish(plx_solver s, const Real *x, Real *t, const Real *b, con
                         double *part) {
     plx_dm dm = s->dm;
     const int st = std::is_same<Real, double>::value ? PLX_FP64 : PLX_FP32;
+    if (!s->range || !s->fixed) return set_error(dm, 1, "solver: work vectors not set up");
     if (int err = launch_apply(dm, s->keys[0], st, true, x, t, PLX_INSERT_VALUES, -1.0, nullptr, true, false)) return err;
     // a sum over the whole mesh needs its partials bounded; the others take a thread per node
     const int blocks = MODE == kFinishDot ? node_blocks(s) : std::max(1, (s->nnodes + 255) / 256);
@@ -786,6 +788,7 @@ static int pcg(plx_solver s, Real *x, Real *r, Real *p, Real *q, Real *z, const 
     plx_dm dm = s->dm;
     // r = b - A x  (caller stored b in r; x == 0 guess skips the apply)
     const bool two = gathered(s);
+    if (two && (!s->p2 || !s->fixed)) return set_error(dm, 1, "solver: work vectors not set up");
     const int nblk = node_blocks(s);
     hipLaunchKernelGGL(pc_start<Real>, two ? dim3(nblk) : red_grid(), dim3(256), 0, dm->stream, s->nnodes, Binv, r, z, p,
                        s->part_a, s->part_b);

@@ -258,3 +258,35 @@ def test_iterates_agree_over_plans(kind, maxit):
     for x, its in out[1:]:
         assert np.abs(x - out[0][0]).max() / scale <= 1e-10
         assert its == out[0][1]
+
+
+@pytest.mark.parametrize("kind", ["hex", "tet"])
+@pytest.mark.parametrize("method", [L.KSP_CG, L.KSP_FGMRES_IR])
+def test_preconditioner_changed_on_one_solver(kind, method):
+    """Multigrid, point-block Jacobi, multigrid and Jacobi again on one solver of a mesh that the
+    two-kernel iteration serves, each solve against a fresh solver's: the same iterations from the same
+    start, rounding apart (order of the LDS additions), to rtol 1e-10: 1e-8 of the solution."""
+    m = (mg.hex_box((9, 14, 11), (0, 0, 0), (6000.0, 6000.0, 6000.0)) if kind == "hex"
+         else mg.tet_p2_box((5, 8, 6), (0, 0, 0), (6000.0, 6000.0, 6000.0)))
+    aux, sizes = mg.elastic_aux(m.num_cells, seed=4, vs_sigma=0.2, vp_vs=1.732)
+    dofs, vals = mg.shear_bcs(m.node_coords, 0.0, 6000.0)
+
+    def solve(dm, solver):
+        x = torch.zeros(3 * m.num_nodes, dtype=torch.float64, device="cuda")
+        dm.insert_boundary_values(torch.from_numpy(vals).cuda(), x)
+        st = solver.solve(x, method=method, rtol=1e-10, maxit=5000)
+        torch.cuda.synchronize()
+        assert st["converged"], st
+        return x.cpu().numpy()
+
+    ref = {}
+    for pc in ("amg", "pbjacobi"):
+        dm, solver = build(m, aux, sizes, dofs)
+        solver.set_preconditioner(pc)
+        ref[pc] = solve(dm, solver)
+    dm, solver = build(m, aux, sizes, dofs)
+    for pc in ("amg", "pbjacobi", "amg", "pbjacobi"):
+        print(f"[solver] change of preconditioner: {kind} method={method} pc={pc}", flush=True)
+        solver.set_preconditioner(pc)
+        x = solve(dm, solver)
+        assert np.abs(x - ref[pc]).max() <= 1e-8 * np.abs(ref[pc]).max(), pc
