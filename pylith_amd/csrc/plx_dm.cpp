@@ -160,9 +160,9 @@ static int build_plan(plx_dm dm, KeyPlan *kp) {
     if ((err = upload(dm, &kp->d_shared_ptr, hp.shared_ptr.data(), hp.shared_ptr.size()))) return err;
     if ((err = upload(dm, &kp->d_shared_slot, hp.shared_slot.data(), hp.shared_slot.size()))) return err;
     if (hp.halo_slots > 0) PLX_HIP(dm, hipMalloc(&kp->d_halo, (size_t)hp.halo_slots * 3 * sizeof(double)));
-    if (dm->cell_type == PLX_TET_P2 && (int64_t)hp.cells.size() >= kPairMinCells) {
-        PairPlan pp;
-        if (build_pair_plan(mv, hp, &pp, &msg)) return set_error(dm, 1, msg);
+    // (a key without a pair plan keeps the tile plan alone)
+    PairPlan pp;
+    if (dm->cell_type == PLX_TET_P2 && (int64_t)hp.cells.size() >= kPairMinCells && !build_pair_plan(mv, hp, &pp, &msg)) {
         PairDev &P = kp->pairs;
         P.num_tiles = pp.num_tiles;
         P.num_pairs = pp.num_pairs;

@@ -8,6 +8,7 @@
 #include <algorithm>
 #include <array>
 #include <cmath>
+#include <iterator>
 #include <system_error>
 #include <thread>
 
@@ -427,10 +428,109 @@ static int plan_cells(const MeshView &m, const TileLimits &lim, HostPlan *hp, st
 // Pair plan.
 // --------------------------------------------------------------------------------------------
 
+namespace {
+struct PairTile {
+    int n = 0;                              // cells
+    std::vector<std::array<int, 4>> match;  // pairs: first cell, second (-1: none), their vertices opposite the face
+    int npaired = 0;                        // those with a second cell come first
+    std::vector<int32_t> nodes;  // sorted distinct, then in local order (owned, shared)
+    std::vector<int32_t> verts;
+    int nown = 0;
+    std::vector<int32_t> cells;  // [pairs][2]
+    std::vector<uint32_t> rec;
+};
+}  // namespace
+
+// Position of x in the sorted v.
+static int place_of(const std::vector<int32_t> &v, int32_t x) {
+    return (int)(std::lower_bound(v.begin(), v.end(), x) - v.begin());
+}
+
+// Local vertices of two cells that share a face, the vertices opposite it (oa, ob) first and the
+// second cell's face turned so that its first vertex is the first cell's; the other two then run the
+// opposite way round in a consistently oriented mesh (else the cells are not paired).
+static bool turn_to_face(const int32_t *va, int oa, const int32_t *vb, int ob, int pa[4], int pb[4]) {
+    static const int kApex[4][4] = {{0, 1, 2, 3}, {1, 0, 3, 2}, {2, 0, 1, 3}, {3, 0, 2, 1}};  // even permutations
+    for (int k = 0; k < 4; ++k) pa[k] = kApex[oa][k];
+    for (int r = 0; r < 3; ++r) {
+        pb[0] = kApex[ob][0];
+        for (int k = 0; k < 3; ++k) pb[1 + k] = kApex[ob][1 + (k + r) % 3];
+        if (vb[pb[1]] == va[pa[1]]) break;
+    }
+    return vb[pb[1]] == va[pa[1]] && vb[pb[2]] == va[pa[3]] && vb[pb[3]] == va[pa[2]];
+}
+
+// The pairs of the cells ids[0 .. n).
+static void match_cells(const MeshView &m, const int32_t *ids, int n, PairTile &T) {
+    const auto vert = [&](int i) { return m.cone + 4 * (size_t)ids[i]; };
+    // faces of the tile: (vertices sorted) -> cell and the vertex opposite
+    std::vector<std::pair<std::array<int32_t, 3>, int32_t>> faces;
+    faces.reserve(4 * (size_t)n);
+    for (int i = 0; i < n; ++i)
+        for (int k = 0; k < 4; ++k) {
+            const int32_t *v = vert(i);
+            std::array<int32_t, 3> f{v[(k + 1) & 3], v[(k + 2) & 3], v[(k + 3) & 3]};
+            std::sort(f.begin(), f.end());
+            faces.push_back({f, 4 * i + k});
+        }
+    std::sort(faces.begin(), faces.end());
+    std::vector<std::array<std::array<int, 3>, 4>> nbr(n);  // (neighbour, my opposite vertex, its)
+    std::vector<int> deg(n, 0);
+    for (size_t f = 0; f + 1 < faces.size(); ++f)
+        if (faces[f].first == faces[f + 1].first) {
+            const int a = faces[f].second >> 2, b = faces[f + 1].second >> 2;
+            if (a != b && deg[a] < 4 && deg[b] < 4) {
+                nbr[a][deg[a]++] = {b, faces[f].second & 3, faces[f + 1].second & 3};
+                nbr[b][deg[b]++] = {a, faces[f + 1].second & 3, faces[f].second & 3};
+            }
+            ++f;
+        }
+    // matching: cells with the fewest free neighbours first, each to its neighbour with the fewest
+    std::vector<int> mate(n, -1), free_deg(deg);
+    std::array<std::vector<int>, 5> bucket;
+    for (int i = n - 1; i >= 0; --i) bucket[free_deg[i]].push_back(i);
+    T.match.clear();
+    for (int d = 1; d <= 4;) {
+        if (bucket[d].empty()) {
+            ++d;
+            continue;
+        }
+        const int a = bucket[d].back();
+        bucket[d].pop_back();
+        if (mate[a] >= 0 || free_deg[a] != d) continue;
+        int best = -1;
+        for (int k = 0; k < deg[a]; ++k) {
+            const int b = nbr[a][k][0];
+            if (mate[b] >= 0) continue;
+            int pa[4], pb[4];
+            if (!turn_to_face(vert(a), nbr[a][k][1], vert(b), nbr[a][k][2], pa, pb)) continue;
+            if (best < 0 || free_deg[b] < free_deg[nbr[a][best][0]]) best = k;
+        }
+        if (best < 0) continue;  // no neighbour it can be turned to: stays single
+        const int b = nbr[a][best][0];
+        mate[a] = b;
+        mate[b] = a;
+        T.match.push_back({a, b, nbr[a][best][1], nbr[a][best][2]});
+        for (int c : {a, b})
+            for (int k = 0; k < deg[c]; ++k) {
+                const int e = nbr[c][k][0];
+                if (mate[e] >= 0) continue;
+                if (--free_deg[e] > 0) bucket[free_deg[e]].push_back(e);
+                if (free_deg[e] > 0 && free_deg[e] < d) d = free_deg[e];
+            }
+    }
+    T.n = n;
+    T.npaired = (int)T.match.size();
+    for (int i = 0; i < n; ++i)
+        if (mate[i] < 0) T.match.push_back({i, -1, 0, 0});
+}
+
 // Cells order[0 .. n) cut into tiles by recursive bisection of their centroids along the longest
-// axis; tile sizes are appended to `sizes` in order.  A cut may move by a sixteenth of its range
-// to the widest gap between centroids there: between layers of cells where the mesh has them.
-static void bisect(const MeshView &m, const std::vector<double> &cen, int32_t *order, int n, std::vector<int32_t> &sizes,
+// axis; the tiles, their cells paired, are appended to `tiles` in order.  A cell left alone takes a
+// pair's place: a part of up to 2 kPairTilePairs cells that does not fit with its pairs is cut on.  A cut
+// may move by a sixteenth of its range to the widest gap between centroids there: between layers of
+// cells where the mesh has them.
+static void bisect(const MeshView &m, const std::vector<double> &cen, int32_t *order, int n, std::vector<PairTile> &tiles_out,
                    int depth) {
     const int most = 2 * kPairTilePairs;
     if (n <= most) {
@@ -442,9 +542,15 @@ static void bisect(const MeshView &m, const std::vector<double> &cen, int32_t *o
             nodes.insert(nodes.end(), m.closure + (size_t)c * m.nb, m.closure + (size_t)(c + 1) * m.nb);
             verts.insert(verts.end(), m.cone + (size_t)c * m.nv, m.cone + (size_t)(c + 1) * m.nv);
         }
-        if (n == 1 || (distinct(nodes) <= kPairTileNodes && distinct(verts) <= kPairTileVerts)) {
-            sizes.push_back(n);
-            return;
+        distinct(nodes);
+        if (n == 1 || ((int)nodes.size() <= kPairTileNodes && distinct(verts) <= kPairTileVerts)) {
+            PairTile T;
+            T.nodes = std::move(nodes);
+            match_cells(m, order, n, T);
+            if ((int)T.match.size() <= kPairTilePairs) {
+                tiles_out.push_back(std::move(T));
+                return;
+            }
         }
     }
     double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
@@ -480,7 +586,7 @@ static void bisect(const MeshView &m, const std::vector<double> &cen, int32_t *o
         }
     }
     if (depth < 3) {
-        std::vector<int32_t> right;
+        std::vector<PairTile> right;
         auto upper = [&] { bisect(m, cen, order + cut, n - cut, right, depth + 1); };
         std::thread t;
         try {
@@ -488,117 +594,32 @@ static void bisect(const MeshView &m, const std::vector<double> &cen, int32_t *o
         } catch (const std::system_error &) {
             upper();
         }
-        bisect(m, cen, order, cut, sizes, depth + 1);
+        bisect(m, cen, order, cut, tiles_out, depth + 1);
         if (t.joinable()) t.join();
-        sizes.insert(sizes.end(), right.begin(), right.end());
+        std::move(right.begin(), right.end(), std::back_inserter(tiles_out));
     } else {
-        bisect(m, cen, order, cut, sizes, depth + 1);
-        bisect(m, cen, order + cut, n - cut, sizes, depth + 1);
+        bisect(m, cen, order, cut, tiles_out, depth + 1);
+        bisect(m, cen, order + cut, n - cut, tiles_out, depth + 1);
     }
 }
 
-namespace {
-struct PairTile {
-    std::vector<int32_t> nodes;  // sorted distinct, then in local order (owned, shared)
-    std::vector<int32_t> verts;
-    int nown = 0;
-    std::vector<int32_t> cells;  // [pairs][2]
-    std::vector<uint32_t> rec;
-};
-}  // namespace
-
-// Pairs, numbering and records of one tile (cells ids[0 .. n); T.nodes its sorted nodes).
-static void build_pair_tile(const MeshView &m, const int32_t *ids, int n, const std::vector<int32_t> &tile_count,
-                            PairTile &T) {
-    auto local = [](const std::vector<int32_t> &v, int32_t x) {
-        return (int)(std::lower_bound(v.begin(), v.end(), x) - v.begin());
-    };
+// Numbering and records of one tile (cells ids[0 .. T.n), paired; T.nodes its sorted nodes).
+static void build_pair_tile(const MeshView &m, const int32_t *ids, const std::vector<int32_t> &tile_count, PairTile &T) {
+    const int n = T.n, np = (int)T.match.size();
     std::vector<int32_t> verts;
     for (int i = 0; i < n; ++i) verts.insert(verts.end(), m.cone + 4 * (size_t)ids[i], m.cone + 4 * (size_t)(ids[i] + 1));
     distinct(verts);
     std::vector<std::array<int, 4>> cv(n);  // tile vertices of each cell
     for (int i = 0; i < n; ++i)
-        for (int k = 0; k < 4; ++k) cv[i][k] = local(verts, m.cone[4 * (size_t)ids[i] + k]);
-    // faces of the tile: (vertices sorted) -> cell and the vertex opposite
-    std::vector<std::pair<uint64_t, int32_t>> faces;
-    for (int i = 0; i < n; ++i)
-        for (int k = 0; k < 4; ++k) {
-            std::array<int, 3> f{cv[i][(k + 1) & 3], cv[i][(k + 2) & 3], cv[i][(k + 3) & 3]};
-            std::sort(f.begin(), f.end());
-            faces.push_back({((uint64_t)f[0] << 40) | ((uint64_t)f[1] << 20) | (uint64_t)f[2], 4 * i + k});
-        }
-    std::sort(faces.begin(), faces.end());
-    std::vector<std::array<std::array<int, 3>, 4>> nbr(n);  // (neighbour, my opposite vertex, its)
-    std::vector<int> deg(n, 0);
-    for (size_t f = 0; f + 1 < faces.size(); ++f)
-        if (faces[f].first == faces[f + 1].first) {
-            const int a = faces[f].second >> 2, b = faces[f + 1].second >> 2;
-            if (a != b && deg[a] < 4 && deg[b] < 4) {
-                nbr[a][deg[a]++] = {b, faces[f].second & 3, faces[f + 1].second & 3};
-                nbr[b][deg[b]++] = {a, faces[f + 1].second & 3, faces[f].second & 3};
-            }
-            ++f;
-        }
-    // the second cell's face turned so that its first vertex is the first cell's; the other two then
-    // run the opposite way round in a consistently oriented mesh (else the cells are not paired)
-    static const int kApex[4][4] = {{0, 1, 2, 3}, {1, 0, 3, 2}, {2, 0, 1, 3}, {3, 0, 2, 1}};  // even permutations
-    auto orient = [&](int a, int oa, int b, int ob, int pa[4], int pb[4]) {
-        for (int k = 0; k < 4; ++k) pa[k] = kApex[oa][k];
-        for (int r = 0; r < 3; ++r) {
-            pb[0] = kApex[ob][0];
-            for (int k = 0; k < 3; ++k) pb[1 + k] = kApex[ob][1 + (k + r) % 3];
-            if (cv[b][pb[1]] == cv[a][pa[1]]) break;
-        }
-        return cv[b][pb[1]] == cv[a][pa[1]] && cv[b][pb[2]] == cv[a][pa[3]] && cv[b][pb[3]] == cv[a][pa[2]];
-    };
-    // matching: cells with the fewest free neighbours first, each to its neighbour with the fewest
-    std::vector<int> mate(n, -1), free_deg(deg);
-    std::vector<std::array<int, 2>> opp(n);
-    std::array<std::vector<int>, 5> bucket;
-    for (int i = n - 1; i >= 0; --i) bucket[free_deg[i]].push_back(i);
-    std::vector<std::array<int, 2>> pairs;  // (first, second)
-    for (int d = 1; d <= 4;) {
-        if (bucket[d].empty()) {
-            ++d;
-            continue;
-        }
-        const int a = bucket[d].back();
-        bucket[d].pop_back();
-        if (mate[a] >= 0 || free_deg[a] != d) continue;
-        int best = -1;
-        for (int k = 0; k < deg[a]; ++k) {
-            const int b = nbr[a][k][0];
-            if (mate[b] >= 0) continue;
-            int pa[4], pb[4];
-            if (!orient(a, nbr[a][k][1], b, nbr[a][k][2], pa, pb)) continue;
-            if (best < 0 || free_deg[b] < free_deg[nbr[a][best][0]]) best = k;
-        }
-        if (best < 0) continue;  // no neighbour it can be turned to: stays single
-        const int b = nbr[a][best][0];
-        mate[a] = b;
-        mate[b] = a;
-        opp[a] = {nbr[a][best][1], nbr[a][best][2]};
-        pairs.push_back({a, b});
-        for (int c : {a, b})
-            for (int k = 0; k < deg[c]; ++k) {
-                const int e = nbr[c][k][0];
-                if (mate[e] >= 0) continue;
-                if (--free_deg[e] > 0) bucket[free_deg[e]].push_back(e);
-                if (free_deg[e] > 0 && free_deg[e] < d) d = free_deg[e];
-            }
-    }
-    const int npaired = (int)pairs.size();
-    for (int i = 0; i < n; ++i)
-        if (mate[i] < 0) pairs.push_back({i, -1});
-    const int np = (int)pairs.size();
+        for (int k = 0; k < 4; ++k) cv[i][k] = place_of(verts, m.cone[4 * (size_t)ids[i] + k]);
     // slots: mesh nodes [14] and tile vertices [5] of each pair
     static const int kEdge[4][4] = {{-1, 4, 5, 6}, {4, -1, 7, 8}, {5, 7, -1, 9}, {6, 8, 9, -1}};
     std::vector<std::array<int32_t, 14>> pn(np);
     std::vector<std::array<int, 5>> pv(np);
     for (int p = 0; p < np; ++p) {
-        const int a = pairs[p][0], b = pairs[p][1];
+        const int a = T.match[p][0], b = T.match[p][1];
         int pa[4] = {0, 1, 2, 3}, pb[4] = {0, 1, 3, 2};
-        if (b >= 0) (void)orient(a, opp[a][0], b, opp[a][1], pa, pb);
+        if (b >= 0) (void)turn_to_face(&m.cone[4 * (size_t)ids[a]], T.match[p][2], &m.cone[4 * (size_t)ids[b]], T.match[p][3], pa, pb);
         const int q = b >= 0 ? b : a;  // alone: the second cell is the mirror image of the first
         const int32_t *ca = m.closure + 10 * (size_t)ids[a], *cb = m.closure + 10 * (size_t)ids[q];
         for (int k = 0; k < 4; ++k) {
@@ -619,7 +640,7 @@ static void build_pair_tile(const MeshView &m, const int32_t *ids, int n, const 
     // targets are distinct
     std::vector<std::array<int32_t, 14>> pl(np);
     for (int p = 0; p < np; ++p)
-        for (int j = 0; j < 14; ++j) pl[p][j] = local(T.nodes, pn[p][j]);
+        for (int j = 0; j < 14; ++j) pl[p][j] = place_of(T.nodes, pn[p][j]);
     std::vector<int> color(np), order(np);
     {
         std::vector<std::array<uint64_t, 2>> used(T.nodes.size(), {0, 0});
@@ -632,7 +653,7 @@ static void build_pair_tile(const MeshView &m, const int32_t *ids, int n, const 
             int c = 0;
             while (c < 127 && ((c < 64 ? (m0 >> c) : (m1 >> (c - 64))) & 1)) ++c;
             for (int32_t k : pl[p]) used[k][c >> 6] |= (uint64_t)1 << (c & 63);
-            color[p] = c + (p < npaired ? 0 : 128);
+            color[p] = c + (p < T.npaired ? 0 : 128);
             order[p] = p;
         }
         std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return color[a] < color[b]; });
@@ -646,7 +667,7 @@ static void build_pair_tile(const MeshView &m, const int32_t *ids, int n, const 
     ord.insert(ord.end(), sh.begin(), sh.end());
     std::vector<int32_t> rank(T.nodes.size());  // sorted position -> local index
     auto ranks = [&](const std::vector<int32_t> &v) {
-        for (size_t k = 0; k < v.size(); ++k) rank[local(T.nodes, v[k])] = (int32_t)k;
+        for (size_t k = 0; k < v.size(); ++k) rank[place_of(T.nodes, v[k])] = (int32_t)k;
     };
     ranks(ord);
     std::vector<std::vector<int32_t>> slot(14, std::vector<int32_t>(np));
@@ -671,8 +692,8 @@ static void build_pair_tile(const MeshView &m, const int32_t *ids, int n, const 
         for (int j = 0; j < 12; ++j) w[j / 3] |= (uint32_t)rank[pl[p][j]] << (10 * (j % 3));
         w[4] = (uint32_t)rank[pl[p][12]] | (uint32_t)rank[pl[p][13]] << 10 | (uint32_t)vslot_id[pv[p][4]] << 20;
         for (int j = 0; j < 4; ++j) w[5] |= (uint32_t)vslot_id[pv[p][j]] << (8 * j);
-        T.cells[2 * (size_t)i] = ids[pairs[p][0]];
-        T.cells[2 * (size_t)i + 1] = pairs[p][1] >= 0 ? ids[pairs[p][1]] : -1;
+        T.cells[2 * (size_t)i] = ids[T.match[p][0]];
+        T.cells[2 * (size_t)i + 1] = T.match[p][1] >= 0 ? ids[T.match[p][1]] : -1;
     }
     T.nodes = std::move(ord);
 }
@@ -681,9 +702,9 @@ static void build_pair_tile(const MeshView &m, const int32_t *ids, int n, const 
 static int64_t tile_nodes_of(const MeshView &m, const std::vector<int32_t> &cells, const std::vector<int32_t> &ptr,
                              std::vector<PairTile> &tiles, std::vector<int32_t> &tile_count) {
     const int nt = (int)ptr.size() - 1;
-    tiles.assign(nt, PairTile());
     parallel_for(nt, [&](int t) {
         std::vector<int32_t> &v = tiles[t].nodes;
+        if (!v.empty()) return;
         for (int i = ptr[t]; i < ptr[t + 1]; ++i)
             v.insert(v.end(), m.closure + (size_t)cells[i] * m.nb, m.closure + (size_t)(cells[i] + 1) * m.nb);
         distinct(v);
@@ -713,18 +734,24 @@ int build_pair_plan(const MeshView &m, const HostPlan &base, PairPlan *pp, std::
                 for (int v = 0; v < 4; ++v) acc += m.coords[3 * (size_t)m.cone[4 * (size_t)c + v] + d];
                 cen[3 * (size_t)c + d] = 0.25 * acc;
             }
-        std::vector<int32_t> sizes;
-        bisect(m, cen, cells.data(), n, sizes, 0);
-        for (int32_t s : sizes) ptr.push_back(ptr.back() + s);
+        bisect(m, cen, cells.data(), n, tiles, 0);
+        for (const PairTile &T : tiles) ptr.push_back(ptr.back() + T.n);
     }
     int64_t halo = tile_nodes_of(m, cells, ptr, tiles, tile_count);
     if (halo > base.halo_slots) {
         cells = base.cells;
         ptr = base.tile_cell_ptr;
+        tiles.assign(base.num_tiles, PairTile());
+        parallel_for(base.num_tiles, [&](int t) { match_cells(m, &cells[ptr[t]], ptr[t + 1] - ptr[t], tiles[t]); });
+        for (const PairTile &T : tiles)
+            if ((int)T.match.size() > kPairTilePairs) {
+                *err = "pair tile over its bounds";
+                return 1;
+            }
         halo = tile_nodes_of(m, cells, ptr, tiles, tile_count);
     }
     const int nt = (int)ptr.size() - 1;
-    parallel_for(nt, [&](int t) { build_pair_tile(m, &cells[ptr[t]], ptr[t + 1] - ptr[t], tile_count, tiles[t]); });
+    parallel_for(nt, [&](int t) { build_pair_tile(m, &cells[ptr[t]], tile_count, tiles[t]); });
     *pp = PairPlan();
     pp->num_tiles = nt;
     pp->halo_slots = halo;

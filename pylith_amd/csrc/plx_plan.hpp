@@ -72,7 +72,8 @@ inline int pair_node(const uint32_t *w, int j) {
 inline int pair_vert(const uint32_t *w, int j) { return j < 4 ? (int)((w[5] >> (8 * j)) & 255u) : (int)((w[4] >> 20) & 255u); }
 
 // Pair plan of the base plan's cells (P2).  The cells are cut by recursive coordinate bisection of their
-// centroids; where that gives no fewer halo slots than the base plan's tiles, those are kept.
+// centroids; where that gives no fewer halo slots than the base plan's tiles, those are kept.  Nonzero
+// with a message where there is none (a tile of the base plan would need more than kPairTilePairs).
 int build_pair_plan(const MeshView &m, const HostPlan &base, PairPlan *pp, std::string *err);
 
 // Gather plan of a small key: tiles own nodes instead of cells.  Each tile holds every cell that touches

@@ -10,6 +10,7 @@ import pytest
 from pylith_amd import _lib as L
 from pylith_amd import meshgen as mg
 from pylith_amd import meshio_ascii
+from general_meshes import delaunay_p2
 
 GOLDEN = os.path.join(os.path.dirname(__file__), "golden")
 
@@ -91,6 +92,29 @@ def pair_cases():
         "tet_renumbered": (mg.renumbered(mg.tet_p2_box(7, (0, 0, 0), (600.0, 600.0, 600.0)), 8), 0),
         "tet_label": (big, 1),
     }
+
+
+def general_pair_case(name):
+    """Meshes whose cells do not all find a partner: nearly full tiles with more than kPairTilePairs pairs and
+    lone cells are cut again."""
+    if name == "label_95":
+        m = mg.tet_p2_box((27, 29, 31), (0, 0, 0), (2700.0, 2900.0, 3100.0))
+        m.labels = (np.random.default_rng(2).random(m.num_cells) < 0.95).astype(np.int32)
+        return m, 1
+    return (delaunay_p2(12500, 1) if name == "delaunay" else delaunay_p2(3000, 4, jitter=0.45)), 0
+
+
+@pytest.mark.parametrize("name", ["delaunay", "delaunay_jitter", "label_95"])
+def test_emulated_pair_kernel_on_general_meshes(name):
+    """As above; det J of the Delaunay cells carries a relative error of a few eps / 0.02, some 1e-14, in either
+    kernel (the vertices enter in another order): 1e-12."""
+    m, label = general_pair_case(name)
+    aux, _ = mg.elastic_aux(m.num_cells, seed=5, vs_sigma=0.2, vp_vs=1.8)
+    u = mg.random_field(m.num_nodes, 3)
+    ref = emulate(m, aux, u, label)
+    assert relerr(emulate(m, aux, u, label, algo=EMULATE_PAIRS), ref) <= 1e-12
+    r32 = emulate(m, aux, u, label, scalar=L.FP32, algo=EMULATE_PAIRS)
+    assert relerr(r32.astype(np.float64), ref) <= 2e-5
 
 
 @pytest.mark.parametrize("name", list(pair_cases()))

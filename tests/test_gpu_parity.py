@@ -12,6 +12,7 @@ torch = pytest.importorskip("torch")
 
 from pylith_amd import meshgen as mg  # noqa: E402
 from pylith_amd import meshio_ascii  # noqa: E402
+from general_meshes import delaunay_p2  # noqa: E402
 
 pytestmark = pytest.mark.gpu
 GOLDEN = os.path.join(os.path.dirname(__file__), "golden")
@@ -166,9 +167,10 @@ def test_p2_tets_config2_64cube(oracle):
 
 # meshes over the line where P2 keys take the pair kernel (65,536 cells): bricks with a remainder, no
 # locality in the numbering, and a key of scattered cells with a second key beside it
-@pytest.mark.parametrize("kind", ["bricks", "random", "scattered_key"])
+@pytest.mark.parametrize("kind", ["bricks", "random", "scattered_key", "delaunay"])
 def test_p2_pair_kernel(oracle, kind):
-    m = mg.tet_p2_box((27, 23, 21), (0, 0, 0), (2700.0, 2300.0, 2100.0))
+    m = (delaunay_p2(12500, 1) if kind == "delaunay"  # (tiles whose cells do not all find a partner)
+         else mg.tet_p2_box((27, 23, 21), (0, 0, 0), (2700.0, 2300.0, 2100.0)))
     if kind == "random":
         m = mg.renumbered(m, 5)
     label = 0
