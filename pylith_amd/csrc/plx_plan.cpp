@@ -446,18 +446,30 @@ static int place_of(const std::vector<int32_t> &v, int32_t x) {
     return (int)(std::lower_bound(v.begin(), v.end(), x) - v.begin());
 }
 
-// Local vertices of two cells that share a face, the vertices opposite it (oa, ob) first and the
-// second cell's face turned so that its first vertex is the first cell's; the other two then run the
-// opposite way round in a consistently oriented mesh (else the cells are not paired).
-static bool turn_to_face(const int32_t *va, int oa, const int32_t *vb, int ob, int pa[4], int pb[4]) {
+// Local node of the edge between two vertices of a P2 tetrahedron.
+static const int kTetEdge[4][4] = {{-1, 4, 5, 6}, {4, -1, 7, 8}, {5, 7, -1, 9}, {6, 8, 9, -1}};
+
+// Local vertices of cells a and b, which share a face, the vertices opposite it (oa, ob) first and b's
+// face turned so that its first vertex is a's; the other two then run the opposite way round in a
+// consistently oriented mesh.  False, and the cells no pair, where they do not, or where the cells'
+// nodes on the face differ (vertices of one place with nodes of their own on either side).
+static bool turn_to_face(const MeshView &m, int32_t a, int oa, int32_t b, int ob, int pa[4], int pb[4]) {
     static const int kApex[4][4] = {{0, 1, 2, 3}, {1, 0, 3, 2}, {2, 0, 1, 3}, {3, 0, 2, 1}};  // even permutations
+    const int32_t *va = m.cone + 4 * (size_t)a, *vb = m.cone + 4 * (size_t)b;
+    const int32_t *ca = m.closure + 10 * (size_t)a, *cb = m.closure + 10 * (size_t)b;
     for (int k = 0; k < 4; ++k) pa[k] = kApex[oa][k];
     for (int r = 0; r < 3; ++r) {
         pb[0] = kApex[ob][0];
         for (int k = 0; k < 3; ++k) pb[1 + k] = kApex[ob][1 + (k + r) % 3];
         if (vb[pb[1]] == va[pa[1]]) break;
     }
-    return vb[pb[1]] == va[pa[1]] && vb[pb[2]] == va[pa[3]] && vb[pb[3]] == va[pa[2]];
+    const int qb[4] = {pb[0], pb[1], pb[3], pb[2]};  // b's vertices in a's order
+    for (int k = 1; k < 4; ++k) {
+        if (vb[qb[k]] != va[pa[k]] || cb[qb[k]] != ca[pa[k]]) return false;
+        const int l = k % 3 + 1;  // and the edge to the next
+        if (cb[kTetEdge[qb[k]][qb[l]]] != ca[kTetEdge[pa[k]][pa[l]]]) return false;
+    }
+    return true;
 }
 
 // The pairs of the cells ids[0 .. n).
@@ -503,7 +515,7 @@ static void match_cells(const MeshView &m, const int32_t *ids, int n, PairTile &
             const int b = nbr[a][k][0];
             if (mate[b] >= 0) continue;
             int pa[4], pb[4];
-            if (!turn_to_face(vert(a), nbr[a][k][1], vert(b), nbr[a][k][2], pa, pb)) continue;
+            if (!turn_to_face(m, ids[a], nbr[a][k][1], ids[b], nbr[a][k][2], pa, pb)) continue;
             if (best < 0 || free_deg[b] < free_deg[nbr[a][best][0]]) best = k;
         }
         if (best < 0) continue;  // no neighbour it can be turned to: stays single
@@ -613,28 +625,27 @@ static void build_pair_tile(const MeshView &m, const int32_t *ids, const std::ve
     for (int i = 0; i < n; ++i)
         for (int k = 0; k < 4; ++k) cv[i][k] = place_of(verts, m.cone[4 * (size_t)ids[i] + k]);
     // slots: mesh nodes [14] and tile vertices [5] of each pair
-    static const int kEdge[4][4] = {{-1, 4, 5, 6}, {4, -1, 7, 8}, {5, 7, -1, 9}, {6, 8, 9, -1}};
     std::vector<std::array<int32_t, 14>> pn(np);
     std::vector<std::array<int, 5>> pv(np);
     for (int p = 0; p < np; ++p) {
         const int a = T.match[p][0], b = T.match[p][1];
         int pa[4] = {0, 1, 2, 3}, pb[4] = {0, 1, 3, 2};
-        if (b >= 0) (void)turn_to_face(&m.cone[4 * (size_t)ids[a]], T.match[p][2], &m.cone[4 * (size_t)ids[b]], T.match[p][3], pa, pb);
+        if (b >= 0) (void)turn_to_face(m, ids[a], T.match[p][2], ids[b], T.match[p][3], pa, pb);
         const int q = b >= 0 ? b : a;  // alone: the second cell is the mirror image of the first
         const int32_t *ca = m.closure + 10 * (size_t)ids[a], *cb = m.closure + 10 * (size_t)ids[q];
         for (int k = 0; k < 4; ++k) {
             pn[p][k] = ca[pa[k]];
             pv[p][k] = cv[a][pa[k]];
         }
-        for (int k = 0; k < 3; ++k) pn[p][4 + k] = ca[kEdge[pa[0]][pa[1 + k]]];
-        pn[p][7] = ca[kEdge[pa[1]][pa[2]]];
-        pn[p][8] = ca[kEdge[pa[1]][pa[3]]];
-        pn[p][9] = ca[kEdge[pa[2]][pa[3]]];
+        for (int k = 0; k < 3; ++k) pn[p][4 + k] = ca[kTetEdge[pa[0]][pa[1 + k]]];
+        pn[p][7] = ca[kTetEdge[pa[1]][pa[2]]];
+        pn[p][8] = ca[kTetEdge[pa[1]][pa[3]]];
+        pn[p][9] = ca[kTetEdge[pa[2]][pa[3]]];
         pn[p][10] = cb[pb[0]];
         pv[p][4] = cv[q][pb[0]];
-        pn[p][11] = cb[kEdge[pb[0]][pb[1]]];  // to x
-        pn[p][12] = cb[kEdge[pb[0]][pb[3]]];  // to y
-        pn[p][13] = cb[kEdge[pb[0]][pb[2]]];  // to z
+        pn[p][11] = cb[kTetEdge[pb[0]][pb[1]]];  // to x
+        pn[p][12] = cb[kTetEdge[pb[0]][pb[3]]];  // to y
+        pn[p][13] = cb[kTetEdge[pb[0]][pb[2]]];  // to z
     }
     // pairs of one colour share no node; sorted by colour (paired ones first) a wave's atomic
     // targets are distinct

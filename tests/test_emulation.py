@@ -132,6 +132,26 @@ def test_emulated_pair_kernel_matches_tile_kernel(name):
     assert relerr(radd - 1.0, ref) <= 1e-11
 
 
+@pytest.mark.parametrize("split", ["edges", "all"])
+def test_emulated_pair_kernel_with_nodes_split_on_a_plane(split):
+    """Cells on either side of a plane share its vertices' coordinates (cone) but not its nodes (closure):
+    all of them, or those of its edges alone.  Faces there do not make pairs."""
+    m = mg.tet_p2_box((4, 3, 2), (0, 0, 0), (4.0, 3.0, 2.0))
+    far = m.node_coords[m.closure].mean(1)[:, 0] > 2.0
+    plane = np.flatnonzero(np.abs(m.node_coords[:, 0] - 2.0) < 1e-9)
+    if split == "edges":
+        plane = np.setdiff1d(plane, m.closure[:, :4])
+    new = np.arange(m.num_nodes)
+    new[plane] = m.num_nodes + np.arange(len(plane))
+    m.closure[far] = new[m.closure[far]]
+    m.node_coords = np.concatenate([m.node_coords, m.node_coords[plane]])
+    aux, _ = mg.elastic_aux(m.num_cells, seed=5, vs_sigma=0.2, vp_vs=1.8)
+    u = mg.random_field(m.num_nodes, 3)
+    ref = emulate(m, aux, u)
+    for algo in (EMULATE_PAIRS, EMULATE_GATHER):
+        assert relerr(emulate(m, aux, u, algo=algo), ref) <= 1e-13
+
+
 EMULATE_GATHER = 101  # PLX_EMULATE_GATHER
 
 
