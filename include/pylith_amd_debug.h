@@ -25,6 +25,9 @@ extern "C" {
 int plx_debug_plan_info(plx_dm dm, int label_value, int part, int *num_tiles, int64_t *halo_slots,
                         int *reordered);
 
+/* Tiles of the key's pair plan and gather plan (0: none). */
+int plx_debug_second_plans(plx_dm dm, int label_value, int part, int *pair_tiles, int *gather_tiles);
+
 /* Z = M R: one multigrid V-cycle on k columns (k in {1, 8, 16, 32, 64}) of a Green's-function handle
  * with the multigrid preconditioner; R, Z: DEVICE [dof][k] in DM order.  R must be complete when the
  * call is made (the handle's own stream reads it); synchronises. */

@@ -144,4 +144,6 @@ SIGNATURES["plx_debug_emulate_apply"] = (_c_int, [_c_int, _c_int, _c_int, _c_int
                                                   _c_int, _c_int])
 SIGNATURES["plx_debug_plan_info"] = (_c_int, [_vp, _c_int, _c_int, ctypes.POINTER(_c_int), _i64p,
                                               ctypes.POINTER(_c_int)])
+SIGNATURES["plx_debug_second_plans"] = (_c_int, [_vp, _c_int, _c_int, ctypes.POINTER(_c_int),
+                                                  ctypes.POINTER(_c_int)])
 SIGNATURES["plx_debug_gf_precondition"] = (_c_int, [_vp, _c_int, _vp, _vp])

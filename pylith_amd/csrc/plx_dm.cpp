@@ -99,6 +99,11 @@ static std::vector<TileHead> tile_heads(const HostPlan &hp) {
 // waves there.  FP64 / FP32 apply, pairs against tiles: 48,000 cells 10.2 / 9.4 against 9.5 / 9.0 us, 83,000
 // 11.6 / 9.9 against 12.1 / 10.7 us, 196,000 17.2 / 14.5 against 20.9 / 17.5 us.
 constexpr int64_t kPairMinCells = 65536;
+// So do keys whose pair tiles hold fewer cells on average (scattered cells: many without a partner, few to a
+// tile's nodes).  FP64, pairs against tiles, at so many cells a pair tile: Delaunay 393 12.5 against 13.9 us,
+// 27 x 29 x 31 x 6 box 405 15.0 against 16.0 us, 80 % of its cells 276 14.2 against 15.0 us; 60 % of 34^3 x 6 232 18.3
+// against 17.8 us, three of six of 42^3 x 6 204 26.4 against 23.9 us, one of six 105 19.7 against 16.6 us.
+constexpr int64_t kPairMinFill = 256;
 
 // Build the key's tile plan on the host (plx_plan.cpp) and upload it.
 static int build_plan(plx_dm dm, KeyPlan *kp) {
@@ -162,7 +167,8 @@ static int build_plan(plx_dm dm, KeyPlan *kp) {
     if (hp.halo_slots > 0) PLX_HIP(dm, hipMalloc(&kp->d_halo, (size_t)hp.halo_slots * 3 * sizeof(double)));
     // (a key without a pair plan keeps the tile plan alone)
     PairPlan pp;
-    if (dm->cell_type == PLX_TET_P2 && (int64_t)hp.cells.size() >= kPairMinCells && !build_pair_plan(mv, hp, &pp, &msg)) {
+    if (dm->cell_type == PLX_TET_P2 && (int64_t)hp.cells.size() >= kPairMinCells && !build_pair_plan(mv, hp, &pp, &msg) &&
+        (int64_t)hp.cells.size() >= kPairMinFill * pp.num_tiles) {
         PairDev &P = kp->pairs;
         P.num_tiles = pp.num_tiles;
         P.num_pairs = pp.num_pairs;
@@ -870,6 +876,14 @@ int plx_debug_plan_info(plx_dm dm, int label_value, int part, int *num_tiles, in
     if (num_tiles) *num_tiles = kp->num_tiles;
     if (halo_slots) *halo_slots = kp->halo_slots;
     if (reordered) *reordered = kp->reordered ? 1 : 0;
+    return 0;
+}
+
+int plx_debug_second_plans(plx_dm dm, int label_value, int part, int *pair_tiles, int *gather_tiles) {
+    KeyPlan *kp = dm ? find_key(dm, label_value, part) : nullptr;
+    if (!kp) return set_error(dm, 1, "unknown key");
+    if (pair_tiles) *pair_tiles = kp->pairs.num_tiles;
+    if (gather_tiles) *gather_tiles = kp->gather.num_tiles;
     return 0;
 }
 

@@ -190,6 +190,29 @@ def test_p2_pair_kernel(oracle, kind):
         assert relerr(r.double().cpu().numpy(), ref) <= tol
 
 
+def second_plans(dm, label=0):
+    """Tiles of the key's pair and gather plans."""
+    import ctypes
+    pairs, gather = ctypes.c_int(-1), ctypes.c_int(-1)
+    assert dm.lib.plx_debug_second_plans(dm.h, label, 0, ctypes.byref(pairs), ctypes.byref(gather)) == 0
+    return pairs.value, gather.value
+
+
+# keys of scattered cells, either side of the line where pair tiles hold too few of them
+@pytest.mark.parametrize("kind,pairs", [("eighty", True), ("sixty", False), ("one_of_six", False)])
+def test_p2_pair_kernel_not_for_scattered_cells(oracle, kind, pairs):
+    n = {"eighty": 27, "sixty": 28, "one_of_six": 42}[kind]
+    m = mg.tet_p2_box(n, (0, 0, 0), (100.0 * n,) * 3)
+    if kind == "one_of_six":
+        m.labels = (np.arange(m.num_cells) % 6 == 0).astype(np.int32)
+    else:
+        m.labels = (np.random.default_rng(2).random(m.num_cells) < (0.8 if kind == "eighty" else 0.6)).astype(np.int32)
+    assert int(m.labels.sum()) >= 65536
+    aux = mg.elastic_aux(m.num_cells, seed=6, vs_sigma=0.2, vp_vs=1.8)
+    dm, _ = check_residual(oracle, m, mg.random_field(m.num_nodes, 9), label=1, aux=aux)
+    assert (second_plans(dm, 1)[0] > 0) == pairs
+
+
 # either side of the line where a key takes the gather plan (38^3 hexes and 6 x 16^3 tets are about the
 # largest), non-affine hexes, and a mesh of affine and other hex tiles
 @pytest.mark.parametrize("kind", ["hex38", "hex41", "hex_warped", "hex_mixed", "tet16", "tet18"])
