@@ -8,7 +8,9 @@
 #include <algorithm>
 #include <array>
 #include <cmath>
+#include <exception>
 #include <iterator>
+#include <mutex>
 #include <system_error>
 #include <thread>
 
@@ -53,27 +55,78 @@ std::vector<int32_t> morton_permutation(const double *xyz, size_t n) {
     return out;
 }
 
+// Joins its threads, whichever way the scope is left.
+struct Threads {
+    std::vector<std::thread> th;
+    ~Threads() { join(); }
+    void join() {
+        for (auto &x : th)
+            if (x.joinable()) x.join();
+    }
+};
+
+// The first exception of work on several threads, to be thrown again by the one that started them.
+struct FirstFailure {
+    std::mutex mu;
+    std::exception_ptr what;
+    template <typename F>
+    void guard(const F &work) {
+        try {
+            work();
+        } catch (...) {
+            std::lock_guard<std::mutex> lock(mu);
+            if (!what) what = std::current_exception();
+        }
+    }
+    void rethrow() const {
+        if (what) std::rethrow_exception(what);
+    }
+};
+
 // body(i) for i in [0, n) on host threads, in contiguous ranges.
 template <typename F>
 static void parallel_for(int n, const F &body) {
     const int nt = std::max(1, std::min({(int)std::thread::hardware_concurrency(), 16, n / 64 + 1}));
-    if (nt == 1) {
-        for (int i = 0; i < n; ++i) body(i);
-        return;
-    }
-    std::vector<std::thread> th;
-    th.reserve(nt);
+    FirstFailure failure;
+    Threads threads;
+    threads.th.reserve(nt);
     for (int t = 0; t < nt; ++t) {
         auto range = [&, t] {
-            for (int i = (int)((int64_t)n * t / nt); i < (int)((int64_t)n * (t + 1) / nt); ++i) body(i);
+            failure.guard([&] {
+                for (int i = (int)((int64_t)n * t / nt); i < (int)((int64_t)n * (t + 1) / nt); ++i) body(i);
+            });
         };
+        if (t + 1 == nt) {  // the last range runs here
+            range();
+            break;
+        }
         try {
-            th.emplace_back(range);
-        } catch (const std::system_error &) {  // no thread to be had: this range runs here
+            threads.th.emplace_back(range);
+        } catch (const std::system_error &) {  // no thread to be had: so does this one
             range();
         }
     }
-    for (auto &x : th) x.join();
+    threads.join();
+    failure.rethrow();
+}
+
+// here() and there(), the latter on a thread of its own if `threaded` and one is to be had.
+template <typename Here, typename There>
+static void both(bool threaded, const Here &here, const There &there) {
+    FirstFailure failure;
+    Threads other;
+    if (threaded) {
+        other.th.reserve(1);
+        try {
+            other.th.emplace_back([&] { failure.guard(there); });
+        } catch (const std::system_error &) {
+            threaded = false;
+        }
+    }
+    here();
+    if (!threaded) there();
+    other.join();
+    failure.rethrow();
 }
 
 static int distinct(std::vector<int32_t> &v) {
@@ -597,22 +650,10 @@ static void bisect(const MeshView &m, const std::vector<double> &cen, int32_t *o
             cut = i;
         }
     }
-    if (depth < 3) {
-        std::vector<PairTile> right;
-        auto upper = [&] { bisect(m, cen, order + cut, n - cut, right, depth + 1); };
-        std::thread t;
-        try {
-            t = std::thread(upper);
-        } catch (const std::system_error &) {
-            upper();
-        }
-        bisect(m, cen, order, cut, tiles_out, depth + 1);
-        if (t.joinable()) t.join();
-        std::move(right.begin(), right.end(), std::back_inserter(tiles_out));
-    } else {
-        bisect(m, cen, order, cut, tiles_out, depth + 1);
-        bisect(m, cen, order + cut, n - cut, tiles_out, depth + 1);
-    }
+    std::vector<PairTile> right;
+    both(depth < 3, [&] { bisect(m, cen, order, cut, tiles_out, depth + 1); },
+         [&] { bisect(m, cen, order + cut, n - cut, right, depth + 1); });
+    std::move(right.begin(), right.end(), std::back_inserter(tiles_out));
 }
 
 // Numbering and records of one tile (cells ids[0 .. T.n), paired; T.nodes its sorted nodes).
@@ -823,15 +864,8 @@ static void bisect_equal(const std::vector<double> &x, int32_t *order, int n, in
         return u < v || (u == v && a < b);
     });
     std::vector<int32_t> right;
-    auto upper = [&] { bisect_equal(x, order + cut, n - cut, parts - left, right, depth + 1); };
-    std::thread t;
-    if (depth < 3 && n > 2000) try {
-            t = std::thread(upper);
-        } catch (const std::system_error &) {
-        }
-    bisect_equal(x, order, cut, left, sizes, depth + 1);
-    if (t.joinable()) t.join();
-    else upper();
+    both(depth < 3 && n > 2000, [&] { bisect_equal(x, order, cut, left, sizes, depth + 1); },
+         [&] { bisect_equal(x, order + cut, n - cut, parts - left, right, depth + 1); });
     sizes.insert(sizes.end(), right.begin(), right.end());
 }
 
