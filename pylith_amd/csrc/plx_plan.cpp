@@ -11,6 +11,7 @@
 #include <exception>
 #include <iterator>
 #include <mutex>
+#include <numeric>
 #include <system_error>
 #include <thread>
 
@@ -83,18 +84,16 @@ struct FirstFailure {
     }
 };
 
-// body(i) for i in [0, n) on host threads, in contiguous ranges.
+// body(lo, hi) over [0, n) on host threads, in contiguous ranges.
 template <typename F>
-static void parallel_for(int n, const F &body) {
+static void parallel_ranges(int n, const F &body) {
     const int nt = std::max(1, std::min({(int)std::thread::hardware_concurrency(), 16, n / 64 + 1}));
     FirstFailure failure;
     Threads threads;
     threads.th.reserve(nt);
     for (int t = 0; t < nt; ++t) {
         auto range = [&, t] {
-            failure.guard([&] {
-                for (int i = (int)((int64_t)n * t / nt); i < (int)((int64_t)n * (t + 1) / nt); ++i) body(i);
-            });
+            failure.guard([&] { body((int)((int64_t)n * t / nt), (int)((int64_t)n * (t + 1) / nt)); });
         };
         if (t + 1 == nt) {  // the last range runs here
             range();
@@ -108,6 +107,13 @@ static void parallel_for(int n, const F &body) {
     }
     threads.join();
     failure.rethrow();
+}
+
+template <typename F>
+static void parallel_for(int n, const F &body) {
+    parallel_ranges(n, [&](int lo, int hi) {
+        for (int i = lo; i < hi; ++i) body(i);
+    });
 }
 
 // here() and there(), the latter on a thread of its own if `threaded` and one is to be had.
@@ -129,7 +135,24 @@ static void both(bool threaded, const Here &here, const There &there) {
     failure.rethrow();
 }
 
+// v's distinct entries (non-negative), sorted.  Entries repeat several times over (a node in every cell around
+// it): the repeats go first, through a table of twice the entries, and only the rest is sorted.
 static int distinct(std::vector<int32_t> &v) {
+    if (v.size() > 64) {
+        int bits = 8;
+        while (((size_t)1 << bits) < 2 * v.size()) ++bits;
+        std::vector<int32_t> table((size_t)1 << bits, -1);
+        size_t kept = 0;
+        for (size_t i = 0; i < v.size(); ++i) {
+            const int32_t x = v[i];
+            size_t at = (uint32_t)x * 2654435769u >> (32 - bits);
+            while (table[at] >= 0 && table[at] != x) at = (at + 1) & (table.size() - 1);
+            if (table[at] == x) continue;
+            table[at] = x;
+            v[kept++] = x;
+        }
+        v.resize(kept);
+    }
     std::sort(v.begin(), v.end());
     v.erase(std::unique(v.begin(), v.end()), v.end());
     return (int)v.size();
@@ -233,16 +256,12 @@ static void balance_banks(std::vector<int32_t> &ids, const std::vector<int> &ran
     for (int k : order) {
         if (res[k] >= 0) continue;
         const int q = range_of[k];
-        int best = -1, best_cost = 0;
-        for (int r = 0; r < 16; ++r) {
-            if (cap[q][r] == 0) continue;
-            int cost = 0;
-            for (int j = item_acc_ptr[k]; j < item_acc_ptr[k + 1]; ++j) cost += 2 * load[item_acc[j]][r] + 1;
-            if (best < 0 || cost < best_cost) {
-                best = r;
-                best_cost = cost;
-            }
-        }
+        int sum[16] = {};
+        for (int j = item_acc_ptr[k]; j < item_acc_ptr[k + 1]; ++j)
+            for (int r = 0; r < 16; ++r) sum[r] += load[item_acc[j]][r];
+        int best = -1;
+        for (int r = 0; r < 16; ++r)
+            if (cap[q][r] > 0 && (best < 0 || sum[r] < sum[best])) best = r;
         res[k] = best;
         cap[q][best]--;
         for (int j = item_acc_ptr[k]; j < item_acc_ptr[k + 1]; ++j) load[item_acc[j]][best]++;
@@ -487,7 +506,8 @@ struct PairTile {
     std::vector<std::array<int, 4>> match;  // pairs: first cell, second (-1: none), their vertices opposite the face
     int npaired = 0;                        // those with a second cell come first
     std::vector<int32_t> nodes;  // sorted distinct, then in local order (owned, shared)
-    std::vector<int32_t> verts;
+    std::vector<int32_t> verts;  // likewise
+    std::vector<std::array<int, 4>> cv;  // each cell's vertices, places in the sorted verts
     int nown = 0;
     std::vector<int32_t> cells;  // [pairs][2]
     std::vector<uint32_t> rec;
@@ -525,19 +545,25 @@ static bool turn_to_face(const MeshView &m, int32_t a, int oa, int32_t b, int ob
     return true;
 }
 
-// The pairs of the cells ids[0 .. n).
+// The vertices (unless there) and pairs of the cells ids[0 .. n).
 static void match_cells(const MeshView &m, const int32_t *ids, int n, PairTile &T) {
-    const auto vert = [&](int i) { return m.cone + 4 * (size_t)ids[i]; };
+    T.n = n;
+    if (T.verts.empty())
+        for (int i = 0; i < n; ++i) T.verts.insert(T.verts.end(), m.cone + 4 * (size_t)ids[i], m.cone + 4 * (size_t)(ids[i] + 1));
+    distinct(T.verts);
+    T.cv.resize(n);
     // faces of the tile: (vertices sorted) -> cell and the vertex opposite
-    std::vector<std::pair<std::array<int32_t, 3>, int32_t>> faces;
+    std::vector<std::pair<uint64_t, int32_t>> faces;
     faces.reserve(4 * (size_t)n);
-    for (int i = 0; i < n; ++i)
+    for (int i = 0; i < n; ++i) {
+        std::array<int, 4> &v = T.cv[i];
+        for (int k = 0; k < 4; ++k) v[k] = place_of(T.verts, m.cone[4 * (size_t)ids[i] + k]);
         for (int k = 0; k < 4; ++k) {
-            const int32_t *v = vert(i);
-            std::array<int32_t, 3> f{v[(k + 1) & 3], v[(k + 2) & 3], v[(k + 3) & 3]};
+            std::array<int, 3> f{v[(k + 1) & 3], v[(k + 2) & 3], v[(k + 3) & 3]};
             std::sort(f.begin(), f.end());
-            faces.push_back({f, 4 * i + k});
+            faces.push_back({((uint64_t)f[0] << 40) | ((uint64_t)f[1] << 20) | (uint64_t)f[2], 4 * i + k});
         }
+    }
     std::sort(faces.begin(), faces.end());
     std::vector<std::array<std::array<int, 3>, 4>> nbr(n);  // (neighbour, my opposite vertex, its)
     std::vector<int> deg(n, 0);
@@ -584,7 +610,6 @@ static void match_cells(const MeshView &m, const int32_t *ids, int n, PairTile &
                 if (free_deg[e] > 0 && free_deg[e] < d) d = free_deg[e];
             }
     }
-    T.n = n;
     T.npaired = (int)T.match.size();
     for (int i = 0; i < n; ++i)
         if (mate[i] < 0) T.match.push_back({i, -1, 0, 0});
@@ -608,9 +633,11 @@ static void bisect(const MeshView &m, const std::vector<double> &cen, int32_t *o
             verts.insert(verts.end(), m.cone + (size_t)c * m.nv, m.cone + (size_t)(c + 1) * m.nv);
         }
         distinct(nodes);
-        if (n == 1 || ((int)nodes.size() <= kPairTileNodes && distinct(verts) <= kPairTileVerts)) {
+        distinct(verts);
+        if (n == 1 || ((int)nodes.size() <= kPairTileNodes && (int)verts.size() <= kPairTileVerts)) {
             PairTile T;
             T.nodes = std::move(nodes);
+            T.verts = std::move(verts);
             match_cells(m, order, n, T);
             if ((int)T.match.size() <= kPairTilePairs) {
                 tiles_out.push_back(std::move(T));
@@ -658,13 +685,9 @@ static void bisect(const MeshView &m, const std::vector<double> &cen, int32_t *o
 
 // Numbering and records of one tile (cells ids[0 .. T.n), paired; T.nodes its sorted nodes).
 static void build_pair_tile(const MeshView &m, const int32_t *ids, const std::vector<int32_t> &tile_count, PairTile &T) {
-    const int n = T.n, np = (int)T.match.size();
-    std::vector<int32_t> verts;
-    for (int i = 0; i < n; ++i) verts.insert(verts.end(), m.cone + 4 * (size_t)ids[i], m.cone + 4 * (size_t)(ids[i] + 1));
-    distinct(verts);
-    std::vector<std::array<int, 4>> cv(n);  // tile vertices of each cell
-    for (int i = 0; i < n; ++i)
-        for (int k = 0; k < 4; ++k) cv[i][k] = place_of(verts, m.cone[4 * (size_t)ids[i] + k]);
+    const int np = (int)T.match.size();
+    const std::vector<int32_t> verts(std::move(T.verts));
+    const std::vector<std::array<int, 4>> cv(std::move(T.cv));
     // slots: mesh nodes [14] and tile vertices [5] of each pair
     std::vector<std::array<int32_t, 14>> pn(np);
     std::vector<std::array<int, 5>> pv(np);
@@ -875,37 +898,46 @@ int build_gather_plan(const MeshView &m, const HostPlan &base, int max_tiles, Ho
     const int nb = m.nb, nv = m.nv;
     // (an early way out: boxes of up to 38^3 hexes or 6 x 16^3 tets fit 512 tiles)
     if (!m.coords || (int64_t)base.cells.size() > (int64_t)max_tiles * (nb == 8 ? 128 : 64)) return 0;
-    // the key's nodes, their positions (mean of the incident cells' centroids) and incident cells
-    std::vector<int32_t> cells(base.cells), nodes;
+    // the key's cells and nodes, ascending; by their places there: each cell's nodes, each node's position (mean
+    // of the incident cells' centroids) and incident cells
+    std::vector<int32_t> cells(base.cells), nodes, rank(m.num_nodes, -1);
     std::sort(cells.begin(), cells.end());
-    std::vector<double> x(3 * (size_t)m.num_nodes, 0.0);
-    std::vector<int32_t> ptr(m.num_nodes + 1, 0), inc;
-    for (int32_t c : cells) {
-        const int32_t *cl = m.closure + (size_t)c * nb, *cn = m.cone + (size_t)c * nv;
+    const int ncell = (int)cells.size();
+    for (int32_t c : cells)
+        for (int b = 0; b < nb; ++b) rank[m.closure[(size_t)c * nb + b]] = 0;
+    for (int i = 0; i < m.num_nodes; ++i)
+        if (rank[i] == 0) {
+            rank[i] = (int32_t)nodes.size();
+            nodes.push_back(i);
+        }
+    const int nnode = (int)nodes.size();
+    std::vector<int32_t> cl((size_t)ncell * nb), ptr(nnode + 1, 0), inc;
+    std::vector<double> x(3 * (size_t)nnode, 0.0);
+    for (int i = 0; i < ncell; ++i) {
+        const int32_t *cn = m.cone + (size_t)cells[i] * nv;
         double mid[3] = {0.0, 0.0, 0.0};
         for (int v = 0; v < nv; ++v)
             for (int d = 0; d < 3; ++d) mid[d] += m.coords[3 * (size_t)cn[v] + d] / nv;
         for (int b = 0; b < nb; ++b) {
-            for (int d = 0; d < 3; ++d) x[3 * (size_t)cl[b] + d] += mid[d];
-            ++ptr[cl[b] + 1];
+            const int32_t g = cl[(size_t)i * nb + b] = rank[m.closure[(size_t)cells[i] * nb + b]];
+            for (int d = 0; d < 3; ++d) x[3 * (size_t)g + d] += mid[d];
+            ++ptr[g + 1];
         }
     }
-    for (int i = 0; i < m.num_nodes; ++i)
-        for (int d = 0; d < 3; ++d)
-            if (ptr[i + 1] > 0) x[3 * (size_t)i + d] /= ptr[i + 1];
-    for (int i = 0; i < m.num_nodes; ++i) {
-        if (ptr[i + 1] > 0) nodes.push_back(i);
+    for (int i = 0; i < nnode; ++i) {
+        for (int d = 0; d < 3; ++d) x[3 * (size_t)i + d] /= ptr[i + 1];
         ptr[i + 1] += ptr[i];
     }
-    inc.resize(ptr[m.num_nodes]);
+    inc.resize(ptr[nnode]);
     {
         std::vector<int32_t> fill(ptr.begin(), ptr.end() - 1);
-        for (int32_t c : cells)
-            for (int b = 0; b < nb; ++b) inc[fill[m.closure[(size_t)c * nb + b]]++] = c;
+        for (int i = 0; i < ncell; ++i)
+            for (int b = 0; b < nb; ++b) inc[fill[cl[(size_t)i * nb + b]]++] = i;
     }
     // as many tiles as allowed (the work of a tile is what a call waits for), not below 32 nodes each
-    const int parts = std::max(1, std::min(max_tiles, (int)nodes.size() / 32));
-    std::vector<int32_t> order(nodes), sizes;
+    const int parts = std::max(1, std::min(max_tiles, nnode / 32));
+    std::vector<int32_t> order(nnode), sizes;
+    std::iota(order.begin(), order.end(), 0);
     bisect_equal(x, order.data(), (int)order.size(), parts, sizes);
     const TileLimits lim = tile_limits(nb == 8 ? 1 : 2);
     gp->tile_cell_ptr.assign(1, 0);
@@ -919,50 +951,73 @@ int build_gather_plan(const MeshView &m, const HostPlan &base, int max_tiles, Ho
         std::vector<uint16_t> lcl, lcn;  // [cells][nb], [cells][nv]
     };
     std::vector<Tile> tiles(sizes.size());
-    parallel_for((int)tiles.size(), [&](int t) {
-        Tile &T = tiles[t];
-        std::vector<int32_t> tc, &tn = T.nodes, &tv = T.verts;
-        tn.assign(order.begin() + first[t], order.begin() + first[t + 1]);
-        std::sort(tn.begin(), tn.end());
-        for (int32_t i : tn) tc.insert(tc.end(), inc.begin() + ptr[i], inc.begin() + ptr[i + 1]);
-        distinct(tc);
-        // the other nodes and the vertices of the tile's cells, and every entry's place in the lists
-        std::vector<int32_t> other, own(tn);
-        for (int32_t c : tc) other.insert(other.end(), m.closure + (size_t)c * nb, m.closure + (size_t)(c + 1) * nb);
-        distinct(other);
-        for (int32_t g : other)
-            if (!std::binary_search(own.begin(), own.end(), g)) tn.push_back(g);
-        const auto node_at = [&](int32_t g) {
-            const auto i = std::lower_bound(own.begin(), own.end(), g);
-            if (i != own.end() && *i == g) return (size_t)(i - own.begin());
-            return (size_t)(std::lower_bound(tn.begin() + own.size(), tn.end(), g) - tn.begin());
-        };
-        if (!m.cone_is_closure) {
-            for (int32_t c : tc) tv.insert(tv.end(), m.cone + (size_t)c * nv, m.cone + (size_t)(c + 1) * nv);
-            distinct(tv);
-        }
-        std::vector<uint16_t> at;
-        for (int32_t c : tc)
-            for (int b = 0; b < nb; ++b) at.push_back((uint16_t)node_at(m.closure[(size_t)c * nb + b]));
-        // tets sorted by colour, so that a wave's atomic targets are mostly distinct (hexes keep mesh order:
-        // neighbouring lanes, spread banks)
+    parallel_ranges((int)tiles.size(), [&](int lo, int hi) {
+        // the tile that last saw each node and cell, and the node's place in it
+        std::vector<int32_t> seen(nnode, -1), place(nnode), cell_seen(ncell, -1), tc, own;
+        std::vector<uint64_t> used;
         std::vector<std::pair<int, int>> by;
-        std::vector<uint64_t> used(tn.size(), 0);
-        for (size_t i = 0; i < tc.size(); ++i) {
-            uint64_t mask = 0;
-            for (int b = 0; b < nb; ++b) mask |= used[at[i * nb + b]];
-            int k = 0;
-            while (k < 63 && ((mask >> k) & 1)) ++k;
-            for (int b = 0; b < nb; ++b) used[at[i * nb + b]] |= (uint64_t)1 << k;
-            by.emplace_back(nb == 8 ? 0 : k, (int)i);
-        }
-        std::sort(by.begin(), by.end());
-        for (const auto &e : by) {
-            const int32_t c = tc[e.second];
-            T.cells.push_back(c);
-            for (int b = 0; b < nb; ++b) T.lcl.push_back(at[(size_t)e.second * nb + b]);
-            for (int b = 0; b < nv && !m.cone_is_closure; ++b)
-                T.lcn.push_back((uint16_t)(std::lower_bound(tv.begin(), tv.end(), m.cone[(size_t)c * nv + b]) - tv.begin()));
+        for (int t = lo; t < hi; ++t) {
+            Tile &T = tiles[t];
+            std::vector<int32_t> &tn = T.nodes, &tv = T.verts;
+            // the tile's nodes, its cells, and the other nodes and the vertices of those
+            tn.assign(order.begin() + first[t], order.begin() + first[t + 1]);
+            std::sort(tn.begin(), tn.end());
+            own = tn;
+            tc.clear();
+            for (int32_t i : own) {
+                seen[i] = t;
+                for (int k = ptr[i]; k < ptr[i + 1]; ++k)
+                    if (cell_seen[inc[k]] != t) {
+                        cell_seen[inc[k]] = t;
+                        tc.push_back(inc[k]);
+                    }
+            }
+            if ((int)tc.size() > kGatherCells) {  // too large (found out below)
+                T.cells = tc;
+                continue;
+            }
+            std::sort(tc.begin(), tc.end());
+            for (int32_t c : tc)
+                for (int b = 0; b < nb; ++b) {
+                    const int32_t g = cl[(size_t)c * nb + b];
+                    if (seen[g] != t) {
+                        seen[g] = t;
+                        tn.push_back(g);
+                    }
+                }
+            std::sort(tn.begin() + own.size(), tn.end());
+            for (size_t k = 0; k < tn.size(); ++k) place[tn[k]] = (int32_t)k;
+            if (!m.cone_is_closure) {
+                for (int32_t c : tc)
+                    tv.insert(tv.end(), m.cone + (size_t)cells[c] * nv, m.cone + (size_t)(cells[c] + 1) * nv);
+                distinct(tv);
+            }
+            // tets sorted by colour, so that a wave's atomic targets are mostly distinct (hexes keep mesh order:
+            // neighbouring lanes, spread banks)
+            by.clear();
+            used.assign(tn.size(), 0);
+            for (size_t i = 0; i < tc.size(); ++i) {
+                int k = 0;
+                if (nb != 8) {
+                    uint64_t mask = 0;
+                    for (int b = 0; b < nb; ++b) mask |= used[place[cl[(size_t)tc[i] * nb + b]]];
+                    while (k < 63 && ((mask >> k) & 1)) ++k;
+                    for (int b = 0; b < nb; ++b) used[place[cl[(size_t)tc[i] * nb + b]]] |= (uint64_t)1 << k;
+                }
+                by.emplace_back(k, (int)i);
+            }
+            std::sort(by.begin(), by.end());
+            T.cells.reserve(tc.size());
+            T.lcl.reserve(tc.size() * nb);
+            T.lcn.reserve(m.cone_is_closure ? 0 : tc.size() * nv);
+            for (const auto &e : by) {
+                const int32_t c = tc[e.second];
+                T.cells.push_back(cells[c]);
+                for (int b = 0; b < nb; ++b) T.lcl.push_back((uint16_t)place[cl[(size_t)c * nb + b]]);
+                for (int b = 0; b < nv && !m.cone_is_closure; ++b)
+                    T.lcn.push_back((uint16_t)place_of(tv, m.cone[(size_t)cells[c] * nv + b]));
+            }
+            for (int32_t &g : tn) g = nodes[g];
         }
     });
     for (size_t t = 0; t < tiles.size(); ++t) {
