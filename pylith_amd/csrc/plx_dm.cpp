@@ -6,6 +6,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <new>
 #include <numeric>
 
 #include "plx_element.hpp"
@@ -33,19 +34,33 @@ static int upload(plx_dm dm, T **dst, const T *src, size_t n) {
     return 0;
 }
 
+static void free_pairs(KeyPlan *k) {
+    PairDev &P = k->pairs;
+    void *ptrs[] = {P.d_heads, P.d_nodes, P.d_verts, P.d_shared_node, P.d_shared_ptr, P.d_shared_slot, P.d_records, P.d_mat64, P.d_mat32};
+    for (void *p : ptrs)
+        if (p) (void)hipFree(p);
+    P = PairDev();
+}
+
+static void free_gather(KeyPlan *k) {
+    GatherDev &G = k->gather;
+    void *ptrs[] = {G.d_heads, G.d_nodes, G.d_verts, G.d_records, G.d_mat64, G.d_mat32};
+    for (void *p : ptrs)
+        if (p) (void)hipFree(p);
+    G = GatherDev();
+}
+
 static void free_plan_arrays(KeyPlan *k) {
     pointfn_release(nullptr, k);
+    free_pairs(k);
+    free_gather(k);
     void *ptrs[] = {k->d_cells,       k->d_tile_cell_ptr, k->d_tile_node_ptr, k->d_tile_nown,
                     k->d_tile_nodes,  k->d_tile_vert_ptr, k->d_tile_verts,    k->d_tile_halo_off,
                     k->d_lclosure,    k->d_lcone,         k->d_shared_node,   k->d_color,
                     k->d_heads,         k->d_records,       k->d_shared_ptr,    k->d_heads_affine,  k->d_heads_general,
                     k->d_shared_slot, k->d_halo,          k->d_mat64,         k->d_mat32,
                     k->d_state,       k->d_gm_mat,        k->d_prestress,     k->d_load_node,
-                    k->d_load64,      k->d_load32,        k->pairs.d_heads,
-                    k->pairs.d_nodes, k->pairs.d_verts,   k->pairs.d_shared_node, k->pairs.d_shared_ptr,
-                    k->pairs.d_shared_slot, k->pairs.d_records, k->pairs.d_mat64, k->pairs.d_mat32,
-                    k->gather.d_heads, k->gather.d_nodes, k->gather.d_verts,  k->gather.d_records,
-                    k->gather.d_mat64, k->gather.d_mat32};
+                    k->d_load64,      k->d_load32};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
     KeyPlan fresh;
@@ -95,6 +110,10 @@ static std::vector<TileHead> tile_heads(const HostPlan &hp) {
     return heads;
 }
 
+static int upload_heads(plx_dm dm, int32_t **d, const std::vector<TileHead> &h) {
+    return upload(dm, reinterpret_cast<TileHead **>(d), h.data(), h.size());
+}
+
 // Keys with fewer cells keep the tile kernel alone: two cells one after another per thread leave too few
 // waves there.  FP64 / FP32 apply, pairs against tiles: 48,000 cells 10.2 / 9.4 against 9.5 / 9.0 us, 83,000
 // 11.6 / 9.9 against 12.1 / 10.7 us, 196,000 17.2 / 14.5 against 20.9 / 17.5 us.
@@ -105,11 +124,21 @@ constexpr int64_t kPairMinCells = 65536;
 // against 17.8 us, three of six of 42^3 x 6 204 26.4 against 23.9 us, one of six 105 19.7 against 16.6 us.
 constexpr int64_t kPairMinFill = 256;
 
+static MeshView mesh_view(plx_dm dm) {
+    return {dm->nb, dm->nv, dm->num_cells, dm->num_nodes, dm->num_vertices,
+            dm->closure.data(), dm->cone.data(), dm->labels.data(),
+            dm->cell_type == PLX_HEX_Q1, dm->coords.data()};
+}
+
+static int num_cus() {
+    int n = 0;
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, 0) != hipSuccess || n <= 0) n = 256;
+    return n;
+}
+
 // Build the key's tile plan on the host (plx_plan.cpp) and upload it.
 static int build_plan(plx_dm dm, KeyPlan *kp) {
-    MeshView mv{dm->nb, dm->nv, dm->num_cells, dm->num_nodes, dm->num_vertices,
-                dm->closure.data(), dm->cone.data(), dm->labels.data(),
-                dm->cell_type == PLX_HEX_Q1, dm->coords.data()};
+    const MeshView mv = mesh_view(dm);
     HostPlan hp;
     std::string msg;
     // P2 tiles keep colour order (the tets of a cube share nodes: colour order keeps a wave's
@@ -120,12 +149,11 @@ static int build_plan(plx_dm dm, KeyPlan *kp) {
     // tile (fewer halo nodes).  Measured on Q1 32^3: 10.5 us per apply at 256-cell tiles against
     // 13.1 us at 512; at 48^3 smaller tiles no longer pay.
     TileLimits lim = tile_limits(dm->cell_type);
-    int ncu = 0;
     {
+        const int ncu = num_cus();
         int64_t nkey = 0;
         for (int c = 0; c < dm->num_cells; ++c)
             if ((dm->labels.empty() ? 0 : dm->labels[c]) == kp->label_value) ++nkey;
-        if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, 0) != hipSuccess || ncu <= 0) ncu = 256;
         int cells = lim.cells;
         while (cells > 64 && nkey < (int64_t)cells * (ncu / 2)) cells >>= 1;
         lim.cells = cells;
@@ -157,39 +185,11 @@ static int build_plan(plx_dm dm, KeyPlan *kp) {
         if ((err = upload(dm, &kp->d_records, rec.data(), rec.size()))) return err;
     }
     const std::vector<TileHead> heads = tile_heads(hp);
-    auto upload_heads = [&](int32_t **d, const std::vector<TileHead> &h) {
-        return upload(dm, reinterpret_cast<TileHead **>(d), h.data(), h.size());
-    };
-    if ((err = upload_heads(&kp->d_heads, heads))) return err;
+    if ((err = upload_heads(dm, &kp->d_heads, heads))) return err;
     if ((err = upload(dm, &kp->d_shared_node, hp.shared_node.data(), hp.shared_node.size()))) return err;
     if ((err = upload(dm, &kp->d_shared_ptr, hp.shared_ptr.data(), hp.shared_ptr.size()))) return err;
     if ((err = upload(dm, &kp->d_shared_slot, hp.shared_slot.data(), hp.shared_slot.size()))) return err;
     if (hp.halo_slots > 0) PLX_HIP(dm, hipMalloc(&kp->d_halo, (size_t)hp.halo_slots * 3 * sizeof(double)));
-    // (a key without a pair plan keeps the tile plan alone)
-    PairPlan pp;
-    if (dm->cell_type == PLX_TET_P2 && (int64_t)hp.cells.size() >= kPairMinCells && !build_pair_plan(mv, hp, &pp, &msg) &&
-        (int64_t)hp.cells.size() >= kPairMinFill * pp.num_tiles) {
-        PairDev &P = kp->pairs;
-        P.num_tiles = pp.num_tiles;
-        P.num_pairs = pp.num_pairs;
-        P.num_shared = (int)pp.shared_node.size();
-        P.halo_slots = pp.halo_slots;
-        std::vector<TileHead> ph(pp.num_tiles);
-        for (int t = 0; t < pp.num_tiles; ++t)
-            ph[t] = {pp.tile_pair_ptr[t], pp.tile_pair_ptr[t + 1] - pp.tile_pair_ptr[t],
-                     pp.tile_node_ptr[t], pp.tile_node_ptr[t + 1] - pp.tile_node_ptr[t],
-                     pp.tile_vert_ptr[t], pp.tile_vert_ptr[t + 1] - pp.tile_vert_ptr[t],
-                     pp.tile_nown[t], pp.tile_halo_off[t]};
-        if ((err = upload_heads(&P.d_heads, ph)) ||
-            (err = upload(dm, &P.d_nodes, pp.tile_nodes.data(), pp.tile_nodes.size())) ||
-            (err = upload(dm, &P.d_verts, pp.tile_verts.data(), pp.tile_verts.size())) ||
-            (err = upload(dm, &P.d_shared_node, pp.shared_node.data(), pp.shared_node.size())) ||
-            (err = upload(dm, &P.d_shared_ptr, pp.shared_ptr.data(), pp.shared_ptr.size())) ||
-            (err = upload(dm, &P.d_shared_slot, pp.shared_slot.data(), pp.shared_slot.size())) ||
-            (err = upload(dm, &P.d_records, pp.records.data(), pp.records.size())))
-            return err;
-        P.cells = std::move(pp.cells);
-    }
     // Q1 tiles whose cells are all parallelepipeds take the modal kernel (geometry is static).
     if (dm->cell_type == PLX_HEX_Q1) {
         std::vector<TileHead> aff, gen;
@@ -207,50 +207,104 @@ static int build_plan(plx_dm dm, KeyPlan *kp) {
         }
         kp->num_tiles_affine = (int)aff.size();
         kp->num_tiles_general = (int)gen.size();
-        if ((err = upload_heads(&kp->d_heads_affine, aff))) return err;
-        if ((err = upload_heads(&kp->d_heads_general, gen))) return err;
+        if ((err = upload_heads(dm, &kp->d_heads_affine, aff))) return err;
+        if ((err = upload_heads(dm, &kp->d_heads_general, gen))) return err;
+    }
+    kp->tile_cell_ptr = std::move(hp.tile_cell_ptr);
+    return 0;
+}
+
+static int upload_pairs(plx_dm dm, const PairPlan &pp, PairDev &P) {
+    P.num_tiles = pp.num_tiles;
+    P.num_pairs = pp.num_pairs;
+    P.num_shared = (int)pp.shared_node.size();
+    P.halo_slots = pp.halo_slots;
+    std::vector<TileHead> ph(pp.num_tiles);
+    for (int t = 0; t < pp.num_tiles; ++t)
+        ph[t] = {pp.tile_pair_ptr[t], pp.tile_pair_ptr[t + 1] - pp.tile_pair_ptr[t],
+                 pp.tile_node_ptr[t], pp.tile_node_ptr[t + 1] - pp.tile_node_ptr[t],
+                 pp.tile_vert_ptr[t], pp.tile_vert_ptr[t + 1] - pp.tile_vert_ptr[t],
+                 pp.tile_nown[t], pp.tile_halo_off[t]};
+    int err = 0;
+    (void)((err = upload_heads(dm, &P.d_heads, ph)) ||
+           (err = upload(dm, &P.d_nodes, pp.tile_nodes.data(), pp.tile_nodes.size())) ||
+           (err = upload(dm, &P.d_verts, pp.tile_verts.data(), pp.tile_verts.size())) ||
+           (err = upload(dm, &P.d_shared_node, pp.shared_node.data(), pp.shared_node.size())) ||
+           (err = upload(dm, &P.d_shared_ptr, pp.shared_ptr.data(), pp.shared_ptr.size())) ||
+           (err = upload(dm, &P.d_shared_slot, pp.shared_slot.data(), pp.shared_slot.size())) ||
+           (err = upload(dm, &P.d_records, pp.records.data(), pp.records.size())));
+    return err;
+}
+
+static int upload_gather(plx_dm dm, const HostPlan &gp, GatherDev &G) {
+    G.num_tiles = gp.num_tiles;
+    for (int32_t k : gp.tile_nown) G.num_owned += k;
+    const std::vector<uint16_t> rec = cell_records(dm, gp);
+    int err = 0;
+    (void)((err = upload_heads(dm, &G.d_heads, tile_heads(gp))) ||
+           (err = upload(dm, &G.d_nodes, gp.tile_nodes.data(), gp.tile_nodes.size())) ||
+           (err = upload(dm, &G.d_verts, gp.tile_verts.data(), gp.tile_verts.size())) ||
+           (err = upload(dm, &G.d_records, rec.data(), rec.size())));
+    return err;
+}
+
+// The pair and gather plans of a key, made beside its tile plan when it first has moduli: not for plug-in kernels,
+// nor for viscoelastic keys without a Jacobian (their residual stays on the tile plan).  (The kernel options, which
+// may rule the plans out too, change at any time, under a stream capture as well.)  Both plans are optional:
+// what cannot be made leaves the tile plan in charge.
+static void make_second_plans(plx_dm dm, KeyPlan *kp) {
+    if (kp->second_plans || (kp->genmax && !kp->jf3)) return;
+    kp->second_plans = true;
+    const MeshView mv = mesh_view(dm);
+    HostPlan base;
+    base.cells = kp->cells;
+    base.tile_cell_ptr = std::move(kp->tile_cell_ptr);
+    kp->tile_cell_ptr.clear();
+    base.num_tiles = kp->num_tiles;
+    base.halo_slots = kp->halo_slots;
+    std::vector<int32_t> at(dm->num_cells, -1);  // mesh cell -> key cell
+    for (size_t i = 0; i < kp->cells.size(); ++i) at[kp->cells[i]] = (int32_t)i;
+    if (dm->cell_type == PLX_TET_P2 && (int64_t)kp->cells.size() >= kPairMinCells) {
+        PairPlan pp;
+        std::string msg;
+        if (!build_pair_plan(mv, base, &pp, &msg) && (int64_t)kp->cells.size() >= kPairMinFill * pp.num_tiles) {
+            kp->pairs.cells = std::move(pp.cells);
+            for (int32_t &c : kp->pairs.cells) c = c >= 0 ? at[c] : -1;
+            if (upload_pairs(dm, pp, kp->pairs)) free_pairs(kp);
+        }
     }
     // Small keys whose elements are cheap (P2, affine hexes): a gather plan of two tiles per CU, all resident at
     // once.  It evaluates the cells on tile boundaries several times but saves the second launch and the
     // halo's way through memory.  FP64 / FP32 apply, gather against tiles + reduce_halo: 12^3 hexes 4.5 / 4.8
     // against 8.0 / 8.3 us, 28^3 5.9 / 5.7 against 8.3 / 8.5, 38^3 (about the largest that fits) 7.3 / 6.6
     // against 9.1 / 8.1; 6 x 8^3 tets 4.7 / 4.7 against 7.4 / 7.2, 6 x 16^3 7.0 / 7.0 against 8.3 / 7.8.  Not for
-    // the quadrature-point element of other hexes: 28^3 16.9 against 14.1 us.
+    // the quadrature-point element of other hexes: 28^3 16.9 against 14.1 us.  Cells of general tets lie in three
+    // tiles and more, and still: Delaunay meshes of 2,771 / 12,129 / 29,863 cells 4.7 / 6.5 / 7.7 against 8.3 / 9.2 / 9.9 us,
+    // and with nothing in the caches 8.4 / 10.5 / 12.2 against 12.7 / 13.6 / 14.6 us (32^3 hexes 10.7 against 13.2).
     if (dm->cell_type != PLX_HEX_Q1 || kp->num_tiles_general == 0) {
         HostPlan gp;
         bool fits = false;
-        if (build_gather_plan(mv, hp, 2 * ncu, &gp, &fits)) return set_error(dm, 1, "gather plan");
-        if (fits) {
-            GatherDev &G = kp->gather;
-            G.num_tiles = gp.num_tiles;
-            for (int32_t k : gp.tile_nown) G.num_owned += k;
-            const std::vector<uint16_t> rec = cell_records(dm, gp);
-            if ((err = upload_heads(&G.d_heads, tile_heads(gp))) ||
-                (err = upload(dm, &G.d_nodes, gp.tile_nodes.data(), gp.tile_nodes.size())) ||
-                (err = upload(dm, &G.d_verts, gp.tile_verts.data(), gp.tile_verts.size())) ||
-                (err = upload(dm, &G.d_records, rec.data(), rec.size())))
-                return err;
-            G.cells = std::move(gp.cells);
+        if (!build_gather_plan(mv, base, 2 * num_cus(), &gp, &fits) && fits) {
+            kp->gather.cells = gp.cells;
+            for (int32_t &c : kp->gather.cells) c = at[c];
+            if (upload_gather(dm, gp, kp->gather)) free_gather(kp);
         }
     }
-    return 0;
 }
 
-int repack_plans(plx_dm dm, KeyPlan *kp, const std::vector<double> &m64, const std::vector<float> &m32) {
-    const int n = (int)kp->cells.size();
+// The key's moduli (lambda, mu: [2][key cells], tile order) in the order of its pair and gather plans.
+static int pack_second_plans(plx_dm dm, KeyPlan *kp, const std::vector<double> &m64, const std::vector<float> &m32) {
+    const size_t n = kp->cells.size();
     int err = 0;
-    if (kp->pairs.num_tiles == 0 && kp->gather.num_tiles == 0) return 0;
-    std::vector<int32_t> at(dm->num_cells, -1);  // mesh cell -> key cell
-    for (int i = 0; i < n; ++i) at[kp->cells[i]] = i;
     if (kp->gather.num_tiles > 0) {
         GatherDev &G = kp->gather;
         const size_t ng = G.cells.size();
         std::vector<double> g64(2 * ng);
         std::vector<float> g32(2 * ng);
-        for (size_t i = 0; i < ng; ++i)
-            for (size_t k = 0; k < 2; ++k) {
-                g64[k * ng + i] = m64[k * n + at[G.cells[i]]];
-                g32[k * ng + i] = m32[k * n + at[G.cells[i]]];
+        for (size_t k = 0; k < 2; ++k)
+            for (size_t i = 0; i < ng; ++i) {
+                g64[k * ng + i] = m64[k * n + G.cells[i]];
+                g32[k * ng + i] = m32[k * n + G.cells[i]];
             }
         if (G.d_mat64) (void)hipFree(G.d_mat64);
         if (G.d_mat32) (void)hipFree(G.d_mat32);
@@ -266,8 +320,8 @@ int repack_plans(plx_dm dm, KeyPlan *kp, const std::vector<double> &m64, const s
         for (size_t i = 0; i < P.cells.size(); ++i)
             if (P.cells[i] >= 0)
                 for (int k = 0; k < 2; ++k) {
-                    p64[2 * i + k] = m64[(size_t)k * n + at[P.cells[i]]];
-                    p32[2 * i + k] = m32[(size_t)k * n + at[P.cells[i]]];
+                    p64[2 * i + k] = m64[k * n + P.cells[i]];
+                    p32[2 * i + k] = m32[k * n + P.cells[i]];
                 }
         if (P.d_mat64) (void)hipFree(P.d_mat64);
         if (P.d_mat32) (void)hipFree(P.d_mat32);
@@ -276,6 +330,30 @@ int repack_plans(plx_dm dm, KeyPlan *kp, const std::vector<double> &m64, const s
         if ((err = upload(dm, &P.d_mat64, p64.data(), p64.size()))) return err;
         if ((err = upload(dm, &P.d_mat32, p32.data(), p32.size()))) return err;
     }
+    return 0;
+}
+
+void update_second_plans(plx_dm dm, KeyPlan *kp, const std::vector<double> &m64, const std::vector<float> &m32) {
+    try {
+        make_second_plans(dm, kp);
+        if (!pack_second_plans(dm, kp, m64, m32)) return;
+    } catch (const std::bad_alloc &) {
+    }
+    // out of memory: the tile plan goes on without them
+    free_pairs(kp);
+    free_gather(kp);
+    (void)hipGetLastError();
+}
+
+// After a change of kernels.
+static int late_second_plans(plx_dm dm, KeyPlan *kp) {
+    if (kp->second_plans || !kp->has_aux || !kp->d_mat64) return 0;
+    const size_t n = kp->cells.size();
+    std::vector<double> m64(2 * n);
+    std::vector<float> m32(2 * n);
+    PLX_HIP(dm, hipMemcpy(m64.data(), kp->d_mat64, m64.size() * sizeof(double), hipMemcpyDeviceToHost));
+    PLX_HIP(dm, hipMemcpy(m32.data(), kp->d_mat32, m32.size() * sizeof(float), hipMemcpyDeviceToHost));
+    update_second_plans(dm, kp, m64, m32);
     return 0;
 }
 
@@ -470,7 +548,7 @@ static int repack_aux(plx_dm dm, KeyPlan *kp) {
     int err = 0;
     if ((err = upload(dm, &kp->d_mat64, m64.data(), m64.size()))) return err;
     if ((err = upload(dm, &kp->d_mat32, m32.data(), m32.size()))) return err;
-    if ((err = repack_plans(dm, kp, m64, m32))) return err;
+    update_second_plans(dm, kp, m64, m32);
     kp->has_aux = true;
     return build_load(dm, kp);
 }
@@ -695,7 +773,7 @@ int plx_dm_add_jacobian(plx_dm dm, int label_value, int part, int jf0, int jf1, 
     kp->jf1 = jf1;
     kp->jf2 = jf2;
     kp->jf3 = jf3;
-    return 0;
+    return late_second_plans(dm, kp);
 }
 
 int plx_dm_create_ordered(plx_dm *out, int cell_type, int num_cells, int num_vertices, int num_nodes,

@@ -286,8 +286,8 @@ int genmax_refresh(plx_dm dm, KeyPlan *kp) {
     PLX_HIP(dm, hipMemcpy(kp->d_mat64, m64.data(), m64.size() * sizeof(double), hipMemcpyHostToDevice));
     PLX_HIP(dm, hipMalloc(&kp->d_mat32, m32.size() * sizeof(float)));
     PLX_HIP(dm, hipMemcpy(kp->d_mat32, m32.data(), m32.size() * sizeof(float), hipMemcpyHostToDevice));
-    int err = repack_plans(dm, kp, m64, m32);
-    if (err || (err = launch_genmax_prestress(dm, kp))) return err;
+    update_second_plans(dm, kp, m64, m32);
+    if (const int err = launch_genmax_prestress(dm, kp)) return err;
     kp->has_aux = true;
     return 0;
 }

@@ -53,7 +53,7 @@ struct TilePlanDev {
 struct PairDev {
     int num_tiles = 0, num_pairs = 0, num_shared = 0;
     int64_t halo_slots = 0;
-    std::vector<int32_t> cells;      // [num_pairs][2] mesh cells (-1: none)
+    std::vector<int32_t> cells;      // [num_pairs][2] places in the key's cells (-1: none)
     int32_t *d_heads = nullptr;      // TileHead of each tile (pairs in place of cells)
     int32_t *d_nodes = nullptr, *d_verts = nullptr;
     int32_t *d_shared_node = nullptr, *d_shared_ptr = nullptr, *d_shared_slot = nullptr;
@@ -65,7 +65,7 @@ struct PairDev {
 // Device arrays of a small key's gather plan (build_gather_plan; num_tiles = 0: none).
 struct GatherDev {
     int num_tiles = 0, num_owned = 0;  // num_owned: the key's nodes
-    std::vector<int32_t> cells;      // tile order, cells on tile boundaries repeated
+    std::vector<int32_t> cells;      // places in the key's cells, those on tile boundaries repeated
     int32_t *d_heads = nullptr, *d_nodes = nullptr, *d_verts = nullptr;
     uint16_t *d_records = nullptr;
     double *d_mat64 = nullptr;       // [2][cells]
@@ -96,6 +96,8 @@ struct KeyPlan {
     bool sorted_by_color = true;
     int32_t *d_heads_affine = nullptr, *d_heads_general = nullptr;  // Q1: those of affine cells / the others
     int num_tiles_affine = 0, num_tiles_general = 0;
+    std::vector<int32_t> tile_cell_ptr;  // host copy, until the pair and gather plans are made
+    bool second_plans = false;           // whether that has been tried
     PairDev pairs;                   // P2: the factored path with LDS atomics
     GatherDev gather;                // small keys: the default algorithm with LDS atomics
     int32_t *d_shared_node = nullptr, *d_shared_ptr = nullptr, *d_shared_slot = nullptr;
@@ -292,8 +294,9 @@ int launch_genmax_prestress(plx_dm dm, KeyPlan *kp);
 int launch_genmax_update(plx_dm dm, KeyPlan *kp, const double *u);
 int genmax_capture(plx_dm dm, KeyPlan *kp);
 int genmax_refresh(plx_dm dm, KeyPlan *kp);
-// The moduli (lambda, mu: [2][key cells], tile order) in the order of the key's pair and gather plans.
-int repack_plans(plx_dm dm, KeyPlan *kp, const std::vector<double> &m64, const std::vector<float> &m32);
+// New moduli (lambda, mu: [2][key cells], tile order) for the key's pair and gather plans, which are made
+// now if they are wanted and not there yet (optional: no error).
+void update_second_plans(plx_dm dm, KeyPlan *kp, const std::vector<double> &m64, const std::vector<float> &m32);
 int validate_geometry(plx_dm dm, int *num_bad);
 
 // Cohesive cells and split-node maps (plx_fault.hip).

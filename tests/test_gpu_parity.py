@@ -213,6 +213,53 @@ def test_p2_pair_kernel_not_for_scattered_cells(oracle, kind, pairs):
     assert (second_plans(dm, 1)[0] > 0) == pairs
 
 
+@pytest.mark.parametrize("cell", ["hex", "tet"])
+def test_second_plans_only_for_keys_that_use_them(oracle, cell):
+    """The plans beside the tile plan come with the moduli (plug-in keys have none) and follow them."""
+    from pylith_amd import _lib as L
+    from pylith_amd.dm import DM
+    m = mg.hex_box(9, (0, 0, 0), (900.0,) * 3) if cell == "hex" else mg.tet_p2_box((27, 23, 21), (0, 0, 0), (2700.0, 2300.0, 2100.0))
+    u = mg.random_field(m.num_nodes, 9)
+    dm = DM(m)
+    dm.add_residual(0, 0, 0, F1)
+    assert second_plans(dm) == (0, 0)
+    for seed in (6, 7):  # new moduli reach them
+        aux, sizes = mg.elastic_aux(m.num_cells, seed=seed, vs_sigma=0.2, vp_vs=1.8)
+        dm.set_auxiliary(0, 0, aux, sizes)
+        assert (second_plans(dm)[0] > 0, second_plans(dm)[1] > 0) == (cell == "tet", cell == "hex")
+        x = dev(u)
+        r = torch.zeros_like(x)
+        dm.compute_residual(0, 0, x, r, mode=1)
+        torch.cuda.synchronize()
+        assert relerr(r.cpu().numpy(), oracle.Problem(m, aux, sizes).residual(u, F1)) <= TOL64
+    dm.close()
+    if cell == "hex":  # a viscoelastic key gets its gather plan (for the action) with the Jacobian, before or after
+        aux, sizes = mg.genmax_aux(m.num_cells, 8, seed=3, log_eta_range=(1e17, 1e19))
+        for late in (False, True):
+            dm = DM(m)
+            dm.add_residual(0, 0, 0, L.F1V_GENMAXWELL_3D)
+            if not late:
+                dm.add_jacobian(0, 0, 0, 0, 0, L.JF3VU_GENMAXWELL_3D)
+            dm.set_auxiliary(0, 0, aux, sizes, per_qp=True)
+            actions = []
+            for dt in (1e7, 3e8):
+                dm.set_constants(0, 0, [dt])
+                assert (second_plans(dm)[1] > 0) == (not late or dt == 3e8)
+                if late:
+                    dm.add_jacobian(0, 0, 0, 0, 0, L.JF3VU_GENMAXWELL_3D)
+                assert second_plans(dm)[1] > 0
+                for acc in (L.ACCUMULATE_AUTO, L.ACCUMULATE_COLORED):
+                    dm.set_kernel_options(L.ALGO_AUTO, acc, 0)
+                    x = dev(u)
+                    r = torch.zeros_like(x)
+                    dm.compute_jacobian_action(0, 0, x, r, mode=1)
+                    torch.cuda.synchronize()
+                    actions.append(r.cpu().numpy())
+            assert relerr(actions[0], actions[1]) <= TOL64 and relerr(actions[2], actions[3]) <= TOL64
+            assert relerr(actions[0], actions[2]) > 1e-6
+            dm.close()
+
+
 # either side of the line where a key takes the gather plan (38^3 hexes and 6 x 16^3 tets are about the
 # largest), non-affine hexes, and a mesh of affine and other hex tiles
 @pytest.mark.parametrize("kind", ["hex38", "hex41", "hex_warped", "hex_mixed", "tet16", "tet18"])
