@@ -565,7 +565,8 @@ __global__ void __launch_bounds__(kPairThreads, 2) apply_pairs(PairArgs A) {
         __builtin_amdgcn_s_setprio(0);
         if (tid < cur.np) {
             int n[14];
-            Real AA[9], AB[9], SA[4][6], SB[4][6], qa, qb;
+            Real AA[9], AB[9], SA[4][6], SB[4][6];
+            double qa, qb;
             {
                 const unsigned w[6] = {cur.rec[0].x, cur.rec[0].y, cur.rec[1].x, cur.rec[1].y, cur.rec[2].x, cur.rec[2].y};
 #pragma unroll
@@ -579,15 +580,10 @@ __global__ void __launch_bounds__(kPairThreads, 2) apply_pairs(PairArgs A) {
 #pragma unroll
                     for (int d = 0; d < 3; ++d) X[v][d] = sX[3 * lv + d];
                 }
-                double Ad[9];
-                qa = (Real)(-A.scale / (30.0 * p2_adjugate(X, Ad)));
-#pragma unroll
-                for (int i = 0; i < 9; ++i) AA[i] = (Real)Ad[i];
+                qa = p2_geometry<Real>(X, A.scale, AA);
                 const double XB[4][3] = {{X[4][0], X[4][1], X[4][2]}, {X[1][0], X[1][1], X[1][2]},
                                          {X[3][0], X[3][1], X[3][2]}, {X[2][0], X[2][1], X[2][2]}};
-                qb = (Real)(-A.scale / (30.0 * p2_adjugate(XB, Ad)));
-#pragma unroll
-                for (int i = 0; i < 9; ++i) AB[i] = (Real)Ad[i];
+                qb = p2_geometry<Real>(XB, A.scale, AB);
             }
             p2_pair_strains<sizeof(Real) == 8, Real>([&](int c, int j) { return sU[3 * n[j] + c]; }, AA, AB, SA, SB);
             p2_vertex_stresses<Real>(qa, cur.mat[0], cur.mat[1], SA);

@@ -213,17 +213,13 @@ int emulate_pairs(const plx::MeshView &mv, const double *coords, const plx::Host
                 m[2 * k] = lam_mu[2 * (size_t)cell];
                 m[2 * k + 1] = lam_mu[2 * (size_t)cell + 1];
             }
-            double Ad[9];
             Real AA[9], AB[9], SA[4][6], SB[4][6];
-            const double da = plx::p2_adjugate(X, Ad);
-            for (int k = 0; k < 9; ++k) AA[k] = (Real)Ad[k];
             const double XB[4][3] = {{X[4][0], X[4][1], X[4][2]}, {X[1][0], X[1][1], X[1][2]},
                                      {X[3][0], X[3][1], X[3][2]}, {X[2][0], X[2][1], X[2][2]}};
-            const double db = plx::p2_adjugate(XB, Ad);
-            for (int k = 0; k < 9; ++k) AB[k] = (Real)Ad[k];
+            const double qa = plx::p2_geometry<Real>(X, 1.0, AA), qb = plx::p2_geometry<Real>(XB, 1.0, AB);
             plx::p2_pair_strains<false, Real>([&](int c, int j) { return sU[3 * n[j] + c]; }, AA, AB, SA, SB);
-            plx::p2_vertex_stresses<Real>((Real)(-1.0 / (30.0 * da)), (Real)m[0], (Real)m[1], SA);
-            plx::p2_vertex_stresses<Real>((Real)(-1.0 / (30.0 * db)), (Real)m[2], (Real)m[3], SB);
+            plx::p2_vertex_stresses<Real>(qa, (Real)m[0], (Real)m[1], SA);
+            plx::p2_vertex_stresses<Real>(qb, (Real)m[2], (Real)m[3], SB);
             plx::p2_pair_contract<false, Real>(SA, SB, AA, AB,
                                                [&](int c, int j, Real v) { sR[3 * n[j] + c] += (double)v; });
         }

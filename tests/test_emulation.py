@@ -152,6 +152,19 @@ def test_emulated_pair_kernel_with_nodes_split_on_a_plane(split):
         assert relerr(emulate(m, aux, u, algo=algo), ref) <= 1e-13
 
 
+@pytest.mark.parametrize("algo", [L.ALGO_FACTORED, EMULATE_PAIRS])
+@pytest.mark.parametrize("h", [1e-14, 1e-11, 1e-8, 1.0, 1e6, 1e9])
+def test_emulated_fp32_p2_element_over_lengths(algo, h):
+    """FP32 with moduli of rock and cells of any length: the products stay inside FP32's range while
+    mu det J does (1e10 h^3 from 1e-32 to 1e37 here)."""
+    m = mg.tet_p2_box((4, 3, 2), (0, 0, 0), (4 * h, 3 * h, 2 * h))
+    aux, _ = mg.elastic_aux(m.num_cells, seed=5, vs_sigma=0.2, vp_vs=1.8)
+    u = 1e3 * h * mg.random_field(m.num_nodes, 3)
+    ref = emulate(m, aux, u)
+    r32 = emulate(m, aux, u, scalar=L.FP32, algo=algo)
+    assert relerr(r32.astype(np.float64), ref) <= 2e-5
+
+
 EMULATE_GATHER = 101  # PLX_EMULATE_GATHER
 
 
