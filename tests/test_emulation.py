@@ -177,6 +177,8 @@ def gather_cases():
         "tet_label": (big, 1),  # nodes of the mesh outside the key
         "hex_max": (mg.hex_box(38, (0, 0, 0), (1.0, 1.0, 1.0)), 0),  # about the largest that fits 512 tiles
         "tet_large": (mg.tet_p2_box(16, (0, 0, 0), (1.0, 1.0, 1.0)), 0),
+        # (on a random mesh det J carries a few eps / 0.02: see the pair kernel's)
+        "delaunay_jitter": (delaunay_p2(1000, 4, jitter=0.3, min_quality=0.1), 0),
         **cases(),
     }
 

@@ -262,10 +262,12 @@ def test_second_plans_only_for_keys_that_use_them(oracle, cell):
 
 # either side of the line where a key takes the gather plan (38^3 hexes and 6 x 16^3 tets are about the
 # largest), non-affine hexes, and a mesh of affine and other hex tiles
-@pytest.mark.parametrize("kind", ["hex38", "hex41", "hex_warped", "hex_mixed", "tet16", "tet18"])
+@pytest.mark.parametrize("kind", ["hex38", "hex41", "hex_warped", "hex_mixed", "tet16", "tet18", "delaunay"])
 def test_gather_plan(oracle, kind):
     n = int(kind[3:]) if kind[3:].isdigit() else 14
-    if kind.startswith("tet"):
+    if kind == "delaunay":  # every cell in some three tiles
+        n, m = 0, delaunay_p2(4000, 1)
+    elif kind.startswith("tet"):
         m = mg.tet_p2_box(n, (0, 0, 0), (100.0 * n,) * 3)
     else:
         m = mg.hex_box(n, (0, 0, 0), (100.0 * n,) * 3)
@@ -277,6 +279,7 @@ def test_gather_plan(oracle, kind):
     aux, sizes = mg.elastic_aux(m.num_cells, seed=6, vs_sigma=0.2, vp_vs=1.8)
     u = mg.random_field(m.num_nodes, 9)
     dm, ref = check_residual(oracle, m, u, aux=(aux, sizes))
+    assert (second_plans(dm)[1] > 0) == (kind in ("hex38", "tet16", "delaunay"))
     dm.set_kernel_options()
     for dt, tol in ((torch.float64, TOL64), (torch.float32, TOL32)):
         x = dev(u, dt)
