@@ -177,7 +177,7 @@ struct Shape<PLX_HEX_Q1, Real> {
 // P2: 4-wave workgroups over the 384-cell tile (cells 0-255 on the first pass, 256-383 on the
 // second), two workgroups per CU at the FP64 kernel's register count (2 waves per SIMD).  One cell
 // per thread in 6-wave workgroups measured slower (63 x 66 x 61 x 6 cells, FP64: 92 us, 96 us with
-// the registers cut to three waves per SIMD, against 80 us).
+// the registers cut to three waves per SIMD, against 80 us on the same build; 76 us now).
 // record: 10 x uint16 closure, 4 x uint16 cone, 2 padding = 2 uint4 words
 template <typename Real>
 struct Shape<PLX_TET_P2, Real> {
@@ -453,11 +453,11 @@ __global__ void __launch_bounds__((Shape<CT, Real>::NT), MINW) apply_tiles(Apply
 // P2 pair kernel: the factored residual / action with LDS atomics, one pair of face-sharing cells per
 // thread (PairPlan).  A pair reads 14 nodes and 5 vertices from LDS and adds to 14 nodes where two
 // cells take 20, 8 and 20, its record is 24 bytes where theirs are 64, and 512-cell tiles leave fewer
-// shared nodes.  63 x 66 x 61 x 6 cells: 74 us against 84 us for the tile kernel (FP32, 40 x 44 x 37 x 6:
-// 17 us against 19 us).
-// The tile kernel above was bound on chip (63 x 66 x 61 x 6 cells: 80 us, 68 us with every gather
-// served from L2, 57 us without its atomics, 42 us without the element): LDS accesses are what
-// pairing cuts.  Same pipeline, with everything but the next tile's ids after the cells: two cells at
+// shared nodes.  63 x 66 x 61 x 6 cells, profiler: 73.6 us and 19.5 us for the halo sums against 75.9 and 21.2 us for
+// the tile kernel (FP32, 40 x 44 x 37 x 6: 17.8 against 19.2 us).
+// The tile kernel above is bound on chip (63 x 66 x 61 x 6 cells, before its extents were fetched two tiles ahead and
+// its loads made unconditional: 80 us, 68 us with every gather served from L2, 57 us without its atomics,
+// 42 us without the element): LDS accesses are what pairing cuts.  Same pipeline, with everything but the next tile's ids after the cells: two cells at
 // once leave no registers for it (between the two halves of the element: 79 us against 74).
 // --------------------------------------------------------------------------------------------
 struct PairArgs {
@@ -808,7 +808,7 @@ bool takes_pairs(plx_dm dm, const KeyPlan *kp) {
            dm->accumulate != PLX_ACCUMULATE_COLORED && dm->min_waves <= 2;
 }
 
-// (build_plan makes a gather plan only where it is the faster one)
+// (a gather plan is made only where it is the faster one: make_second_plans)
 bool takes_gather(plx_dm dm, const KeyPlan *kp) {
     return kp->gather.num_tiles > 0 && kp->gather.d_mat64 && dm->algorithm != PLX_ALGO_QUADRATURE_POINTS &&
            dm->accumulate != PLX_ACCUMULATE_COLORED;

@@ -115,8 +115,9 @@ static int upload_heads(plx_dm dm, int32_t **d, const std::vector<TileHead> &h) 
 }
 
 // Keys with fewer cells keep the tile kernel alone: two cells one after another per thread leave too few
-// waves there.  FP64 / FP32 apply, pairs against tiles: 48,000 cells 10.2 / 9.4 against 9.5 / 9.0 us, 83,000
-// 11.6 / 9.9 against 12.1 / 10.7 us, 196,000 17.2 / 14.5 against 20.9 / 17.5 us.
+// waves there.  FP64 / FP32 apply, pairs against tiles: 34,900 cells 9.9 / 9.3 against 8.9 / 8.2 us, 48,000 10.2 / 9.5
+// against 9.0 / 8.3, 63,800 10.5 / 9.7 against 11.1 / 10.3, 82,800 11.9 / 9.9 against 11.7 / 10.6, 215,000 17.1 / 14.2
+// against 21.1 / 17.2, 391,000 26.9 / 20.9 against 28.0 / 22.6; Delaunay 45,500 11.6 / 9.8 against 11.5 / 9.6.
 constexpr int64_t kPairMinCells = 65536;
 // So do keys whose pair tiles hold fewer cells on average (scattered cells: many without a partner, few to a
 // tile's nodes).  FP64, pairs against tiles, at so many cells a pair tile: Delaunay 393 12.5 against 13.9 us,

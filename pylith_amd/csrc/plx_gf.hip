@@ -203,7 +203,7 @@ __device__ __forceinline__ void col_reduce(double *s, int k) {
     __syncthreads();
 }
 
-// partials[b][r] = sum over this block's (dof, r) of a*b
+// partials[r][b] = sum over block b's (dof, r) of a*b (rows of kGfRed)
 template <typename Real>
 __global__ void __launch_bounds__(256) gf_dot(int64_t ndof, int k, const Real *__restrict__ a,
                                               const Real *__restrict__ b, double *partials) {

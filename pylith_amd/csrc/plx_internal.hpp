@@ -25,7 +25,6 @@ namespace plx {
 
 constexpr int kMaxQuad = 14;
 
-// Device-side arrays of one key's tile plan (passed by value to kernels).
 // Extents of one tile for the tile kernels: cells (or pairs) c0 .. c0 + nc (the colour count in nc's
 // upper half), its nn nodes from n0 (nown owned ones first) and nvt vertices from v0 in the tile
 // lists, first halo slot hoff.
@@ -33,6 +32,7 @@ struct TileHead {
     int32_t c0, nc, n0, nn, v0, nvt, nown, hoff;
 };
 
+// Device-side arrays of one key's tile plan (passed by value to kernels).
 struct TilePlanDev {
     int num_tiles;
     int stride;                      // SoA stride of per-cell arrays (= number of key cells)
