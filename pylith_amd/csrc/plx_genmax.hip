@@ -120,10 +120,16 @@ __global__ void __launch_bounds__(256) genmax_prestress_kernel(GmArgs A) {
 // another on one XCD, so that the cells' indices, moduli and nodes come from its L2 for seven of them, and the
 // state is read before the first store.  STREAM: the state passes by the caches; for keys whose state and
 // state stress exceed half of the 256 MB Infinity Cache, which the solve between two updates fills with its
-// own.  Update and residual, out of the cache, 48 x 45 x 43 cells (178 MB): 118 -> 108 us, streamed 104; 60^3:
-// 236, streamed 228 (191 at once again, 233 not streamed); 32^3 (63 MB): 38, streamed 42.
+// own.  Three waves per SIMD in both forms: at four (128 VGPRs) the reads no longer all go out together.
+// Update, residual and W MB of other traffic in a loop (a solve's place; its stores drain there), without streaming /
+// streamed / streamed at four waves per SIMD / one block per chunk and point, no streaming:
+//   48^3 (202 MB)  W 0: 93 / 99 / 107 / 109 us   W 128: 140 / 121 / 128 / 163   W 512: 217 / 211 / 226 / 241
+//   60^3 (396 MB)  W 0: 210 / 179 / 190 / 243    W 128: 238 / 223 / 242 / 271   W 512: 313 / 300 / 324 / 346
+//   32^3 (60 MB)   W 0: 35 / 42 / 42 / 39        W 128: 51 / 59 / 58 / 54       W 512: 146 / 144 / 146 / 152
+// The kernel by itself does not wait for stores that the caches took: in a time step with a point-block
+// Jacobi solve on 48^3, whose vectors leave most of the state there, 66 / 85 / 92 / 79 us.
 template <bool STREAM>
-__global__ void __launch_bounds__(256, STREAM ? 4 : 3) genmax_update_kernel(GmArgs A, const double *__restrict__ u) {
+__global__ void __launch_bounds__(256, 3) genmax_update_kernel(GmArgs A, const double *__restrict__ u) {
     const int j = blockIdx.x >> 3, q = j & 7;
     const int pos = ((j >> 3) * 8 + (blockIdx.x & 7)) * 256 + threadIdx.x;
     if (pos >= A.n) return;
