@@ -29,7 +29,7 @@
 
 namespace plx {
 
-constexpr int kRedBlocks = 512;
+constexpr int kRedBlocks = 512, kDotBlocks = 2048;
 enum { S_RZ = 0, S_PQ, S_ALPHA, S_BETA, S_RR, S_RZOLD, S_COUNT };
 
 template <typename Real>
@@ -219,7 +219,7 @@ __global__ void __launch_bounds__(256) finish_start(const double *__restrict__ p
 // where it took eight (eleven): at a few 10,000 dofs each kernel is launch and latency, about 3 us
 // whatever it does.  The apply leaves the shared nodes' partial sums; node_finish adds them, masks and
 // takes the dot product in one pass over the nodes; the reductions' last step, a sum of at most
-// kRedBlocks partials, is done by every block of the kernel that needs it instead of by a kernel of
+// kDotBlocks partials, is done by every block of the kernel that needs it instead of by a kernel of
 // its own.  24 x 22 x 25 hexes, FP32 point-block Jacobi: 26 -> 21 us an iteration; multigrid CG on
 // 22 x 24 x 21 x 6 tets: 5.8 -> 5.0 ms a solve.
 // --------------------------------------------------------------------------------------------
@@ -257,9 +257,10 @@ __global__ void __launch_bounds__(256) node_finish(int nnodes, const int2 *__res
             if ((fx >> c) & 1) q[c] = Real(0);
         if (MODE == kFinishDot) {
 #pragma unroll
-            for (int c = 0; c < 3; ++c) {
-                y[o + c] = q[c];
-                acc += (double)x[o + c] * (double)q[c];
+            for (int c = 0; c < 3; ++c) acc += (double)x[o + c] * (double)q[c];
+            if (r.x < r.y || fx) {  // (else y holds q)
+#pragma unroll
+                for (int c = 0; c < 3; ++c) y[o + c] = q[c];
             }
         } else {
             Real rv[3];
@@ -566,6 +567,11 @@ static int ensure_finish(plx_solver s) {
 // step, repeated by every block, stays short on small meshes).
 static int node_blocks(const plx_solver_s *s) { return std::max(1, std::min(kRedBlocks, (s->nnodes + 255) / 256)); }
 
+// Blocks (and partials) of node_finish with the dot product: its chains of dependent loads (range, slot, halo) want
+// more waves than the vector steps.  2.1 million nodes, FP64: 90.8 us in 512 blocks, 43.7 in 2048; an iteration on
+// 64^3 x 6 tets 286 -> 241 us, 128^3 hexes 291 -> 245, 40^3 x 6 72.6 -> 66.8 (4096 blocks 243, 245, 67.2).
+static int dot_blocks(const plx_solver_s *s) { return std::max(1, std::min(kDotBlocks, (s->nnodes + 255) / 256)); }
+
 // t = A x (tile kernel), then node_finish over it.
 template <typename Real, int MODE>
 static int apply_finish(plx_solver s, const Real *x, Real *t, const Real *b, const Real *Dinv, Real sc, Real *out,
@@ -575,7 +581,7 @@ static int apply_finish(plx_solver s, const Real *x, Real *t, const Real *b, con
     if (!s->range || !s->fixed) return set_error(dm, 1, "solver: work vectors not set up");
     if (int err = launch_apply(dm, s->keys[0], st, true, x, t, PLX_INSERT_VALUES, -1.0, nullptr, true, false)) return err;
     // a sum over the whole mesh needs its partials bounded; the others take a thread per node
-    const int blocks = MODE == kFinishDot ? node_blocks(s) : std::max(1, (s->nnodes + 255) / 256);
+    const int blocks = MODE == kFinishDot ? dot_blocks(s) : std::max(1, (s->nnodes + 255) / 256);
     hipLaunchKernelGGL((node_finish<Real, MODE>), dim3(blocks), dim3(256), 0, dm->stream, s->nnodes, s->range,
                        s->sums.slot, static_cast<const Real *>(s->sums.halo), s->fixed, t, x, b, Dinv, sc, out, part);
     PLX_HIP(dm, hipGetLastError());
@@ -737,7 +743,7 @@ static int pcg_amg(plx_solver s, Real *x, Real *r, Real *p, Real *q, Real *z, do
             float *r32 = std::is_same<Real, float>::value ? (float *)r : s->r32;
             float *z32 = std::is_same<Real, float>::value ? (float *)z : s->z32;
             hipLaunchKernelGGL(cg_step_xr<Real>, dim3(nblk), dim3(256), 0, dm->stream, s->n, x, r, p, q, r32, s->part_c,
-                               nblk, s->scal, s->part_b);
+                               dot_blocks(s), s->scal, s->part_b);
             if ((e = gf_vcycle1(s->amg, dm->stream, r32, z32))) return e;
             hipLaunchKernelGGL(rz_partials32<Real>, dim3(nblk), dim3(256), 0, dm->stream, s->n, r, z32, s->part_a);
             hipLaunchKernelGGL((p_step<Real, float>), dim3(nblk), dim3(256), 0, dm->stream, s->n, z32, p, s->part_a,
@@ -821,7 +827,7 @@ static int pcg(plx_solver s, Real *x, Real *r, Real *p, Real *q, Real *z, const 
             const int e = apply_finish<Real, kFinishDot>(s, p, q, nullptr, nullptr, Real(0), nullptr, s->part_c);
             if (e) return e;
             hipLaunchKernelGGL(cg_step<Real>, dim3(nblk), dim3(256), 0, dm->stream, s->nnodes, Binv, x, r, p, q, z,
-                               s->part_c, nblk, s->scal, s->part_a, s->part_b);
+                               s->part_c, dot_blocks(s), s->scal, s->part_a, s->part_b);
             hipLaunchKernelGGL((p_step<Real, Real>), dim3(nblk), dim3(256), 0, dm->stream, s->n, z, p, s->part_a,
                                s->part_b, nblk, s->scal);
             PLX_HIP(dm, hipGetLastError());
@@ -1042,7 +1048,7 @@ int plx_solver_create(plx_solver *out, plx_dm dm, int label_value, int part) {
               hipMalloc(&s->scal, 16 * sizeof(double)) == hipSuccess &&
               hipMalloc(&s->part_a, kRedBlocks * sizeof(double)) == hipSuccess &&
               hipMalloc(&s->part_b, kRedBlocks * sizeof(double)) == hipSuccess &&
-              hipMalloc(&s->part_c, kRedBlocks * sizeof(double)) == hipSuccess;
+              hipMalloc(&s->part_c, kDotBlocks * sizeof(double)) == hipSuccess;
     for (float **v : {&s->x32, &s->r32, &s->p32, &s->q32, &s->z32})
         ok = ok && hipMalloc(v, n * sizeof(float)) == hipSuccess;
     for (double **v : {&s->r64, &s->p64, &s->q64, &s->z64, &s->t64})

@@ -233,14 +233,16 @@ def test_two_materials_solve_matches_dense_direct(oracle, method, pc, kind):
     assert err <= 1e-9, err
 
 
-@pytest.mark.parametrize("kind", ["hex", "hex44", "tet", "tet_pairs"])
+# (hex52 and hex82: more partial sums of the dot product than of the others, and as many as there can be)
+@pytest.mark.parametrize("kind", ["hex", "hex44", "hex52", "hex82", "tet", "tet_pairs"])
 @pytest.mark.parametrize("maxit", [1, 13, 20])
 def test_iterates_agree_over_plans(kind, maxit):
     """The same number of CG iterations over the default plan (gather: two kernels an iteration, or tiles,
     or pairs: four), over the coloured tiles after a change of options on the same solver, and back.
     Rounding differs by some 1e-16 per operation, which 20 iterations amplify little: 1e-10."""
     if kind.startswith("hex"):
-        m = mg.hex_box((44, 41, 42) if kind == "hex44" else (9, 14, 11), (0, 0, 0), (6000.0, 6000.0, 6000.0))
+        n = {"hex": (9, 14, 11), "hex44": (44, 41, 42), "hex52": (52, 53, 51), "hex82": (82, 83, 81)}[kind]
+        m = mg.hex_box(n, (0, 0, 0), (6000.0, 6000.0, 6000.0))
     else:
         m = mg.tet_p2_box((27, 21, 22) if kind == "tet_pairs" else (5, 8, 6), (0, 0, 0), (6000.0, 6000.0, 6000.0))
     aux, sizes = mg.elastic_aux(m.num_cells, seed=4, vs_sigma=0.2, vp_vs=1.732)
