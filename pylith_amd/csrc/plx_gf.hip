@@ -1007,10 +1007,11 @@ static void gf_spmm_launch(plx_gf g, int k, const Real *val, const Real *X, Real
 }
 
 // q = A p and the per-column partials of p.q for the k-column block.  With fewer than kBatchWaves waves of
-// rows (eight per SIMD) the neighbours' loads go out in batches: 16^3 hexes x 16 columns 15.6 -> 11.3 us; a solve with
-// point-block Jacobi on 16^3 x 32 9.0 -> 7.0 ms, 26^3 x 8 12.6 -> 9.8 ms.  More waves hide the loads by
-// themselves: 30^3 x 16 29.2 ms either way, 36^3 x 32 79.5 ms in batches, 75.5 ms without.
-constexpr int64_t kBatchWaves = 8192;
+// rows (six per SIMD; the batched kernel's registers let seven reside, the other's eight) the neighbours' loads go
+// out in batches: 16^3 hexes x 16 columns 15.6 -> 11.3 us.  Solves with point-block Jacobi, serial / batched: 686 waves 5.57 /
+// 4.97 ms, 1267 7.35 / 6.71, 2745 7.60 / 7.22, 4218 12.3 / 11.3, 5071 12.0 / 11.5, 5285 21.3 / 20.8; 6517 24.7 / 25.0,
+// 6612 14.4 / 14.5, 7928 29.4 / 30.4, 8437 16.7 / 17.5; 36^3 x 32 (26,000) 75.5 / 79.5.
+constexpr int64_t kBatchWaves = 6144;
 template <int K>
 static void gf_spmm_dot_launch(plx_gf g) {
     if (K == 64)
