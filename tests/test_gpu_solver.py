@@ -8,6 +8,7 @@ torch = pytest.importorskip("torch")
 
 from pylith_amd import _lib as L  # noqa: E402
 from pylith_amd import meshgen as mg  # noqa: E402
+from general_meshes import delaunay_p2  # noqa: E402
 
 pytestmark = pytest.mark.gpu
 F1, JF3 = 1, 2
@@ -292,3 +293,36 @@ def test_preconditioner_changed_on_one_solver(kind, method):
         solver.set_preconditioner(pc)
         x = solve(dm, solver)
         assert np.abs(x - ref[pc]).max() <= 1e-8 * np.abs(ref[pc]).max(), pc
+
+
+# Delaunay meshes below (gather plan) and above (pair plan) the line of the pair kernel
+@pytest.mark.parametrize("npoints", [1500, 12500])
+@pytest.mark.parametrize("pc", ["pbjacobi", "amg"])
+def test_solve_on_a_general_mesh_agrees_over_plans(npoints, pc):
+    """CG to rtol 1e-10 over the default plan and over the coloured tiles: both solutions are within the
+    residual's reach of the exact one; 1e-6 of the largest displacement leaves the condition number 1e4."""
+    m = delaunay_p2(npoints, 1, min_quality=0.05)
+    # the largest connected part only: cells dropped for their shape leave others hanging
+    from scipy.sparse import coo_matrix
+    from scipy.sparse.csgraph import connected_components
+    e = np.stack([m.closure, np.roll(m.closure, 1, 1)], -1).reshape(-1, 2)
+    _, part = connected_components(coo_matrix((np.ones(len(e)), (e[:, 0], e[:, 1])), shape=(m.num_nodes,) * 2))
+    outside = np.flatnonzero(part != np.bincount(part).argmax())
+    aux, sizes = mg.elastic_aux(m.num_cells, seed=4, vs_sigma=0.2, vp_vs=1.732)
+    x0 = m.node_coords[:, 0]
+    held = np.union1d(np.flatnonzero((x0 < 0.1) | (x0 > 0.9)), outside)
+    dofs = (3 * held[:, None] + np.arange(3)).ravel().astype(np.int32)
+    vals = np.where((x0[held] > 0.9)[:, None] & (np.arange(3) == 1), 1.0, 0.0).ravel()
+    out = []
+    for acc in (L.ACCUMULATE_AUTO, L.ACCUMULATE_COLORED):
+        dm, solver = build(m, aux, sizes, dofs)
+        dm.set_kernel_options(L.ALGO_AUTO, acc)
+        solver.set_preconditioner(pc)
+        print(f"[solver-general] cells={m.num_cells} pc={pc} accumulate={acc}", flush=True)
+        x = torch.zeros(3 * m.num_nodes, dtype=torch.float64, device="cuda")
+        dm.insert_boundary_values(torch.from_numpy(vals).cuda(), x)
+        st = solver.solve(x, method=L.KSP_CG, rtol=1e-10, maxit=20000)
+        torch.cuda.synchronize()
+        assert st["converged"], st
+        out.append(x.cpu().numpy())
+    assert np.abs(out[0] - out[1]).max() <= 1e-6 * np.abs(out[1]).max()
