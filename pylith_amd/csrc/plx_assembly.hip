@@ -94,6 +94,7 @@ struct ApplyArgs {
     int num_list;
     const void *records;       // packed 16-bit local closure (+ cone) per key cell
     const double *prestress;   // Q1: per-point stress added to sigma, [6][8][stride] (nullptr: none)
+    P2Scale p2;
 };
 
 // Cell solution values read from the tile's LDS buffer (component c, local basis b).
@@ -392,7 +393,7 @@ __global__ void __launch_bounds__((Shape<CT, Real>::NT), MINW) apply_tiles(Apply
                     if constexpr (PATH == kPathFactored) {
                         const LdsAcc<Real, 10> acc{sU, {lc[0], lc[1], lc[2], lc[3], lc[4], lc[5], lc[6], lc[7], lc[8], lc[9]}};
                         // LDS atomics take an entry as soon as it is formed
-                        p2_element_linear<Real>(X, acc, lam, mu, [&](int c, int b, Real v) {
+                        p2_element_linear<Real>(X, acc, lam, mu, A.p2, [&](int c, int b, Real v) {
                             if constexpr (DIRECT) atomicAdd(&sR[3 * lc[b] + c], (Acc)v);
                             else re[c][b] = v;
                         });
@@ -469,7 +470,8 @@ struct PairArgs {
     const void *u;
     void *r, *halo;
     int mode;
-    double scale;
+    float area;    // P2Scale
+    double scale;  // with P2Scale's factor
 };
 
 constexpr int kPairThreads = 256, kPairSlots = kPairTileNodes / kPairThreads;
@@ -566,7 +568,7 @@ __global__ void __launch_bounds__(kPairThreads, 2) apply_pairs(PairArgs A) {
         if (tid < cur.np) {
             int n[14];
             Real AA[9], AB[9], SA[4][6], SB[4][6];
-            double qa, qb;
+            Real qa, qb;
             {
                 const unsigned w[6] = {cur.rec[0].x, cur.rec[0].y, cur.rec[1].x, cur.rec[1].y, cur.rec[2].x, cur.rec[2].y};
 #pragma unroll
@@ -580,10 +582,10 @@ __global__ void __launch_bounds__(kPairThreads, 2) apply_pairs(PairArgs A) {
 #pragma unroll
                     for (int d = 0; d < 3; ++d) X[v][d] = sX[3 * lv + d];
                 }
-                qa = p2_geometry<Real>(X, A.scale, AA);
+                qa = p2_geometry<Real>(X, A.scale, A.area, AA);
                 const double XB[4][3] = {{X[4][0], X[4][1], X[4][2]}, {X[1][0], X[1][1], X[1][2]},
                                          {X[3][0], X[3][1], X[3][2]}, {X[2][0], X[2][1], X[2][2]}};
-                qb = p2_geometry<Real>(XB, A.scale, AB);
+                qb = p2_geometry<Real>(XB, A.scale, A.area, AB);
             }
             p2_pair_strains<sizeof(Real) == 8, Real>([&](int c, int j) { return sU[3 * n[j] + c]; }, AA, AB, SA, SB);
             p2_vertex_stresses<Real>(qa, cur.mat[0], cur.mat[1], SA);
@@ -696,7 +698,7 @@ __global__ void __launch_bounds__((Shape<CT, Real>::NT), 2) cg_apply(ApplyArgs A
                 for (int d = 0; d < 3; ++d) X[v][d] = sX[3 * lv + d];
             }
             const LdsAcc<Real, 10> acc{sU, {lc[0], lc[1], lc[2], lc[3], lc[4], lc[5], lc[6], lc[7], lc[8], lc[9]}};
-            p2_element_linear<Real>(X, acc, lam, mu, [&](int c, int b, Real v) { atomicAdd(&sR[3 * lc[b] + c], (double)v); });
+            p2_element_linear<Real>(X, acc, lam, mu, A.p2, [&](int c, int b, Real v) { atomicAdd(&sR[3 * lc[b] + c], (double)v); });
         }
     }
     __syncthreads();
@@ -830,7 +832,8 @@ static int apply_pairs_typed(plx_dm dm, KeyPlan *kp, const void *u, void *r, int
     A.r = r;
     A.halo = halo ? halo : kp->d_halo;
     A.mode = mode;
-    A.scale = scale;
+    A.area = dm->p2_scale.area;
+    A.scale = std::is_same<Real, double>::value ? scale : scale * dm->p2_scale.factor;
     if (dm->num_cu <= 0) PLX_HIP(dm, hipDeviceGetAttribute(&dm->num_cu, hipDeviceAttributeMultiprocessorCount, 0));
     const size_t lds = pair_lds_bytes<Real>();
     const int per_cu = resident_per_cu(reinterpret_cast<const void *>(&apply_pairs<Real>), kPairThreads, lds, 2);
@@ -850,6 +853,7 @@ static int apply_typed(plx_dm dm, KeyPlan *kp, const void *u, void *r, int mode,
     if (!prestress && takes_pairs(dm, kp)) return apply_pairs_typed<Real>(dm, kp, u, r, mode, scale, halo, log, reduce);
     ApplyArgs A;
     A.scale = scale;
+    A.p2 = dm->p2_scale;
     A.prestress = prestress;
     A.p = plan_dev(dm, kp);
     A.color = kp->d_color;
@@ -968,6 +972,7 @@ static int cg_apply_typed(plx_dm dm, KeyPlan *kp, const void *u, void *r, double
     A.u = u;
     A.r = r;
     A.scale = scale;
+    A.p2 = dm->p2_scale;
     A.heads = G.d_heads;
     A.num_list = G.num_tiles;
     A.records = G.d_records;

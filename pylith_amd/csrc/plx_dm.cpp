@@ -643,6 +643,7 @@ int plx_dm_create(plx_dm *out, int cell_type, int num_cells, int num_vertices, i
             return 1;
         }
     dm->coords.assign(coords, coords + (size_t)num_vertices * 3);
+    if (cell_type == PLX_TET_P2) dm->p2_scale = p2_scale(coords, num_vertices, num_cells);
     if (labels)
         dm->labels.assign(labels, labels + num_cells);
     else

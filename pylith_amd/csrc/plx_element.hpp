@@ -4,6 +4,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include "plx_plan.hpp"
+
 namespace plx {
 
 constexpr int kP2Quad = 14;
@@ -674,24 +676,17 @@ __host__ __device__ inline double p2_adjugate(const double X[4][3], double A[9])
 }
 
 // A in Real and the scale of the stresses, times `factor`: the adjugate and -factor / (30 det).  In FP32 A is scaled by
-// a power of two to about 1 (and the scale, which stays in double, by its inverse square): strains would go with
-// the squared length and the scale with its inverse cube, and cells shorter than 5e-10 with moduli of 1e10
-// left the range.  No bit of the result depends on it elsewhere.
+// `area`, a power of two near the inverse of a typical cell's squared length (P2Scale; the factor then carries its
+// inverse square): else strains go with the squared length and the scale with its inverse cube, and cells
+// shorter than 5e-10 with moduli of 1e10 leave the range.  (From each cell's own det instead: the chain through
+// its exponent cost small applies 1 to 3 %.)
 template <typename Real>
-__host__ __device__ inline double p2_geometry(const double X[4][3], double factor, Real A[9]) {
+__host__ __device__ inline Real p2_geometry(const double X[4][3], double factor, float area, Real A[9]) {
     double Ad[9];
     const double det = p2_adjugate(X, Ad);
-    const double q = -factor / (30.0 * det);
-    if (sizeof(Real) == 8) {
 #pragma unroll
-        for (int i = 0; i < 9; ++i) A[i] = (Real)Ad[i];
-        return q;
-    }
-    const int e = 2 * (ilogb(det) / 3);  // 2^e: about the squared length
-    const Real s = (Real)ldexp(1.0, -e);
-#pragma unroll
-    for (int i = 0; i < 9; ++i) A[i] = (Real)Ad[i] * s;
-    return ldexp(q, 2 * e);
+    for (int i = 0; i < 9; ++i) A[i] = sizeof(Real) == 8 ? (Real)Ad[i] : (Real)Ad[i] * (Real)area;
+    return (Real)(-factor / (30.0 * det));
 }
 
 // Strains at the four vertices times det (as A is scaled; xx, yy, zz and twice xy, yz, xz), the part of solution
@@ -738,8 +733,8 @@ __host__ __device__ inline void p2_vertex_strains(const UAcc &U, const Real A[9]
 
 // Stresses of the linear kernels in place of the strains of p2_vertex_strains (isotropic, scaled by q).
 template <typename Real>
-__host__ __device__ inline void p2_vertex_stresses(double q, Real lam, Real mu, Real S[4][6]) {
-    const Real ql = (Real)(q * lam), qm = (Real)(q * mu), qm2 = Real(2) * qm;
+__host__ __device__ inline void p2_vertex_stresses(Real q, Real lam, Real mu, Real S[4][6]) {
+    const Real ql = q * lam, qm = q * mu, qm2 = Real(2) * qm;
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
         const Real ls = ql * (S[v][0] + S[v][1] + S[v][2]);
@@ -844,9 +839,9 @@ __host__ __device__ inline void p2_pair_contract(const Real SA[4][6], const Real
 // moments of the barycentric coordinates in place of the points.
 template <typename Real, typename UAcc, typename Emit>
 __host__ __device__ inline void p2_element_linear(const double X[4][3], const UAcc &U, Real lam, Real mu,
-                                                  const Emit &emit) {
+                                                  const P2Scale &ps, const Emit &emit) {
     Real A[9], S[4][6];
-    const double scale = p2_geometry<Real>(X, 1.0, A);
+    const Real scale = p2_geometry<Real>(X, sizeof(Real) == 8 ? 1.0 : ps.factor, ps.area, A);
     p2_vertex_strains<sizeof(Real) == 8, Real>(U, A, S);
     p2_vertex_stresses<Real>(scale, lam, mu, S);
     p2_sym_contract<sizeof(Real) == 8, Real>(S, A, emit);

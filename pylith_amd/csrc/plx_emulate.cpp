@@ -41,6 +41,7 @@ template <typename Real>
 int emulate(const plx::MeshView &mv, const double *coords, const plx::HostPlan &hp,
             const double *lam_mu, const Real *u, Real *r, int mode, int cell_type, bool linear, bool gather = false) {
     const int nb = mv.nb, nv = mv.nv;
+    const plx::P2Scale ps = plx::p2_scale(coords, mv.num_vertices, mv.num_cells);
     const int stride = (int)hp.cells.size();
     const plx::TileLimits lim = plx::tile_limits(cell_type);
     std::vector<Real> halo((size_t)hp.halo_slots * 3, Real(0));
@@ -120,7 +121,7 @@ int emulate(const plx::MeshView &mv, const double *coords, const plx::HostPlan &
                     for (int c = 0; c < 3; ++c) U[c][b] = sU[3 * lc[b] + c];
                 const auto emit = [&](int c, int b, Real v) { rl[c][b] = v; };
                 if (linear)
-                    plx::p2_element_linear<Real>(X, plx::ArrayAcc3<Real>{U}, lam, mu, emit);
+                    plx::p2_element_linear<Real>(X, plx::ArrayAcc3<Real>{U}, lam, mu, ps, emit);
                 else
                     plx::p2_element<Real, HostTab>(X, U, lam, mu, rl);
                 for (int b = 0; b < nb; ++b)
@@ -172,6 +173,7 @@ int emulate_pairs(const plx::MeshView &mv, const double *coords, const plx::Host
                   const double *lam_mu, const Real *u, Real *r, int mode) {
     std::vector<double> halo(3 * (size_t)pp.halo_slots);
     std::vector<int> seen(mv.num_cells, 0);
+    const plx::P2Scale ps = plx::p2_scale(coords, mv.num_vertices, mv.num_cells);
     CHECK(pp.halo_slots <= hp.halo_slots);
     CHECK((int)pp.tile_pair_ptr.size() == pp.num_tiles + 1 && pp.tile_pair_ptr.back() == pp.num_pairs);
     for (int slot = 0; slot < pp.num_tiles; ++slot) {
@@ -216,7 +218,8 @@ int emulate_pairs(const plx::MeshView &mv, const double *coords, const plx::Host
             Real AA[9], AB[9], SA[4][6], SB[4][6];
             const double XB[4][3] = {{X[4][0], X[4][1], X[4][2]}, {X[1][0], X[1][1], X[1][2]},
                                      {X[3][0], X[3][1], X[3][2]}, {X[2][0], X[2][1], X[2][2]}};
-            const double qa = plx::p2_geometry<Real>(X, 1.0, AA), qb = plx::p2_geometry<Real>(XB, 1.0, AB);
+            const double f = sizeof(Real) == 8 ? 1.0 : ps.factor;
+            const Real qa = plx::p2_geometry<Real>(X, f, ps.area, AA), qb = plx::p2_geometry<Real>(XB, f, ps.area, AB);
             plx::p2_pair_strains<false, Real>([&](int c, int j) { return sU[3 * n[j] + c]; }, AA, AB, SA, SB);
             plx::p2_vertex_stresses<Real>(qa, (Real)m[0], (Real)m[1], SA);
             plx::p2_vertex_stresses<Real>(qb, (Real)m[2], (Real)m[3], SB);

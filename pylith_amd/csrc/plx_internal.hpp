@@ -186,6 +186,7 @@ struct plx_dm_s {
     // the same order); applied to per-point aux on the way in and out
     std::vector<int32_t> quad_perm;
     std::vector<double> coords;
+    plx::P2Scale p2_scale;
     double *d_coords = nullptr;
     int32_t *d_closure = nullptr, *d_cone = nullptr;  // uploaded on first use (set-up kernels)
     hipStream_t stream = nullptr;

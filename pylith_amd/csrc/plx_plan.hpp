@@ -1,6 +1,8 @@
 // plx_plan.hpp -- host-side tile plan (see plx_plan.cpp).
 #pragma once
 
+#include <algorithm>
+#include <cmath>
 #include <cstdint>
 #include <string>
 #include <vector>
@@ -29,6 +31,26 @@ struct MeshView {
     bool cone_is_closure;   // isoparametric Q1: vertices are the nodes, in closure order
     const double *coords = nullptr;  // [num_vertices][3] (spatial reordering of badly ordered keys)
 };
+
+// Powers of two that keep the FP32 element of P2 tetrahedra in range (p2_geometry): area, near the inverse of a typical
+// cell's squared length, for the adjugate of J, and its inverse square for the scale of the stresses.
+struct P2Scale {
+    float area = 1.0f;
+    double factor = 1.0;
+};
+inline P2Scale p2_scale(const double *coords, int64_t num_vertices, int64_t num_cells) {
+    double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300}, size = 0.0;
+    for (int64_t i = 0; i < num_vertices; ++i)
+        for (int d = 0; d < 3; ++d) {
+            lo[d] = std::min(lo[d], coords[3 * i + d]);
+            hi[d] = std::max(hi[d], coords[3 * i + d]);
+        }
+    for (int d = 0; d < 3; ++d) size = std::max(size, hi[d] - lo[d]);
+    const double length = size / std::cbrt((double)num_cells);
+    if (!(length > 0.0) || !std::isfinite(length)) return P2Scale();
+    const int e = std::max(-120, std::min(120, 2 * std::ilogb(length)));
+    return {(float)std::ldexp(1.0, -e), std::ldexp(1.0, 2 * e)};
+}
 
 struct HostPlan {
     int num_tiles = 0;
